@@ -32,7 +32,7 @@ CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall"]
 
 HOST_SRCS = ["imx_mesh.cpp", "imx_trmesh.cpp", "imx_ic.cpp", "imx_sfc.cpp", "imx_gridio.cpp", "imx_plot.cpp", "imx_jacobian.cpp",
              "imx_lte.cpp"]
-HIP_SRCS = ["imx_swm.hip", "imx_mlp.hip", "imx_learn.hip"]
+HIP_SRCS = ["imx_swm.hip", "imx_stage.hip", "imx_mlp.hip", "imx_learn.hip"]
 # the Fortran host's modules, in dependency order
 FORTRAN_SRCS = ("datastruct.f90", "imx_c.f90", "swm_par.f90", "smeshpack.f90", "swm_data.f90", "swm.f90")
 

@@ -49,6 +49,8 @@ struct Alloc {
   }
 };
 
+struct Stage;  // tables of the one-launch-per-stage path (imx_stage.hip)
+
 }  // namespace imx
 
 struct imx_swm {
@@ -226,6 +228,11 @@ struct imx_swm {
   // XCD remap, chosen by imx_swm_tune
   int kbs[3] = {256, 256, 256};
   int kremap[3] = {1, 1, 1};
+  // one launch per stage for the plain scheme; nullptr where the numbering
+  // is not local. stg_stale: the tables no longer match the handle's
+  // staggering, triangle weights or Coriolis parameter.
+  imx::Stage *stg = nullptr;
+  bool stg_stale = false;
 };
 
 // MLP handle: FP32 master parameters with AdamW moments, BF16 fragment
@@ -251,4 +258,17 @@ int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int
 void swm_launch_step(imx_swm *s);
 // waits for the handle's stream; IMX_ESTATE if a step met a vanishing depth
 int swm_check_flag(imx_swm *s, const char *what);
+
+// One launch per RK stage (imx_stage.hip). stage_build makes the block
+// tables from the handle's device tables for blocks of nt threads and leaves
+// s->stg null where the numbering cuts into blocks that are mostly rim;
+// stage_launch evaluates stage 0..3 of (hs, us), or a tendency (stage -1).
+int stage_build(imx_swm *s, int nt);
+void stage_free(imx_swm *s);
+int stage_threads(const imx_swm *s);
+int stage_remap(const imx_swm *s);
+size_t stage_bytes(const imx_swm *s);
+void stage_set_remap(imx_swm *s, int remap);
+template <typename T>
+void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *uout);
 }  // namespace imx

@@ -1,0 +1,680 @@
+// libimx: one launch per RK stage for the plain scheme (trsk10, HTC or HC)
+// on the fused FP32/FP64 handles.
+//
+// The three passes of imx_swm.hip (fast_tri, fast_cell, fast_edge) hand q,
+// phi and the two Coriolis partials of every edge through memory and wait
+// for each other three times per stage. Here a block takes a stretch of the
+// Hilbert-ordered cells and evaluates the whole stage for the edges and
+// cells it owns out of LDS:
+//   local cells   own cells, then the far ends of their owned edges (C: all
+//                 cells whose Bernoulli potential and Coriolis partials the
+//                 own edges need), then the rest of the rings of C (L)
+//   P0  u, u l and the dual length of every edge owned by a local cell, and
+//       h of every local cell, to LDS
+//   P1  PV of every triangle around a cell of C
+//   P2  fast_cell's work for every cell of C; RK update of h on own cells
+//   P3  fast_edge's work and the RK update of u on own edges
+// Nothing but the new state and the accumulators is written. Cells and
+// triangles on the rim are evaluated by every block that needs them (1.2 to
+// 1.4 times the work of the mesh), with the same expressions on the same
+// inputs, so a result does not depend on how the mesh is cut into blocks.
+//
+// Measured (us per RK4 step, three passes -> this): glevel 5 FP32 43 -> 32,
+// glevel 7 78 -> 58, FP64 105 -> 85, glevel 8 191 -> 127, FP64 380 -> 241,
+// glevel 9 948 -> 590. The three passes moved 385 B per cell and stage, 252
+// MB at glevel 8; this moves about 245. What was worth most is the order of
+// the loads: with each phase loading its own tables a block waited five
+// memory latencies in a row and a glevel-8 stage took 45 us; with every load
+// issued before the first barrier it takes 32.
+//
+// Blocks are cut greedily along the curve so that |C| fills the block's
+// threads and |L| its LDS. Ids inside a block are 10-bit, which packs the
+// topology of a cell into 16 bytes; lengths are stored once per edge and the
+// kinetic-energy and vorticity coefficients are formed from them.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "imx_device.h"
+
+#define MX IMX_MAXNB
+#define NXCD 8
+#define HTR_GUARD (1.1920928955078125e-07 / 100000.0)
+// local ids are 10-bit
+#define LID 1023
+// topology word of a cell slot: neighbour | OWN (the cell owns the edge) |
+// K (which of its owner's edges, 2 bits) | signs of the flux and of the
+// Coriolis term
+#define SB_OWN 10
+#define SB_K 11
+#define SB_TTG 13
+#define SB_TNR 14
+// fourth topology word: owner of triangle j (0 cell, 1 nb_j, 2 nb_j+1; 2
+// bits at 2j), k of triangle j (bit 12+j), hexagon (bit 18)
+#define SW_KT 12
+#define SW_HEX 18
+
+// bits of the handle's cell words (imx_swm.hip)
+#define BA_TTG 3
+#define BA_TNR 9
+#define BA_OWN 15
+#define BB_TSEL 12
+#define BB_KT 24
+#define OTH_MASK 0x3FFFFFFF
+#define OTH_V2 30
+
+namespace imx {
+
+template <typename T>
+struct alignas(2 * sizeof(T)) Pair {
+  T x, y;
+};
+template <typename T>
+struct alignas(4 * sizeof(T)) Quad {
+  T x, y, z, w;
+};
+
+// caps of a block of nt threads: cells of C, local cells, triangles
+static constexpr int cap_l(int nt) { return nt + nt / 2 + 64; }
+static constexpr int cap_t(int nt) { return 2 * nt + nt / 2 + 64; }
+
+struct Stage {
+  int nt = 0, nblk = 0, remap = 1;
+  Alloc A;
+  int4 *head = nullptr;      // [nblk] first own cell, own cells, |C|, |L| | triangles << 16
+  int32_t *halo = nullptr;   // [nblk][cap_l] cells of the local ids past the own ones
+  uint4 *topo = nullptr;     // [nblk][nt]
+  void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~
+  void *eld = nullptr;       // [NE] Pair: length, dual length
+  uint16_t *oth = nullptr;   // [NE] local id of the edge's other cell | it is v1 << 10; 0xFFFF dummy
+  uint32_t *tv = nullptr;    // [nblk][cap_t] vertices a, b (10 bits each), edge bits (9), curl signs (3)
+  uint16_t *tslot = nullptr; // [nblk][cap_t] local slot 2 owner + k
+  void *tk = nullptr;        // [nblk][cap_t] Quad: kite weights, 1 / (A_t a)
+  void *tf = nullptr;        // [nblk][cap_t] Coriolis parameter
+};
+
+template <typename T>
+struct StageArgs {
+  const int4 *head;
+  const int32_t *halo;
+  const uint4 *topo;
+  const Quad<T> *cw;
+  const Pair<T> *eld;
+  const uint16_t *oth;
+  const uint32_t *tv;
+  const uint16_t *tslot;
+  const Quad<T> *tk;
+  const T *tf;
+  const double *iaa;
+  const T *hs, *us, *h0, *u0, *gb, *dte;
+  const double *dtc;
+  T *hout, *uout, *acch, *accu, *q, *du_out;
+  double *dh_out;
+  int *flag;
+  double href, dt;
+  T grav, inv_a;
+  int nblk, remap, use_pv, flin, zero_mom;
+  int whole;  // the third stage: its state is a whole step away
+};
+
+__device__ __forceinline__ void kadd(double &s, double &c, double x) {
+  const double t = s + x;
+  if (fabs(s) >= fabs(x)) c += (s - t) + x;
+  else c += (x - t) + s;
+  s = t;
+}
+
+// MODE: 0 the first RK stage, 1 the second and third, 2 the last, 3 a
+// tendency.
+template <typename T, int NT, int MODE>
+__global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
+  constexpr int LC = cap_l(NT), TC = cap_t(NT);
+  constexpr int NH = (LC + NT - 1) / NT, NR = (TC + NT - 1) / NT;
+  __shared__ Pair<T> sU[3 * LC];  // u, dual length
+  __shared__ T sA[3 * LC];        // u l
+  __shared__ T sH[LC], sQ[2 * LC], sPhi[NT], sP[3 * NT], sPo[3 * NT];
+  int b = blockIdx.x;
+  if (a.remap) b = (b % NXCD) * (gridDim.x / NXCD) + b / NXCD;
+  if (b >= a.nblk) return;
+  const int tid = threadIdx.x;
+  // Every load of the stage is issued before the first barrier, in two
+  // generations: the block's tables, which need nothing, and the state,
+  // whose places the first ones give; the phases then run out of registers
+  // and LDS. Lanes past a list read its last entry instead of branching
+  // around the load.
+  const int32_t *halo = a.halo + (size_t)b * LC;
+  int hcell[NH];
+#pragma unroll
+  for (int r = 0; r < NH; ++r) hcell[r] = halo[min(tid + r * NT, LC - 1)];
+  const uint4 tp = a.topo[(size_t)b * NT + tid];
+  const Quad<T> w0 = a.cw[((size_t)b * 2) * NT + tid], w1 = a.cw[((size_t)b * 2 + 1) * NT + tid];
+  const int4 hd = a.head[b];
+  const int own0 = hd.x, nown = hd.y, nC = hd.z, nL = hd.w & 0xFFFF, nTri = hd.w >> 16;
+  const int nh = nL - nown;
+  const T href = (T)a.href;
+  const int oc = own0 + min(tid, nown - 1);
+
+  T hh[NH], hu[NH][3];
+  Pair<T> hl[NH][3];
+#pragma unroll
+  for (int r = 0; r < NH; ++r) {
+    hh[r] = a.hs[hcell[r]];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      hu[r][k] = a.us[3 * hcell[r] + k];
+      hl[r][k] = a.eld[3 * hcell[r] + k];
+    }
+  }
+  const T ho = a.hs[oc];
+  T eu[3];
+  Pair<T> el[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int e = 3 * own0 + min(tid + r * NT, 3 * nown - 1);
+    eu[r] = a.us[e];
+    el[r] = a.eld[e];
+  }
+  uint32_t tv[NR];
+  int tsl[NR];
+  Quad<T> tk[NR];
+  T tf[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const size_t t = (size_t)b * TC + min(tid + r * NT, nTri - 1);
+    tv[r] = a.tv[t];
+    tsl[r] = a.tslot[t];
+    tk[r] = a.tk[t];
+    tf[r] = a.tf[t];
+  }
+  // the RK operands of the own cells and edges
+  const double iaa = a.iaa[oc];
+  T y0 = (T)0, ac = (T)0, v0[3], av[3];
+  uint32_t ow[3];
+  if (MODE != 3) y0 = a.h0[oc];
+  if (MODE == 1 || MODE == 2) ac = a.acch[oc];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int e = 3 * own0 + min(tid + r * NT, 3 * nown - 1);
+    ow[r] = a.oth[e];
+    if (MODE != 3) v0[r] = a.u0[e];
+    if (MODE == 1 || MODE == 2) av[r] = a.accu[e];
+  }
+
+  // P0: the local state to LDS
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    // used here, so the load is not moved into the branch below
+    asm volatile("" : "+v"(eu[r]), "+v"(el[r].x), "+v"(el[r].y));
+    const int i = tid + r * NT;
+    if (i < 3 * nown) {
+      sU[i] = Pair<T>{eu[r], el[r].y};
+      sA[i] = eu[r] * el[r].x;
+    }
+  }
+  if (tid < nown) sH[tid] = ho;
+#pragma unroll
+  for (int r = 0; r < NH; ++r)
+    if (tid + r * NT < nh) {
+      const int lc = nown + tid + r * NT;
+      sH[lc] = hh[r];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        sU[3 * lc + k] = Pair<T>{hu[r][k], hl[r][k].y};
+        sA[3 * lc + k] = hu[r][k] * hl[r][k].x;
+      }
+    }
+  __syncthreads();
+
+  // P1: PV at triangles
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (tid + r * NT >= nTri) continue;
+    const uint32_t v = tv[r];
+    const int sl = tsl[r];
+    const Quad<T> k = tk[r];
+    T eta = tf[r];
+    const int o = sl >> 1, va = v & LID, vb = (v >> 10) & LID;
+    const int eb = v >> 20;
+    const int e0 = 3 * ((eb & 1) ? o : va) + ((eb >> 1) & 3);
+    const int e1 = 3 * (((eb >> 3) & 1) ? va : vb) + ((eb >> 4) & 3);
+    const int e2 = 3 * (((eb >> 6) & 1) ? vb : o) + ((eb >> 7) & 3);
+    if (!a.flin) {
+      const T c0 = sA[e0], c1 = sA[e1], c2 = sA[e2];
+      T z = (eb >> 9) & 1 ? -c0 : c0;
+      z += (eb >> 10) & 1 ? -c1 : c1;
+      z += (eb >> 11) & 1 ? -c2 : c2;
+      eta += z * k.w;
+    }
+    T hsum = k.x * sH[o];
+    hsum += k.y * sH[va];
+    hsum += k.z * sH[vb];
+    const T ht = href + hsum;
+    T qq = (T)0;
+    if (a.use_pv) {
+      if (fabs((double)ht) < HTR_GUARD) a.flag[0] = 1;
+      else qq = eta / ht;
+    }
+    sQ[sl] = qq;
+    // the field a caller may read: the last stage's, or a tendency's
+    if (MODE >= 2 && o < nown) a.q[2 * own0 + sl] = qq;
+  }
+  __syncthreads();
+
+  // P2: cells
+  if (tid < nC) {
+    const uint32_t wj[3] = {tp.x, tp.y, tp.z};
+    const bool hex = (tp.w >> SW_HEX) & 1;
+    int nb[MX], ed[MX];
+    uint32_t f[MX];
+#pragma unroll
+    for (int j = 0; j < MX; ++j) {
+      f[j] = wj[j / 2] >> (16 * (j % 2));
+      nb[j] = f[j] & LID;
+      ed[j] = 3 * (((f[j] >> SB_OWN) & 1) ? tid : nb[j]) + ((f[j] >> SB_K) & 3);
+    }
+    const T hc = sH[tid];
+    double dv = 0.0, dvc = 0.0;
+    T ke = (T)0;
+    T G[MX];
+#pragma unroll
+    for (int j = 0; j < MX; ++j) {
+      const bool valid = (j < MX - 1) || hex;
+      const Pair<T> u = sU[ed[j]];
+      // both cells of an edge form the same product, so the mass flux
+      // cancels exactly between them
+      double g = (double)u.x * (a.href + 0.5 * ((double)hc + (double)sH[nb[j]])) * (double)u.y;
+      if ((f[j] >> SB_TTG) & 1) g = -g;
+      if (!valid) g = 0.0;
+      kadd(dv, dvc, g);
+      G[j] = (T)g;
+      ke += valid ? sA[ed[j]] * (u.x * u.y) : (T)0;
+    }
+    T qt[MX];
+#pragma unroll
+    for (int j = 0; j < MX; ++j) {
+      const int ts = (tp.w >> (2 * j)) & 3;
+      const int to = (ts == 0) ? tid : (ts == 1) ? nb[j] : nb[(j + 1) % MX];
+      qt[j] = sQ[2 * to + ((tp.w >> (SW_KT + j)) & 1)];
+    }
+    // a pentagon's padded slot may name a triangle that is not local
+    if (!hex) qt[MX - 1] = (T)0;
+    T pot = a.grav * hc;
+    if (a.gb) pot += a.gb[tid < nown ? own0 + tid : halo[tid - nown]];
+    sPhi[tid] = (pot + ke * w1.z) * a.inv_a;
+    if (tid < nown) {
+      const int c = own0 + tid;
+      const double dh = -(dv + dvc) * iaa;
+      const double dt = a.dtc ? a.dtc[c] : a.dt;
+      if (MODE == 3) {
+        a.dh_out[c] = dh;
+      } else if (MODE < 2) {
+        const double ca = a.whole ? dt : 0.5 * dt;
+        const double cb = MODE == 0 ? dt / 6.0 : dt / 3.0;
+        a.hout[c] = (T)((double)y0 + ca * dh);
+        a.acch[c] = MODE == 0 ? (T)(cb * dh) : (T)((double)ac + cb * dh);
+      } else {
+        a.hout[c] = (T)((double)y0 + ((double)ac + (dt / 6.0) * dh));
+      }
+    }
+    // PV at the cell's edges: edge j lies between ring triangles j-1 and j
+    T qe[MX];
+    qe[0] = (T)0.5 * ((hex ? qt[MX - 1] : qt[MX - 2]) + qt[0]);
+#pragma unroll
+    for (int j = 1; j < MX; ++j) qe[j] = (T)0.5 * (qt[j - 1] + qt[j]);
+    // TRiSK weights from prefix sums of the kite areas:
+    // w(i,j) = S_j - S_i - 1/2 (j>i), tot - S_i + S_j - 1/2 (j<i), w(i,i) = 0
+    const T R[MX] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
+    T S[MX + 1];
+    S[0] = (T)0;
+#pragma unroll
+    for (int j = 0; j < MX; ++j) S[j + 1] = S[j] + R[j];
+    const T tot = S[MX];
+#pragma unroll
+    for (int i = 0; i < MX; ++i) {
+      T acc = (T)0;
+#pragma unroll
+      for (int j = 0; j < MX; ++j)
+        if (j != i) {
+          const T w = ((j > i) ? (S[j] - S[i]) : (tot - S[i] + S[j])) - (T)0.5;
+          acc += G[j] * (qe[i] + qe[j]) * w;
+        }
+      T P = (T)0.5 * acc;
+      if ((f[i] >> SB_TNR) & 1) P = -P;
+      if (i < MX - 1 || hex) {
+        if ((f[i] >> SB_OWN) & 1) {
+          if (tid < nown) sP[ed[i]] = P;
+        } else if (nb[i] < nown) {
+          sPo[ed[i]] = P;
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // P3: own edges
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int i = tid + r * NT;
+    if (i >= 3 * nown) continue;
+    const int e = 3 * own0 + i;
+    const uint32_t w = ow[r];
+    if (w == 0xFFFFu) continue;
+    const int o = i / 3, c2 = w & LID;
+    const bool own_v2 = (w >> SB_OWN) & 1;
+    const T d = own_v2 ? sPhi[o] - sPhi[c2] : sPhi[c2] - sPhi[o];
+    T du = -(d + (sP[i] + sPo[i])) / el[r].x;
+    if (a.zero_mom) du = (T)0;
+    const T dt = a.dte ? a.dte[e] : (T)a.dt;
+    if (MODE == 3) {
+      a.du_out[e] = du;
+    } else if (MODE < 2) {
+      const T ca = a.whole ? dt : (T)0.5 * dt;
+      const T cb = MODE == 0 ? dt / (T)6 : dt / (T)3;
+      a.uout[e] = v0[r] + ca * du;
+      a.accu[e] = MODE == 0 ? cb * du : av[r] + cb * du;
+    } else {
+      a.uout[e] = v0[r] + (av[r] + (dt / (T)6) * du);
+    }
+  }
+}
+
+// ------------------------------------------------------------- host side ---
+template <typename X>
+static bool down(std::vector<X> &h, const void *d, size_t n) {
+  h.resize(n);
+  return n == 0 || hipMemcpy(h.data(), d, n * sizeof(X), hipMemcpyDeviceToHost) == hipSuccess;
+}
+
+void stage_free(imx_swm *s) {
+  if (!s->stg) return;
+  s->stg->A.release();
+  delete s->stg;
+  s->stg = nullptr;
+}
+
+int stage_threads(const imx_swm *s) { return s->stg ? s->stg->nt : 0; }
+void stage_set_remap(imx_swm *s, int remap) {
+  if (s->stg) s->stg->remap = remap;
+}
+size_t stage_bytes(const imx_swm *s) { return s->stg ? s->stg->A.bytes : 0; }
+int stage_remap(const imx_swm *s) { return s->stg ? s->stg->remap : 0; }
+
+// A block's local cells and triangles: small open-addressing tables that are
+// emptied by raising the stamp (a block holds far fewer entries than slots).
+struct LocalSet {
+  static constexpr int kSlots = 1 << 13;
+  struct Entry {
+    int32_t stamp = 0, key = 0, id = 0, in_c = 0;
+  };
+  std::vector<Entry> e{(size_t)kSlots};
+  std::vector<int32_t> keys;
+  int32_t stamp = 1;
+  void clear() {
+    ++stamp;
+    keys.clear();
+  }
+  // the entry of key, added when absent
+  Entry &at(int32_t key) {
+    uint32_t p = (uint32_t)key * 2654435761u >> 19;
+    while (e[p].stamp == stamp && e[p].key != key) p = (p + 1) & (kSlots - 1);
+    if (e[p].stamp != stamp) {
+      e[p] = Entry{stamp, key, 0, 0};
+      keys.push_back(key);
+    }
+    return e[p];
+  }
+};
+struct LocalSets {
+  LocalSet L, tri;
+  int nC = 0;
+  void clear() {
+    L.clear();
+    tri.clear();
+    nC = 0;
+  }
+};
+
+template <typename T>
+static int build(imx_swm *s, int nt) {
+  const int nv = s->nv, NE = s->NE, NTri = s->NT;
+  const int LC = cap_l(nt), TC = cap_t(nt);
+  const double ea = s->o.erad;
+  std::vector<int32_t> nbr, bA, bB, oth, tab, teb;
+  std::vector<T> R, ika, ceta, kap, tf;
+  std::vector<double> leng, dleng, tarea;
+  if (!down(nbr, s->x_c_nb, (size_t)MX * nv) || !down(bA, s->x_c_bitsA, nv) || !down(bB, s->x_c_bitsB, nv) ||
+      !down(oth, s->x_e_oth, NE) || !down(tab, s->x_t_ab, (size_t)2 * NTri) || !down(teb, s->x_t_eb, NTri) ||
+      !down(R, s->x_c_R, (size_t)MX * nv) || !down(ika, s->x_c_ika, nv) ||
+      !down(ceta, s->x_t_ceta, (size_t)3 * NTri) || !down(kap, s->x_t_kap, (size_t)3 * NTri) ||
+      !down(tf, s->x_t_f, NTri) || !down(leng, s->e_leng, NE) || !down(dleng, s->e_dleng, NE) ||
+      !down(tarea, s->t_area, NTri))
+    return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
+
+  auto tri_of = [&](int c, int j) {
+    const int ts = (bB[c] >> (BB_TSEL + 2 * j)) & 3;
+    const int to = ts == 0 ? c : ts == 1 ? nbr[(size_t)j * nv + c] : nbr[(size_t)((j + 1) % MX) * nv + c];
+    return 2 * to + ((bB[c] >> (BB_KT + j)) & 1);
+  };
+  // adds own cell c to the sets of the current block; false past a cap
+  auto add = [&](LocalSets &w, int c) {
+    auto in_c = [&](int k) {
+      LocalSet::Entry &q = w.L.at(k);
+      if (q.in_c) return;
+      q.in_c = 1;
+      ++w.nC;
+      const int n = bA[k] & 7;
+      for (int j = 0; j < n; ++j) {
+        (void)w.L.at(nbr[(size_t)j * nv + k]);
+        (void)w.tri.at(tri_of(k, j));
+      }
+    };
+    in_c(c);
+    const int n = bA[c] & 7;
+    for (int j = 0; j < n; ++j)
+      if ((bA[c] >> (BA_OWN + j)) & 1) in_c(nbr[(size_t)j * nv + c]);
+    return w.nC <= nt && (int)w.L.keys.size() <= LC && (int)w.tri.keys.size() <= TC;
+  };
+
+  // cut the curve into at most 16 segments, one host thread each, and every
+  // segment greedily into blocks
+  const int seg = std::max(64 * nt, (nv + 15) / 16), nseg = (nv + seg - 1) / seg;
+  auto each_segment = [&](auto fn) {
+    std::vector<std::thread> th;
+    for (int g = 0; g < nseg; ++g) th.emplace_back([&fn, g] { fn(g); });
+    for (auto &x : th) x.join();
+  };
+  std::vector<std::vector<int32_t>> cuts(nseg);
+  std::vector<char> fine(nseg, 1);
+  each_segment([&](int g) {
+    const int c0 = g * seg, c1 = std::min(nv, c0 + seg);
+    LocalSets w;
+    int first = c0;
+    cuts[g].push_back(first);
+    for (int c = c0; c < c1 && fine[g]; ++c) {
+      if (add(w, c)) continue;
+      first = c;
+      cuts[g].push_back(first);
+      w.clear();
+      fine[g] = add(w, c);  // a single cell within the caps
+    }
+  });
+  std::vector<int32_t> start, seg0;
+  for (int g = 0; g < nseg; ++g) {
+    seg0.push_back((int32_t)start.size());
+    start.insert(start.end(), cuts[g].begin(), cuts[g].end());
+  }
+  const int nblk = (int)start.size();
+  seg0.push_back(nblk);
+  start.push_back(nv);
+  // Numberings that are not local (a mesh in its caller's order) cut into
+  // blocks that are mostly rim: the three passes run instead.
+  for (char ok : fine)
+    if (!ok) return IMX_OK;
+  if (nblk > 1 && (int64_t)nblk * nt > (int64_t)3 * nv) return IMX_OK;
+
+  std::vector<int4> head(nblk);
+  std::vector<int32_t> halo((size_t)nblk * LC, 0);
+  std::vector<uint4> topo((size_t)nblk * nt, uint4{0, 0, 0, 0});
+  std::vector<Quad<T>> cw((size_t)nblk * 2 * nt, Quad<T>{0, 0, 0, 0}), tk((size_t)nblk * TC, Quad<T>{0, 0, 0, 0});
+  std::vector<Pair<T>> eld(NE);
+  std::vector<uint16_t> loth(NE, 0xFFFF), tslot((size_t)nblk * TC, 0);
+  std::vector<uint32_t> tv((size_t)nblk * TC, 0);
+  std::vector<T> tfv((size_t)nblk * TC, (T)0);
+  for (int e = 0; e < NE; ++e) eld[e] = Pair<T>{(T)leng[e], (T)dleng[e]};
+  each_segment([&](int g) {
+    LocalSets w;
+    for (int b = seg0[g]; b < seg0[g + 1]; ++b) {
+      const int o0 = start[b], nown = start[b + 1] - o0;
+      w.clear();
+      for (int c = o0; c < o0 + nown; ++c) (void)add(w, c);
+      // own cells, the rest of C, the rest of L, each ascending; own
+      // triangles first
+      auto own = [&](int k) { return k >= o0 && k < o0 + nown; };
+      std::vector<int32_t> cells = w.L.keys, tris = w.tri.keys;
+      auto rank = [&](int k) { return own(k) ? 0 : w.L.at(k).in_c ? 1 : 2; };
+      std::sort(cells.begin(), cells.end(), [&](int x, int y) {
+        const int rx = rank(x), ry = rank(y);
+        return rx != ry ? rx < ry : x < y;
+      });
+      std::sort(tris.begin(), tris.end(), [&](int x, int y) {
+        const bool ox = own(x / 2), oy = own(y / 2);
+        return ox != oy ? ox : x < y;
+      });
+      const int nL = (int)cells.size(), nC = w.nC;
+      for (int k = 0; k < nL; ++k) w.L.at(cells[k]).id = k;
+      auto id = [&](int k) { return (uint32_t)w.L.at(k).id; };
+      for (int k = nown; k < nL; ++k) halo[(size_t)b * LC + k - nown] = cells[k];
+      head[b] = int4{o0, nown, nC, nL | (int)tris.size() << 16};
+      for (int k = 0; k < nC; ++k) {
+        const int c = cells[k];
+        const bool hex = (bA[c] & 7) == MX;
+        uint32_t f[MX], t3 = (uint32_t)hex << SW_HEX;
+        T r[MX];
+        for (int j = 0; j < MX; ++j) {
+          f[j] = id(nbr[(size_t)j * nv + c]);
+          f[j] |= ((bA[c] >> (BA_OWN + j)) & 1u) << SB_OWN;
+          f[j] |= ((bB[c] >> (2 * j)) & 3u) << SB_K;
+          f[j] |= ((bA[c] >> (BA_TTG + j)) & 1u) << SB_TTG;
+          f[j] |= ((bA[c] >> (BA_TNR + j)) & 1u) << SB_TNR;
+          t3 |= ((bB[c] >> (BB_TSEL + 2 * j)) & 3u) << (2 * j);
+          t3 |= ((bB[c] >> (BB_KT + j)) & 1u) << (SW_KT + j);
+          r[j] = R[(size_t)j * nv + c];
+        }
+        topo[(size_t)b * nt + k] = uint4{f[0] | f[1] << 16, f[2] | f[3] << 16, f[4] | f[5] << 16, t3};
+        cw[((size_t)b * 2) * nt + k] = Quad<T>{r[0], r[1], r[2], r[3]};
+        // ika = 1 / sum (l l~ / 4)
+        cw[((size_t)b * 2 + 1) * nt + k] = Quad<T>{r[4], r[5], (T)0.25 * ika[c], (T)0};
+      }
+      for (int k = 0; k < (int)tris.size(); ++k) {
+        const int t = tris[k];
+        const size_t p = (size_t)b * TC + k;
+        uint32_t v = id(tab[t]) | id(tab[(size_t)NTri + t]) << 10;
+        v |= (uint32_t)(teb[t] & 511) << 20;
+        for (int m = 0; m < 3; ++m) v |= (ceta[(size_t)m * NTri + t] < 0 ? 1u : 0u) << (29 + m);
+        tv[p] = v;
+        tslot[p] = (uint16_t)(2 * id(t / 2) + t % 2);
+        tk[p] = Quad<T>{kap[t], kap[(size_t)NTri + t], kap[(size_t)2 * NTri + t], (T)(1.0 / (tarea[t] * ea))};
+        tfv[p] = tf[t];
+      }
+      for (int e = 3 * o0; e < 3 * (o0 + nown); ++e) {
+        if (oth[e] < 0) continue;
+        loth[e] = (uint16_t)(id(oth[e] & OTH_MASK) | ((uint32_t)(oth[e] >> OTH_V2) & 1u) << SB_OWN);
+      }
+    }
+  });
+
+  Stage *g = s->stg = new Stage();
+  Alloc &A = g->A;
+  g->nt = nt;
+  g->nblk = nblk;
+  g->head = A.put(head);
+  g->halo = A.put(halo);
+  g->topo = A.put(topo);
+  g->cw = A.put(cw);
+  g->eld = A.put(eld);
+  g->oth = A.put(loth);
+  g->tv = A.put(tv);
+  g->tslot = A.put(tslot);
+  g->tk = A.put(tk);
+  g->tf = A.put(tfv);
+  if (A.err != hipSuccess) {
+    const std::string why = hipGetErrorString(A.err);
+    stage_free(s);
+    return set_error(IMX_EDEVICE, "stage tables: " + why);
+  }
+  return IMX_OK;
+}
+
+int stage_build(imx_swm *s, int nt) {
+  stage_free(s);
+  return s->single ? build<float>(s, nt) : build<double>(s, nt);
+}
+
+template <typename T, int NT>
+static void launch_nt(const StageArgs<T> &a, int stage, int grid, hipStream_t st) {
+  switch (stage) {
+    case 0: fast_stage<T, NT, 0><<<grid, NT, 0, st>>>(a); break;
+    case 1:
+    case 2: fast_stage<T, NT, 1><<<grid, NT, 0, st>>>(a); break;
+    case 3: fast_stage<T, NT, 2><<<grid, NT, 0, st>>>(a); break;
+    default: fast_stage<T, NT, 3><<<grid, NT, 0, st>>>(a); break;
+  }
+}
+
+template <typename T>
+void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *uout) {
+  const Stage &g = *s->stg;
+  StageArgs<T> a;
+  a.head = g.head;
+  a.halo = g.halo;
+  a.topo = g.topo;
+  a.cw = (const Quad<T> *)g.cw;
+  a.eld = (const Pair<T> *)g.eld;
+  a.oth = g.oth;
+  a.tv = g.tv;
+  a.tslot = g.tslot;
+  a.tk = (const Quad<T> *)g.tk;
+  a.tf = (const T *)g.tf;
+  a.iaa = s->x_c_iaa;
+  a.hs = hs;
+  a.us = us;
+  a.h0 = (const T *)s->h0;
+  a.u0 = (const T *)s->u0;
+  a.gb = (const T *)s->x_gb;
+  a.dte = (const T *)s->dt_e;
+  a.dtc = s->dt_c;
+  a.hout = hout;
+  a.uout = uout;
+  a.acch = (T *)s->acch;
+  a.accu = (T *)s->accu;
+  a.q = (T *)s->q;
+  a.du_out = (T *)s->du_out;
+  a.dh_out = s->dh_out;
+  a.flag = s->flag;
+  a.href = s->href;
+  a.dt = s->o.dt;
+  a.grav = (T)s->o.grav;
+  a.inv_a = (T)(1.0 / s->o.erad);
+  a.nblk = g.nblk;
+  a.remap = g.remap;
+  a.whole = stage == 2;
+  a.use_pv = s->o.testcase >= 2;
+  a.flin = s->f_lin ? 1 : 0;
+  a.zero_mom = s->o.testcase <= 1;
+  const int grid = (g.nblk + NXCD - 1) / NXCD * NXCD;
+  switch (g.nt) {
+    case 128: launch_nt<T, 128>(a, stage, grid, s->stream); break;
+    case 512:
+      if constexpr (sizeof(T) == 4) launch_nt<T, 512>(a, stage, grid, s->stream);
+      break;
+    default: launch_nt<T, 256>(a, stage, grid, s->stream); break;
+  }
+}
+template void stage_launch<float>(imx_swm *, int, const float *, const float *, float *, float *);
+template void stage_launch<double>(imx_swm *, int, const double *, const double *, double *, double *);
+
+}  // namespace imx

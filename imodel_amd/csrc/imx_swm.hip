@@ -1655,6 +1655,14 @@ static void launch_ref_step(imx_swm *s) {
     default: CALL(256); break;   \
   }
 
+// The scheme imx_stage.hip evaluates in one launch per stage: trsk10's
+// methods without options, HTC or HC, with any topography and Coriolis term.
+static bool plain_scheme(const imx_swm *s) {
+  return !(s->f_gass || s->f_melv || s->f_perhx || s->f_nopv || s->f_apvm || s->f_bary || s->f_pered || s->f_gk ||
+           s->f_dtred || s->f_diff || s->f_hyper);
+}
+static bool stage_on(const imx_swm *s) { return s->stg && !s->stg_stale && plain_scheme(s); }
+
 // One FAST stage: stage<0 evaluates the tendency of (hs, us) into dh_out/du_out.
 template <typename T>
 static void launch_fast_stage(imx_swm *s, int stage, const T *hs, const T *us, T *hout,
@@ -1663,6 +1671,12 @@ static void launch_fast_stage(imx_swm *s, int stage, const T *hs, const T *us, T
   hipStream_t st = s->stream;
   const T href = (T)s->href;
   if (evs) (void)hipEventRecord(evs[0], st);
+  if (stage_on(s)) {
+    stage_launch<T>(s, stage, hs, us, hout, uout);
+    if (evs)
+      for (int k = 1; k < 4; ++k) (void)hipEventRecord(evs[k], st);
+    return;
+  }
   if (s->f_pxhc)  // before fast_tri, whose dtred term reads these depths
     fast_hc_he<T, 256><<<grid_bs(NE, 256), 256, 0, st>>>(s->kremap[2], NE, s->x_e_oth, (const T *)s->x_px_hb,
                                                          s->x_px_hv, hs, href, (T *)s->x_px_he);
@@ -2522,6 +2536,22 @@ static int validate_desc(const imx_mesh_desc &d) {
   return IMX_OK;
 }
 
+// Threads of a block of the one-launch stage: small blocks until there are
+// enough cells to give every CU one (glevel 5, FP32, per step: 128 threads
+// 32.0 us, 256 36 us), then 256, where the rim is 1.3 times the work and five
+// blocks fit a CU (glevel 8: 127 us against 131 with 128 and 129 with 512).
+static int stage_default(const imx_swm *s) { return s->nv < 30000 ? 128 : 256; }
+
+// The stage tables follow the handle's staggering, triangle weights and
+// Coriolis parameter; they are made again when the plain scheme is back.
+static int stage_refresh(imx_swm *s) {
+  s->stg_stale = s->stg != nullptr;
+  if (!s->stg_stale || !plain_scheme(s)) return IMX_OK;
+  const int rc = stage_build(s, stage_threads(s));
+  s->stg_stale = false;
+  return rc;
+}
+
 static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
                   const int32_t *group = nullptr, const double *dt_cell = nullptr,
                   const double *dt_edge = nullptr, const Layout *pre = nullptr) {
@@ -2706,7 +2736,7 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
     }
   }
   HIPTRY(hipDeviceSynchronize(), "imx_swm_create");
-  return IMX_OK;
+  return s->fast ? stage_build(s, stage_default(s)) : IMX_OK;
 }
 
 static int check_flag(imx_swm *s, const char *what) {
@@ -2854,26 +2884,62 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   HIPTRY(hipMemcpyAsync(su, s->u0, es * s->NE, hipMemcpyDeviceToDevice, s->stream), "tune");
   std::vector<hipEvent_t> ev(16);
   for (auto &e : ev) HIPTRY(hipEventCreate(&e), "event");
+  // one step's time at the present launch shapes, over nsteps (the first
+  // pass warms up): the events (j, j + 1) of each stage
+  auto timed = [&](int j0, int j1, double &acc) -> int {
+    acc = 0.0;
+    for (int it = 0; it <= nsteps; ++it) {
+      if (s->single) launch_fast_step<float>(s, &ev);
+      else launch_fast_step<double>(s, &ev);
+      HIPTRY(hipEventSynchronize(ev[15]), "event");
+      if (it == 0) continue;
+      for (int st = 0; st < 4; ++st) {
+        float f = 0.f;
+        HIPTRY(hipEventElapsedTime(&f, ev[4 * st + j0], ev[4 * st + j1]), "event");
+        acc += f;
+      }
+    }
+    return IMX_OK;
+  };
   const int bss[4] = {64, 128, 256, 512};
-  for (int k = 0; k < 3; ++k) {
+  int rc = IMX_OK;
+  if (stage_on(s)) {
+    // one launch per stage: block threads (which cut the mesh anew) x remap
+    double best = 1e30;
+    int bb = stage_threads(s), br = 1;
+    for (int bs : {128, 256, 512}) {
+      if (bs == 512 && !s->single) continue;  // over 64 KB of LDS
+      if ((rc = stage_build(s, bs))) break;
+      if (!s->stg) continue;
+      for (int r = 0; r < 2 && !rc; ++r) {
+        stage_set_remap(s, r);
+        double acc;
+        rc = timed(0, 1, acc);
+        if (!rc && acc < best) {
+          best = acc;
+          bb = bs;
+          br = r;
+        }
+      }
+      if (rc) break;
+    }
+    if (!s->stg || stage_threads(s) != bb) {
+      const int r2 = stage_build(s, bb);
+      if (!rc) rc = r2;
+    }
+    stage_set_remap(s, br);
+    s->kbs[1] = bb;
+    s->kremap[1] = br;
+  } else {
+  for (int k = 0; k < 3 && !rc; ++k) {
     double best = 1e30;
     int bb = s->kbs[k], br = s->kremap[k];
     for (int bi = 0; bi < 4; ++bi)
       for (int r = 0; r < 2; ++r) {
         s->kbs[k] = bss[bi];
         s->kremap[k] = r;
-        double acc = 0.0;
-        for (int it = 0; it <= nsteps; ++it) {  // first pass warms up
-          if (s->single) launch_fast_step<float>(s, &ev);
-          else launch_fast_step<double>(s, &ev);
-          HIPTRY(hipEventSynchronize(ev[15]), "event");
-          if (it == 0) continue;
-          for (int st = 0; st < 4; ++st) {
-            float f = 0.f;
-            HIPTRY(hipEventElapsedTime(&f, ev[4 * st + k], ev[4 * st + k + 1]), "event");
-            acc += f;
-          }
-        }
+        double acc;
+        if ((rc = timed(k, k + 1, acc))) break;
         if (acc < best) {
           best = acc;
           bb = bss[bi];
@@ -2883,6 +2949,7 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
     s->kbs[k] = bb;
     s->kremap[k] = br;
   }
+  }
   for (auto &e : ev) (void)hipEventDestroy(e);
   HIPTRY(hipMemcpyAsync(s->h0, sh, es * s->nv, hipMemcpyDeviceToDevice, s->stream), "tune");
   HIPTRY(hipMemcpyAsync(s->u0, su, es * s->NE, hipMemcpyDeviceToDevice, s->stream), "tune");
@@ -2890,6 +2957,7 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   (void)hipFree(sh);
   (void)hipFree(su);
   drop_graph(s);
+  if (rc) return rc;
   if (out)
     for (int k = 0; k < 3; ++k) {
       out[2 * k] = s->kbs[k];
@@ -3014,7 +3082,7 @@ int imx_swm_set_coriolis(imx_swm *s, int32_t fsphere, double fcte) {
   }
   s->f_lin = fsphere == IMX_F_LINEAR;
   imx::drop_graph(s);  // the captured step holds the previous flag
-  return IMX_OK;
+  return s->fast ? imx::stage_refresh(s) : IMX_OK;
 }
 
 int imx_swm_get_state(imx_swm *s, double *h, double *u) {
@@ -3603,8 +3671,9 @@ int imx_swm_set_scheme(imx_swm *s, const imx_mesh_desc *d, const imx_scheme *sc)
     s->sc_hyper = r.k4 != 0.0;
     s->sc = r;
     imx::drop_graph(s);
+    const int rs = imx::stage_refresh(s);
     if (rc) return imx::set_error(rc, why + " (the handle is back on the default scheme)");
-    return IMX_OK;
+    return rs;
   }
   const int nv = s->nv, NE = s->NE, NT = s->NT;
   const std::vector<int32_t> &cn = s->lay.cell_new, &en = s->lay.edge_new, &tn = s->lay.tri_new;
@@ -3761,13 +3830,13 @@ int imx_swm_profile(imx_swm *s, int32_t nsteps, double *ms, int32_t *nk) {
   }
   for (auto &e : ev) (void)hipEventDestroy(e);
   for (int j = 0; j < 3; ++j) ms[j] = acc[j] / (4.0 * (nsteps > 0 ? nsteps : 1));
-  *nk = 3;
+  *nk = imx::stage_on(s) ? 1 : 3;
   return imx::check_flag(s, "imx_swm_profile");
 }
 
 const char *imx_swm_kernel_name(imx_swm *s, int32_t k) {
-  (void)s;
   if (k < 0 || k > 2) return "";
+  if (s && s->fast && imx::stage_on(s)) return k == 0 ? "fast_stage" : "";
   return kFastNames[k];
 }
 
@@ -3852,7 +3921,7 @@ int imx_swm_info(imx_swm *s, int64_t out[8]) {
   out[0] = s->nv;
   out[1] = s->ne;
   out[2] = s->nt;
-  out[3] = (int64_t)s->A.bytes;
+  out[3] = (int64_t)(s->A.bytes + imx::stage_bytes(s));
   out[4] = s->o.precision;
   out[5] = s->o.use_sfc;
   out[6] = s->o.use_graph;
@@ -3904,6 +3973,7 @@ void imx_swm_destroy(imx_swm *s) {
   if (!s) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   imx::drop_graph(s);
+  imx::stage_free(s);
   s->A.release();
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
