@@ -49,6 +49,56 @@ struct Alloc {
   }
 };
 
+// Captured steps: graphs of 1, 4 and 16 steps, so that a run of many steps
+// pays one graph launch (6.8 us on the device, whatever the graph holds) per
+// sixteen. Each is captured when a run first needs it.
+struct StepGraphs {
+  static constexpr int kSizes = 3;
+  static constexpr int kSteps[kSizes] = {16, 4, 1};
+  hipGraph_t graph[kSizes] = {};
+  hipGraphExec_t exec[kSizes] = {};
+  void drop() {
+    for (int k = 0; k < kSizes; ++k) {
+      if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
+      if (graph[k]) (void)hipGraphDestroy(graph[k]);
+      exec[k] = nullptr;
+      graph[k] = nullptr;
+    }
+  }
+  // captures what a run of nsteps launches; one(): enqueues a step, 0 or an
+  // IMX_E* code, which is returned (a hipError_t comes back in err)
+  template <typename F>
+  int ensure(int nsteps, hipStream_t st, F one, hipError_t &err) {
+    err = hipSuccess;
+    for (int k = 0; k < kSizes; ++k) {
+      const int count = nsteps / kSteps[k];
+      nsteps -= count * kSteps[k];
+      if (count == 0 || exec[k]) continue;
+      if ((err = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal)) != hipSuccess) return 0;
+      int rc = 0;
+      for (int i = 0; i < kSteps[k] && rc == 0; ++i) rc = one();
+      hipGraph_t g = nullptr;
+      err = hipStreamEndCapture(st, &g);
+      if (rc == 0 && err == hipSuccess) err = hipGraphInstantiate(&exec[k], g, nullptr, nullptr, 0);
+      if (rc != 0 || err != hipSuccess) {
+        if (g) (void)hipGraphDestroy(g);
+        exec[k] = nullptr;
+        return rc;
+      }
+      graph[k] = g;
+    }
+    return 0;
+  }
+  hipError_t launch(int nsteps, hipStream_t st) {
+    for (int k = 0; k < kSizes; ++k)
+      for (; nsteps >= kSteps[k]; nsteps -= kSteps[k]) {
+        const hipError_t e = hipGraphLaunch(exec[k], st);
+        if (e != hipSuccess) return e;
+      }
+    return hipSuccess;
+  }
+};
+
 struct Stage;  // tables of the one-launch-per-stage path (imx_stage.hip)
 
 }  // namespace imx
@@ -59,8 +109,7 @@ struct imx_swm {
   int NE = 0, NT = 0;          // internal edge/triangle slots (3 nv, 2 nv)
   imx::Layout lay;             // caller -> internal maps
   hipStream_t stream = nullptr;
-  hipGraphExec_t gexec = nullptr;
-  hipGraph_t graph = nullptr;
+  imx::StepGraphs graphs;
   // bumped whenever the step's kernel sequence or arguments change (scheme,
   // tuning, topography, h_ref): graphs captured over the step by other
   // objects (imx_learn) compare it with the value they captured at

@@ -20,7 +20,7 @@
 // fits D F to the dh target through D (the gradient D^T r is handed to the
 // MLP backward pass). The correction is skipped (plain step kept) when its
 // RMS exceeds a bound. The corrected step (save, RK4 step, features, MLP,
-// correction) is one hipGraph launch.
+// correction) is captured; one graph launch runs up to 16 of them.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
@@ -61,8 +61,7 @@ struct imx_learn {
   double *bound = nullptr;  // [2] RMS bound, limiter mode (IMX_LIMIT_*)
   double *lh = nullptr;     // [1] h loss of the last training epoch
   int *nfb = nullptr;       // [1] limited steps since the counter was cleared
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  imx::StepGraphs graphs;
   const short *gX = nullptr;  // MLP input buffer the graph was captured with
   uint64_t gen = 0;           // the step handle's generation at capture
   // device sample store: normalised features, scaled targets
@@ -295,12 +294,7 @@ static int lfail(hipError_t e, const char *what) {
     if (_e != hipSuccess) return imx::lfail(_e, what); \
   } while (0)
 
-static void learn_drop_graph(imx_learn *L) {
-  if (L->gexec) (void)hipGraphExecDestroy(L->gexec);
-  if (L->graph) (void)hipGraphDestroy(L->graph);
-  L->gexec = nullptr;
-  L->graph = nullptr;
-}
+static void learn_drop_graph(imx_learn *L) { L->graphs.drop(); }
 
 // enqueue: save x_n, one plain step
 template <typename T>
@@ -360,33 +354,25 @@ static int learn_sample(imx_learn *L) {
   return IMX_OK;
 }
 
-static int learn_ensure_graph(imx_learn *L) {
+static int learn_ensure_graphs(imx_learn *L, int nsteps) {
   int rc = mlp_reserve(L->m, L->NE);
   if (rc) return rc;
   // recapture when the MLP scratch moved or the handle's step changed
   // (scheme, tuning, topography, h_ref)
-  if (L->gexec && L->gX == L->m->X && L->gen == L->s->generation) return IMX_OK;
-  learn_drop_graph(L);
-  hipStream_t st = L->s->stream;
-  LTRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "learn graph capture");
-  if (L->s->single) {
-    learn_enqueue_sample<float>(L);
-    rc = learn_enqueue_correct<float>(L);
-  } else {
-    learn_enqueue_sample<double>(L);
-    rc = learn_enqueue_correct<double>(L);
-  }
-  hipGraph_t gr = nullptr;
-  hipError_t e = hipStreamEndCapture(st, &gr);
-  if (rc) {
-    if (gr) (void)hipGraphDestroy(gr);
-    return rc;
-  }
-  LTRY(e, "learn graph capture end");
-  L->graph = gr;
-  LTRY(hipGraphInstantiate(&L->gexec, L->graph, nullptr, nullptr, 0), "learn graph instantiate");
+  if (L->gX != L->m->X || L->gen != L->s->generation) learn_drop_graph(L);
   L->gX = L->m->X;
   L->gen = L->s->generation;
+  hipError_t e;
+  rc = L->graphs.ensure(nsteps, L->s->stream, [&] {
+    if (L->s->single) {
+      learn_enqueue_sample<float>(L);
+      return learn_enqueue_correct<float>(L);
+    }
+    learn_enqueue_sample<double>(L);
+    return learn_enqueue_correct<double>(L);
+  }, e);
+  if (rc) return rc;
+  LTRY(e, "learn graph capture");
   return IMX_OK;
 }
 
@@ -611,11 +597,11 @@ int imx_learn_set_limiter(imx_learn *L, int32_t mode) {
 int imx_learn_step(imx_learn *L, int32_t nsteps, double bound, int32_t *nlimited) {
   if (!L || nsteps < 0) return imx::set_error(IMX_EINVAL, "imx_learn_step: bad argument");
   imx_swm *s = L->s;
-  int rc = imx::learn_ensure_graph(L);
+  int rc = imx::learn_ensure_graphs(L, nsteps);
   if (rc) return rc;
   LTRY(hipMemcpyAsync(L->bound, &bound, 8, hipMemcpyHostToDevice, s->stream), "learn step");
   LTRY(hipMemsetAsync(L->nfb, 0, 4, s->stream), "learn step");
-  for (int k = 0; k < nsteps; ++k) LTRY(hipGraphLaunch(L->gexec, s->stream), "learn step");
+  LTRY(L->graphs.launch(nsteps, s->stream), "learn step");
   int nfb = 0;
   LTRY(hipMemcpyAsync(&nfb, L->nfb, 4, hipMemcpyDeviceToHost, s->stream), "learn step");
   rc = imx::swm_check_flag(s, "imx_learn_step");

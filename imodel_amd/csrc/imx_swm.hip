@@ -2806,26 +2806,21 @@ int swm_stencil_rings(const imx_swm *s) {
 
 static void drop_graph(imx_swm *s) {
   ++s->generation;  // graphs captured elsewhere over this handle's step are stale too
-  if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
-  if (s->graph) (void)hipGraphDestroy(s->graph);
-  s->gexec = nullptr;
-  s->graph = nullptr;
+  s->graphs.drop();
 }
 
-static int ensure_graph(imx_swm *s) {
-  if (s->gexec) return IMX_OK;
-  HIPTRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal), "graph capture");
-  launch_step(s);
-  HIPTRY(hipStreamEndCapture(s->stream, &s->graph), "graph capture end");
-  HIPTRY(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0), "graph instantiate");
-  return IMX_OK;
+static int ensure_graphs(imx_swm *s, int nsteps) {
+  hipError_t e;
+  const int rc = s->graphs.ensure(nsteps, s->stream, [&] { launch_step(s); return 0; }, e);
+  HIPTRY(e, "step graph capture");
+  return rc;
 }
 
 static int run_steps(imx_swm *s, int nsteps) {
   if (s->o.use_graph) {
-    int rc = ensure_graph(s);
+    int rc = ensure_graphs(s, nsteps);
     if (rc) return rc;
-    for (int k = 0; k < nsteps; ++k) HIPTRY(hipGraphLaunch(s->gexec, s->stream), "hipGraphLaunch");
+    HIPTRY(s->graphs.launch(nsteps, s->stream), "hipGraphLaunch");
   } else {
     for (int k = 0; k < nsteps; ++k) launch_step(s);
     HIPTRY(hipGetLastError(), "step launch");
@@ -3795,7 +3790,7 @@ int imx_swm_step_timed(imx_swm *s, int32_t nsteps, double *ms) {
   if (!s || !ms) return imx::set_error(IMX_EINVAL, "imx_swm_step_timed: NULL argument");
   if (nsteps < 0) return imx::set_error(IMX_EINVAL, "imx_swm_step_timed: nsteps < 0");
   if (s->o.use_graph) {
-    int rc = imx::ensure_graph(s);  // instantiation stays outside the timed region
+    int rc = imx::ensure_graphs(s, nsteps);  // instantiation stays outside the timed region
     if (rc) return rc;
   }
   HIPTRY(hipEventRecord(s->ev0, s->stream), "event");
