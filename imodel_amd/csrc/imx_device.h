@@ -108,6 +108,12 @@ struct imx_swm {
   int nv = 0, ne = 0, nt = 0;  // caller counts
   int NE = 0, NT = 0;          // internal edge/triangle slots (3 nv, 2 nv)
   imx::Layout lay;             // caller -> internal maps
+  int32_t *d_cell = nullptr, *d_edge = nullptr;  // the cell and edge maps on the device
+  // pinned memory the kernels read states from and write them to in caller
+  // order (at most kHostStage bytes: larger states go through it in parts)
+  static constexpr size_t kHostStage = (size_t)64 << 20;
+  void *hstage = nullptr;
+  size_t hstage_bytes = 0;
   hipStream_t stream = nullptr;
   imx::StepGraphs graphs;
   // bumped whenever the step's kernel sequence or arguments change (scheme,
@@ -208,7 +214,7 @@ struct imx_swm {
   void *x_gb_buf = nullptr;
   bool has_topo = false;
   double topo_sb = 0.0, topo_sb2 = 0.0;  // sum A b, sum A b^2 (unit-sphere areas)
-  int *flag = nullptr;
+  int *flag = nullptr;  // vanishing depth met; pinned host memory, written by the kernels
   double *part = nullptr, *diag = nullptr;
   int nparts = 0;
 

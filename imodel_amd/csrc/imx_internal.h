@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -10,21 +11,26 @@
 
 namespace imx {
 
-// fn(i0, i1) over [0, n) split across up to 16 host threads; each index is
-// handled by exactly one thread, so per-element results do not depend on
-// the split (reductions stay serial in the callers).
+// fn(i0, i1) over [0, n) split across up to 16 host threads, at least grain
+// indices each; each index is handled by exactly one thread, so per-element
+// results do not depend on the split (reductions stay serial in the callers).
 template <typename F>
-void parallel_ranges(int n, F fn) {
+void parallel_ranges(int n, F fn, int grain = 4096) {
   const int hw = (int)std::thread::hardware_concurrency();
-  const int nt = std::max(1, std::min({16, hw > 0 ? hw : 1, n / 4096 + 1}));
+  const int nt = std::max(1, std::min({16, hw > 0 ? hw : 1, n / grain + 1}));
   if (nt == 1) {
     fn(0, n);
     return;
   }
   std::vector<std::thread> th;
+  th.reserve(nt);
   for (int t = 0; t < nt; ++t) {
     const int i0 = (int)((int64_t)n * t / nt), i1 = (int)((int64_t)n * (t + 1) / nt);
-    th.emplace_back([=] { fn(i0, i1); });
+    try {
+      th.emplace_back([=] { fn(i0, i1); });
+    } catch (const std::system_error &) {
+      fn(i0, i1);  // no more threads: this one does the range
+    }
   }
   for (auto &x : th) x.join();
 }

@@ -34,7 +34,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -482,13 +484,18 @@ static int build(imx_swm *s, int nt) {
   // cut the curve into at most 16 segments, one host thread each, and every
   // segment greedily into blocks
   const int seg = std::max(64 * nt, (nv + 15) / 16), nseg = (nv + seg - 1) / seg;
-  auto each_segment = [&](auto fn) {
-    std::vector<std::thread> th;
-    for (int g = 0; g < nseg; ++g) th.emplace_back([&fn, g] { fn(g); });
-    for (auto &x : th) x.join();
-  };
   std::vector<std::vector<int32_t>> cuts(nseg);
   std::vector<char> fine(nseg, 1);
+  std::atomic<bool> memory{true};
+  auto each_segment = [&](auto fn) {
+    parallel_ranges(nseg, [&](int g0, int g1) {
+      try {
+        for (int g = g0; g < g1; ++g) fn(g);
+      } catch (const std::bad_alloc &) {
+        memory = false;
+      }
+    }, 1);
+  };
   each_segment([&](int g) {
     const int c0 = g * seg, c1 = std::min(nv, c0 + seg);
     LocalSets w;
@@ -502,6 +509,8 @@ static int build(imx_swm *s, int nt) {
       fine[g] = add(w, c);  // a single cell within the caps
     }
   });
+  const char *out_of = "stage tables: host out of memory";
+  if (!memory) return set_error(IMX_ENOMEM, out_of);
   std::vector<int32_t> start, seg0;
   for (int g = 0; g < nseg; ++g) {
     seg0.push_back((int32_t)start.size());
@@ -587,6 +596,7 @@ static int build(imx_swm *s, int nt) {
     }
   });
 
+  if (!memory) return set_error(IMX_ENOMEM, out_of);
   Stage *g = s->stg = new Stage();
   Alloc &A = g->A;
   g->nt = nt;
@@ -611,7 +621,11 @@ static int build(imx_swm *s, int nt) {
 
 int stage_build(imx_swm *s, int nt) {
   stage_free(s);
-  return s->single ? build<float>(s, nt) : build<double>(s, nt);
+  try {
+    return s->single ? build<float>(s, nt) : build<double>(s, nt);
+  } catch (const std::bad_alloc &) {
+    return set_error(IMX_ENOMEM, "stage tables: host out of memory");
+  }
 }
 
 template <typename T, int NT>

@@ -1364,6 +1364,32 @@ __global__ __launch_bounds__(BS) void fast_edge(int remap, int NE, const int32_t
   }
 }
 
+// ======================================================= caller's order ==
+// Values i0 .. i0 + m of a state in the caller's order (nh cells, then edges)
+// between the staging area and their places: reads and writes of the staging
+// area, over the host link, are consecutive.
+template <typename T>
+__global__ __launch_bounds__(TPB) void state_in(int i0, int m, int nh, const int32_t *__restrict__ cell,
+                                                const int32_t *__restrict__ edge, const T *__restrict__ src,
+                                                T *__restrict__ h, T *__restrict__ u) {
+  const int k = blockIdx.x * TPB + threadIdx.x;
+  if (k >= m) return;
+  const int i = i0 + k;
+  const T v = src[k];
+  if (i < nh) h[cell[i]] = v;
+  else u[edge[i - nh]] = v;
+}
+
+template <typename D, typename TH, typename TU>
+__global__ __launch_bounds__(TPB) void state_out(int i0, int m, int nh, const int32_t *__restrict__ cell,
+                                                 const int32_t *__restrict__ edge, const TH *__restrict__ h,
+                                                 const TU *__restrict__ u, D *__restrict__ dst) {
+  const int k = blockIdx.x * TPB + threadIdx.x;
+  if (k >= m) return;
+  const int i = i0 + k;
+  dst[k] = i < nh ? (D)h[cell[i]] : (D)u[edge[i - nh]];
+}
+
 // ============================================================ diagnostics ==
 // FP64 reductions of the current state (h = href + hs, u) with wavefront
 // shuffles + LDS, one partial per block, then a one-block final pass.
@@ -2670,7 +2696,10 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
   s->f_var = t_f;
   s->t_trhx = A.put(t_trhx);
   s->bt = A.put(std::vector<double>(nv, 0.0));
-  s->flag = A.put(std::vector<int>(1, 0));
+  s->d_cell = A.put(s->lay.cell_new);
+  s->d_edge = A.put(s->lay.edge_new);
+  HIPTRY(hipHostMalloc((void **)&s->flag, sizeof(int), hipHostMallocDefault), "hipHostMalloc");
+  *s->flag = 0;
   s->nparts = (nv + TPB - 1) / TPB + (NE + TPB - 1) / TPB + (NT + TPB - 1) / TPB;
   s->part = A.get<double>((size_t)s->nparts * NPART);
   s->diag = A.get<double>(NPART);
@@ -2740,12 +2769,10 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
 }
 
 static int check_flag(imx_swm *s, const char *what) {
-  int f = 0;
-  HIPTRY(hipMemcpyAsync(&f, s->flag, sizeof(int), hipMemcpyDeviceToHost, s->stream), what);
   HIPTRY(hipStreamSynchronize(s->stream), what);
-  if (f) {
-    int z = 0;
-    HIPTRY(hipMemcpy(s->flag, &z, sizeof(int), hipMemcpyHostToDevice), what);
+  volatile int *f = s->flag;
+  if (*f) {
+    *f = 0;
     return set_error(IMX_ESTATE, std::string(what) +
                                      ": division by zero, |h_tr| < epsilon/1e5 "
                                      "(swm_operators.f90:1603)");
@@ -2753,32 +2780,89 @@ static int check_flag(imx_swm *s, const char *what) {
   return IMX_OK;
 }
 
+// The pinned staging area, for n values of the given size (or what of them
+// fits kHostStage); made at its first use, kept with the handle.
+static int host_stage(imx_swm *s, size_t n, size_t size) {
+  const size_t want = std::min(n * size, imx_swm::kHostStage);
+  if (want <= s->hstage_bytes) return IMX_OK;
+  if (s->hstage) (void)hipHostFree(s->hstage);
+  s->hstage = nullptr;
+  s->hstage_bytes = 0;
+  HIPTRY(hipHostMalloc(&s->hstage, want, hipHostMallocDefault), "host staging");
+  s->hstage_bytes = want;
+  return IMX_OK;
+}
+
+// host values per thread from which a copy is worth splitting
+static constexpr int kHostGrain = 1 << 17;
+
+// A caller's state (nh cell values from cell c0 of the caller's numbering,
+// nu edge values from edge e0) to internal order: the host rounds h - href
+// and u into the staging area in the caller's order, a sequential pass, and
+// state_in puts every value in its place, so the scattered writes are the
+// device's. The call returns when the device has the state.
 template <typename T>
-static int upload_state(imx_swm *s, const double *h, const double *u, T *hd, T *ud) {
-  std::vector<T> hb(s->nv, (T)0), ub(s->NE, (T)0);
-  for (int i = 0; i < s->nv; ++i) hb[s->lay.cell_new[i]] = (T)(h[i] - s->href);
-  for (int l = 0; l < s->ne; ++l) ub[s->lay.edge_new[l]] = (T)u[l];
-  HIPTRY(hipMemcpyAsync(hd, hb.data(), hb.size() * sizeof(T), hipMemcpyHostToDevice, s->stream),
-         "upload h");
-  HIPTRY(hipMemcpyAsync(ud, ub.data(), ub.size() * sizeof(T), hipMemcpyHostToDevice, s->stream),
-         "upload u");
+static int upload_state(imx_swm *s, const double *h, const double *u, T *hd, T *ud, int c0, int nh, int e0, int nu) {
+  const int n = nh + nu;
+  int rc = host_stage(s, n, sizeof(T));
+  if (rc) return rc;
+  T *st = (T *)s->hstage;
+  const int part = (int)std::min<size_t>(n, s->hstage_bytes / sizeof(T));
+  const double href = s->href;
+  for (int i0 = 0; i0 < n; i0 += part) {
+    const int m = std::min(part, n - i0);
+    parallel_ranges(m, [=](int a, int b) {
+      const int cells = std::min(std::max(nh - i0, a), b);
+      for (int k = a; k < cells; ++k) st[k] = (T)(h[i0 + k] - href);
+      for (int k = cells; k < b; ++k) st[k] = (T)u[i0 + k - nh];
+    }, kHostGrain);
+    state_in<T><<<(m + TPB - 1) / TPB, TPB, 0, s->stream>>>(i0, m, nh, s->d_cell + c0, s->d_edge + e0, st, hd, ud);
+    HIPTRY(hipGetLastError(), "upload");
+    if (i0 + m < n) HIPTRY(hipStreamSynchronize(s->stream), "upload");
+  }
+  return IMX_OK;
+}
+
+// The way back: state_out writes the values in the caller's order, as D, to
+// the staging area; the host adds href to the cells' ones. With `what` the
+// caller's arrays are written only when no kernel met a vanishing depth.
+template <typename D, typename TH, typename TU>
+static int download_state(imx_swm *s, double *h, double *u, const TH *hd, const TU *ud, double href, int c0, int nh,
+                          int e0, int nu, const char *what = nullptr) {
+  if (!h) nh = 0;
+  if (!u) nu = 0;
+  const int n = nh + nu;
+  int rc = host_stage(s, n, sizeof(D));
+  if (rc) return rc;
+  D *st = (D *)s->hstage;
+  const int part = (int)std::min<size_t>(n, s->hstage_bytes / sizeof(D));
+  for (int i0 = 0; i0 < n; i0 += part) {
+    const int m = std::min(part, n - i0);
+    state_out<D, TH, TU><<<(m + TPB - 1) / TPB, TPB, 0, s->stream>>>(i0, m, nh, s->d_cell + c0, s->d_edge + e0, hd, ud,
+                                                                    st);
+    HIPTRY(hipGetLastError(), "download");
+    HIPTRY(hipStreamSynchronize(s->stream), "download");
+    if (what && (rc = check_flag(s, what))) return rc;
+    parallel_ranges(m, [=](int a, int b) {
+      const int cells = std::min(std::max(nh - i0, a), b);
+      for (int k = a; k < cells; ++k) h[i0 + k] = (double)st[k] + href;
+      for (int k = cells; k < b; ++k) u[i0 + k - nh] = (double)st[k];
+    }, kHostGrain);
+  }
+  return IMX_OK;
+}
+
+template <typename T>
+static int set_state(imx_swm *s, const double *h, const double *u, T *hd, T *ud) {
+  const int rc = upload_state<T>(s, h, u, hd, ud, 0, s->nv, 0, s->ne);
+  if (rc) return rc;
   HIPTRY(hipStreamSynchronize(s->stream), "upload");
   return IMX_OK;
 }
 
 template <typename T>
-static int download_state(imx_swm *s, double *h, double *u, const T *hd, const T *ud) {
-  std::vector<T> hb(s->nv), ub(s->NE);
-  HIPTRY(hipMemcpyAsync(hb.data(), hd, hb.size() * sizeof(T), hipMemcpyDeviceToHost, s->stream),
-         "download h");
-  HIPTRY(hipMemcpyAsync(ub.data(), ud, ub.size() * sizeof(T), hipMemcpyDeviceToHost, s->stream),
-         "download u");
-  HIPTRY(hipStreamSynchronize(s->stream), "download");
-  if (h)
-    for (int i = 0; i < s->nv; ++i) h[i] = (double)hb[s->lay.cell_new[i]] + s->href;
-  if (u)
-    for (int l = 0; l < s->ne; ++l) u[l] = (double)ub[s->lay.edge_new[l]];
-  return IMX_OK;
+static int get_state(imx_swm *s, double *h, double *u, const T *hd, const T *ud) {
+  return download_state<T>(s, h, u, hd, ud, s->href, 0, s->nv, 0, s->ne);
 }
 
 static void drop_graph(imx_swm *s);
@@ -3003,10 +3087,10 @@ int imx_swm_create(const imx_mesh_desc *d, const imx_swm_opts *o, imx_swm **out)
 
 int imx_swm_set_state(imx_swm *s, const double *h, const double *u) {
   if (!s || !h || !u) return imx::set_error(IMX_EINVAL, "imx_swm_set_state: NULL argument");
-  if (!s->fast) return imx::upload_state<double>(s, h, u, s->rh, s->ru);
+  if (!s->fast) return imx::set_state<double>(s, h, u, s->rh, s->ru);
   imx::set_href(s, h);
-  if (s->single) return imx::upload_state<float>(s, h, u, (float *)s->h0, (float *)s->u0);
-  return imx::upload_state<double>(s, h, u, (double *)s->h0, (double *)s->u0);
+  if (s->single) return imx::set_state<float>(s, h, u, (float *)s->h0, (float *)s->u0);
+  return imx::set_state<double>(s, h, u, (double *)s->h0, (double *)s->u0);
 }
 
 int imx_swm_set_topography(imx_swm *s, const double *bt) {
@@ -3082,44 +3166,37 @@ int imx_swm_set_coriolis(imx_swm *s, int32_t fsphere, double fcte) {
 
 int imx_swm_get_state(imx_swm *s, double *h, double *u) {
   if (!s) return imx::set_error(IMX_EINVAL, "imx_swm_get_state: NULL handle");
-  if (!s->fast) return imx::download_state<double>(s, h, u, s->rh, s->ru);
-  if (s->single) return imx::download_state<float>(s, h, u, (float *)s->h0, (float *)s->u0);
-  return imx::download_state<double>(s, h, u, (double *)s->h0, (double *)s->u0);
+  if (!s->fast) return imx::get_state<double>(s, h, u, s->rh, s->ru);
+  if (s->single) return imx::get_state<float>(s, h, u, (float *)s->h0, (float *)s->u0);
+  return imx::get_state<double>(s, h, u, (double *)s->h0, (double *)s->u0);
 }
 
 int imx_swm_tendency(imx_swm *s, const double *h, const double *u, double *masseq,
                      double *momeq) {
   if (!s || !h || !u || !masseq || !momeq)
     return imx::set_error(IMX_EINVAL, "imx_swm_tendency: NULL argument");
+  const int nv = s->nv, ne = s->ne;
+  const char *me = "imx_swm_tendency";
   int rc;
-  std::vector<double> mb(s->nv), fb(s->NE);
   if (!s->fast) {
-    if ((rc = imx::upload_state<double>(s, h, u, s->rhn, s->run))) return rc;
+    if ((rc = imx::upload_state<double>(s, h, u, s->rhn, s->run, 0, nv, 0, ne))) return rc;
     imx::launch_ref_tendency(s, s->rhn, s->run, s->massf, s->momf);
-    if ((rc = imx::check_flag(s, "imx_swm_tendency"))) return rc;
-    HIPTRY(hipMemcpy(mb.data(), s->massf, s->nv * sizeof(double), hipMemcpyDeviceToHost), "tendency");
-    HIPTRY(hipMemcpy(fb.data(), s->momf, s->NE * sizeof(double), hipMemcpyDeviceToHost), "tendency");
+    if ((rc = imx::download_state<double>(s, masseq, momeq, s->massf, s->momf, 0.0, 0, nv, 0, ne, me))) return rc;
   } else {
     imx::set_href(s, h);
     if (s->single) {
-      if ((rc = imx::upload_state<float>(s, h, u, (float *)s->hA, (float *)s->uA))) return rc;
+      if ((rc = imx::upload_state<float>(s, h, u, (float *)s->hA, (float *)s->uA, 0, nv, 0, ne))) return rc;
       imx::launch_fast_stage<float>(s, -1, (const float *)s->hA, (const float *)s->uA, nullptr,
                                     nullptr, nullptr);
-      if ((rc = imx::check_flag(s, "imx_swm_tendency"))) return rc;
-      std::vector<float> ff(s->NE);
-      HIPTRY(hipMemcpy(ff.data(), s->du_out, s->NE * sizeof(float), hipMemcpyDeviceToHost), "tendency");
-      for (int l = 0; l < s->NE; ++l) fb[l] = ff[l];
+      rc = imx::download_state<double>(s, masseq, momeq, s->dh_out, (const float *)s->du_out, 0.0, 0, nv, 0, ne, me);
     } else {
-      if ((rc = imx::upload_state<double>(s, h, u, (double *)s->hA, (double *)s->uA))) return rc;
+      if ((rc = imx::upload_state<double>(s, h, u, (double *)s->hA, (double *)s->uA, 0, nv, 0, ne))) return rc;
       imx::launch_fast_stage<double>(s, -1, (const double *)s->hA, (const double *)s->uA, nullptr,
                                      nullptr, nullptr);
-      if ((rc = imx::check_flag(s, "imx_swm_tendency"))) return rc;
-      HIPTRY(hipMemcpy(fb.data(), s->du_out, s->NE * sizeof(double), hipMemcpyDeviceToHost), "tendency");
+      rc = imx::download_state<double>(s, masseq, momeq, s->dh_out, (const double *)s->du_out, 0.0, 0, nv, 0, ne, me);
     }
-    HIPTRY(hipMemcpy(mb.data(), s->dh_out, s->nv * sizeof(double), hipMemcpyDeviceToHost), "tendency");
+    if (rc) return rc;
   }
-  for (int i = 0; i < s->nv; ++i) masseq[i] = mb[s->lay.cell_new[i]];
-  for (int l = 0; l < s->ne; ++l) momeq[l] = fb[s->lay.edge_new[l]];
   return IMX_OK;
 }
 
@@ -3970,6 +4047,8 @@ void imx_swm_destroy(imx_swm *s) {
   imx::drop_graph(s);
   imx::stage_free(s);
   s->A.release();
+  if (s->hstage) (void)hipHostFree(s->hstage);
+  if (s->flag) (void)hipHostFree(s->flag);
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
   if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -4000,14 +4079,8 @@ namespace imx {
 template <typename T>
 static int ens_upload(imx_ens *E, int i, const double *h, const double *u) {
   imx_swm *s = E->s;
-  const int nc = E->nv[i], c0 = E->c0[i];
-  std::vector<T> hb(nc, (T)0), ub((size_t)3 * nc, (T)0);
-  for (int k = 0; k < nc; ++k) hb[s->lay.cell_new[E->cv0[i] + k] - c0] = (T)(h[k] - s->href);
-  for (int l = 0; l < E->ne[i]; ++l) ub[s->lay.edge_new[E->ce0[i] + l] - 3 * c0] = (T)u[l];
-  HIPTRY(hipMemcpyAsync((T *)s->h0 + c0, hb.data(), hb.size() * sizeof(T), hipMemcpyHostToDevice,
-                        s->stream), "imx_ens_set_state");
-  HIPTRY(hipMemcpyAsync((T *)s->u0 + (size_t)3 * c0, ub.data(), ub.size() * sizeof(T),
-                        hipMemcpyHostToDevice, s->stream), "imx_ens_set_state");
+  const int rc = upload_state<T>(s, h, u, (T *)s->h0, (T *)s->u0, E->cv0[i], E->nv[i], E->ce0[i], E->ne[i]);
+  if (rc) return rc;
   HIPTRY(hipStreamSynchronize(s->stream), "imx_ens_set_state");
   return IMX_OK;
 }
@@ -4015,18 +4088,8 @@ static int ens_upload(imx_ens *E, int i, const double *h, const double *u) {
 template <typename T>
 static int ens_download(imx_ens *E, int i, double *h, double *u) {
   imx_swm *s = E->s;
-  const int nc = E->nv[i], c0 = E->c0[i];
-  std::vector<T> hb(nc), ub((size_t)3 * nc);
-  HIPTRY(hipMemcpyAsync(hb.data(), (const T *)s->h0 + c0, hb.size() * sizeof(T),
-                        hipMemcpyDeviceToHost, s->stream), "imx_ens_get_state");
-  HIPTRY(hipMemcpyAsync(ub.data(), (const T *)s->u0 + (size_t)3 * c0, ub.size() * sizeof(T),
-                        hipMemcpyDeviceToHost, s->stream), "imx_ens_get_state");
-  HIPTRY(hipStreamSynchronize(s->stream), "imx_ens_get_state");
-  if (h)
-    for (int k = 0; k < nc; ++k) h[k] = (double)hb[s->lay.cell_new[E->cv0[i] + k] - c0] + s->href;
-  if (u)
-    for (int l = 0; l < E->ne[i]; ++l) u[l] = (double)ub[s->lay.edge_new[E->ce0[i] + l] - 3 * c0];
-  return IMX_OK;
+  return download_state<T>(s, h, u, (const T *)s->h0, (const T *)s->u0, s->href, E->cv0[i], E->nv[i], E->ce0[i],
+                           E->ne[i]);
 }
 
 }  // namespace imx
