@@ -19,13 +19,16 @@
 // 1.4 times the work of the mesh), with the same expressions on the same
 // inputs, so a result does not depend on how the mesh is cut into blocks.
 //
-// Measured (us per RK4 step, three passes -> this): glevel 5 FP32 43 -> 32,
-// glevel 7 78 -> 58, FP64 105 -> 85, glevel 8 191 -> 127, FP64 380 -> 241,
-// glevel 9 948 -> 590. The three passes moved 385 B per cell and stage, 252
-// MB at glevel 8; this moves about 245. What was worth most is the order of
-// the loads: with each phase loading its own tables a block waited five
-// memory latencies in a row and a glevel-8 stage took 45 us; with every load
-// issued before the first barrier it takes 32.
+// Measured (us per RK4 step, three passes -> this; 16-step graphs on both
+// sides would take 6 off the first figures): glevel 5 FP32 43 -> 19.7, glevel
+// 7 78 -> 43.5, FP64 105 -> 68, glevel 8 191 -> 110.6, FP64 380 -> 211,
+// glevel 9 948 -> 547. The three passes moved 252 MB per stage at glevel 8;
+// this moves 181 (FETCH_SIZE x 2 + WRITE_SIZE) at 6.6 TB/s, against 7.8 for a
+// copy that stays in the last-level cache. What bounds it there: the vector
+// units are busy 47 % of the time (693 instructions a wave), memory most of
+// the rest. What was worth most: every load issued before the first barrier
+// (with each phase loading its own tables a glevel-8 stage took 45 us instead
+// of 32), then fewer vector instructions (32 -> 27.6).
 //
 // Blocks are cut greedily along the curve so that |C| fills the block's
 // threads and |L| its LDS. Ids inside a block are 10-bit, which packs the
@@ -48,13 +51,13 @@
 #define HTR_GUARD (1.1920928955078125e-07 / 100000.0)
 // local ids are 10-bit
 #define LID 1023
-// topology word of a cell slot: neighbour | OWN (the cell owns the edge) |
-// K (which of its owner's edges, 2 bits) | signs of the flux and of the
-// Coriolis term
+// topology half word of a cell slot: neighbour | OWN (the cell owns the edge)
+// | K (which of its owner's edges, 2 bits) | signs of the Coriolis term and,
+// in the top bit, of the flux
 #define SB_OWN 10
 #define SB_K 11
-#define SB_TTG 13
 #define SB_TNR 14
+#define SB_TTG 15
 // fourth topology word: owner of triangle j (0 cell, 1 nb_j, 2 nb_j+1; 2
 // bits at 2j), k of triangle j (bit 12+j), hexagon (bit 18)
 #define SW_KT 12
@@ -80,7 +83,8 @@ struct alignas(4 * sizeof(T)) Quad {
   T x, y, z, w;
 };
 
-// caps of a block of nt threads: cells of C, local cells, triangles
+// caps of a block of nt threads: local cells (and at most nt past the own
+// ones, at most nt in C), triangles
 static constexpr int cap_l(int nt) { return nt + nt / 2 + 64; }
 static constexpr int cap_t(int nt) { return 2 * nt + nt / 2 + 64; }
 
@@ -88,7 +92,7 @@ struct Stage {
   int nt = 0, nblk = 0, remap = 1;
   Alloc A;
   int4 *head = nullptr;      // [nblk] first own cell, own cells, |C|, |L| | triangles << 16
-  int32_t *halo = nullptr;   // [nblk][cap_l] cells of the local ids past the own ones
+  int32_t *halo = nullptr;   // [nblk][nt] cells of the local ids past the own ones
   uint4 *topo = nullptr;     // [nblk][nt]
   void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~
   void *eld = nullptr;       // [NE] Pair: length, dual length
@@ -117,17 +121,47 @@ struct StageArgs {
   T *hout, *uout, *acch, *accu, *q, *du_out;
   double *dh_out;
   int *flag;
-  double href, dt;
-  T grav, inv_a;
+  double href, ca, cb;  // the stage's step and its weight in the sum (ensembles: per cell)
+  T grav, inv_a, cat, cbt;
   int nblk, remap, use_pv, flin, zero_mom;
   int whole;  // the third stage: its state is a whole step away
 };
 
-__device__ __forceinline__ void kadd(double &s, double &c, double x) {
+// Compensated summation: c gathers the exact rounding errors of s (Knuth's
+// two-sum, which needs no branch on the larger operand).
+__device__ __forceinline__ void two_sum(double &s, double &c, double x) {
   const double t = s + x;
-  if (fabs(s) >= fabs(x)) c += (s - t) + x;
-  else c += (x - t) + s;
+  const double y = t - s;
+  c += (s - (t - y)) + (x - y);
   s = t;
+}
+
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// x with its sign changed when bit 31 of m is set (the other bits are 0)
+__device__ __forceinline__ float flip(float x, uint32_t m) { return __uint_as_float(__float_as_uint(x) ^ m); }
+__device__ __forceinline__ double flip(double x, uint32_t m) {
+  return __longlong_as_double(__double_as_longlong(x) ^ ((long long)m << 32));
+}
+// 1/x to about an ulp: the hardware's estimate and Newton steps
+__device__ __forceinline__ float recip(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+__device__ __forceinline__ double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+// element i of a table, by a 32-bit byte offset (tables are under 4 GiB; see
+// stage_build): one scalar base and one vector register for the address
+template <typename X>
+__device__ __forceinline__ X at(const X *p, uint32_t i) {
+  return *(const X *)((const char *)p + (uint32_t)(i * (uint32_t)sizeof(X)));
+}
+template <typename X>
+__device__ __forceinline__ void put(X *p, uint32_t i, X v) {
+  *(X *)((char *)p + (uint32_t)(i * (uint32_t)sizeof(X))) = v;
 }
 
 // MODE: 0 the first RK stage, 1 the second and third, 2 the last, 3 a
@@ -135,10 +169,10 @@ __device__ __forceinline__ void kadd(double &s, double &c, double x) {
 template <typename T, int NT, int MODE>
 __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
   constexpr int LC = cap_l(NT), TC = cap_t(NT);
-  constexpr int NH = (LC + NT - 1) / NT, NR = (TC + NT - 1) / NT;
-  __shared__ Pair<T> sU[3 * LC];  // u, dual length
-  __shared__ T sA[3 * LC];        // u l
-  __shared__ T sH[LC], sQ[2 * LC], sPhi[NT], sP[3 * NT], sPo[3 * NT];
+  constexpr int NR = (TC + NT - 1) / NT;
+  __shared__ T sU[3 * LC], sD[3 * LC], sA[3 * LC];  // u, dual length, u l
+  __shared__ T sH[LC], sQ[2 * LC], sPhi[NT], sPP[6 * NT];
+  T *sP = sPP, *sPo = sPP + 3 * NT;  // partials of the own edges' owners and other cells
   int b = blockIdx.x;
   if (a.remap) b = (b % NXCD) * (gridDim.x / NXCD) + b / NXCD;
   if (b >= a.nblk) return;
@@ -148,63 +182,63 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
   // whose places the first ones give; the phases then run out of registers
   // and LDS. Lanes past a list read its last entry instead of branching
   // around the load.
-  const int32_t *halo = a.halo + (size_t)b * LC;
-  int hcell[NH];
-#pragma unroll
-  for (int r = 0; r < NH; ++r) hcell[r] = halo[min(tid + r * NT, LC - 1)];
-  const uint4 tp = a.topo[(size_t)b * NT + tid];
-  const Quad<T> w0 = a.cw[((size_t)b * 2) * NT + tid], w1 = a.cw[((size_t)b * 2 + 1) * NT + tid];
+  const int32_t *halo = a.halo + (size_t)b * NT;
+  const int hcell = at(halo, tid);
+  const uint4 tp = at(a.topo + (size_t)b * NT, tid);
+  const Quad<T> *cw = a.cw + (size_t)b * 2 * NT;
+  const Quad<T> w0 = at(cw, tid), w1 = at(cw + NT, tid);
   const int4 hd = a.head[b];
   const int own0 = hd.x, nown = hd.y, nC = hd.z, nL = hd.w & 0xFFFF, nTri = hd.w >> 16;
   const int nh = nL - nown;
   const T href = (T)a.href;
-  const int oc = own0 + min(tid, nown - 1);
+  const int oc = min(tid, nown - 1);
 
-  T hh[NH], hu[NH][3];
-  Pair<T> hl[NH][3];
+  const T hh = at(a.hs, hcell);
+  T hu[3];
+  Pair<T> hl[3];
 #pragma unroll
-  for (int r = 0; r < NH; ++r) {
-    hh[r] = a.hs[hcell[r]];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      hu[r][k] = a.us[3 * hcell[r] + k];
-      hl[r][k] = a.eld[3 * hcell[r] + k];
-    }
+  for (int k = 0; k < 3; ++k) {
+    hu[k] = at(a.us, 3 * hcell + k);
+    hl[k] = at(a.eld, 3 * hcell + k);
   }
-  const T ho = a.hs[oc];
+  const T ho = at(a.hs + own0, oc);
   T eu[3];
   Pair<T> el[3];
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
-    const int e = 3 * own0 + min(tid + r * NT, 3 * nown - 1);
-    eu[r] = a.us[e];
-    el[r] = a.eld[e];
+    const int e = min(tid + r * NT, 3 * nown - 1);
+    eu[r] = at(a.us + 3 * (size_t)own0, e);
+    el[r] = at(a.eld + 3 * (size_t)own0, e);
   }
+  // the state first: P0 waits for it alone
+  __builtin_amdgcn_sched_barrier(0);
   uint32_t tv[NR];
   int tsl[NR];
   Quad<T> tk[NR];
   T tf[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
-    const size_t t = (size_t)b * TC + min(tid + r * NT, nTri - 1);
-    tv[r] = a.tv[t];
-    tsl[r] = a.tslot[t];
-    tk[r] = a.tk[t];
-    tf[r] = a.tf[t];
+    const int t = min(tid + r * NT, nTri - 1);
+    tv[r] = at(a.tv + (size_t)b * TC, t);
+    tsl[r] = at(a.tslot + (size_t)b * TC, t);
+    tk[r] = at(a.tk + (size_t)b * TC, t);
+    tf[r] = at(a.tf + (size_t)b * TC, t);
   }
   // the RK operands of the own cells and edges
-  const double iaa = a.iaa[oc];
+  __builtin_amdgcn_sched_barrier(0);
+  const double iaa = at(a.iaa + own0, oc);
   T y0 = (T)0, ac = (T)0, v0[3], av[3];
   uint32_t ow[3];
-  if (MODE != 3) y0 = a.h0[oc];
-  if (MODE == 1 || MODE == 2) ac = a.acch[oc];
+  if (MODE != 3) y0 = at(a.h0 + own0, oc);
+  if (MODE == 1 || MODE == 2) ac = at((const T *)a.acch + own0, oc);
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
-    const int e = 3 * own0 + min(tid + r * NT, 3 * nown - 1);
-    ow[r] = a.oth[e];
-    if (MODE != 3) v0[r] = a.u0[e];
-    if (MODE == 1 || MODE == 2) av[r] = a.accu[e];
+    const int e = min(tid + r * NT, 3 * nown - 1);
+    ow[r] = at(a.oth + 3 * (size_t)own0, e);
+    if (MODE != 3) v0[r] = at(a.u0 + 3 * (size_t)own0, e);
+    if (MODE == 1 || MODE == 2) av[r] = at((const T *)a.accu + 3 * (size_t)own0, e);
   }
+  __builtin_amdgcn_sched_barrier(0);
 
   // P0: the local state to LDS
 #pragma unroll
@@ -213,22 +247,22 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     asm volatile("" : "+v"(eu[r]), "+v"(el[r].x), "+v"(el[r].y));
     const int i = tid + r * NT;
     if (i < 3 * nown) {
-      sU[i] = Pair<T>{eu[r], el[r].y};
+      sU[i] = eu[r];
+      sD[i] = el[r].y;
       sA[i] = eu[r] * el[r].x;
     }
   }
   if (tid < nown) sH[tid] = ho;
+  if (tid < nh) {
+    const int lc = nown + tid;
+    sH[lc] = hh;
 #pragma unroll
-  for (int r = 0; r < NH; ++r)
-    if (tid + r * NT < nh) {
-      const int lc = nown + tid + r * NT;
-      sH[lc] = hh[r];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        sU[3 * lc + k] = Pair<T>{hu[r][k], hl[r][k].y};
-        sA[3 * lc + k] = hu[r][k] * hl[r][k].x;
-      }
+    for (int k = 0; k < 3; ++k) {
+      sU[3 * lc + k] = hu[k];
+      sD[3 * lc + k] = hl[k].y;
+      sA[3 * lc + k] = hu[k] * hl[k].x;
     }
+  }
   __syncthreads();
 
   // P1: PV at triangles
@@ -245,10 +279,9 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     const int e1 = 3 * (((eb >> 3) & 1) ? va : vb) + ((eb >> 4) & 3);
     const int e2 = 3 * (((eb >> 6) & 1) ? vb : o) + ((eb >> 7) & 3);
     if (!a.flin) {
-      const T c0 = sA[e0], c1 = sA[e1], c2 = sA[e2];
-      T z = (eb >> 9) & 1 ? -c0 : c0;
-      z += (eb >> 10) & 1 ? -c1 : c1;
-      z += (eb >> 11) & 1 ? -c2 : c2;
+      T z = flip(sA[e0], (v << 2) & 0x80000000u);
+      z += flip(sA[e1], (v << 1) & 0x80000000u);
+      z += flip(sA[e2], v & 0x80000000u);
       eta += z * k.w;
     }
     T hsum = k.x * sH[o];
@@ -262,7 +295,7 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     }
     sQ[sl] = qq;
     // the field a caller may read: the last stage's, or a tendency's
-    if (MODE >= 2 && o < nown) a.q[2 * own0 + sl] = qq;
+    if (MODE >= 2 && o < nown) put(a.q + 2 * (size_t)own0, sl, qq);
   }
   __syncthreads();
 
@@ -274,9 +307,10 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     uint32_t f[MX];
 #pragma unroll
     for (int j = 0; j < MX; ++j) {
-      f[j] = wj[j / 2] >> (16 * (j % 2));
-      nb[j] = f[j] & LID;
-      ed[j] = 3 * (((f[j] >> SB_OWN) & 1) ? tid : nb[j]) + ((f[j] >> SB_K) & 3);
+      // the slot's half word in the upper half: signs by plain masks
+      f[j] = j % 2 ? wj[j / 2] : wj[j / 2] << 16;
+      nb[j] = (f[j] >> 16) & LID;
+      ed[j] = 3 * (((f[j] >> (16 + SB_OWN)) & 1) ? tid : nb[j]) + ((f[j] >> (16 + SB_K)) & 3);
     }
     const T hc = sH[tid];
     double dv = 0.0, dvc = 0.0;
@@ -285,15 +319,20 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
 #pragma unroll
     for (int j = 0; j < MX; ++j) {
       const bool valid = (j < MX - 1) || hex;
-      const Pair<T> u = sU[ed[j]];
+      const T u = sU[ed[j]], dl = sD[ed[j]];
       // both cells of an edge form the same product, so the mass flux
       // cancels exactly between them
-      double g = (double)u.x * (a.href + 0.5 * ((double)hc + (double)sH[nb[j]])) * (double)u.y;
-      if ((f[j] >> SB_TTG) & 1) g = -g;
-      if (!valid) g = 0.0;
-      kadd(dv, dvc, g);
+      double g = (double)flip(u, f[j] & 0x80000000u) *
+                 fma_(0.5, (double)hc + (double)sH[nb[j]], a.href) * (double)dl;
+      T k = sA[ed[j]] * (u * dl);
+      if (!valid) {
+        g = 0.0;
+        k = (T)0;
+      }
+      if (j == 0) dv = g;
+      else two_sum(dv, dvc, g);
       G[j] = (T)g;
-      ke += valid ? sA[ed[j]] * (u.x * u.y) : (T)0;
+      ke += k;
     }
     T qt[MX];
 #pragma unroll
@@ -305,21 +344,24 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     // a pentagon's padded slot may name a triangle that is not local
     if (!hex) qt[MX - 1] = (T)0;
     T pot = a.grav * hc;
-    if (a.gb) pot += a.gb[tid < nown ? own0 + tid : halo[tid - nown]];
+    if (a.gb) pot += at(a.gb, tid < nown ? own0 + tid : halo[tid - nown]);
     sPhi[tid] = (pot + ke * w1.z) * a.inv_a;
     if (tid < nown) {
-      const int c = own0 + tid;
       const double dh = -(dv + dvc) * iaa;
-      const double dt = a.dtc ? a.dtc[c] : a.dt;
+      // the step over the stage's share of it (1, 2 halves) and over 6 or 3
+      double ca = a.ca, cb = a.cb;
+      if (a.dtc) {
+        const double dt = at(a.dtc + own0, tid);
+        ca = a.whole ? dt : 0.5 * dt;
+        cb = MODE == 1 ? dt / 3.0 : dt / 6.0;
+      }
       if (MODE == 3) {
-        a.dh_out[c] = dh;
+        put(a.dh_out + own0, tid, dh);
       } else if (MODE < 2) {
-        const double ca = a.whole ? dt : 0.5 * dt;
-        const double cb = MODE == 0 ? dt / 6.0 : dt / 3.0;
-        a.hout[c] = (T)((double)y0 + ca * dh);
-        a.acch[c] = MODE == 0 ? (T)(cb * dh) : (T)((double)ac + cb * dh);
+        put(a.hout + own0, tid, (T)((double)y0 + ca * dh));
+        put(a.acch + own0, tid, MODE == 0 ? (T)(cb * dh) : (T)((double)ac + cb * dh));
       } else {
-        a.hout[c] = (T)((double)y0 + ((double)ac + (dt / 6.0) * dh));
+        put(a.hout + own0, tid, (T)((double)y0 + ((double)ac + cb * dh)));
       }
     }
     // PV at the cell's edges: edge j lies between ring triangles j-1 and j
@@ -328,31 +370,31 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
 #pragma unroll
     for (int j = 1; j < MX; ++j) qe[j] = (T)0.5 * (qt[j - 1] + qt[j]);
     // TRiSK weights from prefix sums of the kite areas:
-    // w(i,j) = S_j - S_i - 1/2 (j>i), tot - S_i + S_j - 1/2 (j<i), w(i,i) = 0
+    // w(i,j) = S_j - S_i - 1/2 (j>i), S_6 - S_i + S_j - 1/2 (j<i), w(i,i) = 0
     const T R[MX] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
     T S[MX + 1];
     S[0] = (T)0;
 #pragma unroll
     for (int j = 0; j < MX; ++j) S[j + 1] = S[j] + R[j];
-    const T tot = S[MX];
+    const T rest = S[MX] - (T)0.5;
+    // P_i = sum_j G_j (q_i + q_j)/2 w(i,j) = (q_i sum_j G_j w + sum_j G_j q_j w)/2
+    T H[MX];
+#pragma unroll
+    for (int j = 0; j < MX; ++j) H[j] = G[j] * qe[j];
 #pragma unroll
     for (int i = 0; i < MX; ++i) {
-      T acc = (T)0;
+      T x = (T)0, y = (T)0;
 #pragma unroll
       for (int j = 0; j < MX; ++j)
         if (j != i) {
-          const T w = ((j > i) ? (S[j] - S[i]) : (tot - S[i] + S[j])) - (T)0.5;
-          acc += G[j] * (qe[i] + qe[j]) * w;
+          const T w = (j > i) ? (S[j] - S[i]) - (T)0.5 : rest - (S[i] - S[j]);
+          x = fma_(G[j], w, x);
+          y = fma_(H[j], w, y);
         }
-      T P = (T)0.5 * acc;
-      if ((f[i] >> SB_TNR) & 1) P = -P;
-      if (i < MX - 1 || hex) {
-        if ((f[i] >> SB_OWN) & 1) {
-          if (tid < nown) sP[ed[i]] = P;
-        } else if (nb[i] < nown) {
-          sPo[ed[i]] = P;
-        }
-      }
+      const T P = flip((T)0.5 * fma_(qe[i], x, y), (f[i] << 1) & 0x80000000u);
+      // for the block's own edges: by its owner or by its other cell
+      T *to = (f[i] >> (16 + SB_OWN)) & 1 ? sP : sPo;
+      if (ed[i] < 3 * nown && (i < MX - 1 || hex)) to[ed[i]] = P;
     }
   }
   __syncthreads();
@@ -362,24 +404,26 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
   for (int r = 0; r < 3; ++r) {
     const int i = tid + r * NT;
     if (i >= 3 * nown) continue;
-    const int e = 3 * own0 + i;
     const uint32_t w = ow[r];
     if (w == 0xFFFFu) continue;
     const int o = i / 3, c2 = w & LID;
     const bool own_v2 = (w >> SB_OWN) & 1;
     const T d = own_v2 ? sPhi[o] - sPhi[c2] : sPhi[c2] - sPhi[o];
-    T du = -(d + (sP[i] + sPo[i])) / el[r].x;
+    T du = -(d + (sP[i] + sPo[i])) * recip(el[r].x);
     if (a.zero_mom) du = (T)0;
-    const T dt = a.dte ? a.dte[e] : (T)a.dt;
+    T ca = a.cat, cb = a.cbt;
+    if (a.dte) {
+      const T dt = at(a.dte + 3 * (size_t)own0, i);
+      ca = a.whole ? dt : (T)0.5 * dt;
+      cb = MODE == 1 ? dt / (T)3 : dt / (T)6;
+    }
     if (MODE == 3) {
-      a.du_out[e] = du;
+      put(a.du_out + 3 * (size_t)own0, i, du);
     } else if (MODE < 2) {
-      const T ca = a.whole ? dt : (T)0.5 * dt;
-      const T cb = MODE == 0 ? dt / (T)6 : dt / (T)3;
-      a.uout[e] = v0[r] + ca * du;
-      a.accu[e] = MODE == 0 ? cb * du : av[r] + cb * du;
+      put(a.uout + 3 * (size_t)own0, i, v0[r] + ca * du);
+      put(a.accu + 3 * (size_t)own0, i, MODE == 0 ? cb * du : av[r] + cb * du);
     } else {
-      a.uout[e] = v0[r] + (av[r] + (dt / (T)6) * du);
+      put(a.uout + 3 * (size_t)own0, i, v0[r] + (av[r] + cb * du));
     }
   }
 }
@@ -432,11 +476,11 @@ struct LocalSet {
 };
 struct LocalSets {
   LocalSet L, tri;
-  int nC = 0;
+  int nC = 0, own = 0;
   void clear() {
     L.clear();
     tri.clear();
-    nC = 0;
+    nC = own = 0;
   }
 };
 
@@ -478,7 +522,9 @@ static int build(imx_swm *s, int nt) {
     const int n = bA[c] & 7;
     for (int j = 0; j < n; ++j)
       if ((bA[c] >> (BA_OWN + j)) & 1) in_c(nbr[(size_t)j * nv + c]);
-    return w.nC <= nt && (int)w.L.keys.size() <= LC && (int)w.tri.keys.size() <= TC;
+    ++w.own;
+    const int nL = (int)w.L.keys.size();
+    return w.nC <= nt && nL <= LC && nL - w.own <= nt && (int)w.tri.keys.size() <= TC;
   };
 
   // cut the curve into at most 16 segments, one host thread each, and every
@@ -524,9 +570,11 @@ static int build(imx_swm *s, int nt) {
   for (char ok : fine)
     if (!ok) return IMX_OK;
   if (nblk > 1 && (int64_t)nblk * nt > (int64_t)3 * nv) return IMX_OK;
+  // the kernel addresses its tables by 32-bit byte offsets
+  if ((uint64_t)NE * sizeof(Pair<T>) >> 32) return IMX_OK;
 
   std::vector<int4> head(nblk);
-  std::vector<int32_t> halo((size_t)nblk * LC, 0);
+  std::vector<int32_t> halo((size_t)nblk * nt, 0);
   std::vector<uint4> topo((size_t)nblk * nt, uint4{0, 0, 0, 0});
   std::vector<Quad<T>> cw((size_t)nblk * 2 * nt, Quad<T>{0, 0, 0, 0}), tk((size_t)nblk * TC, Quad<T>{0, 0, 0, 0});
   std::vector<Pair<T>> eld(NE);
@@ -556,7 +604,7 @@ static int build(imx_swm *s, int nt) {
       const int nL = (int)cells.size(), nC = w.nC;
       for (int k = 0; k < nL; ++k) w.L.at(cells[k]).id = k;
       auto id = [&](int k) { return (uint32_t)w.L.at(k).id; };
-      for (int k = nown; k < nL; ++k) halo[(size_t)b * LC + k - nown] = cells[k];
+      for (int k = nown; k < nL; ++k) halo[(size_t)b * nt + k - nown] = cells[k];
       head[b] = int4{o0, nown, nC, nL | (int)tris.size() << 16};
       for (int k = 0; k < nC; ++k) {
         const int c = cells[k];
@@ -670,7 +718,12 @@ void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *u
   a.dh_out = s->dh_out;
   a.flag = s->flag;
   a.href = s->href;
-  a.dt = s->o.dt;
+  const double dt = s->o.dt;
+  const T dtt = (T)dt;
+  a.ca = stage == 2 ? dt : 0.5 * dt;
+  a.cb = stage == 1 || stage == 2 ? dt / 3.0 : dt / 6.0;
+  a.cat = stage == 2 ? dtt : (T)0.5 * dtt;
+  a.cbt = stage == 1 || stage == 2 ? dtt / (T)3 : dtt / (T)6;
   a.grav = (T)s->o.grav;
   a.inv_a = (T)(1.0 / s->o.erad);
   a.nblk = g.nblk;

@@ -2562,18 +2562,27 @@ static int validate_desc(const imx_mesh_desc &d) {
   return IMX_OK;
 }
 
-// Threads of a block of the one-launch stage: small blocks until there are
-// enough cells to give every CU one (glevel 5, FP32, per step: 128 threads
-// 32.0 us, 256 36 us), then 256, where the rim is 1.3 times the work and five
-// blocks fit a CU (glevel 8: 127 us against 131 with 128 and 129 with 512).
-static int stage_default(const imx_swm *s) { return s->nv < 30000 ? 128 : 256; }
+// Threads of a block of the one-launch stage and whether its blocks are
+// remapped so that each XCD walks its own stretch of the curve. us per stage,
+// launch included (block threads, remap):
+//   glevel 5 FP32   128: 7.8    256: 8.3    512: 9.1
+//   glevel 6 FP64   128: 9.8    256: 9.2
+//   glevel 8 FP32   128: 33.1   256: 30.1   512: 31.6   256, no remap: 36.9
+//   glevel 9 FP32   128: 162    256: 142    512: 137    512, no remap: 137
+//   glevel 9 FP64   128: 278    256: 254                256, no remap: 245
+// Small blocks until there is one of the larger ones for every other CU;
+// beyond the last-level cache (some 250 B per FP32 cell) the least rim is
+// best, and eight separate stretches of memory no longer pay.
+static bool stage_large(const imx_swm *s) { return (size_t)s->nv * (s->single ? 4 : 8) > ((size_t)8 << 20); }
+static int stage_default(const imx_swm *s) { return s->nv < 30000 ? 128 : stage_large(s) && s->single ? 512 : 256; }
 
 // The stage tables follow the handle's staggering, triangle weights and
 // Coriolis parameter; they are made again when the plain scheme is back.
 static int stage_refresh(imx_swm *s) {
   s->stg_stale = s->stg != nullptr;
   if (!s->stg_stale || !plain_scheme(s)) return IMX_OK;
-  const int rc = stage_build(s, stage_threads(s));
+  const int remap = stage_remap(s), rc = stage_build(s, stage_threads(s));
+  stage_set_remap(s, remap);
   s->stg_stale = false;
   return rc;
 }
@@ -2765,7 +2774,11 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
     }
   }
   HIPTRY(hipDeviceSynchronize(), "imx_swm_create");
-  return s->fast ? stage_build(s, stage_default(s)) : IMX_OK;
+  if (s->fast) {
+    if ((rc = stage_build(s, stage_default(s)))) return rc;
+    stage_set_remap(s, stage_large(s) ? 0 : 1);
+  }
+  return IMX_OK;
 }
 
 static int check_flag(imx_swm *s, const char *what) {
@@ -2985,7 +2998,7 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   if (stage_on(s)) {
     // one launch per stage: block threads (which cut the mesh anew) x remap
     double best = 1e30;
-    int bb = stage_threads(s), br = 1;
+    int bb = stage_threads(s), br = stage_remap(s);
     for (int bs : {128, 256, 512}) {
       if (bs == 512 && !s->single) continue;  // over 64 KB of LDS
       if ((rc = stage_build(s, bs))) break;
