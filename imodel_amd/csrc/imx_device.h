@@ -296,10 +296,9 @@ struct imx_mlp {
   float *P = nullptr, *M = nullptr, *V = nullptr, *G = nullptr, *part = nullptr, *lossp = nullptr;
   short *Ff = nullptr, *Fb = nullptr;  // K16 fragments of the training kernels
   short *Ff32 = nullptr;                // K32 fragments of the inference kernel
-  short *X = nullptr, *AT = nullptr, *DZT = nullptr;
+  short *X = nullptr;
   float *T = nullptr, *w = nullptr, *Y = nullptr, *Xf = nullptr;
   int64_t cap = 0;  // edges the scratch holds
-  int nsplit = 16;
   int64_t t = 0;    // optimiser step
   hipStream_t stream = nullptr;
 };
@@ -307,8 +306,9 @@ struct imx_mlp {
 namespace imx {
 int mlp_reserve(imx_mlp *m, int64_t n);
 int mlp_forward_dev(imx_mlp *m, int64_t n, const short *X, float *Y, hipStream_t st);
-int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int apply, double *loss,
+int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int apply, float *loss_part,
                   int gmask);
+int mlp_loss(imx_mlp *m, int64_t n, const float *loss_part, int passes, double *loss);
 // one fused RK4 step of a FAST handle, enqueued on its stream (no graph)
 void swm_launch_step(imx_swm *s);
 // waits for the handle's stream; IMX_ESTATE if a step met a vanishing depth

@@ -39,6 +39,7 @@
 #define LTPB 256
 #define LPART 1024  // blocks of the correction-norm pass
 #define SREC 32    // words per edge stencil record (128 bytes)
+static constexpr int kLossSteps = 16;  // a fit returns the mean loss of its last steps
 
 struct imx_learn {
   imx_swm *s = nullptr;
@@ -59,7 +60,8 @@ struct imx_learn {
   double *part = nullptr;   // [LPART] partial sums of the correction norm
   double *rms = nullptr;    // [1] correction RMS of the last step
   double *bound = nullptr;  // [2] RMS bound, limiter mode (IMX_LIMIT_*)
-  double *lh = nullptr;     // [1] h loss of the last training epoch
+  double *lh = nullptr;     // [kLossSteps] h losses of a fit's last steps
+  float *lossu = nullptr;   // [kLossSteps][(NE + 63) / 64] their u loss partials
   int *nfb = nullptr;       // [1] limited steps since the counter was cleared
   imx::StepGraphs graphs;
   const short *gX = nullptr;  // MLP input buffer the graph was captured with
@@ -204,6 +206,7 @@ __global__ __launch_bounds__(1024) void learn_norm2(int na, const float *__restr
     for (int e = threadIdx.x; e < na; e += 1024) s += (double)w[e] * (double)a[sa * e] * (double)a[sa * e];
   double t = 0.0;
   if (b)
+#pragma unroll 8
     for (int c = threadIdx.x; c < nb; c += 1024) t += (double)b[c] * (double)b[c];
   s += sb * t;
   __shared__ double red[1024];
@@ -493,7 +496,8 @@ int imx_learn_create(imx_swm *s, imx_mlp *m, const imx_mesh_desc *d, imx_learn *
   L->part = A.get<double>(LPART);
   L->rms = A.get<double>(1);
   L->bound = A.put(std::vector<double>{1e300, (double)IMX_LIMIT_FALLBACK});
-  L->lh = A.get<double>(1);
+  L->lh = A.get<double>(kLossSteps);
+  L->lossu = A.get<float>((size_t)kLossSteps * ((NE + 63) / 64));
   L->nfb = A.get<int>(1);
   if (A.err != hipSuccess) {
     int rc = imx::lfail(A.err, "imx_learn_create");
@@ -569,9 +573,10 @@ int imx_learn_train(imx_learn *L, const double *du, const double *dh, int32_t ep
     if (last) learn_norm2<<<1, 1024, 0, st>>>(0, nullptr, 1, nullptr, nv, L->dhc, 1.0 / nv, 0, L->lh);
     learn_divT<<<g, LTPB, 0, st>>>(NE, s->e_v, L->de, L->dhc, 2.f / (float)nv, m->T);
     LTRY(hipGetLastError(), "learn train");
-    rc = imx::mlp_train_dev(m, NE, nullptr, lr, wd, 1, last ? &lu : nullptr, 2);
+    rc = imx::mlp_train_dev(m, NE, nullptr, lr, wd, 1, nullptr, 2);
     if (rc) return rc;
   }
+  if ((rc = imx::mlp_loss(m, NE, nullptr, 1, &lu))) return rc;
   double lh = 0.0;
   LTRY(hipMemcpyAsync(&lh, L->lh, 8, hipMemcpyDeviceToHost, st), "learn train");
   LTRY(hipStreamSynchronize(st), "learn train");
@@ -661,8 +666,7 @@ int imx_learn_fit(imx_learn *L, int32_t nsteps, float lr0, float lr1, float wd, 
   LTRY(hipStreamSynchronize(s->stream), "imx_learn_fit");
   LTRY(hipMemcpyAsync(m->w, L->wv, (size_t)NE * 4, hipMemcpyDeviceToDevice, st), "imx_learn_fit");
   const int g = (NE + LTPB - 1) / LTPB, gc = (nv + LTPB - 1) / LTPB;
-  const int tail = nsteps < 16 ? nsteps : 16;
-  double su = 0.0, sh = 0.0;
+  const int tail = nsteps < kLossSteps ? nsteps : kLossSteps, nb = (NE + 63) / 64;
   uint64_t x = seed;
   for (int k = 0; k < nsteps; ++k) {
     x += 0x9E3779B97F4A7C15ull;  // SplitMix64
@@ -674,25 +678,26 @@ int imx_learn_fit(imx_learn *L, int32_t nsteps, float lr0, float lr1, float wd, 
     const short *X = L->Xb + (size_t)j * L->xstride;
     const float lr = nsteps > 1 ? lr0 + (lr1 - lr0) * (float)k / (float)(nsteps - 1) : lr0;
     const bool last = k >= nsteps - tail;
+    const int slot = k - (nsteps - tail);
     rc = imx::mlp_forward_dev(m, NE, X, L->Y, st);
     if (rc) return rc;
     learn_div<<<gc, LTPB, 0, st>>>(nv, s->c_nnb, s->c_ed, L->dc, L->Y, L->thb + (size_t)j * nv, L->dhc);
-    if (last) learn_norm2<<<1, 1024, 0, st>>>(0, nullptr, 1, nullptr, nv, L->dhc, 1.0 / nv, 0, L->lh);
+    if (last) learn_norm2<<<1, 1024, 0, st>>>(0, nullptr, 1, nullptr, nv, L->dhc, 1.0 / nv, 0, L->lh + slot);
     learn_targets<<<g, LTPB, 0, st>>>(NE, s->e_v, L->de, L->dhc, 2.f / (float)nv,
                                       L->tub + (size_t)j * NE, m->T);
     LTRY(hipGetLastError(), "imx_learn_fit");
-    double lu = 0.0;
-    rc = imx::mlp_train_dev(m, NE, X, lr, wd, 1, last ? &lu : nullptr, 2);
+    // the last steps' losses stay on the device until the end
+    rc = imx::mlp_train_dev(m, NE, X, lr, wd, 1, last ? L->lossu + (size_t)slot * nb : nullptr, 2);
     if (rc) return rc;
-    if (last) {
-      double lh = 0.0;
-      LTRY(hipMemcpyAsync(&lh, L->lh, 8, hipMemcpyDeviceToHost, st), "imx_learn_fit");
-      LTRY(hipStreamSynchronize(st), "imx_learn_fit");
-      su += lu;
-      sh += lh;
-    }
   }
-  LTRY(hipStreamSynchronize(st), "imx_learn_fit");
+  double lu[kLossSteps], lh[kLossSteps];
+  if ((rc = imx::mlp_loss(m, NE, L->lossu, tail, lu))) return rc;
+  LTRY(hipMemcpy(lh, L->lh, tail * sizeof(double), hipMemcpyDeviceToHost), "imx_learn_fit");
+  double su = 0.0, sh = 0.0;
+  for (int k = 0; k < tail; ++k) {
+    su += lu[k];
+    sh += lh[k];
+  }
   if (loss) {
     loss[0] = su / tail;
     loss[1] = sh / tail;

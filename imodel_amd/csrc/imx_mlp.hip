@@ -12,8 +12,8 @@
 // chunk t of the next layer, so activations never leave registers between
 // layers. The backward data pass (dA^T = W dZ^T) has the same shape with a
 // second, transposed weight fragment set. Weight gradients
-// dW = A^T(features x edges) . dZ(edges x features) contract over edges and
-// read activations/gradients stored feature-major by the training kernel.
+// dW = A^T(features x edges) . dZ(edges x features) contract over edges, in
+// the same kernel, from LDS.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
@@ -27,22 +27,6 @@
 
 #include "imx_mlp_dev.h"
 
-// Y^T tiles (NT x 16 edges) = W^T (N x K) X^T (K x 16), from fragments
-// Wf[(n*KT + kc)*64 + lane] and input fragments xin[kc].
-template <int KT, int NT>
-__device__ __forceinline__ void layer_fwd(const v4s *__restrict__ Wf, const float *__restrict__ b,
-                                          const v4s (&xin)[KT], v4f (&z)[NT], int lane) {
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    v4f acc;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = b[n * 16 + 4 * (lane / 16) + i];
-#pragma unroll
-    for (int kc = 0; kc < KT; ++kc) acc = mfma(Wf[(n * KT + kc) * 64 + lane], xin[kc], acc);
-    z[n] = acc;
-  }
-}
-
 // load the 3 input fragments of 16 edges (rows of X, 48 bf16 each)
 __device__ __forceinline__ void load_x(const short *__restrict__ X, int64_t e0, int64_t n, int lane,
                                        v4s (&x)[3]) {
@@ -54,202 +38,341 @@ __device__ __forceinline__ void load_x(const short *__restrict__ X, int64_t e0, 
   }
 }
 
-// Training pass over a batch: forward, weighted MSE loss
+// Training pass: forward, weighted MSE loss
 //   L = sum_e w_e sum_o (y_eo - t_eo)^2,
-// backward through every layer; stores (feature-major, bf16) the layer
-// inputs A0^T = X^T .. A3^T and the pre-activation gradients dZ1^T .. dZ4^T
-// for the weight-gradient kernel, and one loss partial per block.
-// Output o with bit o of gmask set takes T[e][o] as dL/dy_eo itself (a loss
-// defined outside the network, e.g. through a divergence) and adds nothing
-// to the loss partial.
-__global__ __launch_bounds__(64 * MLP_WAVES) void mlp_train(
-    int64_t n, int64_t npad, const short *__restrict__ X, const float *__restrict__ T,
-    const float *__restrict__ w, int gmask, const v4s *__restrict__ Wf, const v4s *__restrict__ Wb,
-    const float *__restrict__ P, short *__restrict__ AT, short *__restrict__ DZT,
-    float *__restrict__ loss_part) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int64_t e0 = ((int64_t)blockIdx.x * MLP_WAVES + wave) * 16;
-  __shared__ float lred[MLP_WAVES];
-  float lsum = 0.f;
-  if (e0 < npad) {
-    const int64_t e = e0 + (lane % 16);
-    const bool live = e < n;
-    v4s x[3];
-    load_x(X, e0, n, lane, x);
-    v4f z1[8], z2[8], z3[8];
-    v4s a1[8], a2[8], a3[8];
-    layer_fwd<3, 8>(Wf + FF_1 / 4, P + P_B1, x, z1, lane);
+// backward through every layer, and the weight and bias gradients, in one
+// kernel. Output o with bit o of gmask set takes T[e][o] as dL/dy_eo itself
+// (a loss defined outside the network, e.g. through a divergence) and adds
+// nothing to the loss.
+//
+// A block takes 64 edges at a time. Four of its eight waves, 16 edges each,
+// evaluate the layers forward and backward and leave the layer inputs
+// A0 = X .. A3 and the pre-activation gradients dZ1 .. dZ4 in LDS,
+// feature-major (the transposition the weight gradients need). The other four
+// contract them over the 64 edges, one phase behind, with the gradient tiles
+// in accumulators over all of the block's edges, and fetch the next layer's
+// weight fragments into LDS while one layer runs. The block writes its
+// gradient once; the optimiser kernel sums the blocks' partials in order.
+//   gradient wave g: output tiles 2g, 2g + 1 of layers 1-3 with all input
+//   tiles, input tiles 2g, 2g + 1 of layer 4; biases as products with ones.
+// One block per CU (161 KB of LDS), two waves per SIMD: one busy with
+// activations, one with MFMAs and LDS.
+//
+// Against the form that stored A and dZ in memory (1.7 KB per edge, in
+// 32-byte pieces) and contracted them in a second and third kernel: 754 us ->
+// 90 at glevel 6 (122,886 edges; 320 TFLOP/s). What bounds it now is one
+// layer wave's own chain of LDS reads, MFMAs and activations, 29 k cycles a
+// batch, of which the matrix cores are busy 6 k. With both roles in four waves the
+// accumulators and the layers in flight spilled, and every wait for a spilled
+// value or a bias also waited for the weights on their way: 282 us. The
+// derivative is formed with the activation and shares its exponential and
+// reciprocal.
+#define TR_STRIDE 68  // bf16 per LDS row: 64 edges and a pad of 8 bytes
+#define TR_A 0        // rows: layer inputs 48 + 3 x 128
+#define TR_DA 432     // dZ of layers 3 and 1
+#define TR_DB 560     // dZ of layer 2
+#define TR_D4 688     // dZ4, 16 rows of which 2 are live
+#define TR_ROWS 704
+#define TR_BLOCKS 256
+#define TR_ILV 4     // MFMA chains a wave runs side by side
+#define TR_THREADS (2 * 64 * MLP_WAVES)
+
+// activation (BF16, as the next layer's input) and its derivative
+__device__ __forceinline__ v4s gelu_both(const v4f &z, v4f &d) {
+  float g[4];
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a1[t][i] = f2bf(gelu(z1[t][i]));
-    layer_fwd<8, 8>(Wf + FF_2 / 4, P + P_B2, a1, z2, lane);
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a2[t][i] = f2bf(gelu(z2[t][i]));
-    layer_fwd<8, 8>(Wf + FF_3 / 4, P + P_B3, a2, z3, lane);
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a3[t][i] = f2bf(gelu(z3[t][i]));
-    v4f y = {0.f, 0.f, 0.f, 0.f};
-    if (lane < 16) {
-      y[0] = P[P_B4];
-      y[1] = P[P_B4 + 1];
-    }
-#pragma unroll
-    for (int kc = 0; kc < 8; ++kc) y = mfma(Wf[(FF_4 / 4) + kc * 64 + lane], a3[kc], y);
-    // dL/dy (features 0,1 live in lanes 0..15, elements 0,1)
-    v4s dz4 = {0, 0, 0, 0};
-    if (lane < 16 && live) {
-      const float we = w[e];
-      const float r0 = y[0] - T[e * 2], r1 = y[1] - T[e * 2 + 1];
-      lsum = ((gmask & 1) ? 0.f : we * r0 * r0) + ((gmask & 2) ? 0.f : we * r1 * r1);
-      dz4[0] = f2bf((gmask & 1) ? T[e * 2] : 2.f * we * r0);
-      dz4[1] = f2bf((gmask & 2) ? T[e * 2 + 1] : 2.f * we * r1);
-    }
-    // stores: feature-major [row][npad]; a wave writes its 16 edge columns
-    const int64_t col = e0 + (lane % 16);
-    auto store4 = [&](short *base, int row0, v4s v) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) base[(int64_t)(row0 + 4 * (lane / 16) + i) * npad + col] = v[i];
-    };
-    // layer inputs A0 (X, 48 rows), A1..A3 (128 rows each)
-#pragma unroll
-    for (int kc = 0; kc < 3; ++kc) store4(AT, kc * 16, x[kc]);
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      store4(AT + (int64_t)48 * npad, t * 16, a1[t]);
-      store4(AT + (int64_t)176 * npad, t * 16, a2[t]);
-      store4(AT + (int64_t)304 * npad, t * 16, a3[t]);
-    }
-    // dZ4 (16 rows, 2 live)
-    store4(DZT + (int64_t)384 * npad, 0, dz4);
-    // dA3^T = W4 dZ4^T, dZ3 = dA3 * gelu'(z3)
-    v4s dz[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = mfma(Wb[(FB_4 / 4) + m * 64 + lane], dz4, acc);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dz[m][i] = f2bf(acc[i] * gelu_d(z3[m][i]));
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) store4(DZT + (int64_t)256 * npad, t * 16, dz[t]);
-    // dA2^T = W3 dZ3^T, dZ2
-    v4s dzn[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kc = 0; kc < 8; ++kc) acc = mfma(Wb[(FB_3 / 4) + (m * 8 + kc) * 64 + lane], dz[kc], acc);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dzn[m][i] = f2bf(acc[i] * gelu_d(z2[m][i]));
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) store4(DZT + (int64_t)128 * npad, t * 16, dzn[t]);
-    // dA1^T = W2 dZ2^T, dZ1
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kc = 0; kc < 8; ++kc) acc = mfma(Wb[(FB_2 / 4) + (m * 8 + kc) * 64 + lane], dzn[kc], acc);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dz[m][i] = f2bf(acc[i] * gelu_d(z1[m][i]));
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) store4(DZT, t * 16, dz[t]);
+  for (int i = 0; i < 4; ++i) {
+    const float x = z[i], s = gelu_s(x);
+    g[i] = x * s;
+    float t = s + g[i] * (1.0f - s) * GELU_C2 * __builtin_fmaf(3.0f * GELU_A, x * x, 1.0f);
+    asm volatile("" : "+v"(t));  // now: left to its use, x and s would be kept instead
+    d[i] = t;
   }
-  // loss partial: wave sum, then block
+  uint32_t p[2] = {f2bf2(g[0], g[1]), f2bf2(g[2], g[3])};
+  return __builtin_bit_cast(v4s, p);
+}
+
+// rows 16 t + 4 (lane / 16) + i of one edge column
+__device__ __forceinline__ void put_rows(short *lds, int row0, int col, int lane, v4s v) {
+  short *p = lds + (row0 + 4 * (lane / 16)) * TR_STRIDE + col;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
-  if (lane == 0) lred[wave] = lsum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int q = 0; q < MLP_WAVES; ++q) s += lred[q];
-    loss_part[blockIdx.x] = s;
+  for (int i = 0; i < 4; ++i) p[i * TR_STRIDE] = v[i];
+}
+// One hidden layer of 16 edges, a tile of 16 features at a time: pre-activations
+// from fragments Wf[(n*KT + kc)*64 + lane] and input fragments xin[kc], the
+// activation (to the next layer and to rows row0 of LDS) and its derivative.
+template <int KT>
+__device__ __forceinline__ void layer_act(const v4s *Wf, const float *b, const v4s (&xin)[KT], v4s (&a)[8], v4f (&d)[8],
+                                          short *lds, int row0, int col, int lane) {
+#pragma unroll
+  for (int n = 0; n < 8; n += TR_ILV) {  // independent chains side by side
+    v4f z[TR_ILV];
+#pragma unroll
+    for (int q = 0; q < TR_ILV; ++q) z[q] = *reinterpret_cast<const v4f *>(b + (n + q) * 16 + 4 * (lane / 16));
+#pragma unroll
+    for (int kc = 0; kc < KT; ++kc)
+#pragma unroll
+      for (int q = 0; q < TR_ILV; ++q) z[q] = mfma(Wf[((n + q) * KT + kc) * 64 + lane], xin[kc], z[q]);
+#pragma unroll
+    for (int q = 0; q < TR_ILV; ++q) {
+      a[n + q] = gelu_both(z[q], d[n + q]);
+      put_rows(lds, row0 + 16 * (n + q), col, lane, a[n + q]);
+    }
+  }
+}
+// K32 operand: row lane % 16 of a 16-row tile, 8 edges of chunk c
+__device__ __forceinline__ v8s get_rows(const short *lds, int row0, int c, int lane) {
+  const v4s *p = reinterpret_cast<const v4s *>(lds + (row0 + lane % 16) * TR_STRIDE + 32 * c + 8 * (lane / 16));
+  return __builtin_shufflevector(p[0], p[1], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// gradient tiles of one layer: MT input tiles x NB output tiles of this wave
+template <int MT, int NB>
+__device__ __forceinline__ void grad_tiles(const short *lds, int a_row, int dz_row, int lane, v4f (&acc)[NB][MT],
+                                           v4f (&bias)[NB]) {
+  const short one = 0x3F80;
+  const v8s ones = {one, one, one, one, one, one, one, one};
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    v8s dz[NB];
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      dz[q] = get_rows(lds, dz_row + 16 * q, c, lane);
+      bias[q] = mfma32(ones, dz[q], bias[q]);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const v8s x = get_rows(lds, a_row + 16 * m, c, lane);
+#pragma unroll
+      for (int q = 0; q < NB; ++q) acc[q][m] = mfma32(x, dz[q], acc[q][m]);
+    }
   }
 }
 
-// Weight gradients: one wave per (layer, in-tile, out-tile, edge split);
-// dW[in][out] = sum_e A^T[in][e] dZ^T[out][e] on MFMA, one FP32 partial
-// tile per split (reduced deterministically by the optimiser kernel).
-__constant__ int c_wg_layer_tiles[5] = {0, 24, 88, 152, 160};  // prefix of 3x8, 8x8, 8x8, 8x1
-
-__global__ __launch_bounds__(64 * MLP_WAVES) void mlp_wgrad(int64_t npad, int nsplit,
-                                                            const short *__restrict__ AT,
-                                                            const short *__restrict__ DZT,
-                                                            float *__restrict__ part) {
-  const int lane = threadIdx.x & 63;
-  const int gw = blockIdx.x * MLP_WAVES + (threadIdx.x >> 6);
-  const int tile = gw / nsplit, split = gw % nsplit;
-  if (tile >= 160) return;
-  int layer = 0;
-  while (tile >= c_wg_layer_tiles[layer + 1]) ++layer;
-  const int lt = tile - c_wg_layer_tiles[layer];
-  // layer geometry: input rows in AT, dz rows in DZT, out tiles, param offset
-  const int a_row = (layer == 0) ? 0 : 48 + (layer - 1) * 128;
-  const int dz_row = layer * 128;
-  const int n_out_t = (layer == 3) ? 1 : 8;
-  const int nout = (layer == 3) ? MLP_OUT : MLP_H;
-  const int poff = (layer == 0) ? P_W1 : (layer == 1) ? P_W2 : (layer == 2) ? P_W3 : P_W4;
-  const int mt = lt / n_out_t, nt = lt % n_out_t;
-  const int64_t per = ((npad / 16 + nsplit - 1) / nsplit) * 16;
-  const int64_t k0 = split * per, k1 = (k0 + per < npad) ? k0 + per : npad;
-  v4f acc = {0.f, 0.f, 0.f, 0.f};
-  const short *ar = AT + (int64_t)(a_row + mt * 16 + lane % 16) * npad;
-  const short *br = DZT + (int64_t)(dz_row + nt * 16 + lane % 16) * npad;
-  for (int64_t k = k0; k < k1; k += 16) {
-    const v4s a = *reinterpret_cast<const v4s *>(ar + k + 4 * (lane / 16));
-    const v4s b = *reinterpret_cast<const v4s *>(br + k + 4 * (lane / 16));
-    acc = mfma(a, b, acc);
+// dz (128 features) = (W dZ_next) g'(z): one layer of the backward pass
+template <int KT>
+__device__ __forceinline__ void back_layer(const v4s *__restrict__ Wb, const v4s (&dzn)[KT], const v4f (&d)[8],
+                                           v4s (&dz)[8], int lane) {
+#pragma unroll
+  for (int m = 0; m < 8; m += TR_ILV) {
+    v4f acc[TR_ILV];
+#pragma unroll
+    for (int q = 0; q < TR_ILV; ++q) acc[q] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kc = 0; kc < KT; ++kc)
+#pragma unroll
+      for (int q = 0; q < TR_ILV; ++q) acc[q] = mfma(Wb[((m + q) * KT + kc) * 64 + lane], dzn[kc], acc[q]);
+#pragma unroll
+    for (int q = 0; q < TR_ILV; ++q) {
+      const v4f g = acc[q] * d[m + q];
+      uint32_t p[2] = {f2bf2(g[0], g[1]), f2bf2(g[2], g[3])};
+      dz[m + q] = __builtin_bit_cast(v4s, p);
+    }
   }
-  // D[in = mt*16 + 4(l/16)+i][out = nt*16 + l%16]
-  const int outc = nt * 16 + lane % 16;
-  if (outc < nout)
+}
+
+// One layer's weight fragments from memory straight to LDS (16 bytes per lane,
+// no registers), a quarter of them by each of four waves; in flight until
+// the wave's s_waitcnt.
+template <int COUNT>
+__device__ __forceinline__ void tr_fetch(const short *__restrict__ src, short *dst, int wave) {
+  constexpr int kWave = COUNT / MLP_WAVES;  // bf16 per wave
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < kWave; i += 512)
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) void *)(src + wave * kWave + i + lane * 8),
+        (__attribute__((address_space(3))) void *)(dst + wave * kWave + i), 16, 0, 0);
+}
+__device__ __forceinline__ void tr_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+__global__ __launch_bounds__(TR_THREADS) void mlp_train(
+    int64_t n, int nbatch, const short *__restrict__ X, const float *__restrict__ T,
+    const float *__restrict__ w, int gmask, const short *__restrict__ Wf, const short *__restrict__ Wb,
+    const float *__restrict__ P, float *__restrict__ part, float *__restrict__ loss_part) {
+  __shared__ __align__(16) short lds[TR_ROWS * TR_STRIDE];
+  __shared__ __align__(16) short wbuf[2][MLP_H * MLP_H];  // the layer in use and the next
+  __shared__ __align__(16) float lb[3 * MLP_H];           // biases of layers 1-3
+  __shared__ float lred[MLP_WAVES];
+  const int lane = threadIdx.x & 63;
+  const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = role & (MLP_WAVES - 1);
+  const v4f zero = {0.f, 0.f, 0.f, 0.f};
+  for (int i = threadIdx.x; i < 3 * MLP_H; i += TR_THREADS)
+    lb[i] = P[(i < MLP_H ? P_B1 : i < 2 * MLP_H ? P_B2 - MLP_H : P_B3 - 2 * MLP_H) + i];
+  // Both roles pass the same barriers: one before the loop, five per batch,
+  // one after it. wbuf[cur] holds layers 1 and 3 forward and 2 backward.
+  int cur = 0;
+  if (role < MLP_WAVES) {  // layers
+    const int col = 16 * wave + lane % 16;
+    const v4s *W4 = reinterpret_cast<const v4s *>(Wf + FF_4), *B4 = reinterpret_cast<const v4s *>(Wb + FB_4);
+    v4s w4[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w4[k] = W4[k * 64 + lane];
+    const float y0 = lane < 16 ? P[P_B4] : 0.f, y1 = lane < 16 ? P[P_B4 + 1] : 0.f;
+    auto frag = [&](int which) { return reinterpret_cast<const v4s *>(wbuf[which]); };
+    __syncthreads();
+    for (int b = blockIdx.x; b < nbatch; b += gridDim.x) {
+      const int64_t e = (int64_t)b * 64 + col;
+      const bool live = lane < 16 && e < n;
+      v4s x[3];
+      load_x(X, (int64_t)b * 64 + 16 * wave, n, lane, x);
+      const float we = live ? w[e] : 0.f, t0 = live ? T[e * 2] : 0.f, t1 = live ? T[e * 2 + 1] : 0.f;
+      v4f d1[8], d2[8], d3[8];
+      v4s a1[8], a2[8];
+      __syncthreads();  // layer 1's weights
+      layer_act<3>(frag(cur), lb, x, a1, d1, lds, TR_A + 48, col, lane);
+      __syncthreads();  // layer 2's; the previous batch's layer-1 gradient has read X
+#pragma unroll
+      for (int kc = 0; kc < 3; ++kc) put_rows(lds, TR_A + kc * 16, col, lane, x[kc]);
+      layer_act<8>(frag(cur ^ 1), lb + MLP_H, a1, a2, d2, lds, TR_A + 176, col, lane);
+      __syncthreads();  // layer 3's
+      layer_act<8>(frag(cur), lb + 2 * MLP_H, a2, a1, d3, lds, TR_A + 304, col, lane);
+      v4f y = {y0, y1, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < 8; ++kc) y = mfma(w4[kc], a1[kc], y);
+      // dL/dy (features 0,1 live in lanes 0..15, elements 0,1)
+      v4s dz4[1] = {{0, 0, 0, 0}};
+      float lsum = 0.f;
+      if (live) {
+        const float r0 = y[0] - t0, r1 = y[1] - t1;
+        lsum = ((gmask & 1) ? 0.f : we * r0 * r0) + ((gmask & 2) ? 0.f : we * r1 * r1);
+        dz4[0][0] = f2bf((gmask & 1) ? t0 : 2.f * we * r0);
+        dz4[0][1] = f2bf((gmask & 2) ? t1 : 2.f * we * r1);
+      }
+      put_rows(lds, TR_D4, col, lane, dz4[0]);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
+      if (lane == 0) lred[wave] = lsum;
+      v4s dz[8], dzn[8];
+      back_layer<1>(B4, dz4, d3, dz, lane);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) put_rows(lds, TR_DA + 16 * t, col, lane, dz[t]);
+      __syncthreads();  // layer 3's backward; A, dZ4, dZ3 to the gradients
+      if (threadIdx.x == 0) {
+        float s = 0.f;
+        for (int q = 0; q < MLP_WAVES; ++q) s += lred[q];
+        loss_part[b] = s;
+      }
+      back_layer<8>(frag(cur ^ 1), dz, d2, dzn, lane);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) put_rows(lds, TR_DB + 16 * t, col, lane, dzn[t]);
+      __syncthreads();  // layer 2's backward; dZ2; dZ3 is read: its rows take dZ1
+      back_layer<8>(frag(cur), dzn, d1, dz, lane);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) put_rows(lds, TR_DA + 16 * t, col, lane, dz[t]);
+      cur ^= 1;
+    }
+    __syncthreads();
+    return;
+  }
+
+  // gradients and weight fetches
+  v4f g1[2][3], g2[2][8], g3[2][8], g4[1][2], b1[2], b2[2], b3[2], b4[1];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    b1[q] = b2[q] = b3[q] = g4[0][q] = zero;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) g2[q][m] = g3[q][m] = zero;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) g1[q][m] = zero;
+  }
+  b4[0] = zero;
+  tr_fetch<MLP_IN * MLP_H>(Wf + FF_1, wbuf[0], wave);
+  __syncthreads();
+  for (int b = blockIdx.x; b < nbatch; b += gridDim.x) {
+    tr_wait();
+    __syncthreads();  // layer 1 runs
+    tr_fetch<MLP_H * MLP_H>(Wf + FF_2, wbuf[cur ^ 1], wave);
+    if (b != blockIdx.x) grad_tiles<3, 2>(lds, TR_A, TR_DA + 32 * wave, lane, g1, b1);
+    tr_wait();
+    __syncthreads();  // layer 2
+    tr_fetch<MLP_H * MLP_H>(Wf + FF_3, wbuf[cur], wave);
+    tr_wait();
+    __syncthreads();  // layers 3 and 4, dZ3
+    tr_fetch<MLP_H * MLP_H>(Wb + FB_3, wbuf[cur ^ 1], wave);
+    tr_wait();
+    __syncthreads();  // dZ2
+    tr_fetch<MLP_H * MLP_H>(Wb + FB_2, wbuf[cur], wave);
+    grad_tiles<2, 1>(lds, TR_A + 304 + 32 * wave, TR_D4, lane, g4, b4);
+    grad_tiles<8, 2>(lds, TR_A + 176, TR_DA + 32 * wave, lane, g3, b3);
+    tr_wait();
+    __syncthreads();  // dZ1
+    tr_fetch<MLP_IN * MLP_H>(Wf + FF_1, wbuf[cur ^ 1], wave);  // of the next batch
+    grad_tiles<8, 2>(lds, TR_A + 48, TR_DB + 32 * wave, lane, g2, b2);
+    cur ^= 1;
+  }
+  tr_wait();  // the last fetch, which no batch uses
+  __syncthreads();
+  grad_tiles<3, 2>(lds, TR_A, TR_DA + 32 * wave, lane, g1, b1);
+  // the block's partial: D[in = 16 mt + 4 (l/16) + i][out = 16 nt + l % 16]
+  float *q = part + (int64_t)blockIdx.x * P_N;
+  const int in0 = 4 * (lane / 16), lo = lane % 16;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int out = 32 * wave + 16 * k + lo;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int inr = mt * 16 + 4 * (lane / 16) + i;
-      part[(int64_t)split * P_N + poff + inr * nout + outc] = acc[i];
+#pragma unroll
+      for (int m = 0; m < 3; ++m) q[P_W1 + (16 * m + in0 + i) * MLP_H + out] = g1[k][m][i];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        q[P_W2 + (16 * m + in0 + i) * MLP_H + out] = g2[k][m][i];
+        q[P_W3 + (16 * m + in0 + i) * MLP_H + out] = g3[k][m][i];
+      }
+      if (lo < MLP_OUT) q[P_W4 + (32 * wave + 16 * k + in0 + i) * MLP_OUT + lo] = g4[0][k][i];
     }
-}
-
-// Bias gradients: db[f] = sum_e dZ^T[f][e], one block per bias entry row;
-// written into split 0's partial slots (other splits hold 0 there).
-__global__ __launch_bounds__(256) void mlp_bgrad(int64_t npad, const short *__restrict__ DZT,
-                                                 float *__restrict__ part) {
-  const int r = blockIdx.x;  // 0..385: b1 (128), b2, b3, b4 (2)
-  int row, poff;
-  if (r < 128) { row = r; poff = P_B1 + r; }
-  else if (r < 256) { row = r; poff = P_B2 + (r - 128); }
-  else if (r < 384) { row = r; poff = P_B3 + (r - 256); }
-  else { row = 384 + (r - 384); poff = P_B4 + (r - 384); }
-  float s = 0.f;
-  for (int64_t e = threadIdx.x; e < npad; e += 256) s += bf2f(DZT[(int64_t)row * npad + e]);
-  __shared__ float red[256];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+    if (lane < 16) {
+      q[P_B1 + out] = b1[k][0];
+      q[P_B2 + out] = b2[k][0];
+      q[P_B3 + out] = b3[k][0];
+    }
   }
-  if (threadIdx.x == 0) part[poff] = red[0];
+  if (wave == 0 && lane < MLP_OUT) q[P_B4 + lane] = b4[0][0];
 }
 
-// AdamW (decoupled weight decay on the matrices, not the biases), summing
-// the split partials; then the BF16 fragment copies are rebuilt.
-__global__ __launch_bounds__(256) void mlp_adamw(int nsplit, const float *__restrict__ part,
+// The places of weight (row, col) of a layer in the fragment copies (the
+// inverse of mlp_pack's maps; layer 0-3, N output features)
+__device__ __forceinline__ void put_weight(int layer, int row, int col, short v, short *Ff, short *Fb, short *Ff32) {
+  const int KT = layer == 0 ? 3 : 8;
+  const int fbase = layer == 0 ? FF_1 : layer == 1 ? FF_2 : layer == 2 ? FF_3 : FF_4;
+  Ff[fbase + (((col / 16) * KT + row / 16) * 64 + (row % 16) / 4 * 16 + col % 16) * 4 + row % 4] = v;
+  if (layer > 0) {
+    const int bbase = layer == 1 ? FB_2 : layer == 2 ? FB_3 : FB_4, KB = layer == 3 ? 1 : 8;
+    Fb[bbase + (((row / 16) * KB + col / 16) * 64 + (col % 16) / 4 * 16 + row % 16) * 4 + col % 4] = v;
+  }
+  // K32: slot i of lane group g holds row kappa32(g, i) of its chunk
+  const int r = row % 32, lane = (r % 16) / 4 * 16 + col % 16, i = r % 4 + (r < 16 ? 0 : 4);
+  if (layer == 0)
+    Ff32[(col / 16) * 768 + (row < 32 ? lane * 8 + i : 512 + lane * 4 + row % 4)] = v;
+  else
+    Ff32[fbase + (col / 16) * 2048 + (row / 32) * 512 + lane * 8 + i] = v;
+}
+
+// AdamW (decoupled weight decay on the matrices, not the biases) on the sum
+// of the blocks' partials, and the updated weights' places in the BF16
+// fragment copies: 64 parameters per block, eight threads each over an eighth
+// of the partials, added in a fixed order.
+#define AW_GROUPS 8
+__global__ __launch_bounds__(64 * AW_GROUPS) void mlp_adamw(int nsplit, const float *__restrict__ part,
                                                  float *__restrict__ P, float *__restrict__ M,
                                                  float *__restrict__ V, float *__restrict__ G, float lr,
                                                  float b1, float b2, float eps, float wd, float bc1,
-                                                 float bc2, int apply) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= P_N) return;
+                                                 float bc2, int apply, short *__restrict__ Ff,
+                                                 short *__restrict__ Fb, short *__restrict__ Ff32) {
+  const int lane = threadIdx.x & 63, p = blockIdx.x * 64 + lane, grp = threadIdx.x >> 6;
+  __shared__ float red[AW_GROUPS][64];
   float g = 0.f;
-  for (int s = 0; s < nsplit; ++s) g += part[(int64_t)s * P_N + p];
+  if (p < P_N) {
+#pragma unroll 8
+    for (int s = grp; s < nsplit; s += AW_GROUPS) g += part[(int64_t)s * P_N + p];
+  }
+  red[grp][lane] = g;
+  __syncthreads();
+  if (grp || p >= P_N) return;
+  g = 0.f;
+#pragma unroll
+  for (int k = 0; k < AW_GROUPS; ++k) g += red[k][lane];
   G[p] = g;
   if (!apply) return;
   const bool is_bias = (p >= P_B1 && p < P_W2) || (p >= P_B2 && p < P_W3) || (p >= P_B3 && p < P_W4) ||
@@ -262,6 +385,11 @@ __global__ __launch_bounds__(256) void mlp_adamw(int nsplit, const float *__rest
   if (!is_bias) x -= lr * wd * x;
   x -= lr * (m / bc1) / (sqrtf(v / bc2) + eps);
   P[p] = x;
+  if (is_bias) return;
+  const int layer = p < P_W2 ? 0 : p < P_W3 ? 1 : p < P_W4 ? 2 : 3;
+  const int q = p - (layer == 0 ? P_W1 : layer == 1 ? P_W2 : layer == 2 ? P_W3 : P_W4);
+  const int N = layer == 3 ? MLP_OUT : MLP_H;
+  put_weight(layer, q / N, q % N, f2bf(x), Ff, Fb, Ff32);
 }
 
 // fragment copies from the FP32 master (forward: W^T tiles; backward: W tiles)
@@ -356,18 +484,14 @@ int mlp_reserve(imx_mlp *m, int64_t n) {
   const int64_t npad = ((n + 63) / 64) * 64;
   if (npad <= m->cap) return IMX_OK;
   (void)hipFree(m->X);
-  (void)hipFree(m->AT);
-  (void)hipFree(m->DZT);
   (void)hipFree(m->T);
   (void)hipFree(m->w);
   (void)hipFree(m->Y);
   (void)hipFree(m->Xf);
   (void)hipFree(m->lossp);
-  m->X = m->AT = m->DZT = nullptr;
+  m->X = nullptr;
   m->T = m->w = m->Y = m->Xf = m->lossp = nullptr;
   MTRY(hipMalloc(&m->X, npad * MLP_IN * 2), "mlp scratch");
-  MTRY(hipMalloc(&m->AT, npad * 432 * 2), "mlp scratch");
-  MTRY(hipMalloc(&m->DZT, npad * 400 * 2), "mlp scratch");
   MTRY(hipMalloc(&m->T, npad * 2 * 4), "mlp scratch");
   MTRY(hipMalloc(&m->w, npad * 4), "mlp scratch");
   MTRY(hipMalloc(&m->Y, npad * 2 * 4), "mlp scratch");
@@ -415,40 +539,37 @@ int mlp_forward_dev(imx_mlp *m, int64_t n, const short *X, float *Y, hipStream_t
   return IMX_OK;
 }
 
-// One training pass on the device batch X (m->X when NULL), m->T, m->w (n edges).
-int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int apply, double *loss,
+// One training pass on the device batch X (m->X when NULL), m->T, m->w (n
+// edges), enqueued on m's stream; loss_part [(n + 63) / 64] takes the loss
+// partials (m->lossp when NULL).
+int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int apply, float *loss_part,
                   int gmask) {
-  const int64_t npad = ((n + 63) / 64) * 64;
-  const int64_t blocks = npad / 64;
+  const int nbatch = (int)((n + 63) / 64), blocks = nbatch < TR_BLOCKS ? nbatch : TR_BLOCKS;
   hipStream_t st = m->stream;
-  // zero the padding columns of the stored tensors (rows beyond n in the batch)
-  mlp_train<<<(unsigned)blocks, 64 * MLP_WAVES, 0, st>>>(n, npad, X ? X : m->X, m->T, m->w, gmask, (const v4s *)m->Ff,
-                                                        (const v4s *)m->Fb, m->P, m->AT, m->DZT, m->lossp);
+  mlp_train<<<blocks, TR_THREADS, 0, st>>>(n, nbatch, X ? X : m->X, m->T, m->w, gmask, m->Ff, m->Fb, m->P,
+                                               m->part, loss_part ? loss_part : m->lossp);
   MTRY(hipGetLastError(), "mlp_train");
-  MTRY(hipMemsetAsync(m->part, 0, (size_t)m->nsplit * P_N * 4, st), "mlp part");
-  const int waves = 160 * m->nsplit;
-  mlp_wgrad<<<(waves + MLP_WAVES - 1) / MLP_WAVES, 64 * MLP_WAVES, 0, st>>>(npad, m->nsplit, m->AT, m->DZT,
-                                                                          m->part);
-  mlp_bgrad<<<386, 256, 0, st>>>(npad, m->DZT, m->part);
-  MTRY(hipGetLastError(), "mlp_wgrad");
   m->t += apply ? 1 : 0;
   const float b1 = 0.9f, b2 = 0.999f;
   const float bc1 = 1.f - powf(b1, (float)(m->t > 0 ? m->t : 1));
   const float bc2 = 1.f - powf(b2, (float)(m->t > 0 ? m->t : 1));
-  mlp_adamw<<<(P_N + 255) / 256, 256, 0, st>>>(m->nsplit, m->part, m->P, m->M, m->V, m->G, lr, b1, b2,
-                                                1e-8f, wd, bc1, bc2, apply);
+  mlp_adamw<<<(P_N + 63) / 64, 64 * AW_GROUPS, 0, st>>>(blocks, m->part, m->P, m->M, m->V, m->G, lr, b1, b2, 1e-8f,
+                                                        wd, bc1, bc2, apply, m->Ff, m->Fb, m->Ff32);
   MTRY(hipGetLastError(), "mlp_adamw");
-  if (apply) {
-    int rc = mlp_pack_launch(m);
-    if (rc) return rc;
-  }
-  if (loss) {
-    std::vector<float> lp(blocks);
-    MTRY(hipMemcpyAsync(lp.data(), m->lossp, blocks * 4, hipMemcpyDeviceToHost, st), "loss");
-    MTRY(hipStreamSynchronize(st), "loss");
+  return IMX_OK;
+}
+
+// Sum of the loss partials of passes over n edges (waits for m's stream).
+int mlp_loss(imx_mlp *m, int64_t n, const float *loss_part, int passes, double *loss) {
+  const int64_t nb = (n + 63) / 64;
+  std::vector<float> lp((size_t)nb * passes);
+  MTRY(hipMemcpyAsync(lp.data(), loss_part ? loss_part : m->lossp, lp.size() * 4, hipMemcpyDeviceToHost, m->stream),
+       "loss");
+  MTRY(hipStreamSynchronize(m->stream), "loss");
+  for (int k = 0; k < passes; ++k) {
     double s = 0.0;
-    for (float v : lp) s += v;
-    *loss = s;
+    for (int64_t b = 0; b < nb; ++b) s += lp[k * nb + b];
+    loss[k] = s;
   }
   return IMX_OK;
 }
@@ -468,7 +589,7 @@ int imx_mlp_create(uint64_t seed, imx_mlp **out) {
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&m->P, P_N * 4) != hipSuccess || hipMalloc(&m->M, P_N * 4) != hipSuccess ||
       hipMalloc(&m->V, P_N * 4) != hipSuccess || hipMalloc(&m->G, P_N * 4) != hipSuccess ||
-      hipMalloc(&m->part, (size_t)m->nsplit * P_N * 4) != hipSuccess ||
+      hipMalloc(&m->part, (size_t)TR_BLOCKS * P_N * 4) != hipSuccess ||
       hipMalloc(&m->Ff, FF_N * 2) != hipSuccess || hipMalloc(&m->Fb, FB_N * 2) != hipSuccess ||
       hipMalloc(&m->Ff32, FF_N * 2) != hipSuccess) {
     rc = imx::set_error(IMX_EDEVICE, "imx_mlp_create: device allocation failed");
@@ -557,7 +678,8 @@ int imx_mlp_train(imx_mlp *m, int64_t n, const float *X, const float *T, const f
       hipMemcpyAsync(m->w, w, n * 4, hipMemcpyHostToDevice, st) != hipSuccess)
     return imx::set_error(IMX_EDEVICE, "imx_mlp_train: upload");
   f32_to_bf16<<<(unsigned)((n * MLP_IN + 255) / 256), 256, 0, st>>>(n * MLP_IN, m->Xf, m->X);
-  rc = imx::mlp_train_dev(m, n, nullptr, lr, wd, apply, loss, gmask);
+  rc = imx::mlp_train_dev(m, n, nullptr, lr, wd, apply, nullptr, gmask);
+  if (!rc && loss) rc = imx::mlp_loss(m, n, nullptr, 1, loss);
   if (rc) return rc;
   if (grad && (hipMemcpyAsync(grad, m->G, P_N * 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
                hipStreamSynchronize(st) != hipSuccess))
@@ -593,7 +715,7 @@ void imx_mlp_destroy(imx_mlp *m) {
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   float *fs[] = {m->P, m->M, m->V, m->G, m->part, m->lossp, m->T, m->w, m->Y, m->Xf};
   for (float *p : fs) (void)hipFree(p);
-  short *ss[] = {m->Ff, m->Fb, m->Ff32, m->X, m->AT, m->DZT};
+  short *ss[] = {m->Ff, m->Fb, m->Ff32, m->X};
   for (short *p : ss) (void)hipFree(p);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
