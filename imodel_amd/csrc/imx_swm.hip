@@ -49,6 +49,11 @@ __device__ __forceinline__ int xcd_index() {
   return lb * TPB + threadIdx.x;
 }
 
+// The same for a part of a launch: block pb of nb (a multiple of NXCD).
+__device__ __forceinline__ int part_index(int pb, int nb) {
+  return ((pb % NXCD) * (nb / NXCD) + pb / NXCD) * (int)blockDim.x + (int)threadIdx.x;
+}
+
 // Same with a compile-time block size; remap = 0 keeps the hardware order
 // (a choice the autotuner makes per kernel).
 template <int BS>
@@ -69,17 +74,32 @@ static inline int grid_bs(int n, int bs) {
 #define HTR_GUARD (1.1920928955078125e-07 / 100000.0)
 
 // ============================================================ REF kernels ==
+// What ode_rk4 does with a tendency value (swm.f90:2647-2678), by the kernel
+// that has just formed it: the next stage's state y + dt k / 2 or y + dt k, or
+// the step's y + dt (k0 + 2 k1 + 2 k2 + k3) / 6.
+struct RefRk {
+  int kind = 0;  // 0 nothing, 1 half a step, 2 a whole one, 3 the sum
+  const double *y = nullptr;
+  double *out = nullptr;
+  const double *k0 = nullptr, *k1 = nullptr, *k2 = nullptr;
+  double dt = 0.0;
+  __device__ __forceinline__ void update(int i, double k) const {
+    if (kind == 1) out[i] = y[i] + dt * k / 2.0;
+    else if (kind == 2) out[i] = y[i] + dt * k;
+    else if (kind == 3) out[i] = y[i] + dt * (k0[i] + 2.0 * k1[i] + 2.0 * k2[i] + k) / 6.0;
+  }
+};
+
 // scalar_hx2ed + scalar_elem_product (swm_operators.f90:88-114, :1567-1573):
 // the average of the two cells, or (HC with pxt16) barycentric weights hb of
 // the cells hv of the triangle holding the dual edge midpoint
-__global__ __launch_bounds__(TPB) void ref_edge_flux(int ne, const int32_t *__restrict__ e_v,
+__device__ __forceinline__ void ref_edge_flux(int l, int ne, const int32_t *__restrict__ e_v,
                                                      const double *__restrict__ hb,
                                                      const int32_t *__restrict__ hv,
                                                      const double *__restrict__ h,
                                                      const double *__restrict__ u,
                                                      double *__restrict__ h_ed,
                                                      double *__restrict__ uh) {
-  const int l = xcd_index();
   if (l >= ne || e_v[l] < 0) return;
   double he;
   if (hb) {
@@ -98,7 +118,7 @@ __global__ __launch_bounds__(TPB) void ref_edge_flux(int ne, const int32_t *__re
 // h at triangles: trsk area weights (hmode 0), barycentric coordinates t_w
 // (1, pxt16), or edge values weighted by the edge's sub-triangle areas t_w
 // (2, gass18: scalar_edtr2trcc, swm_operators.f90:286-346)
-__global__ __launch_bounds__(TPB) void ref_tri(int nt, const int32_t *__restrict__ t_ed,
+__device__ __forceinline__ void ref_tri(int k, int nt, const int32_t *__restrict__ t_ed,
                                                const int8_t *__restrict__ t_tg,
                                                const int32_t *__restrict__ t_v,
                                                const double *__restrict__ t_area,
@@ -113,7 +133,6 @@ __global__ __launch_bounds__(TPB) void ref_tri(int nt, const int32_t *__restrict
                                                double *__restrict__ zeta,
                                                double *__restrict__ h_tr,
                                                double *__restrict__ q_tr, int *__restrict__ flag) {
-  const int k = xcd_index();
   if (k >= nt || t_ed[k] < 0) return;
   double e = 0.0;
 #pragma unroll
@@ -156,7 +175,7 @@ __global__ __launch_bounds__(TPB) void ref_tri(int nt, const int32_t *__restrict
 // The vorticity at edges (eta_ed, scalar_tr2ed of eta with the same
 // interpolation, swm.f90:2465) is written when eta_ed is not NULL (the level
 // model's Coriolis term reads it).
-__global__ __launch_bounds__(TPB) void ref_edge_q(int ne, int qmode, const int32_t *__restrict__ e_sh,
+__device__ __forceinline__ void ref_edge_q(int l, int ne, int qmode, const int32_t *__restrict__ e_sh,
                                                   const double *__restrict__ e_dw,
                                                   const double *__restrict__ t_area,
                                                   const double *__restrict__ eta,
@@ -164,7 +183,6 @@ __global__ __launch_bounds__(TPB) void ref_edge_q(int ne, int qmode, const int32
                                                   const double *__restrict__ q_tr,
                                                   double *__restrict__ q_ed, double *__restrict__ eta_ed,
                                                   int *__restrict__ flag) {
-  const int l = xcd_index();
   if (l >= ne || e_sh[l] < 0) return;
   const int k1 = e_sh[l], k2 = e_sh[ne + l];
   if (qmode == 1) {
@@ -216,7 +234,7 @@ __global__ __launch_bounds__(TPB) void ref_ketr(int nt, const int32_t *__restric
 
 // div_hx(uh), div_hx(u), kinetic_energy_hx, g(h+b)+K
 // (swm_operators.f90:613-661, :1132-1217; swm.f90:2533-2536)
-__global__ __launch_bounds__(TPB) void ref_cell(int nv, const int32_t *__restrict__ c_nnb,
+__device__ __forceinline__ void ref_cell(int i, int nv, const int32_t *__restrict__ c_nnb,
                                                 const int32_t *__restrict__ c_ed,
                                                 const int8_t *__restrict__ c_ttg,
                                                 const double *__restrict__ c_area,
@@ -224,7 +242,7 @@ __global__ __launch_bounds__(TPB) void ref_cell(int nv, const int32_t *__restric
                                                 const double *__restrict__ e_dleng,
                                                 const double *__restrict__ u,
                                                 const double *__restrict__ uh,
-                                                const double *__restrict__ h,
+                                                const double *h,
                                                 const double *__restrict__ bt, int kmode,
                                                 const double *__restrict__ vhx,
                                                 const double *__restrict__ vuh,
@@ -235,20 +253,30 @@ __global__ __launch_bounds__(TPB) void ref_cell(int nv, const int32_t *__restric
                                                 double *__restrict__ masseq,
                                                 double *__restrict__ divu,
                                                 double *__restrict__ ke,
-                                                double *__restrict__ ghbk) {
-  const int i = xcd_index();
+                                                double *__restrict__ ghbk, const RefRk &rk) {
   if (i >= nv) return;
   const int n = c_nnb[i];
   double s = 0.0, sd = 0.0, k = 0.0, ca = 0.0;
-  for (int j = 0; j < n; ++j) {
-    const int l = c_ed[j * nv + i];
-    const double sg = (double)c_ttg[j * nv + i];
-    s = s + sg * uh[l] * e_dleng[l];
-    sd = sd + sg * u[l] * e_dleng[l];
-    const double ed_area = 0.25 * e_leng[l] * e_dleng[l];
+  // all gathers in flight together; the sums stay in ring order
+  double gu[MX], guh[MX], gl[MX], gd[MX], sgn[MX];
+#pragma unroll
+  for (int j = 0; j < MX; ++j) {
+    const int l = c_ed[j * nv + i];  // padded slots name edge slot 0
+    sgn[j] = (double)c_ttg[j * nv + i];
+    gu[j] = u[l];
+    guh[j] = uh[l];
+    gl[j] = e_leng[l];
+    gd[j] = e_dleng[l];
+  }
+#pragma unroll
+  for (int j = 0; j < MX; ++j) {
+    if (j >= n) continue;
+    s = s + sgn[j] * guh[j] * gd[j];
+    sd = sd + sgn[j] * gu[j] * gd[j];
+    const double ed_area = 0.25 * gl[j] * gd[j];
     ca = ca + ed_area;
     // melv (HTC): sum of ed_area uh u
-    k = (kmode == IMX_REC_MELV) ? k + ed_area * uh[l] * u[l] : k + ed_area * (u[l] * u[l]);
+    k = (kmode == IMX_REC_MELV) ? k + ed_area * guh[j] * gu[j] : k + ed_area * (gu[j] * gu[j]);
   }
   const double dv = s / c_area[i] / erad;
   divuh[i] = dv;
@@ -279,47 +307,119 @@ __global__ __launch_bounds__(TPB) void ref_cell(int nv, const int32_t *__restric
   }
   ke[i] = kk;
   ghbk[i] = grav * (h[i] + bt[i]) + kk;
+  rk.update(i, -dv);  // may overwrite h[i], which no other cell reads
+}
+
+// Two operators that do not read each other's results share a launch: flux
+// and depth at edges with the triangles (which take gass18's depth from the
+// edges: there the triangles come second), and PV at edges with the cells.
+// A launch costs 1.8 us of the step's 80 at glevel 5.
+struct RefPre {
+  int ne, nt, nbe;  // nbe blocks of edges, then blocks of triangles
+  const int32_t *e_v;
+  const double *hb;
+  const int32_t *hv;
+  const double *h, *u;
+  double *h_ed, *uh;
+  const int32_t *t_ed;
+  const int8_t *t_tg;
+  const int32_t *t_v;
+  const double *t_area, *t_f, *t_trhx, *e_leng;
+  int hmode;
+  const double *t_w;
+  double erad;
+  int use_pv, flin;
+  double *eta, *zeta, *h_tr, *q_tr;
+  int *flag;
+};
+__global__ __launch_bounds__(TPB) void ref_pre(const RefPre a) {
+  if ((int)blockIdx.x < a.nbe)
+    ref_edge_flux(part_index(blockIdx.x, a.nbe), a.ne, a.e_v, a.hb, a.hv, a.h, a.u, a.h_ed, a.uh);
+  else
+    ref_tri(part_index(blockIdx.x - a.nbe, gridDim.x - a.nbe), a.nt, a.t_ed, a.t_tg, a.t_v, a.t_area, a.t_f, a.t_trhx,
+            a.e_leng, a.u, a.h, a.hmode, a.t_w, a.h_ed, a.erad, a.use_pv, a.flin, a.eta, a.zeta, a.h_tr, a.q_tr,
+            a.flag);
+}
+
+struct RefMid {
+  int ne, nv, nbe;  // nbe blocks of edges, then blocks of cells
+  int qmode;
+  const int32_t *e_sh;
+  const double *e_dw, *t_area, *eta, *h_tr, *q_tr;
+  double *q_ed, *eta_ed;
+  int *flag;
+  const int32_t *c_nnb, *c_ed;
+  const int8_t *c_ttg;
+  const double *c_area, *e_leng, *e_dleng, *u, *uh, *h, *bt;
+  int kmode;
+  const double *vhx, *vuh, *ketr;
+  const int32_t *c_tr;
+  const double *c_hxtr;
+  double gcoef, erad, grav;
+  double *divuh, *masseq, *divu, *ke, *ghbk;
+  RefRk rk;
+};
+__global__ __launch_bounds__(TPB) void ref_mid(const RefMid a) {
+  if ((int)blockIdx.x < a.nbe)
+    ref_edge_q(part_index(blockIdx.x, a.nbe), a.ne, a.qmode, a.e_sh, a.e_dw, a.t_area, a.eta, a.h_tr, a.q_tr, a.q_ed,
+               a.eta_ed, a.flag);
+  else
+    ref_cell(part_index(blockIdx.x - a.nbe, gridDim.x - a.nbe), a.nv, a.c_nnb, a.c_ed, a.c_ttg, a.c_area, a.e_leng,
+             a.e_dleng, a.u, a.uh, a.h, a.bt, a.kmode, a.vhx, a.vuh, a.ketr, a.c_tr, a.c_hxtr, a.gcoef, a.erad, a.grav,
+             a.divuh, a.masseq, a.divu, a.ke, a.ghbk, a.rk);
 }
 
 // grad_ed (HTC) + coriolis_ed (trsk, PV form) -> momeq
 // (swm_operators.f90:535-542, :1283-1309; swm.f90:2542, :2567)
+// All ring ids are loaded before the gathers and all gathers before the sum,
+// which stays in the reference's order; GASS: the gass Coriolis term's linking
+// edges (e_ed3). Bound by the term tables (252 B per edge) at glevel 8.
+template <bool GASS>
 __global__ __launch_bounds__(TPB) void ref_edge_mom(
-    int ne, int nv, const int32_t *__restrict__ e_v, const int8_t *__restrict__ e_loc,
-    const double *__restrict__ e_leng, const double *__restrict__ e_dleng,
-    const int32_t *__restrict__ c_nnb, const int32_t *__restrict__ c_ed,
-    const int8_t *__restrict__ c_ttg, const int8_t *__restrict__ c_tnr,
-    const int32_t *__restrict__ e_tk, const double *__restrict__ e_tw, const double *__restrict__ e_tdl,
-    const int8_t *__restrict__ e_ts, const double *__restrict__ ghbk,
-    const double *__restrict__ uh, const double *__restrict__ q_ed,
-    const int32_t *__restrict__ e_ed3, const int8_t *__restrict__ e_gs, double erad,
-    int zero_mom, double *__restrict__ grad, double *__restrict__ uhq,
-    double *__restrict__ momeq) {
-  const int l = xcd_index();
+    int ne, const int32_t *__restrict__ e_v, const double *__restrict__ e_leng, const int32_t *__restrict__ e_tk,
+    const double *__restrict__ e_tw, const double *__restrict__ e_tdl, const int8_t *__restrict__ e_ts,
+    const double *__restrict__ ghbk, const double *__restrict__ uh, const double *__restrict__ q_ed,
+    const int32_t *__restrict__ e_ed3, const int8_t *__restrict__ e_gs, double erad, int zero_mom,
+    double *__restrict__ grad, double *__restrict__ uhq, double *__restrict__ momeq, RefRk rk) {
+  const int l = part_index(blockIdx.x, gridDim.x);
   if (l >= ne || e_v[l] < 0) return;
-  // grad_ed: HC orients the difference by edhx%nr (e_gs)
-  const double gs = e_gs ? (double)e_gs[l] : 1.0;
-  const double g = gs * (ghbk[e_v[ne + l]] - ghbk[e_v[l]]) / e_leng[l] / erad;
-  grad[l] = g;
-  double s = 0.0;
-  const double ql = q_ed[l];
   // the terms in the reference's order (cell 1 then cell 2, each cell's
   // edges in ring order), ring edges and weights from the edge-major term
   // tables (coalesced) instead of the cell-major weight table
+  int k[2 * MX], k3[2 * MX];
+#pragma unroll
+  for (int t = 0; t < 2 * MX; ++t) {
+    k[t] = e_tk[t * ne + l];
+    k3[t] = GASS ? e_ed3[t * ne + l] : -1;
+  }
+  const double ql = q_ed[l], len = e_leng[l];
+  double gu[2 * MX], gq[2 * MX];
+#pragma unroll
+  for (int t = 0; t < 2 * MX; ++t) {
+    const int kt = k[t] < 0 ? l : k[t];
+    gu[t] = uh[kt];
+    // gass18: q of the rhombus linking edges l and k where there is one
+    gq[t] = q_ed[GASS && k3[t] >= 0 ? k3[t] : kt];
+  }
+  // grad_ed: HC orients the difference by edhx%nr (e_gs)
+  const double gs = e_gs ? (double)e_gs[l] : 1.0;
+  const double g = gs * (ghbk[e_v[ne + l]] - ghbk[e_v[l]]) / len / erad;
+  grad[l] = g;
+  double s = 0.0;
   // the sign of a term is dsign(1, ttgout(j) tnrccw(ei)) (HTC) or
   // dsign(1, hx%nr(j) hx%nr(ei)) (HC), tabulated per term
 #pragma unroll
   for (int t = 0; t < 2 * MX; ++t) {
-    const int k = e_tk[t * ne + l];
-    if (k < 0) continue;
     const double signcor = (double)e_ts[t * ne + l];
-    // gass18: q of the rhombus linking edges l and k where there is one
-    const int e3 = e_ed3 ? e_ed3[t * ne + l] : -1;
-    const double qtmp = e3 >= 0 ? q_ed[e3] : 0.5 * (ql + q_ed[k]);
-    s = s + uh[k] * qtmp * e_tdl[t * ne + l] * e_tw[t * ne + l] * signcor;
+    const double qtmp = GASS && k3[t] >= 0 ? gq[t] : 0.5 * (ql + gq[t]);
+    const double term = gu[t] * qtmp * e_tdl[t * ne + l] * e_tw[t * ne + l] * signcor;
+    if (k[t] >= 0) s = s + term;
   }
-  const double p = s / e_leng[l];
+  const double p = s / len;
   uhq[l] = p;
-  momeq[l] = zero_mom ? 0.0 : (-g) - p;
+  const double f = zero_mom ? 0.0 : (-g) - p;
+  momeq[l] = f;
+  rk.update(l, f);
 }
 
 // ---- scheme options of the REF path (APVM, diffusion, hyperdiffusion) ----
@@ -665,23 +765,11 @@ __global__ __launch_bounds__(TPB) void ref_edge_mom_pered(
   momeq[l] = zero_mom ? 0.0 : (-g) - p;
 }
 
-// ode_rk4 combinations (swm.f90:2647-2678)
-__global__ __launch_bounds__(TPB) void ref_rk_stage(int n, const double *__restrict__ y,
-                                                    const double *__restrict__ k, double dt,
-                                                    int half, double *__restrict__ yn) {
-  const int i = xcd_index();
-  if (i >= n) return;
-  yn[i] = half ? y[i] + dt * k[i] / 2.0 : y[i] + dt * k[i];
-}
-
-__global__ __launch_bounds__(TPB) void ref_rk_final(int n, double *__restrict__ y,
-                                                    const double *__restrict__ k0,
-                                                    const double *__restrict__ k1,
-                                                    const double *__restrict__ k2,
-                                                    const double *__restrict__ k3, double dt) {
-  const int i = xcd_index();
-  if (i >= n) return;
-  y[i] = y[i] + dt * (k0[i] + 2.0 * k1[i] + 2.0 * k2[i] + k3[i]) / 6.0;
+// The same for edges whose tendency a later kernel has changed or whose
+// neighbours' momentum kernel reads the stage's u.
+__global__ __launch_bounds__(TPB) void ref_rk(int n, const double *__restrict__ f, RefRk rk) {
+  const int i = part_index(blockIdx.x, gridDim.x);
+  if (i < n) rk.update(i, f[i]);
 }
 
 // =========================================================== FAST kernels ==
@@ -1563,29 +1651,35 @@ static std::vector<T> cvt(const std::vector<double> &a) {
 }
 
 // --------------------------------------------------------------- launches --
-static void launch_ref_tendency(imx_swm *s, const double *h, const double *u, double *masseq,
-                                double *momeq) {
+// The RK use of the tendency (of h and of u) goes to the kernels that form it;
+// true when the momentum's is left to the caller.
+static bool launch_ref_tendency(imx_swm *s, const double *h, const double *u, double *masseq,
+                                double *momeq, const RefRk &rkh = RefRk(), const RefRk &rku = RefRk()) {
   const int nv = s->nv, NE = s->NE, NT = s->NT;
   hipStream_t st = s->stream;
+  // small blocks until there are enough for every CU
+  const int bs = NE < 262144 ? 64 : TPB;
   // the method triple: scalar interpolation, Coriolis, kinetic energy
   const int sint = s->sc_sint, cor = s->sc_cor, rec = s->sc_rec;
   // the staggering's signs and Perot edge points (HC: hx%nr, edhx%c, ...)
   const bool hc = s->sc_hc;
-  const int8_t *csg = hc ? s->hc_c : s->c_ttg, *ctn = hc ? s->hc_c : s->c_tnr;
+  const int8_t *csg = hc ? s->hc_c : s->c_ttg;
   const int8_t *tsg = hc ? s->hc_t : s->t_tg, *egs = hc ? s->hc_g : nullptr;
   const int8_t *ett = hc ? s->hc_tt : s->e_nrs;
   const double *epc = hc ? s->hc_pc : s->e_c;
   const int qmode = sint == IMX_SINT_GASS ? (hc ? 3 : 2) : (!hc && sint == IMX_SINT_BARY ? 1 : 0);
   const bool hbary = hc && sint == IMX_SINT_BARY;
-  ref_edge_flux<<<grid_for(NE), TPB, 0, st>>>(NE, s->e_v, hbary ? s->hc_hb : nullptr, s->hc_hv, h, u,
-                                              s->f_h_ed, s->f_uh);
-  ref_tri<<<grid_for(NT), TPB, 0, st>>>(NT, s->t_ed, tsg, s->t_v, s->t_area, s->t_f,
-                                        s->t_trhx, s->e_leng, u, h, sint, s->t_w, s->f_h_ed,
-                                        s->o.erad, s->o.testcase >= 2, s->f_lin ? 1 : 0, s->f_eta, s->f_zeta,
-                                        s->f_h_tr, s->f_q_tr, s->flag);
-  ref_edge_q<<<grid_for(NE), TPB, 0, st>>>(NE, qmode, s->e_sh, s->e_dw, s->t_area, s->f_eta, s->f_h_tr,
-                                           s->f_q_tr, s->f_q_ed, s->sc_nopv ? s->f_eta_ed : nullptr,
-                                           s->flag);
+  RefPre pre{NE, NT, grid_bs(NE, bs), s->e_v, hbary ? s->hc_hb : nullptr, s->hc_hv, h, u, s->f_h_ed, s->f_uh,
+             s->t_ed, tsg, s->t_v, s->t_area, s->t_f, s->t_trhx, s->e_leng, sint, s->t_w, s->o.erad,
+             s->o.testcase >= 2, s->f_lin ? 1 : 0, s->f_eta, s->f_zeta, s->f_h_tr, s->f_q_tr, s->flag};
+  const int gt = grid_bs(NT, bs);
+  if (sint == IMX_SINT_GASS) {  // the triangles read the edges' depths
+    ref_pre<<<pre.nbe, bs, 0, st>>>(pre);
+    pre.nbe = 0;
+    ref_pre<<<gt, bs, 0, st>>>(pre);
+  } else {
+    ref_pre<<<pre.nbe + gt, bs, 0, st>>>(pre);
+  }
   // Perot velocity at cells: APVM, the pxt16 and Melvin kinetic energies
   // (vector_edhx2hx_perot, swm.f90:2516)
   if (s->sc_apvm || rec == IMX_REC_PERHX || (hc && rec == IMX_REC_MELV))
@@ -1596,6 +1690,12 @@ static void launch_ref_tendency(imx_swm *s, const double *h, const double *u, do
                                                s->e_dleng, s->c_area, s->f_uh, s->f_vuh);
   if (rec == IMX_REC_GASS)  // kinetic_energy_tr (swm.f90:2521-2523)
     ref_ketr<<<grid_for(NT), TPB, 0, st>>>(NT, s->t_ed, s->t_ka, s->t_area, u, s->f_ketr);
+  const RefMid mid{NE, nv, grid_bs(NE, bs), qmode, s->e_sh, s->e_dw, s->t_area, s->f_eta, s->f_h_tr, s->f_q_tr,
+                   s->f_q_ed, s->sc_nopv ? s->f_eta_ed : nullptr, s->flag, s->c_nnb, s->c_ed, csg, s->c_area,
+                   s->e_leng, s->e_dleng, u, s->f_uh, h, s->bt, rec, s->f_vhx,
+                   (hc && rec == IMX_REC_MELV) ? s->f_vuh : nullptr, s->f_ketr, s->c_tr, s->c_hxtr, s->sc_gcoef,
+                   s->o.erad, s->o.grav, s->f_divuh, masseq, s->f_divu, s->f_ke, s->f_ghbk, rkh};
+  ref_mid<<<mid.nbe + grid_bs(nv, bs), bs, 0, st>>>(mid);
   if (cor == IMX_COR_DTRED)  // vhq_tr (swm.f90:2501-2503)
     ref_lte_tr<<<grid_for(NT), TPB, 0, st>>>(NT, NE, s->t_ed, tsg, epc, s->t_c, s->e_leng, s->t_area, s->f_uh,
                                              s->f_q_tr, s->f_vhq);
@@ -1609,11 +1709,6 @@ static void launch_ref_tendency(imx_swm *s, const double *h, const double *u, do
     ref_apvm_q<<<grid_for(NE), TPB, 0, st>>>(NE, NT, nv, s->e_sh, s->e_v, s->f_qg_tr, s->f_vhx,
                                              s->sc.pvspar, s->o.dt, s->f_q_ed);
   }
-  ref_cell<<<grid_for(nv), TPB, 0, st>>>(nv, s->c_nnb, s->c_ed, csg, s->c_area, s->e_leng,
-                                         s->e_dleng, u, s->f_uh, h, s->bt, rec, s->f_vhx,
-                                         (hc && rec == IMX_REC_MELV) ? s->f_vuh : nullptr, s->f_ketr, s->c_tr,
-                                         s->c_hxtr, s->sc_gcoef, s->o.erad, s->o.grav, s->f_divuh, masseq,
-                                         s->f_divu, s->f_ke, s->f_ghbk);
   if (cor == IMX_COR_DTRED)
     ref_edge_mom_dtred<<<grid_for(NE), TPB, 0, st>>>(NE, NT, s->e_v, s->e_sh, s->e_leng, s->e_dw, s->e_c, s->e_nr,
                                                      s->f_vhq, s->f_ghbk, egs, hc ? 1 : 0, s->o.erad,
@@ -1624,14 +1719,23 @@ static void launch_ref_tendency(imx_swm *s, const double *h, const double *u, do
                                                      s->c_area, s->f_ghbk, s->f_uh, s->f_q_ed, egs,
                                                      hc ? 1.0 : -1.0, s->o.erad, s->o.testcase <= 1,
                                                      s->f_grad, s->f_uhq, momeq);
-  else
-    ref_edge_mom<<<grid_for(NE), TPB, 0, st>>>(NE, nv, s->e_v, s->e_loc, s->e_leng, s->e_dleng,
-                                               s->c_nnb, s->c_ed, csg, ctn, s->e_tk, s->e_tw, s->e_tdl,
-                                               hc ? s->hc_ts : s->e_ts, s->f_ghbk,
-                                               s->sc_nopv ? u : s->f_uh,             // level model:
-                                               s->sc_nopv ? s->f_eta_ed : s->f_q_ed,  // u and eta
-                                               cor == IMX_COR_GASS ? s->e_ed3 : nullptr, egs, s->o.erad,
-                                               s->o.testcase <= 1, s->f_grad, s->f_uhq, momeq);
+  else {
+    // the level model reads u and eta in place of uh and q: u of the stage,
+    // which the update would overwrite under its neighbours
+    const bool fold = !s->sc_nopv && !s->sc_diff && !s->sc_hyper;
+    const double *fu = s->sc_nopv ? u : s->f_uh, *fq = s->sc_nopv ? s->f_eta_ed : s->f_q_ed;
+    const int8_t *ts = hc ? s->hc_ts : s->e_ts;
+    const RefRk rk = fold ? rku : RefRk();
+    if (cor == IMX_COR_GASS)
+      ref_edge_mom<true><<<grid_bs(NE, bs), bs, 0, st>>>(NE, s->e_v, s->e_leng, s->e_tk, s->e_tw, s->e_tdl, ts,
+                                                         s->f_ghbk, fu, fq, s->e_ed3, egs, s->o.erad,
+                                                         s->o.testcase <= 1, s->f_grad, s->f_uhq, momeq, rk);
+    else
+      ref_edge_mom<false><<<grid_bs(NE, bs), bs, 0, st>>>(NE, s->e_v, s->e_leng, s->e_tk, s->e_tw, s->e_tdl, ts,
+                                                          s->f_ghbk, fu, fq, nullptr, egs, s->o.erad,
+                                                          s->o.testcase <= 1, s->f_grad, s->f_uhq, momeq, rk);
+    if (fold) return false;
+  }
   if (s->sc_diff || s->sc_hyper) {
     // diffusion_ed of u (momeq + lapu with K2), then with K4 diffusion_ed of
     // lapu's divergence and vorticity (momeq - lap_lapu) (swm.f90:2575-2590);
@@ -1650,26 +1754,27 @@ static void launch_ref_tendency(imx_swm *s, const double *h, const double *u, do
                                             live ? 2 : 0, s->f_lap2, momeq);
     }
   }
+  return true;
 }
 
 static void launch_ref_step(imx_swm *s) {
   const int nv = s->nv, NE = s->NE;
-  const double dt = s->o.dt;
-  hipStream_t st = s->stream;
   double *m[4], *f[4];
   for (int k = 0; k < 4; ++k) {
     m[k] = s->massf + (size_t)k * nv;
     f[k] = s->momf + (size_t)k * NE;
   }
-  launch_ref_tendency(s, s->rh, s->ru, m[0], f[0]);
-  for (int k = 0; k < 3; ++k) {
-    const int half = (k < 2);
-    ref_rk_stage<<<grid_for(NE), TPB, 0, st>>>(NE, s->ru, f[k], dt, half, s->run);
-    ref_rk_stage<<<grid_for(nv), TPB, 0, st>>>(nv, s->rh, m[k], dt, half, s->rhn);
-    launch_ref_tendency(s, s->rhn, s->run, m[k + 1], f[k + 1]);
+  for (int k = 0; k < 4; ++k) {
+    RefRk rh, ru;
+    rh.kind = ru.kind = k < 2 ? 1 : k;
+    rh.dt = ru.dt = s->o.dt;
+    rh.y = s->rh, ru.y = s->ru;
+    rh.out = k < 3 ? s->rhn : s->rh, ru.out = k < 3 ? s->run : s->ru;
+    rh.k0 = m[0], rh.k1 = m[1], rh.k2 = m[2];
+    ru.k0 = f[0], ru.k1 = f[1], ru.k2 = f[2];
+    if (launch_ref_tendency(s, k ? s->rhn : s->rh, k ? s->run : s->ru, m[k], f[k], rh, ru))
+      ref_rk<<<grid_for(NE), TPB, 0, s->stream>>>(NE, f[k], ru);
   }
-  ref_rk_final<<<grid_for(NE), TPB, 0, st>>>(NE, s->ru, f[0], f[1], f[2], f[3], dt);
-  ref_rk_final<<<grid_for(nv), TPB, 0, st>>>(nv, s->rh, m[0], m[1], m[2], m[3], dt);
 }
 
 // Block-size dispatch of the fused kernels (the autotuner's search space).
