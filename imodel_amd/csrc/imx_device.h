@@ -296,6 +296,7 @@ struct imx_mlp {
   float *P = nullptr, *M = nullptr, *V = nullptr, *G = nullptr, *part = nullptr, *lossp = nullptr;
   short *Ff = nullptr, *Fb = nullptr;  // K16 fragments of the training kernels
   short *Ff32 = nullptr;                // K32 fragments of the inference kernel
+  short *F1g = nullptr;                 // layer 1 of them for features gathered in the kernel
   short *X = nullptr;
   float *T = nullptr, *w = nullptr, *Y = nullptr, *Xf = nullptr;
   int64_t cap = 0;  // edges the scratch holds
@@ -309,8 +310,9 @@ int mlp_forward_dev(imx_mlp *m, int64_t n, const short *X, float *Y, hipStream_t
 int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int apply, float *loss_part,
                   int gmask);
 int mlp_loss(imx_mlp *m, int64_t n, const float *loss_part, int passes, double *loss);
-// one fused RK4 step of a FAST handle, enqueued on its stream (no graph)
-void swm_launch_step(imx_swm *s);
+// one fused RK4 step of a FAST handle, enqueued on its stream (no graph); the
+// state after it goes to hout and uout (the handle's own arrays when null)
+void swm_launch_step(imx_swm *s, void *hout = nullptr, void *uout = nullptr);
 // waits for the handle's stream; IMX_ESTATE if a step met a vanishing depth
 int swm_check_flag(imx_swm *s, const char *what);
 

@@ -19,8 +19,8 @@
 // sum_c A_c h_c is unchanged. Training fits du to its target directly and
 // fits D F to the dh target through D (the gradient D^T r is handed to the
 // MLP backward pass). The correction is skipped (plain step kept) when its
-// RMS exceeds a bound. The corrected step (save, RK4 step, features, MLP,
-// correction) is captured; one graph launch runs up to 16 of them.
+// RMS exceeds a bound. The corrected step (RK4 step, network with the features
+// formed in its kernel, correction) is captured; one graph launch runs up to 16 of them.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
@@ -51,7 +51,8 @@ struct imx_learn {
   float *de = nullptr;      // [2][NE] coefficient of F_e in (D F) at e_v[0/1][e]
   void *hn = nullptr, *un = nullptr;  // state before the step (T)
   float *raw = nullptr;     // [NE][NF]
-  float *mu = nullptr, *sig = nullptr;
+  float *mu = nullptr, *sig = nullptr, *norm = nullptr;  // norm: FeatLoader's order
+  void *hq = nullptr, *uq = nullptr;  // state after the plain step of a corrected one (T)
   float tsu = 1.f, tsh = 1.f;
   float *Y = nullptr;       // [NE][2]
   float *wv = nullptr;      // [NE] 1/ne on real edges
@@ -64,7 +65,6 @@ struct imx_learn {
   float *lossu = nullptr;   // [kLossSteps][(NE + 63) / 64] their u loss partials
   int *nfb = nullptr;       // [1] limited steps since the counter was cleared
   imx::StepGraphs graphs;
-  const short *gX = nullptr;  // MLP input buffer the graph was captured with
   uint64_t gen = 0;           // the step handle's generation at capture
   // device sample store: normalised features, scaled targets
   int cap = 0, count = 0;
@@ -84,14 +84,20 @@ __global__ __launch_bounds__(LTPB) void learn_save(int nv, int NE, const T *__re
   if (i < nv) hn[i] = h[i];
 }
 
-// Features of (saved state un/hn, plain step up/hp), one thread per edge
-// slot: the 128-byte stencil record is read with vector loads and all 42
-// state gathers are issued before any is used, so a thread keeps its
-// loads in flight together (one feature per thread would chain a record
-// read and a gather for every feature). Record words: 0-10 ring edges
-// (id << 1 | sign bit, -1 pad; word 0 is the edge itself, -1 for a dummy
-// slot), 11-20 stencil cells (-1 pad), 21-26 geometry features (FP32
-// bits). Dummy slots get all-zero raw features.
+// Stencil record of an edge, 32 words in four quarters of 8, one per lane
+// group of the network kernel (mlp_feature_slot): words 0-4 the quarter's ids
+// j = 0..4 (id << 1 | sign, -1 pad), word 5 id 5 (quarter 3), words 6, 7 two
+// geometry features (FP32 bits; quarters 0-2). Dummy slots: no ids, zeros.
+__host__ __device__ inline int rec_edge(int k) { return k / 5 * 8 + k % 5; }
+__host__ __device__ inline int rec_cell(int k) { return k < 4 ? 17 + k : 20 + k; }
+__host__ __device__ inline int rec_geo(int k) { return k / 2 * 8 + 6 + k % 2; }
+
+// Features of (saved state un/hn, plain step up/hp) for sampling and
+// training, one thread per edge slot: the stencil record is read with vector
+// loads and all 42 state gathers are issued before any is used, so a thread
+// keeps its loads in flight together (one feature per thread would chain a
+// record read and a gather for every feature). Dummy slots get all-zero raw
+// features.
 template <typename T>
 __global__ __launch_bounds__(LTPB) void learn_featx(int NE, const int32_t *__restrict__ stn,
                                                     const T *__restrict__ un, const T *__restrict__ hn,
@@ -101,48 +107,48 @@ __global__ __launch_bounds__(LTPB) void learn_featx(int NE, const int32_t *__res
                                                     float *__restrict__ raw, short *__restrict__ X) {
   const int e = blockIdx.x * LTPB + threadIdx.x;
   if (e >= NE) return;
-  int32_t r[28];
+  int32_t r[SREC];
   const int4 *rv = reinterpret_cast<const int4 *>(stn + (int64_t)e * SREC);
 #pragma unroll
-  for (int q = 0; q < 7; ++q) {
+  for (int q = 0; q < SREC / 4; ++q) {
     const int4 v = rv[q];
     r[4 * q] = v.x;
     r[4 * q + 1] = v.y;
     r[4 * q + 2] = v.z;
     r[4 * q + 3] = v.w;
   }
-  const bool real = r[0] >= 0;
   float f[NF];
   T a[NSE], b[NSE], c0[NSC], c1[NSC];
 #pragma unroll
   for (int k = 0; k < NSE; ++k) {
-    const int w = r[k];
-    const int ek = (real && w >= 0) ? (w >> 1) : 0;
+    const int w = r[rec_edge(k)];
+    const int ek = w >= 0 ? w >> 1 : 0;
     a[k] = un[ek];
     b[k] = up[ek];
   }
 #pragma unroll
   for (int k = 0; k < NSC; ++k) {
-    const int c = (real && r[NSE + k] >= 0) ? r[NSE + k] : 0;
+    const int w = r[rec_cell(k)];
+    const int c = w >= 0 ? w >> 1 : 0;
     c0[k] = hn[c];
     c1[k] = hp[c];
   }
 #pragma unroll
   for (int k = 0; k < NSE; ++k) {
-    const int w = r[k];
-    const bool ok = real && w >= 0;
+    const int w = r[rec_edge(k)];
+    const bool ok = w >= 0;
     const float sg = (w & 1) ? -1.f : 1.f;
     f[k] = ok ? sg * (float)a[k] : 0.f;
     f[NSE + k] = ok ? sg * (float)(b[k] - a[k]) : 0.f;
   }
 #pragma unroll
   for (int k = 0; k < NSC; ++k) {
-    const bool ok = real && r[NSE + k] >= 0;
+    const bool ok = r[rec_cell(k)] >= 0;
     f[2 * NSE + k] = ok ? (float)c0[k] : 0.f;
     f[2 * NSE + NSC + k] = ok ? (float)(c1[k] - c0[k]) : 0.f;
   }
 #pragma unroll
-  for (int k = 0; k < 6; ++k) f[2 * NSE + 2 * NSC + k] = real ? __int_as_float(r[NSE + NSC + k]) : 0.f;
+  for (int k = 0; k < 6; ++k) f[2 * NSE + 2 * NSC + k] = __int_as_float(r[rec_geo(k)]);
   const int64_t o = (int64_t)e * NF;
   if (raw) {
     float4 *rw = reinterpret_cast<float4 *>(raw + o);
@@ -160,6 +166,77 @@ __global__ __launch_bounds__(LTPB) void learn_featx(int NE, const int32_t *__res
     }
   }
 }
+
+// Input fragments of the network formed in its own kernel: the features of
+// learn_featx in the slots of mlp_feature_slot. The four lanes of an edge read
+// its record as consecutive 32-byte quarters and gather six ids each; the
+// normalised row (96 bytes written and read per edge) never exists: 385 us at
+// glevel 8 instead of 147 for the rows and 301 for the network on them. The
+// kernel is bound by its activations, two waves a SIMD; fetching the next
+// tile's record, or its gathers too, a tile ahead did not help (395 us, and
+// 424 with registers spilled). norm: per lane group 12 means, 12 deviations.
+template <typename T>
+struct FeatLoader {
+  static constexpr int kNorm = 24;
+  const int32_t *stn;
+  const T *un, *hn, *up, *hp;
+  const float *norm;
+  __device__ __forceinline__ void prepare(float *sh) const {
+    for (int i = threadIdx.x; i < 4 * kNorm; i += blockDim.x) sh[64 * (i / kNorm) + i % kNorm] = norm[i];
+  }
+  template <int ET>
+  __device__ __forceinline__ void operator()(int64_t e0, int64_t n, int lane, v4s (&x)[3][ET], const float *sh) const {
+    const int g = lane / 16;
+    // id 0 is an edge's in groups 0-2, the others in groups 0 and 1
+    const T *a0 = g < 3 ? un : hn, *b0 = g < 3 ? up : hp, *a1 = g < 2 ? un : hn, *b1 = g < 2 ? up : hp;
+    int w[ET][8];
+    T a[ET][6], b[ET][6];
+#pragma unroll
+    for (int t = 0; t < ET; ++t) {
+      int64_t e = e0 + 16 * t + lane % 16;
+      if (e >= n) e = n - 1;
+      const int4 *r = reinterpret_cast<const int4 *>(stn + e * SREC + 8 * g);
+      const int4 p = r[0], q = r[1];
+      w[t][0] = p.x, w[t][1] = p.y, w[t][2] = p.z, w[t][3] = p.w;
+      w[t][4] = q.x, w[t][5] = q.y, w[t][6] = q.z, w[t][7] = q.w;
+    }
+#pragma unroll
+    for (int t = 0; t < ET; ++t)
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        const int id = w[t][j] < 0 ? 0 : w[t][j] >> 1;
+        a[t][j] = (j ? a1 : a0)[id];
+        b[t][j] = (j ? b1 : b0)[id];
+      }
+    const float *m = sh + 64 * g;
+#pragma unroll
+    for (int t = 0; t < ET; ++t) {
+      float f[12];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        const bool ok = w[t][j] >= 0;
+        const float sg = (w[t][j] & 1) ? -1.f : 1.f;
+        f[2 * j] = ok ? sg * (float)a[t][j] : 0.f;
+        f[2 * j + 1] = ok ? sg * (float)(b[t][j] - a[t][j]) : 0.f;
+      }
+      if (g < 3) {
+        f[10] = __int_as_float(w[t][6]);
+        f[11] = __int_as_float(w[t][7]);
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        float q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int s = 4 * k + i;
+          q[i] = (f[s] - m[s]) / m[12 + s];
+        }
+        const uint32_t v[2] = {f2bf2(q[0], q[1]), f2bf2(q[2], q[3])};
+        x[k][t] = __builtin_bit_cast(v4s, v);
+      }
+    }
+  }
+};
 
 // out_c = (D F)_c - t_c (t may be NULL), F = the flux output Y[.][1]
 __global__ __launch_bounds__(LTPB) void learn_div(int nv, const int32_t *__restrict__ c_nnb,
@@ -251,13 +328,15 @@ __global__ __launch_bounds__(LTPB) void learn_div_part(int nv, int NE, const int
 }
 
 // every block sums the LPART partials (fixed order: the same RMS in every
-// block), then applies u += Y0/tsu and h += (D F)/tsh unless RMS > bound
+// block), then the state u, h becomes the plain step's up, hp plus Y0/tsu and
+// (D F)/tsh, or the plain step's where RMS > bound
 template <typename T>
 __global__ __launch_bounds__(LTPB) void learn_apply(int nv, int NE, const float *__restrict__ wv,
                                                     const float *__restrict__ Y,
                                                     const float *__restrict__ dhc, float inv_tsu,
                                                     float inv_tsh, const double *__restrict__ part,
-                                                    const double *__restrict__ bound, T *u, T *h,
+                                                    const double *__restrict__ bound, const T *__restrict__ up,
+                                                    const T *__restrict__ hp, T *__restrict__ u, T *__restrict__ h,
                                                     double *__restrict__ rms, int *__restrict__ nfb) {
   __shared__ double red[LTPB];
   double p = 0.0;
@@ -281,9 +360,9 @@ __global__ __launch_bounds__(LTPB) void learn_apply(int nv, int NE, const float 
     rms[0] = r;
     if (!ok) nfb[0] = nfb[0] + 1;  // one thread of the grid counts
   }
-  if (!(sc > 0.f)) return;
-  if (i < NE && wv[i] > 0.f) u[i] = (T)((float)u[i] + sc * (Y[2 * i] * inv_tsu));
-  if (i < nv) h[i] = (T)((float)h[i] + sc * (dhc[i] * inv_tsh));
+  const bool on = sc > 0.f;
+  if (i < NE && wv[i] > 0.f) u[i] = on ? (T)((float)up[i] + sc * (Y[2 * i] * inv_tsu)) : up[i];
+  if (i < nv) h[i] = on ? (T)((float)hp[i] + sc * (dhc[i] * inv_tsh)) : hp[i];
 }
 
 namespace imx {
@@ -332,20 +411,23 @@ static void learn_free_store(imx_learn *L) {
   L->cap = L->count = 0;
 }
 
-// enqueue: features -> MLP -> correction (with the RMS bound) on the state
+// enqueue: one corrected step: the plain step into hq, uq, the network on
+// features gathered from both states, the correction (with the RMS bound)
+// back into the handle's state
 template <typename T>
-static int learn_enqueue_correct(imx_learn *L) {
+static int learn_enqueue_step(imx_learn *L) {
   imx_swm *s = L->s;
   hipStream_t st = s->stream;
-  learn_enqueue_featx_t<T>(L, st, nullptr, L->m->X);
-  int rc = mlp_forward_dev(L->m, L->NE, L->m->X, L->Y, st);
-  if (rc) return rc;
+  swm_launch_step(s, L->hq, L->uq);
+  const FeatLoader<T> ld{L->stn, (const T *)s->u0, (const T *)s->h0, (const T *)L->uq, (const T *)L->hq, L->norm};
+  LTRY(mlp_fwd_launch(L->m->F1g, L->m->Ff32, L->m->P, L->NE, ld, L->Y, st), "mlp_fwd_lds");
   const int nmax = s->nv > L->NE ? s->nv : L->NE;
   learn_div_part<<<LPART, LTPB, 0, st>>>(s->nv, L->NE, s->c_nnb, s->c_ed, L->dc, L->Y, L->wv, L->dhc,
                                          L->part);
   learn_apply<T><<<(nmax + LTPB - 1) / LTPB, LTPB, 0, st>>>(s->nv, L->NE, L->wv, L->Y, L->dhc,
                                                            1.f / L->tsu, 1.f / L->tsh, L->part, L->bound,
-                                                           (T *)s->u0, (T *)s->h0, L->rms, L->nfb);
+                                                           (const T *)L->uq, (const T *)L->hq, (T *)s->u0,
+                                                           (T *)s->h0, L->rms, L->nfb);
   LTRY(hipGetLastError(), "learn_apply");
   return IMX_OK;
 }
@@ -358,25 +440,31 @@ static int learn_sample(imx_learn *L) {
 }
 
 static int learn_ensure_graphs(imx_learn *L, int nsteps) {
-  int rc = mlp_reserve(L->m, L->NE);
-  if (rc) return rc;
-  // recapture when the MLP scratch moved or the handle's step changed
-  // (scheme, tuning, topography, h_ref)
-  if (L->gX != L->m->X || L->gen != L->s->generation) learn_drop_graph(L);
-  L->gX = L->m->X;
+  // recapture when the handle's step changed (scheme, tuning, topography, h_ref)
+  if (L->gen != L->s->generation) learn_drop_graph(L);
   L->gen = L->s->generation;
   hipError_t e;
-  rc = L->graphs.ensure(nsteps, L->s->stream, [&] {
-    if (L->s->single) {
-      learn_enqueue_sample<float>(L);
-      return learn_enqueue_correct<float>(L);
-    }
-    learn_enqueue_sample<double>(L);
-    return learn_enqueue_correct<double>(L);
+  const int rc = L->graphs.ensure(nsteps, L->s->stream, [&] {
+    return L->s->single ? learn_enqueue_step<float>(L) : learn_enqueue_step<double>(L);
   }, e);
   if (rc) return rc;
   LTRY(e, "learn graph capture");
   return IMX_OK;
+}
+
+// FeatLoader's normalisation from the features' means and deviations
+static std::vector<float> learn_norm(const float *mu, const float *sig) {
+  constexpr int K = FeatLoader<float>::kNorm;
+  std::vector<float> v(4 * K, 0.f);
+  for (int q = 0; q < 4; ++q)
+    for (int s = 0; s < 12; ++s) v[K * q + 12 + s] = 1.f;
+  for (int f = 0; f < NF; ++f) {
+    int g, s;
+    mlp_feature_slot(f, &g, &s);
+    v[K * g + s] = mu[f];
+    v[K * g + 12 + s] = sig[f];
+  }
+  return v;
 }
 
 }  // namespace imx
@@ -399,7 +487,8 @@ int imx_learn_create(imx_swm *s, imx_mlp *m, const imx_mesh_desc *d, imx_learn *
   const std::vector<int32_t> &cn = s->lay.cell_new, &en = s->lay.edge_new;
   std::vector<int32_t> stn((size_t)SREC * NE, 0);
   for (int e = 0; e < NE; ++e)
-    for (int k = 0; k < NSE + NSC; ++k) stn[(size_t)e * SREC + k] = -1;
+    for (int k = 0; k < SREC; ++k)
+      if (k % 8 < 6) stn[(size_t)e * SREC + k] = -1;
   std::vector<float> wv(NE, 0.f);
   std::vector<float> dc((size_t)6 * nv, 0.f), de((size_t)2 * NE, 0.f);
   double ml = 0, md = 0, ma = 0;
@@ -431,7 +520,7 @@ int imx_learn_create(imx_swm *s, imx_mlp *m, const imx_mesh_desc *d, imx_learn *
       for (int j = 0; j < d->v_nnb[cell[q]]; ++j)
         if (d->v_ed[MX * cell[q] + j] == eo + 1) slot[q] = j;
     int32_t *rec = stn.data() + (size_t)e * SREC;
-    rec[0] = e << 1;
+    rec[rec_edge(0)] = e << 1;
     int k = 1;
     for (int q = 0; q < 2; ++q) {
       const int c = cell[q], n = d->v_nnb[c], i = slot[q];
@@ -439,7 +528,7 @@ int imx_learn_create(imx_swm *s, imx_mlp *m, const imx_mesh_desc *d, imx_learn *
         if (t >= n) continue;  // pentagon: one slot stays padded
         const int j = (i + t) % n;
         const int neg = d->hx_ttgout[MX * c + j] * d->hx_tnrccw[MX * c + i] < 0 ? 1 : 0;
-        rec[k] = (en[d->v_ed[MX * c + j] - 1] << 1) | neg;
+        rec[rec_edge(k)] = (en[d->v_ed[MX * c + j] - 1] << 1) | neg;
       }
     }
     // cells: c1, c2, left apex, right apex, other ring cells of c1 and c2
@@ -471,12 +560,12 @@ int imx_learn_create(imx_swm *s, imx_mlp *m, const imx_mesh_desc *d, imx_learn *
         cl[kc] = d->v_nb[MX * c + (i + t) % n] - 1;
       }
     }
-    for (int q = 0; q < NSC; ++q) rec[NSE + q] = cl[q] >= 0 ? cn[cl[q]] : -1;
+    for (int q = 0; q < NSC; ++q) rec[rec_cell(q)] = cl[q] >= 0 ? cn[cl[q]] << 1 : -1;
     const double z = d->ed_c[3 * eo + 2];
     const float geo[6] = {(float)z, (float)std::sqrt(std::max(0.0, 1 - z * z)),
                           (float)(d->ed_leng[eo] / ml), (float)(d->edhx_leng[eo] / md),
                           (float)(d->hx_areag[cell[0]] / ma), (float)(d->hx_areag[cell[1]] / ma)};
-    std::memcpy(rec + NSE + NSC, geo, sizeof(geo));
+    for (int q = 0; q < 6; ++q) std::memcpy(rec + rec_geo(q), geo + q, 4);
     wv[e] = 1.f / (float)d->ne;
   }
   imx::Alloc &A = L->A;
@@ -490,6 +579,12 @@ int imx_learn_create(imx_swm *s, imx_mlp *m, const imx_mesh_desc *d, imx_learn *
   L->raw = A.get<float>((size_t)NE * NF);
   L->mu = A.put(std::vector<float>(NF, 0.f));
   L->sig = A.put(std::vector<float>(NF, 1.f));
+  {
+    const std::vector<float> zero(NF, 0.f), one(NF, 1.f);
+    L->norm = A.put(imx::learn_norm(zero.data(), one.data()));
+  }
+  L->hq = A.get<char>(es * nv);
+  L->uq = A.get<char>(es * NE);
   L->Y = A.get<float>((size_t)2 * NE);
   L->dhc = A.get<float>(nv);
   L->th = A.get<float>(nv);
@@ -531,6 +626,8 @@ int imx_learn_set_scaling(imx_learn *L, const float *mu, const float *sig, float
     if (!(sig[j] > 0)) return imx::set_error(IMX_EINVAL, "imx_learn_set_scaling: sig must be positive");
   LTRY(hipMemcpy(L->mu, mu, NF * 4, hipMemcpyHostToDevice), "learn scaling");
   LTRY(hipMemcpy(L->sig, sig, NF * 4, hipMemcpyHostToDevice), "learn scaling");
+  const std::vector<float> norm = imx::learn_norm(mu, sig);
+  LTRY(hipMemcpy(L->norm, norm.data(), norm.size() * 4, hipMemcpyHostToDevice), "learn scaling");
   L->tsu = tscale_u;
   L->tsh = tscale_h;
   imx::learn_drop_graph(L);  // the scales are launch arguments of the graph

@@ -333,7 +333,8 @@ __global__ __launch_bounds__(TR_THREADS) void mlp_train(
 
 // The places of weight (row, col) of a layer in the fragment copies (the
 // inverse of mlp_pack's maps; layer 0-3, N output features)
-__device__ __forceinline__ void put_weight(int layer, int row, int col, short v, short *Ff, short *Fb, short *Ff32) {
+__device__ __forceinline__ void put_weight(int layer, int row, int col, short v, short *Ff, short *Fb, short *Ff32,
+                                           short *F1g) {
   const int KT = layer == 0 ? 3 : 8;
   const int fbase = layer == 0 ? FF_1 : layer == 1 ? FF_2 : layer == 2 ? FF_3 : FF_4;
   Ff[fbase + (((col / 16) * KT + row / 16) * 64 + (row % 16) / 4 * 16 + col % 16) * 4 + row % 4] = v;
@@ -343,9 +344,13 @@ __device__ __forceinline__ void put_weight(int layer, int row, int col, short v,
   }
   // K32: slot i of lane group g holds row kappa32(g, i) of its chunk
   const int r = row % 32, lane = (r % 16) / 4 * 16 + col % 16, i = r % 4 + (r < 16 ? 0 : 4);
-  if (layer == 0)
+  if (layer == 0) {
     Ff32[(col / 16) * 768 + (row < 32 ? lane * 8 + i : 512 + lane * 4 + row % 4)] = v;
-  else
+    int g, s;
+    mlp_feature_slot(row, &g, &s);
+    const int gl = g * 16 + col % 16;
+    F1g[(col / 16) * 768 + (s < 8 ? gl * 8 + s : 512 + gl * 4 + s - 8)] = v;
+  } else
     Ff32[fbase + (col / 16) * 2048 + (row / 32) * 512 + lane * 8 + i] = v;
 }
 
@@ -359,7 +364,8 @@ __global__ __launch_bounds__(64 * AW_GROUPS) void mlp_adamw(int nsplit, const fl
                                                  float *__restrict__ V, float *__restrict__ G, float lr,
                                                  float b1, float b2, float eps, float wd, float bc1,
                                                  float bc2, int apply, short *__restrict__ Ff,
-                                                 short *__restrict__ Fb, short *__restrict__ Ff32) {
+                                                 short *__restrict__ Fb, short *__restrict__ Ff32,
+                                                 short *__restrict__ F1g) {
   const int lane = threadIdx.x & 63, p = blockIdx.x * 64 + lane, grp = threadIdx.x >> 6;
   __shared__ float red[AW_GROUPS][64];
   float g = 0.f;
@@ -389,7 +395,7 @@ __global__ __launch_bounds__(64 * AW_GROUPS) void mlp_adamw(int nsplit, const fl
   const int layer = p < P_W2 ? 0 : p < P_W3 ? 1 : p < P_W4 ? 2 : 3;
   const int q = p - (layer == 0 ? P_W1 : layer == 1 ? P_W2 : layer == 2 ? P_W3 : P_W4);
   const int N = layer == 3 ? MLP_OUT : MLP_H;
-  put_weight(layer, q / N, q % N, f2bf(x), Ff, Fb, Ff32);
+  put_weight(layer, q / N, q % N, f2bf(x), Ff, Fb, Ff32, F1g);
 }
 
 // fragment copies from the FP32 master (forward: W^T tiles; backward: W tiles)
@@ -399,8 +405,16 @@ __global__ __launch_bounds__(64 * AW_GROUPS) void mlp_adamw(int nsplit, const fl
 __device__ __forceinline__ int kappa32(int g, int i) { return i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4); }
 
 __global__ __launch_bounds__(256) void mlp_pack(const float *__restrict__ P, short *__restrict__ Ff,
-                                                short *__restrict__ Fb, short *__restrict__ Ff32) {
+                                                short *__restrict__ Fb, short *__restrict__ Ff32,
+                                                short *__restrict__ F1g) {
   const int q = blockIdx.x * 256 + threadIdx.x;
+  if (q < MLP_IN * MLP_H) {  // layer 1 for gathered features
+    const int row = q / MLP_H, col = q % MLP_H;
+    int g, s;
+    mlp_feature_slot(row, &g, &s);
+    const int gl = g * 16 + col % 16;
+    F1g[(col / 16) * 768 + (s < 8 ? gl * 8 + s : 512 + gl * 4 + s - 8)] = f2bf(P[P_W1 + q]);
+  }
   // inference (K32) fragments: index -> (layer, output tile, chunk, lane, i)
   if (q < FF_N) {
     int row, col, N, poff;
@@ -527,7 +541,7 @@ void mlp_initial_params(uint64_t seed, std::vector<float> &P) {
 
 int mlp_pack_launch(imx_mlp *m) {
   const int n = FF_N > FB_N ? FF_N : FB_N;
-  mlp_pack<<<(n + 255) / 256, 256, 0, m->stream>>>(m->P, m->Ff, m->Fb, m->Ff32);
+  mlp_pack<<<(n + 255) / 256, 256, 0, m->stream>>>(m->P, m->Ff, m->Fb, m->Ff32, m->F1g);
   MTRY(hipGetLastError(), "mlp_pack");
   return IMX_OK;
 }
@@ -535,7 +549,7 @@ int mlp_pack_launch(imx_mlp *m) {
 // Forward on device buffers (X bf16 [n][48]) -> Y fp32 [n][2].
 int mlp_forward_dev(imx_mlp *m, int64_t n, const short *X, float *Y, hipStream_t st) {
   if (n <= 0) return IMX_OK;
-  MTRY(mlp_fwd_launch(m->Ff32, m->P, n, RowLoader{X}, Y, st), "mlp_fwd_lds");
+  MTRY(mlp_fwd_launch(m->Ff32, m->Ff32, m->P, n, RowLoader{X}, Y, st), "mlp_fwd_lds");
   return IMX_OK;
 }
 
@@ -554,7 +568,7 @@ int mlp_train_dev(imx_mlp *m, int64_t n, const short *X, float lr, float wd, int
   const float bc1 = 1.f - powf(b1, (float)(m->t > 0 ? m->t : 1));
   const float bc2 = 1.f - powf(b2, (float)(m->t > 0 ? m->t : 1));
   mlp_adamw<<<(P_N + 63) / 64, 64 * AW_GROUPS, 0, st>>>(blocks, m->part, m->P, m->M, m->V, m->G, lr, b1, b2, 1e-8f,
-                                                        wd, bc1, bc2, apply, m->Ff, m->Fb, m->Ff32);
+                                                        wd, bc1, bc2, apply, m->Ff, m->Fb, m->Ff32, m->F1g);
   MTRY(hipGetLastError(), "mlp_adamw");
   return IMX_OK;
 }
@@ -591,7 +605,7 @@ int imx_mlp_create(uint64_t seed, imx_mlp **out) {
       hipMalloc(&m->V, P_N * 4) != hipSuccess || hipMalloc(&m->G, P_N * 4) != hipSuccess ||
       hipMalloc(&m->part, (size_t)TR_BLOCKS * P_N * 4) != hipSuccess ||
       hipMalloc(&m->Ff, FF_N * 2) != hipSuccess || hipMalloc(&m->Fb, FB_N * 2) != hipSuccess ||
-      hipMalloc(&m->Ff32, FF_N * 2) != hipSuccess) {
+      hipMalloc(&m->Ff32, FF_N * 2) != hipSuccess || hipMalloc(&m->F1g, FF_2 * 2) != hipSuccess) {
     rc = imx::set_error(IMX_EDEVICE, "imx_mlp_create: device allocation failed");
   } else {
     (void)hipMemcpy(m->P, P.data(), P_N * 4, hipMemcpyHostToDevice);
@@ -715,7 +729,7 @@ void imx_mlp_destroy(imx_mlp *m) {
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   float *fs[] = {m->P, m->M, m->V, m->G, m->part, m->lossp, m->T, m->w, m->Y, m->Xf};
   for (float *p : fs) (void)hipFree(p);
-  short *ss[] = {m->Ff, m->Fb, m->Ff32, m->X};
+  short *ss[] = {m->Ff, m->Fb, m->Ff32, m->F1g, m->X};
   for (short *p : ss) (void)hipFree(p);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;

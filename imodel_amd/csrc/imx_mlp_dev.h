@@ -38,6 +38,34 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // size): per output tile of layer 1 a K32 fragment of 64 lanes x 8 bf16
 // then a K16 fragment of 64 x 4; layers 2..4 (K = 128) four K32 fragments
 // per output tile, tile-major.
+// Layer 1 has a third copy, for features that the kernel gathers itself: lane
+// group g of a wave forms twelve of an edge's 48 features, slots s = 0..11,
+// from its quarter of the edge's stencil record,
+//   group 0: ring edges 0-4, 1: ring edges 5-9, 2: ring edge 10 and cells 0-3,
+//   3: cells 4-9; slots 2 j, 2 j + 1 are the value at id j and its increment,
+//   slots 10, 11 of groups 0-2 the geometry features 2 g, 2 g + 1,
+// and the operand's k order follows (slots 0-7 the K32 chunk, 8-11 the tail).
+__host__ __device__ inline void mlp_feature_slot(int f, int *g, int *s) {
+  if (f >= 42) {
+    *g = (f - 42) / 2;
+    *s = 10 + (f - 42) % 2;
+    return;
+  }
+  int j, t;  // id, value or increment
+  if (f < 22) {
+    const int k = f % 11;
+    t = f / 11;
+    *g = k / 5;
+    j = k % 5;
+  } else {
+    const int c = (f - 22) % 10;
+    t = (f - 22) / 10;
+    *g = c < 4 ? 2 : 3;
+    j = c < 4 ? c + 1 : c - 4;
+  }
+  *s = 2 * j + t;
+}
+
 // backward fragments (layers 2..4, transposed)
 #define FB_2 0
 #define FB_3 (FB_2 + MLP_H * MLP_H)
@@ -111,9 +139,11 @@ __device__ __forceinline__ uint32_t f2bf2(float lo, float hi) {
 // and the packed weights follow the same permutation (mlp_pack), which
 // leaves each dot product unchanged.
 //
-// ld(e0, n, lane, x) fills the input fragments x[kc][t] of edges
-// e0 + 16 t + lane % 16 (features 16 kc + 4 (lane / 16) + i), zeros past n;
-// x[0], x[1] form K32 chunk 0 of the first layer and x[2] its K16 tail.
+// ld(e0, n, lane, x, sh) fills the input fragments x[kc][t] of edges
+// e0 + 16 t + lane % 16 (in the order of layer 1's fragments W1; rows past n
+// are not stored); x[0], x[1] form K32 chunk 0 of the first layer and x[2] its
+// K16 tail. sh: LDS that ld.prepare fills, 56 floats from sh + 64 g for lane
+// group g.
 #define MLP_FWD_WAVES 4
 // GELU of activation tiles z0, z1 (features 16 m .. 16 m + 31) as the K32
 // operand of their chunk
@@ -157,10 +187,16 @@ __device__ __forceinline__ void layer_pipe(const short *Ws, const float *__restr
 
 template <int ET, class Loader>
 __global__ __launch_bounds__(64 * MLP_FWD_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
-void mlp_fwd_lds(int64_t n, Loader ld, const v8s *__restrict__ Wf, const float *__restrict__ P,
-                 float *__restrict__ Y) {
+void mlp_fwd_lds(int64_t n, Loader ld, const v8s *__restrict__ W1, const v8s *__restrict__ Wf,
+                 const float *__restrict__ P, float *__restrict__ Y) {
   __shared__ v8s Wv[FF_N / 8];
-  for (int i = threadIdx.x; i < FF_N / 8; i += 64 * MLP_FWD_WAVES) Wv[i] = Wf[i];
+  for (int i = threadIdx.x; i < FF_N / 8; i += 64 * MLP_FWD_WAVES) Wv[i] = i < FF_2 / 8 ? W1[i] : Wf[i];
+  __syncthreads();
+  // two blocks per CU leave no LDS beside the fragments: the loader's
+  // constants take the place of output rows 2-15 of layer 4, of which the
+  // tile has 16 and the network 2
+  float *sh = reinterpret_cast<float *>(Wv + FF_4 / 8 + 2);
+  ld.prepare(sh);
   __syncthreads();
   const short *Ws = reinterpret_cast<const short *>(Wv);
   const int lane = threadIdx.x & 63;
@@ -173,7 +209,7 @@ void mlp_fwd_lds(int64_t n, Loader ld, const v8s *__restrict__ Wf, const float *
     // 80 KB fragment set would be held in registers
     asm volatile("" ::: "memory");
     v4s x[3][ET];
-    ld(e0, n, lane, x);
+    ld(e0, n, lane, x, sh);
     v4f z[8][ET], z2[8][ET];
     // layer 1: per output tile one K32 fragment (features 0..31) then one
     // K16 fragment (32..47), 768 bf16. The tail runs as a K32 MFMA with
@@ -231,8 +267,9 @@ void mlp_fwd_lds(int64_t n, Loader ld, const v8s *__restrict__ Wf, const float *
 // input fragments from stored BF16 rows X[n][48]
 struct RowLoader {
   const short *X;
+  __device__ __forceinline__ void prepare(float *) const {}
   template <int ET>
-  __device__ __forceinline__ void operator()(int64_t e0, int64_t n, int lane, v4s (&x)[3][ET]) const {
+  __device__ __forceinline__ void operator()(int64_t e0, int64_t n, int lane, v4s (&x)[3][ET], const float *) const {
 #pragma unroll
     for (int t = 0; t < ET; ++t) {
       const int64_t e = e0 + 16 * t + (lane % 16);
@@ -251,14 +288,15 @@ struct RowLoader {
 // tiles on, two sets (1024 blocks) balance the tail better (measured on
 // random weights: 7-10 % faster at 1.97 M edges, 15 % slower at 123 k).
 template <class Loader>
-inline hipError_t mlp_fwd_launch(const short *Ff32, const float *P, int64_t n, Loader ld, float *Y,
-                                 hipStream_t st) {
+inline hipError_t mlp_fwd_launch(const short *F1, const short *Ff32, const float *P, int64_t n, Loader ld,
+                                 float *Y, hipStream_t st) {
   constexpr int ET = 2;
   const int64_t ntiles = (n + 16 * ET - 1) / (16 * ET);
   int64_t blocks = (ntiles + MLP_FWD_WAVES - 1) / MLP_FWD_WAVES;
   const int64_t cap = ntiles >= 32768 ? 1024 : 512;
   if (blocks > cap) blocks = cap;
   if (blocks < 1) blocks = 1;
-  mlp_fwd_lds<ET, Loader><<<(unsigned)blocks, 64 * MLP_FWD_WAVES, 0, st>>>(n, ld, (const v8s *)Ff32, P, Y);
+  mlp_fwd_lds<ET, Loader>
+      <<<(unsigned)blocks, 64 * MLP_FWD_WAVES, 0, st>>>(n, ld, (const v8s *)F1, (const v8s *)Ff32, P, Y);
   return hipGetLastError();
 }

@@ -1897,13 +1897,13 @@ static void launch_fast_stage(imx_swm *s, int stage, const T *hs, const T *us, T
 }
 
 template <typename T>
-static void launch_fast_step(imx_swm *s, std::vector<hipEvent_t> *evs) {
+static void launch_fast_step(imx_swm *s, std::vector<hipEvent_t> *evs, T *hfin = nullptr, T *ufin = nullptr) {
   T *h0 = (T *)s->h0, *hA = (T *)s->hA, *hB = (T *)s->hB;
   T *u0 = (T *)s->u0, *uA = (T *)s->uA, *uB = (T *)s->uB;
   const T *hin[4] = {h0, hA, hB, hA};
   const T *uin[4] = {u0, uA, uB, uA};
-  T *hout[4] = {hA, hB, hA, h0};
-  T *uout[4] = {uA, uB, uA, u0};
+  T *hout[4] = {hA, hB, hA, hfin ? hfin : h0};
+  T *uout[4] = {uA, uB, uA, ufin ? ufin : u0};
   for (int st = 0; st < 4; ++st)
     launch_fast_stage<T>(s, st, hin[st], uin[st], hout[st], uout[st],
                          evs ? &(*evs)[4 * st] : nullptr);
@@ -1915,7 +1915,10 @@ static void launch_step(imx_swm *s) {
   else launch_fast_step<double>(s, nullptr);
 }
 
-void swm_launch_step(imx_swm *s) { launch_step(s); }
+void swm_launch_step(imx_swm *s, void *hout, void *uout) {
+  if (s->single) launch_fast_step<float>(s, nullptr, (float *)hout, (float *)uout);
+  else launch_fast_step<double>(s, nullptr, (double *)hout, (double *)uout);
+}
 
 // Diagnostics of the cells [c0, c1) and the edge/triangle slots they own.
 template <typename T>
