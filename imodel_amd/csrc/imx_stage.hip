@@ -1,5 +1,5 @@
-// libimx: one launch per RK stage for the plain scheme (trsk10, HTC or HC)
-// on the fused FP32/FP64 handles.
+// libimx: one launch per RK stage for the plain scheme (trsk10, HTC or HC),
+// without or with APVM, on the fused FP32/FP64 handles.
 //
 // The three passes of imx_swm.hip (fast_tri, fast_cell, fast_edge) hand q,
 // phi and the two Coriolis partials of every edge through memory and wait
@@ -14,6 +14,10 @@
 //   P1  PV of every triangle around a cell of C
 //   P2  fast_cell's work for every cell of C; RK update of h on own cells
 //   P3  fast_edge's work and the RK update of u on own edges
+// APVM adds the Perot velocity at every cell of L and grad q at the triangles
+// around C, between P1 and P2; for these the block also holds the rings of L
+// and the PV of every triangle around a cell of L, and takes the weights from
+// tables in its own order.
 // Nothing but the new state and the accumulators is written. Cells and
 // triangles on the rim are evaluated by every block that needs them (1.2 to
 // 1.4 times the work of the mesh), with the same expressions on the same
@@ -29,6 +33,13 @@
 // the rest. What was worth most: every load issued before the first barrier
 // (with each phase loading its own tables a glevel-8 stage took 45 us instead
 // of 32), then fewer vector instructions (32 -> 27.6).
+//
+// APVM, four passes -> this: glevel 5 FP32 64 -> 24.3, glevel 7 126 -> 77,
+// FP64 204 -> 165, glevel 8 459 -> 285, FP64 839 -> 686, glevel 9 1858 -> 1124.
+// The passes read three-component weights as four words and wrote the
+// velocities, gradients and partials; this moves 371 MB per stage at glevel 8
+// (about 330 of it tables, 1.45 times the mesh's for the rim) at 5.1 TB/s, a
+// large copy's rate: the tables no longer fit the last-level cache.
 //
 // Blocks are cut greedily along the curve so that |C| fills the block's
 // threads and |L| its LDS. Ids inside a block are 10-bit, which packs the
@@ -82,18 +93,26 @@ template <typename T>
 struct alignas(4 * sizeof(T)) Quad {
   T x, y, z, w;
 };
+template <typename T>
+struct Tri {
+  T x, y, z;
+};
 
 // caps of a block of nt threads: local cells (and at most nt past the own
-// ones, at most nt in C), triangles
-static constexpr int cap_l(int nt) { return nt + nt / 2 + 64; }
-static constexpr int cap_t(int nt) { return 2 * nt + nt / 2 + 64; }
+// ones, at most nt in C), cells of L, triangles, triangles around C
+static constexpr int cap_a(int nt) { return nt + nt / 2 + 64; }
+static constexpr int cap_l(int nt, bool ap) { return ap ? nt + nt / 4 + 64 : nt; }
+static constexpr int cap_t(int nt, bool ap) { return ap ? 3 * nt : 2 * nt + nt / 2 + 64; }
+static constexpr int cap_g(int nt) { return 2 * nt + nt / 4 + 32; }
 
 struct Stage {
   int nt = 0, nblk = 0, remap = 1;
+  bool ap = false;
   Alloc A;
-  int4 *head = nullptr;      // [nblk] first own cell, own cells, |C|, |L| | triangles << 16
+  int4 *head = nullptr;      // [nblk] first own cell, own cells | |L| << 16, |C| | triangles around C << 16,
+                             // local cells | triangles << 16
   int32_t *halo = nullptr;   // [nblk][nt] cells of the local ids past the own ones
-  uint4 *topo = nullptr;     // [nblk][nt]
+  uint4 *topo = nullptr;     // [nblk][cap_l]
   void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~
   void *eld = nullptr;       // [NE] Pair: length, dual length
   uint16_t *oth = nullptr;   // [NE] local id of the edge's other cell | it is v1 << 10; 0xFFFF dummy
@@ -101,6 +120,9 @@ struct Stage {
   uint16_t *tslot = nullptr; // [nblk][cap_t] local slot 2 owner + k
   void *tk = nullptr;        // [nblk][cap_t] Quad: kite weights, 1 / (A_t a)
   void *tf = nullptr;        // [nblk][cap_t] Coriolis parameter
+  void *wc = nullptr;        // APVM: [nblk][6][cap_l] Tri: Perot weights of a cell's velocity
+  void *wt = nullptr;        // APVM: [nblk][3][cap_g] Tri: those of grad q at a triangle
+  ushort4 *tn = nullptr;     // APVM: [nblk][cap_g] local slots of the triangles across and its own
 };
 
 template <typename T>
@@ -115,6 +137,8 @@ struct StageArgs {
   const uint16_t *tslot;
   const Quad<T> *tk;
   const T *tf;
+  const Tri<T> *wc, *wt;
+  const ushort4 *tn;
   const double *iaa;
   const T *hs, *us, *h0, *u0, *gb, *dte;
   const double *dtc;
@@ -122,7 +146,7 @@ struct StageArgs {
   double *dh_out;
   int *flag;
   double href, ca, cb;  // the stage's step and its weight in the sum (ensembles: per cell)
-  T grav, inv_a, cat, cbt;
+  T grav, inv_a, cat, cbt, pvsdt;
   int nblk, remap, use_pv, flin, zero_mom;
   int whole;  // the third stage: its state is a whole step away
 };
@@ -165,13 +189,14 @@ __device__ __forceinline__ void put(X *p, uint32_t i, X v) {
 }
 
 // MODE: 0 the first RK stage, 1 the second and third, 2 the last, 3 a
-// tendency.
-template <typename T, int NT, int MODE>
-__global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
-  constexpr int LC = cap_l(NT), TC = cap_t(NT);
-  constexpr int NR = (TC + NT - 1) / NT;
+// tendency. AP: with APVM.
+template <typename T, int NT, int MODE, bool AP>
+__global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const StageArgs<T> a) {
+  constexpr int LC = cap_a(NT), CL = cap_l(NT, AP), TC = cap_t(NT, AP), GC = cap_g(NT);
+  constexpr int NR = (TC + NT - 1) / NT, NG = (GC + NT - 1) / NT;
   __shared__ T sU[3 * LC], sD[3 * LC], sA[3 * LC];  // u, dual length, u l
   __shared__ T sH[LC], sQ[2 * LC], sPhi[NT], sPP[6 * NT];
+  __shared__ Tri<T> sV[AP ? CL : 1], sG[AP ? 2 * CL : 1];  // Perot velocity at cells, grad q at triangles
   T *sP = sPP, *sPo = sPP + 3 * NT;  // partials of the own edges' owners and other cells
   int b = blockIdx.x;
   if (a.remap) b = (b % NXCD) * (gridDim.x / NXCD) + b / NXCD;
@@ -184,12 +209,13 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
   // around the load.
   const int32_t *halo = a.halo + (size_t)b * NT;
   const int hcell = at(halo, tid);
-  const uint4 tp = at(a.topo + (size_t)b * NT, tid);
+  const uint4 *topo = a.topo + (size_t)b * CL;
+  const uint4 tp = at(topo, tid);
   const Quad<T> *cw = a.cw + (size_t)b * 2 * NT;
   const Quad<T> w0 = at(cw, tid), w1 = at(cw + NT, tid);
   const int4 hd = a.head[b];
-  const int own0 = hd.x, nown = hd.y, nC = hd.z, nL = hd.w & 0xFFFF, nTri = hd.w >> 16;
-  const int nh = nL - nown;
+  const int own0 = hd.x, nown = hd.y & 0xFFFF, nL = hd.y >> 16, nC = hd.z & 0xFFFF, nG = hd.z >> 16;
+  const int nTri = hd.w >> 16, nh = (hd.w & 0xFFFF) - nown;
   const T href = (T)a.href;
   const int oc = min(tid, nown - 1);
 
@@ -223,6 +249,18 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     tsl[r] = at(a.tslot + (size_t)b * TC, t);
     tk[r] = at(a.tk + (size_t)b * TC, t);
     tf[r] = at(a.tf + (size_t)b * TC, t);
+  }
+  uint4 tpl;
+  Tri<T> wc[2][MX];
+  if constexpr (AP) {
+    const Tri<T> *w = a.wc + (size_t)b * MX * CL;
+    const int i = min(tid + NT, CL - 1);
+    tpl = at(topo, i);
+#pragma unroll
+    for (int j = 0; j < MX; ++j) {
+      wc[0][j] = at(w + j * CL, tid);
+      wc[1][j] = at(w + j * CL, i);
+    }
   }
   // the RK operands of the own cells and edges
   __builtin_amdgcn_sched_barrier(0);
@@ -263,8 +301,40 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
       sA[3 * lc + k] = hu[k] * hl[k].x;
     }
   }
+  ushort4 tn[NG];
+  Tri<T> wt[NG][3];
+  if constexpr (AP) {
+#pragma unroll
+    for (int r = 0; r < NG; ++r) {
+      const int t = min(tid + r * NT, nG - 1);
+      tn[r] = at(a.tn + (size_t)b * GC, t);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) wt[r][m] = at(a.wt + ((size_t)b * 3 + m) * GC, t);
+    }
+  }
   __syncthreads();
 
+  if constexpr (AP) {
+    // Perot velocity at the cells of L (a pentagon's padded slot has a zero
+    // weight)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int i = tid + r * NT;
+      if (i >= nL) continue;
+      const uint4 t4 = r ? tpl : tp;
+      const uint32_t wj[3] = {t4.x, t4.y, t4.z};
+      Tri<T> v{(T)0, (T)0, (T)0};
+#pragma unroll
+      for (int j = 0; j < MX; ++j) {
+        const uint32_t f = j % 2 ? wj[j / 2] >> 16 : wj[j / 2];
+        const T u = sU[3 * ((f >> SB_OWN) & 1 ? i : (int)(f & LID)) + ((f >> SB_K) & 3)];
+        v.x = fma_(wc[r][j].x, u, v.x);
+        v.y = fma_(wc[r][j].y, u, v.y);
+        v.z = fma_(wc[r][j].z, u, v.z);
+      }
+      sV[i] = v;
+    }
+  }
   // P1: PV at triangles
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
@@ -298,6 +368,25 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     if (MODE >= 2 && o < nown) put(a.q + 2 * (size_t)own0, sl, qq);
   }
   __syncthreads();
+
+  if constexpr (AP) {
+    // grad q at the triangles around C
+#pragma unroll
+    for (int r = 0; r < NG; ++r) {
+      if (tid + r * NT >= nG) continue;
+      const T qt = sQ[tn[r].w];
+      const T d[3] = {sQ[tn[r].x] - qt, sQ[tn[r].y] - qt, sQ[tn[r].z] - qt};
+      Tri<T> g{(T)0, (T)0, (T)0};
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        g.x = fma_(wt[r][m].x, d[m], g.x);
+        g.y = fma_(wt[r][m].y, d[m], g.y);
+        g.z = fma_(wt[r][m].z, d[m], g.z);
+      }
+      sG[tn[r].w] = g;
+    }
+    __syncthreads();
+  }
 
   // P2: cells
   if (tid < nC) {
@@ -335,11 +424,13 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
       ke += k;
     }
     T qt[MX];
+    int ts[MX];
 #pragma unroll
     for (int j = 0; j < MX; ++j) {
-      const int ts = (tp.w >> (2 * j)) & 3;
-      const int to = (ts == 0) ? tid : (ts == 1) ? nb[j] : nb[(j + 1) % MX];
-      qt[j] = sQ[2 * to + ((tp.w >> (SW_KT + j)) & 1)];
+      const int sel = (tp.w >> (2 * j)) & 3;
+      const int to = (sel == 0) ? tid : (sel == 1) ? nb[j] : nb[(j + 1) % MX];
+      ts[j] = 2 * to + ((tp.w >> (SW_KT + j)) & 1);
+      qt[j] = sQ[ts[j]];
     }
     // a pentagon's padded slot may name a triangle that is not local
     if (!hex) qt[MX - 1] = (T)0;
@@ -369,6 +460,19 @@ __global__ __launch_bounds__(NT) void fast_stage(const StageArgs<T> a) {
     qe[0] = (T)0.5 * ((hex ? qt[MX - 1] : qt[MX - 2]) + qt[0]);
 #pragma unroll
     for (int j = 1; j < MX; ++j) qe[j] = (T)0.5 * (qt[j - 1] + qt[j]);
+    if constexpr (AP) {
+      // q_e -= pvspar dt (grad q(t_{j-1}) + grad q(t_j)) . (v(c) + v(nb_j))
+      if (!hex) ts[MX - 1] = ts[MX - 2];  // the ring's last triangle, and in place of the pad
+      const Tri<T> vs = sV[tid];
+      Tri<T> gp = sG[ts[MX - 1]];
+#pragma unroll
+      for (int j = 0; j < MX; ++j) {
+        const Tri<T> g = sG[ts[j]], v = sV[nb[j]];
+        qe[j] -= a.pvsdt * ((gp.x + g.x) * (vs.x + v.x) + (gp.y + g.y) * (vs.y + v.y) + (gp.z + g.z) * (vs.z + v.z));
+        gp = g;
+      }
+      if (!hex) qe[MX - 1] = (T)0;
+    }
     // TRiSK weights from prefix sums of the kite areas:
     // w(i,j) = S_j - S_i - 1/2 (j>i), S_6 - S_i + S_j - 1/2 (j<i), w(i,i) = 0
     const T R[MX] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
@@ -443,18 +547,18 @@ void stage_free(imx_swm *s) {
 }
 
 int stage_threads(const imx_swm *s) { return s->stg ? s->stg->nt : 0; }
+bool stage_apvm(const imx_swm *s) { return s->stg && s->stg->ap; }
 void stage_set_remap(imx_swm *s, int remap) {
   if (s->stg) s->stg->remap = remap;
 }
 size_t stage_bytes(const imx_swm *s) { return s->stg ? s->stg->A.bytes : 0; }
-int stage_remap(const imx_swm *s) { return s->stg ? s->stg->remap : 0; }
 
 // A block's local cells and triangles: small open-addressing tables that are
 // emptied by raising the stamp (a block holds far fewer entries than slots).
 struct LocalSet {
   static constexpr int kSlots = 1 << 13;
   struct Entry {
-    int32_t stamp = 0, key = 0, id = 0, in_c = 0;
+    int32_t stamp = 0, key = 0, id = 0, level = 0;  // cells: 1 in L, 2 in C; triangles: 1 around C
   };
   std::vector<Entry> e{(size_t)kSlots};
   std::vector<int32_t> keys;
@@ -476,18 +580,19 @@ struct LocalSet {
 };
 struct LocalSets {
   LocalSet L, tri;
-  int nC = 0, own = 0;
+  int nC = 0, nL = 0, nG = 0, own = 0;
   void clear() {
     L.clear();
     tri.clear();
-    nC = own = 0;
+    nC = nL = nG = own = 0;
   }
 };
 
 template <typename T>
 static int build(imx_swm *s, int nt) {
   const int nv = s->nv, NE = s->NE, NTri = s->NT;
-  const int LC = cap_l(nt), TC = cap_t(nt);
+  const bool ap = s->f_apvm;
+  const int LC = cap_a(nt), CL = cap_l(nt, ap), TC = cap_t(nt, ap), GC = cap_g(nt);
   const double ea = s->o.erad;
   std::vector<int32_t> nbr, bA, bB, oth, tab, teb;
   std::vector<T> R, ika, ceta, kap, tf;
@@ -499,6 +604,11 @@ static int build(imx_swm *s, int nt) {
       !down(tf, s->x_t_f, NTri) || !down(leng, s->e_leng, NE) || !down(dleng, s->e_dleng, NE) ||
       !down(tarea, s->t_area, NTri))
     return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
+  std::vector<Quad<T>> awc, awt;
+  std::vector<int32_t> atn;
+  if (ap && (!down(awc, s->x_ap_wc, (size_t)MX * nv) || !down(awt, s->x_ap_wt, (size_t)3 * NTri) ||
+             !down(atn, s->x_ap_tnb, (size_t)3 * NTri)))
+    return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
 
   auto tri_of = [&](int c, int j) {
     const int ts = (bB[c] >> (BB_TSEL + 2 * j)) & 3;
@@ -507,15 +617,31 @@ static int build(imx_swm *s, int nt) {
   };
   // adds own cell c to the sets of the current block; false past a cap
   auto add = [&](LocalSets &w, int c) {
-    auto in_c = [&](int k) {
+    auto in_l = [&](int k) {
       LocalSet::Entry &q = w.L.at(k);
-      if (q.in_c) return;
-      q.in_c = 1;
-      ++w.nC;
+      if (q.level) return;
+      q.level = 1;
+      ++w.nL;
+      if (!ap) return;
+      // APVM takes the velocity at k and the PV of the triangles around it
       const int n = bA[k] & 7;
       for (int j = 0; j < n; ++j) {
         (void)w.L.at(nbr[(size_t)j * nv + k]);
         (void)w.tri.at(tri_of(k, j));
+      }
+    };
+    auto in_c = [&](int k) {
+      in_l(k);
+      LocalSet::Entry &q = w.L.at(k);
+      if (q.level == 2) return;
+      q.level = 2;
+      ++w.nC;
+      const int n = bA[k] & 7;
+      for (int j = 0; j < n; ++j) {
+        in_l(nbr[(size_t)j * nv + k]);
+        LocalSet::Entry &t = w.tri.at(tri_of(k, j));
+        w.nG += !t.level;
+        t.level = 1;
       }
     };
     in_c(c);
@@ -523,8 +649,9 @@ static int build(imx_swm *s, int nt) {
     for (int j = 0; j < n; ++j)
       if ((bA[c] >> (BA_OWN + j)) & 1) in_c(nbr[(size_t)j * nv + c]);
     ++w.own;
-    const int nL = (int)w.L.keys.size();
-    return w.nC <= nt && nL <= LC && nL - w.own <= nt && (int)w.tri.keys.size() <= TC;
+    const int nA = (int)w.L.keys.size();
+    return w.nC <= nt && nA <= LC && nA - w.own <= nt && (int)w.tri.keys.size() <= TC &&
+           (!ap || (w.nL <= CL && w.nG <= GC));
   };
 
   // cut the curve into at most 16 segments, one host thread each, and every
@@ -575,12 +702,15 @@ static int build(imx_swm *s, int nt) {
 
   std::vector<int4> head(nblk);
   std::vector<int32_t> halo((size_t)nblk * nt, 0);
-  std::vector<uint4> topo((size_t)nblk * nt, uint4{0, 0, 0, 0});
+  std::vector<uint4> topo((size_t)nblk * CL, uint4{0, 0, 0, 0});
   std::vector<Quad<T>> cw((size_t)nblk * 2 * nt, Quad<T>{0, 0, 0, 0}), tk((size_t)nblk * TC, Quad<T>{0, 0, 0, 0});
   std::vector<Pair<T>> eld(NE);
   std::vector<uint16_t> loth(NE, 0xFFFF), tslot((size_t)nblk * TC, 0);
   std::vector<uint32_t> tv((size_t)nblk * TC, 0);
   std::vector<T> tfv((size_t)nblk * TC, (T)0);
+  std::vector<Tri<T>> wc(ap ? (size_t)nblk * MX * CL : 0, Tri<T>{0, 0, 0}),
+      wt(ap ? (size_t)nblk * 3 * GC : 0, Tri<T>{0, 0, 0});
+  std::vector<ushort4> tn(ap ? (size_t)nblk * GC : 0, ushort4{0, 0, 0, 0});
   for (int e = 0; e < NE; ++e) eld[e] = Pair<T>{(T)leng[e], (T)dleng[e]};
   each_segment([&](int g) {
     LocalSets w;
@@ -588,25 +718,26 @@ static int build(imx_swm *s, int nt) {
       const int o0 = start[b], nown = start[b + 1] - o0;
       w.clear();
       for (int c = o0; c < o0 + nown; ++c) (void)add(w, c);
-      // own cells, the rest of C, the rest of L, each ascending; own
-      // triangles first
+      // own cells, the rest of C, the rest of L, the others, each ascending;
+      // own triangles, the others around C, the others
       auto own = [&](int k) { return k >= o0 && k < o0 + nown; };
       std::vector<int32_t> cells = w.L.keys, tris = w.tri.keys;
-      auto rank = [&](int k) { return own(k) ? 0 : w.L.at(k).in_c ? 1 : 2; };
+      auto rank = [&](int k) { return own(k) ? 0 : 3 - w.L.at(k).level; };
+      auto trank = [&](int k) { return own(k / 2) ? 0 : 2 - w.tri.at(k).level; };
       std::sort(cells.begin(), cells.end(), [&](int x, int y) {
         const int rx = rank(x), ry = rank(y);
         return rx != ry ? rx < ry : x < y;
       });
       std::sort(tris.begin(), tris.end(), [&](int x, int y) {
-        const bool ox = own(x / 2), oy = own(y / 2);
-        return ox != oy ? ox : x < y;
+        const int rx = trank(x), ry = trank(y);
+        return rx != ry ? rx < ry : x < y;
       });
-      const int nL = (int)cells.size(), nC = w.nC;
-      for (int k = 0; k < nL; ++k) w.L.at(cells[k]).id = k;
+      const int nA = (int)cells.size(), nL = w.nL, nC = w.nC;
+      for (int k = 0; k < nA; ++k) w.L.at(cells[k]).id = k;
       auto id = [&](int k) { return (uint32_t)w.L.at(k).id; };
-      for (int k = nown; k < nL; ++k) halo[(size_t)b * nt + k - nown] = cells[k];
-      head[b] = int4{o0, nown, nC, nL | (int)tris.size() << 16};
-      for (int k = 0; k < nC; ++k) {
+      for (int k = nown; k < nA; ++k) halo[(size_t)b * nt + k - nown] = cells[k];
+      head[b] = int4{o0, nown | nL << 16, nC | w.nG << 16, nA | (int)tris.size() << 16};
+      for (int k = 0; k < (ap ? nL : nC); ++k) {
         const int c = cells[k];
         const bool hex = (bA[c] & 7) == MX;
         uint32_t f[MX], t3 = (uint32_t)hex << SW_HEX;
@@ -621,7 +752,12 @@ static int build(imx_swm *s, int nt) {
           t3 |= ((bB[c] >> (BB_KT + j)) & 1u) << (SW_KT + j);
           r[j] = R[(size_t)j * nv + c];
         }
-        topo[(size_t)b * nt + k] = uint4{f[0] | f[1] << 16, f[2] | f[3] << 16, f[4] | f[5] << 16, t3};
+        topo[(size_t)b * CL + k] = uint4{f[0] | f[1] << 16, f[2] | f[3] << 16, f[4] | f[5] << 16, t3};
+        for (int j = 0; ap && j < MX; ++j) {
+          const Quad<T> &q = awc[(size_t)j * nv + c];
+          wc[((size_t)b * MX + j) * CL + k] = Tri<T>{q.x, q.y, q.z};
+        }
+        if (k >= nC) continue;
         cw[((size_t)b * 2) * nt + k] = Quad<T>{r[0], r[1], r[2], r[3]};
         // ika = 1 / sum (l l~ / 4)
         cw[((size_t)b * 2 + 1) * nt + k] = Quad<T>{r[4], r[5], (T)0.25 * ika[c], (T)0};
@@ -636,6 +772,14 @@ static int build(imx_swm *s, int nt) {
         tslot[p] = (uint16_t)(2 * id(t / 2) + t % 2);
         tk[p] = Quad<T>{kap[t], kap[(size_t)NTri + t], kap[(size_t)2 * NTri + t], (T)(1.0 / (tarea[t] * ea))};
         tfv[p] = tf[t];
+        if (!ap || k >= w.nG) continue;
+        auto slot = [&](int i) { return (unsigned short)(2 * id(i / 2) + i % 2); };
+        tn[(size_t)b * GC + k] = ushort4{slot(atn[t]), slot(atn[(size_t)NTri + t]), slot(atn[(size_t)2 * NTri + t]),
+                                         slot(t)};
+        for (int m = 0; m < 3; ++m) {
+          const Quad<T> &q = awt[(size_t)m * NTri + t];
+          wt[((size_t)b * 3 + m) * GC + k] = Tri<T>{q.x, q.y, q.z};
+        }
       }
       for (int e = 3 * o0; e < 3 * (o0 + nown); ++e) {
         if (oth[e] < 0) continue;
@@ -659,6 +803,12 @@ static int build(imx_swm *s, int nt) {
   g->tslot = A.put(tslot);
   g->tk = A.put(tk);
   g->tf = A.put(tfv);
+  g->ap = ap;
+  if (ap) {
+    g->wc = A.put(wc);
+    g->wt = A.put(wt);
+    g->tn = A.put(tn);
+  }
   if (A.err != hipSuccess) {
     const std::string why = hipGetErrorString(A.err);
     stage_free(s);
@@ -676,14 +826,25 @@ int stage_build(imx_swm *s, int nt) {
   }
 }
 
-template <typename T, int NT>
+template <typename T, int NT, bool AP>
 static void launch_nt(const StageArgs<T> &a, int stage, int grid, hipStream_t st) {
   switch (stage) {
-    case 0: fast_stage<T, NT, 0><<<grid, NT, 0, st>>>(a); break;
+    case 0: fast_stage<T, NT, 0, AP><<<grid, NT, 0, st>>>(a); break;
     case 1:
-    case 2: fast_stage<T, NT, 1><<<grid, NT, 0, st>>>(a); break;
-    case 3: fast_stage<T, NT, 2><<<grid, NT, 0, st>>>(a); break;
-    default: fast_stage<T, NT, 3><<<grid, NT, 0, st>>>(a); break;
+    case 2: fast_stage<T, NT, 1, AP><<<grid, NT, 0, st>>>(a); break;
+    case 3: fast_stage<T, NT, 2, AP><<<grid, NT, 0, st>>>(a); break;
+    default: fast_stage<T, NT, 3, AP><<<grid, NT, 0, st>>>(a); break;
+  }
+}
+
+template <typename T, bool AP>
+static void launch_threads(const StageArgs<T> &a, int nt, int stage, int grid, hipStream_t st) {
+  switch (nt) {
+    case 128: launch_nt<T, 128, AP>(a, stage, grid, st); break;
+    case 512:
+      if constexpr (sizeof(T) == 4) launch_nt<T, 512, AP>(a, stage, grid, st);
+      break;
+    default: launch_nt<T, 256, AP>(a, stage, grid, st); break;
   }
 }
 
@@ -701,6 +862,10 @@ void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *u
   a.tslot = g.tslot;
   a.tk = (const Quad<T> *)g.tk;
   a.tf = (const T *)g.tf;
+  a.wc = (const Tri<T> *)g.wc;
+  a.wt = (const Tri<T> *)g.wt;
+  a.tn = g.tn;
+  a.pvsdt = (T)(s->sc.pvspar * s->o.dt);
   a.iaa = s->x_c_iaa;
   a.hs = hs;
   a.us = us;
@@ -733,13 +898,8 @@ void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *u
   a.flin = s->f_lin ? 1 : 0;
   a.zero_mom = s->o.testcase <= 1;
   const int grid = (g.nblk + NXCD - 1) / NXCD * NXCD;
-  switch (g.nt) {
-    case 128: launch_nt<T, 128>(a, stage, grid, s->stream); break;
-    case 512:
-      if constexpr (sizeof(T) == 4) launch_nt<T, 512>(a, stage, grid, s->stream);
-      break;
-    default: launch_nt<T, 256>(a, stage, grid, s->stream); break;
-  }
+  if (g.ap) launch_threads<T, true>(a, g.nt, stage, grid, s->stream);
+  else launch_threads<T, false>(a, g.nt, stage, grid, s->stream);
 }
 template void stage_launch<float>(imx_swm *, int, const float *, const float *, float *, float *);
 template void stage_launch<double>(imx_swm *, int, const double *, const double *, double *, double *);

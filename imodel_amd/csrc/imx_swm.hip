@@ -1786,13 +1786,16 @@ static void launch_ref_step(imx_swm *s) {
     default: CALL(256); break;   \
   }
 
-// The scheme imx_stage.hip evaluates in one launch per stage: trsk10's
-// methods without options, HTC or HC, with any topography and Coriolis term.
-static bool plain_scheme(const imx_swm *s) {
-  return !(s->f_gass || s->f_melv || s->f_perhx || s->f_nopv || s->f_apvm || s->f_bary || s->f_pered || s->f_gk ||
-           s->f_dtred || s->f_diff || s->f_hyper);
+// The schemes imx_stage.hip evaluates in one launch per stage: trsk10's
+// methods without options or with APVM, HTC or HC, with any topography and
+// Coriolis term.
+static bool stage_scheme(const imx_swm *s) {
+  return !(s->f_gass || s->f_melv || s->f_perhx || s->f_nopv || s->f_bary || s->f_pered || s->f_gk || s->f_dtred ||
+           s->f_diff || s->f_hyper);
 }
-static bool stage_on(const imx_swm *s) { return s->stg && !s->stg_stale && plain_scheme(s); }
+static bool stage_on(const imx_swm *s) {
+  return s->stg && !s->stg_stale && stage_scheme(s) && stage_apvm(s) == s->f_apvm;
+}
 
 // One FAST stage: stage<0 evaluates the tendency of (hs, us) into dh_out/du_out.
 template <typename T>
@@ -2680,19 +2683,40 @@ static int validate_desc(const imx_mesh_desc &d) {
 //   glevel 9 FP64   128: 278    256: 254                256, no remap: 245
 // Small blocks until there is one of the larger ones for every other CU;
 // beyond the last-level cache (some 250 B per FP32 cell) the least rim is
-// best, and eight separate stretches of memory no longer pay.
+// best, and eight separate stretches of memory no longer pay. With APVM a cell
+// takes twice the bytes and the rim is a ring wider (us per step):
+//   glevel 5 FP32   128: 24.3
+//   glevel 6 FP32   256: 29.7   512: 40.3
+//   glevel 7 FP32   256: 76.8   512: 82.7
+//   glevel 8 FP32   256: 317    512: 291   512, no remap: 285
+//   glevel 8 FP64   256: 695               256, no remap: 686
+//   glevel 9 FP32   256: 1206              512, no remap: 1124
 static bool stage_large(const imx_swm *s) { return (size_t)s->nv * (s->single ? 4 : 8) > ((size_t)8 << 20); }
-static int stage_default(const imx_swm *s) { return s->nv < 30000 ? 128 : stage_large(s) && s->single ? 512 : 256; }
+static void stage_defaults(imx_swm *s) {
+  s->stg_nt[0] = s->nv < 30000 ? 128 : stage_large(s) && s->single ? 512 : 256;
+  s->stg_remap[0] = stage_large(s) ? 0 : 1;
+  const bool apvm_large = (size_t)s->nv * (s->single ? 4 : 8) > ((size_t)2 << 20);
+  s->stg_nt[1] = s->nv < 30000 ? 128 : apvm_large && s->single ? 512 : 256;
+  s->stg_remap[1] = apvm_large ? 0 : 1;
+}
 
-// The stage tables follow the handle's staggering, triangle weights and
-// Coriolis parameter; they are made again when the plain scheme is back.
-static int stage_refresh(imx_swm *s) {
-  s->stg_stale = s->stg != nullptr;
-  if (!s->stg_stale || !plain_scheme(s)) return IMX_OK;
-  const int remap = stage_remap(s), rc = stage_build(s, stage_threads(s));
-  stage_set_remap(s, remap);
+// (Re)builds the stage tables for the handle's scheme: they follow its
+// staggering, triangle weights and Coriolis parameter, and are made again
+// when a scheme that has them is back.
+static int stage_make(imx_swm *s) {
+  const int rc = stage_build(s, s->stg_nt[s->f_apvm]);
+  stage_set_remap(s, s->stg_remap[s->f_apvm]);
   s->stg_stale = false;
   return rc;
+}
+static int stage_refresh(imx_swm *s) {
+  s->stg_stale = true;
+  if (!s->stg_local || !stage_scheme(s)) return IMX_OK;
+  const int rc = stage_make(s);
+  if (!s->f_apvm || !rc) return rc;
+  // no room for APVM's tables: the three passes need none
+  (void)hipGetLastError();
+  return IMX_OK;
 }
 
 static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
@@ -2883,8 +2907,9 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
   }
   HIPTRY(hipDeviceSynchronize(), "imx_swm_create");
   if (s->fast) {
-    if ((rc = stage_build(s, stage_default(s)))) return rc;
-    stage_set_remap(s, stage_large(s) ? 0 : 1);
+    stage_defaults(s);
+    if ((rc = stage_make(s))) return rc;
+    s->stg_local = s->stg != nullptr;
   }
   return IMX_OK;
 }
@@ -3106,7 +3131,7 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   if (stage_on(s)) {
     // one launch per stage: block threads (which cut the mesh anew) x remap
     double best = 1e30;
-    int bb = stage_threads(s), br = stage_remap(s);
+    int &bb = s->stg_nt[s->f_apvm], &br = s->stg_remap[s->f_apvm];
     for (int bs : {128, 256, 512}) {
       if (bs == 512 && !s->single) continue;  // over 64 KB of LDS
       if ((rc = stage_build(s, bs))) break;
@@ -3123,10 +3148,8 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
       }
       if (rc) break;
     }
-    if (!s->stg || stage_threads(s) != bb) {
-      const int r2 = stage_build(s, bb);
-      if (!rc) rc = r2;
-    }
+    const int r2 = !s->stg || stage_threads(s) != bb ? stage_make(s) : IMX_OK;
+    if (!rc) rc = r2;
     stage_set_remap(s, br);
     s->kbs[1] = bb;
     s->kremap[1] = br;
