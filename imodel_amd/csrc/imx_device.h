@@ -283,13 +283,13 @@ struct imx_swm {
   // XCD remap, chosen by imx_swm_tune
   int kbs[3] = {256, 256, 256};
   int kremap[3] = {1, 1, 1};
-  // one launch per stage for the plain scheme and APVM; stg_local: the
-  // numbering is local. stg_stale: the tables no longer match the handle's
-  // staggering, triangle weights or Coriolis parameter. stg_nt, stg_remap:
-  // block threads and XCD remap of the plain scheme and of APVM.
+  // one launch per stage; stg_local: the numbering is local. stg_stale: the
+  // tables no longer match the handle's staggering, triangle weights or
+  // Coriolis parameter. stg_nt, stg_remap: block threads and XCD remap of
+  // each scheme it has (one_launch_scheme).
   imx::Stage *stg = nullptr;
   bool stg_stale = false, stg_local = false;
-  int stg_nt[2] = {256, 256}, stg_remap[2] = {1, 1};
+  int stg_nt[4] = {256, 256, 256, 256}, stg_remap[4] = {1, 1, 1, 1};
 };
 
 // MLP handle: FP32 master parameters with AdamW moments, BF16 fragment
@@ -322,10 +322,10 @@ int swm_check_flag(imx_swm *s, const char *what);
 // tables from the handle's device tables for blocks of nt threads and leaves
 // s->stg null where the numbering cuts into blocks that are mostly rim;
 // stage_launch evaluates stage 0..3 of (hs, us), or a tendency (stage -1).
-int stage_build(imx_swm *s, int nt);
+int stage_build(imx_swm *s, int nt, int scheme);
 void stage_free(imx_swm *s);
 int stage_threads(const imx_swm *s);
-bool stage_apvm(const imx_swm *s);
+int stage_scheme(const imx_swm *s);
 size_t stage_bytes(const imx_swm *s);
 void stage_set_remap(imx_swm *s, int remap);
 template <typename T>

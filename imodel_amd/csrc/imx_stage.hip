@@ -1,5 +1,5 @@
-// libimx: one launch per RK stage for the plain scheme (trsk10, HTC or HC),
-// without or with APVM, on the fused FP32/FP64 handles.
+// libimx: one launch per RK stage on the fused FP32/FP64 handles, for trsk10's
+// methods (HTC or HC), alone, with APVM or with diffusion, and for pxt16's (HTC).
 //
 // The three passes of imx_swm.hip (fast_tri, fast_cell, fast_edge) hand q,
 // phi and the two Coriolis partials of every edge through memory and wait
@@ -18,6 +18,9 @@
 // around C, between P1 and P2; for these the block also holds the rings of L
 // and the PV of every triangle around a cell of L, and takes the weights from
 // tables in its own order.
+// pxt16 replaces the Coriolis partials by two Perot vectors of every cell of
+// C, which P3 reads; diffusion adds K zeta at the triangles and its jump at
+// the own edges.
 // Nothing but the new state and the accumulators is written. Cells and
 // triangles on the rim are evaluated by every block that needs them (1.2 to
 // 1.4 times the work of the mesh), with the same expressions on the same
@@ -40,6 +43,9 @@
 // velocities, gradients and partials; this moves 371 MB per stage at glevel 8
 // (about 330 of it tables, 1.45 times the mesh's for the rim) at 5.1 TB/s, a
 // large copy's rate: the tables no longer fit the last-level cache.
+// pxt16, three passes -> this: glevel 5 FP32 52 -> 19.7, glevel 7 105 -> 56.6,
+// FP64 159 -> 87, glevel 8 378 -> 158, FP64 659 -> 377. Diffusion: 53 -> 21.7,
+// 89 -> 48.9, 124 -> 74, 223 -> 119, 488 -> 236.
 //
 // Blocks are cut greedily along the curve so that |C| fills the block's
 // threads and |L| its LDS. Ids inside a block are 10-bit, which packs the
@@ -53,6 +59,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "imx_device.h"
@@ -73,11 +80,13 @@
 // bits at 2j), k of triangle j (bit 12+j), hexagon (bit 18)
 #define SW_KT 12
 #define SW_HEX 18
+#define SW_FZ 19  // sign of the tangential diffusion at edge j (bit 19 + j)
 
 // bits of the handle's cell words (imx_swm.hip)
 #define BA_TTG 3
 #define BA_TNR 9
 #define BA_OWN 15
+#define BA_FZ 21
 #define BB_TSEL 12
 #define BB_KT 24
 #define OTH_MASK 0x3FFFFFFF
@@ -100,6 +109,7 @@ struct Tri {
 
 // caps of a block of nt threads: local cells (and at most nt past the own
 // ones, at most nt in C), cells of L, triangles, triangles around C
+static constexpr int kPlain = 0, kApvm = 1, kPerot = 2, kDiff = 3;  // stage_build's schemes
 static constexpr int cap_a(int nt) { return nt + nt / 2 + 64; }
 static constexpr int cap_l(int nt, bool ap) { return ap ? nt + nt / 4 + 64 : nt; }
 static constexpr int cap_t(int nt, bool ap) { return ap ? 3 * nt : 2 * nt + nt / 2 + 64; }
@@ -107,22 +117,25 @@ static constexpr int cap_g(int nt) { return 2 * nt + nt / 4 + 32; }
 
 struct Stage {
   int nt = 0, nblk = 0, remap = 1;
-  bool ap = false;
+  int scheme = kPlain;
   Alloc A;
   int4 *head = nullptr;      // [nblk] first own cell, own cells | |L| << 16, |C| | triangles around C << 16,
                              // local cells | triangles << 16
   int32_t *halo = nullptr;   // [nblk][nt] cells of the local ids past the own ones
   uint4 *topo = nullptr;     // [nblk][cap_l]
-  void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~
+  void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~, with diffusion K / A;
+                             // pxt16: PV weights of the earlier triangle at edges 0-3; 4, 5
   void *eld = nullptr;       // [NE] Pair: length, dual length
   uint16_t *oth = nullptr;   // [NE] local id of the edge's other cell | it is v1 << 10; 0xFFFF dummy
   uint32_t *tv = nullptr;    // [nblk][cap_t] vertices a, b (10 bits each), edge bits (9), curl signs (3)
   uint16_t *tslot = nullptr; // [nblk][cap_t] local slot 2 owner + k
   void *tk = nullptr;        // [nblk][cap_t] Quad: kite weights, 1 / (A_t a)
   void *tf = nullptr;        // [nblk][cap_t] Coriolis parameter
-  void *wc = nullptr;        // APVM: [nblk][6][cap_l] Tri: Perot weights of a cell's velocity
+  void *wc = nullptr;        // APVM, pxt16: [nblk][6][cap_l] Tri: Perot weights of a cell's velocity
   void *wt = nullptr;        // APVM: [nblk][3][cap_g] Tri: those of grad q at a triangle
   ushort4 *tn = nullptr;     // APVM: [nblk][cap_g] local slots of the triangles across and its own
+  void *en = nullptr;        // pxt16: [NE] Tri: normal of the Coriolis term
+  void *tkt = nullptr;       // diffusion: [nblk][cap_t] coefficient at triangles
 };
 
 template <typename T>
@@ -137,8 +150,6 @@ struct StageArgs {
   const uint16_t *tslot;
   const Quad<T> *tk;
   const T *tf;
-  const Tri<T> *wc, *wt;
-  const ushort4 *tn;
   const double *iaa;
   const T *hs, *us, *h0, *u0, *gb, *dte;
   const double *dtc;
@@ -146,9 +157,19 @@ struct StageArgs {
   double *dh_out;
   int *flag;
   double href, ca, cb;  // the stage's step and its weight in the sum (ensembles: per cell)
-  T grav, inv_a, cat, cbt, pvsdt;
+  T grav, inv_a, cat, cbt;
   int nblk, remap, use_pv, flin, zero_mom;
   int whole;  // the third stage: its state is a whole step away
+};
+// the operands of the options, which the plain scheme's kernel does not take:
+// with them its arguments are a cache line longer and a glevel-6 step 1.3 %
+// slower
+template <typename T>
+struct StageOpts : StageArgs<T> {
+  const Tri<T> *wc, *wt, *en;
+  const T *tkt;
+  const ushort4 *tn;
+  T pvsdt;
 };
 
 // Compensated summation: c gathers the exact rounding errors of s (Knuth's
@@ -189,15 +210,20 @@ __device__ __forceinline__ void put(X *p, uint32_t i, X v) {
 }
 
 // MODE: 0 the first RK stage, 1 the second and third, 2 the last, 3 a
-// tendency. AP: with APVM.
-template <typename T, int NT, int MODE, bool AP>
-__global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const StageArgs<T> a) {
+// tendency. SCHEME: trsk10's methods (kPlain), with APVM or diffusion, or
+// pxt16's (kPerot).
+template <typename T, int NT, int MODE, int SCHEME, class Args>
+__global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast_stage(const Args a) {
+  constexpr bool AP = SCHEME == kApvm, PX = SCHEME == kPerot, DF = SCHEME == kDiff;
   constexpr int LC = cap_a(NT), CL = cap_l(NT, AP), TC = cap_t(NT, AP), GC = cap_g(NT);
   constexpr int NR = (TC + NT - 1) / NT, NG = (GC + NT - 1) / NT;
   __shared__ T sU[3 * LC], sD[3 * LC], sA[3 * LC];  // u, dual length, u l
   __shared__ T sH[LC], sQ[2 * LC], sPhi[NT], sPP[6 * NT];
   __shared__ Tri<T> sV[AP ? CL : 1], sG[AP ? 2 * CL : 1];  // Perot velocity at cells, grad q at triangles
   T *sP = sPP, *sPo = sPP + 3 * NT;  // partials of the own edges' owners and other cells
+  Tri<T> *sAB = reinterpret_cast<Tri<T> *>(sPP);  // pxt16: Perot vectors of u h, u h q at the cells of C
+  __shared__ T sE[PX || DF ? 3 * NT : 1];  // own edges: PV (pxt16), the jump of K zeta (diffusion)
+  __shared__ T sZ[DF ? 2 * LC : 1];        // K zeta
   int b = blockIdx.x;
   if (a.remap) b = (b % NXCD) * (gridDim.x / NXCD) + b / NXCD;
   if (b >= a.nblk) return;
@@ -251,7 +277,14 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
     tf[r] = at(a.tf + (size_t)b * TC, t);
   }
   uint4 tpl;
-  Tri<T> wc[2][MX];
+  T tkt[NR];
+  if constexpr (DF)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) tkt[r] = at(a.tkt + (size_t)b * TC, min(tid + r * NT, nTri - 1));
+  Tri<T> wc[AP ? 2 : 1][MX];
+  if constexpr (PX)
+#pragma unroll
+    for (int j = 0; j < MX; ++j) wc[0][j] = at(a.wc + (size_t)b * MX * CL + j * CL, tid);
   if constexpr (AP) {
     const Tri<T> *w = a.wc + (size_t)b * MX * CL;
     const int i = min(tid + NT, CL - 1);
@@ -267,12 +300,14 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
   const double iaa = at(a.iaa + own0, oc);
   T y0 = (T)0, ac = (T)0, v0[3], av[3];
   uint32_t ow[3];
+  Tri<T> en[3];
   if (MODE != 3) y0 = at(a.h0 + own0, oc);
   if (MODE == 1 || MODE == 2) ac = at((const T *)a.acch + own0, oc);
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
     const int e = min(tid + r * NT, 3 * nown - 1);
     ow[r] = at(a.oth + 3 * (size_t)own0, e);
+    if constexpr (PX) en[r] = at(a.en + 3 * (size_t)own0, e);
     if (MODE != 3) v0[r] = at(a.u0 + 3 * (size_t)own0, e);
     if (MODE == 1 || MODE == 2) av[r] = at((const T *)a.accu + 3 * (size_t)own0, e);
   }
@@ -348,11 +383,13 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
     const int e0 = 3 * ((eb & 1) ? o : va) + ((eb >> 1) & 3);
     const int e1 = 3 * (((eb >> 3) & 1) ? va : vb) + ((eb >> 4) & 3);
     const int e2 = 3 * (((eb >> 6) & 1) ? vb : o) + ((eb >> 7) & 3);
-    if (!a.flin) {
+    if (DF || !a.flin) {
       T z = flip(sA[e0], (v << 2) & 0x80000000u);
       z += flip(sA[e1], (v << 1) & 0x80000000u);
       z += flip(sA[e2], v & 0x80000000u);
-      eta += z * k.w;
+      z *= k.w;
+      if (!a.flin) eta += z;
+      if constexpr (DF) sZ[sl] = tkt[r] * z;
     }
     T hsum = k.x * sH[o];
     hsum += k.y * sH[va];
@@ -404,15 +441,17 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
     const T hc = sH[tid];
     double dv = 0.0, dvc = 0.0;
     T ke = (T)0;
-    T G[MX];
+    T G[MX];  // mass flux; pxt16: u h
+    Tri<T> v{(T)0, (T)0, (T)0};
+    double du = 0.0;
 #pragma unroll
     for (int j = 0; j < MX; ++j) {
       const bool valid = (j < MX - 1) || hex;
       const T u = sU[ed[j]], dl = sD[ed[j]];
       // both cells of an edge form the same product, so the mass flux
       // cancels exactly between them
-      double g = (double)flip(u, f[j] & 0x80000000u) *
-                 fma_(0.5, (double)hc + (double)sH[nb[j]], a.href) * (double)dl;
+      const double he = fma_(0.5, (double)hc + (double)sH[nb[j]], a.href);
+      double g = (double)flip(u, f[j] & 0x80000000u) * he * (double)dl;
       T k = sA[ed[j]] * (u * dl);
       if (!valid) {
         g = 0.0;
@@ -420,9 +459,22 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
       }
       if (j == 0) dv = g;
       else two_sum(dv, dvc, g);
-      G[j] = (T)g;
-      ke += k;
+      if constexpr (PX) {
+        // perhx: the kinetic energy of the Perot velocity (a pentagon's
+        // padded slot has a zero weight)
+        G[j] = u * (T)he;
+        v.x = fma_(wc[0][j].x, u, v.x);
+        v.y = fma_(wc[0][j].y, u, v.y);
+        v.z = fma_(wc[0][j].z, u, v.z);
+      } else {
+        G[j] = (T)g;
+        ke += k;
+      }
+      if constexpr (DF) du += valid ? (double)flip(u, f[j] & 0x80000000u) * (double)dl : 0.0;
     }
+    T K = PX ? (v.x * v.x + v.y * v.y + v.z * v.z) / (T)2 : ke * w1.z;
+    // the normal part of the diffusion: grad(K div u) folds into the potential
+    if constexpr (DF) K -= (T)(du * (double)w1.w);
     T qt[MX];
     int ts[MX];
 #pragma unroll
@@ -436,7 +488,7 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
     if (!hex) qt[MX - 1] = (T)0;
     T pot = a.grav * hc;
     if (a.gb) pot += at(a.gb, tid < nown ? own0 + tid : halo[tid - nown]);
-    sPhi[tid] = (pot + ke * w1.z) * a.inv_a;
+    sPhi[tid] = (pot + K) * a.inv_a;
     if (tid < nown) {
       const double dh = -(dv + dvc) * iaa;
       // the step over the stage's share of it (1, 2 halves) and over 6 or 3
@@ -457,9 +509,16 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
     }
     // PV at the cell's edges: edge j lies between ring triangles j-1 and j
     T qe[MX];
-    qe[0] = (T)0.5 * ((hex ? qt[MX - 1] : qt[MX - 2]) + qt[0]);
+    const T ql = hex ? qt[MX - 1] : qt[MX - 2];
+    if constexpr (PX) {
+      const T w[MX] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
 #pragma unroll
-    for (int j = 1; j < MX; ++j) qe[j] = (T)0.5 * (qt[j - 1] + qt[j]);
+      for (int j = 0; j < MX; ++j) qe[j] = w[j] * (j ? qt[j - 1] : ql) + ((T)1 - w[j]) * qt[j];
+    } else {
+      qe[0] = (T)0.5 * (ql + qt[0]);
+#pragma unroll
+      for (int j = 1; j < MX; ++j) qe[j] = (T)0.5 * (qt[j - 1] + qt[j]);
+    }
     if constexpr (AP) {
       // q_e -= pvspar dt (grad q(t_{j-1}) + grad q(t_j)) . (v(c) + v(nb_j))
       if (!hex) ts[MX - 1] = ts[MX - 2];  // the ring's last triangle, and in place of the pad
@@ -473,32 +532,58 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
       }
       if (!hex) qe[MX - 1] = (T)0;
     }
-    // TRiSK weights from prefix sums of the kite areas:
-    // w(i,j) = S_j - S_i - 1/2 (j>i), S_6 - S_i + S_j - 1/2 (j<i), w(i,i) = 0
-    const T R[MX] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
-    T S[MX + 1];
-    S[0] = (T)0;
+    if constexpr (PX) {
+      // pered: the Perot reconstruction here of uh (q_e + q_l) / 2 for an edge
+      // l is (q_l A + B) / 2 with A = P(uh) and B = P(uh q); P3 takes both
+      // cells' A and B with q_l
+      Tri<T> A{(T)0, (T)0, (T)0}, B{(T)0, (T)0, (T)0};
 #pragma unroll
-    for (int j = 0; j < MX; ++j) S[j + 1] = S[j] + R[j];
-    const T rest = S[MX] - (T)0.5;
-    // P_i = sum_j G_j (q_i + q_j)/2 w(i,j) = (q_i sum_j G_j w + sum_j G_j q_j w)/2
-    T H[MX];
+      for (int j = 0; j < MX; ++j) {
+        const T uq = G[j] * qe[j];
+        A.x = fma_(wc[0][j].x, G[j], A.x);
+        A.y = fma_(wc[0][j].y, G[j], A.y);
+        A.z = fma_(wc[0][j].z, G[j], A.z);
+        B.x = fma_(wc[0][j].x, uq, B.x);
+        B.y = fma_(wc[0][j].y, uq, B.y);
+        B.z = fma_(wc[0][j].z, uq, B.z);
+        if (tid < nown && ((f[j] >> (16 + SB_OWN)) & 1) && (j < MX - 1 || hex)) sE[ed[j]] = qe[j];
+      }
+      sAB[tid] = A;
+      sAB[NT + tid] = B;
+    } else {
+      const T R[MX] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
+      // TRiSK weights from prefix sums of the kite areas:
+      // w(i,j) = S_j - S_i - 1/2 (j>i), S_6 - S_i + S_j - 1/2 (j<i), w(i,i) = 0
+      T S[MX + 1];
+      S[0] = (T)0;
 #pragma unroll
-    for (int j = 0; j < MX; ++j) H[j] = G[j] * qe[j];
+      for (int j = 0; j < MX; ++j) S[j + 1] = S[j] + R[j];
+      const T rest = S[MX] - (T)0.5;
+      // P_i = sum_j G_j (q_i + q_j)/2 w(i,j) = (q_i sum_j G_j w + sum_j G_j q_j w)/2
+      T H[MX];
 #pragma unroll
-    for (int i = 0; i < MX; ++i) {
-      T x = (T)0, y = (T)0;
+      for (int j = 0; j < MX; ++j) H[j] = G[j] * qe[j];
 #pragma unroll
-      for (int j = 0; j < MX; ++j)
-        if (j != i) {
-          const T w = (j > i) ? (S[j] - S[i]) - (T)0.5 : rest - (S[i] - S[j]);
-          x = fma_(G[j], w, x);
-          y = fma_(H[j], w, y);
+      for (int i = 0; i < MX; ++i) {
+        T x = (T)0, y = (T)0;
+#pragma unroll
+        for (int j = 0; j < MX; ++j)
+          if (j != i) {
+            const T w = (j > i) ? (S[j] - S[i]) - (T)0.5 : rest - (S[i] - S[j]);
+            x = fma_(G[j], w, x);
+            y = fma_(H[j], w, y);
+          }
+        const T P = flip((T)0.5 * fma_(qe[i], x, y), (f[i] << 1) & 0x80000000u);
+        // for the block's own edges: by its owner or by its other cell
+        T *to = (f[i] >> (16 + SB_OWN)) & 1 ? sP : sPo;
+        if (ed[i] < 3 * nown && (i < MX - 1 || hex)) to[ed[i]] = P;
+        if constexpr (DF) {
+          // the tangential part: the jump of K zeta between the edge's triangles
+          const T jump = sZ[ts[i]] - sZ[ts[i ? i - 1 : hex ? MX - 1 : MX - 2]];
+          if (tid < nown && ((f[i] >> (16 + SB_OWN)) & 1) && (i < MX - 1 || hex))
+            sE[ed[i]] = flip(jump, (tp.w << (31 - SW_FZ - i)) & 0x80000000u);
         }
-      const T P = flip((T)0.5 * fma_(qe[i], x, y), (f[i] << 1) & 0x80000000u);
-      // for the block's own edges: by its owner or by its other cell
-      T *to = (f[i] >> (16 + SB_OWN)) & 1 ? sP : sPo;
-      if (ed[i] < 3 * nown && (i < MX - 1 || hex)) to[ed[i]] = P;
+      }
     }
   }
   __syncthreads();
@@ -513,7 +598,19 @@ __global__ __launch_bounds__(NT, AP && NT == 512 ? 4 : 1) void fast_stage(const 
     const int o = i / 3, c2 = w & LID;
     const bool own_v2 = (w >> SB_OWN) & 1;
     const T d = own_v2 ? sPhi[o] - sPhi[c2] : sPhi[c2] - sPhi[o];
-    T du = -(d + (sP[i] + sPo[i])) * recip(el[r].x);
+    T du;
+    if constexpr (PX) {
+      const T ql = sE[i];
+      const Tri<T> A1 = sAB[o], A2 = sAB[c2], B1 = sAB[NT + o], B2 = sAB[NT + c2];
+      const T uhq = (T)0.25 * (en[r].x * (ql * (A1.x + A2.x) + (B1.x + B2.x)) +
+                               en[r].y * (ql * (A1.y + A2.y) + (B1.y + B2.y)) +
+                               en[r].z * (ql * (A1.z + A2.z) + (B1.z + B2.z)));
+      du = -d * recip(el[r].x) - uhq;
+    } else {
+      T P = sP[i] + sPo[i];
+      if constexpr (DF) P += el[r].x * recip(el[r].y) * a.inv_a * sE[i];
+      du = -(d + P) * recip(el[r].x);
+    }
     if (a.zero_mom) du = (T)0;
     T ca = a.cat, cb = a.cbt;
     if (a.dte) {
@@ -547,7 +644,7 @@ void stage_free(imx_swm *s) {
 }
 
 int stage_threads(const imx_swm *s) { return s->stg ? s->stg->nt : 0; }
-bool stage_apvm(const imx_swm *s) { return s->stg && s->stg->ap; }
+int stage_scheme(const imx_swm *s) { return s->stg ? s->stg->scheme : -1; }
 void stage_set_remap(imx_swm *s, int remap) {
   if (s->stg) s->stg->remap = remap;
 }
@@ -589,9 +686,9 @@ struct LocalSets {
 };
 
 template <typename T>
-static int build(imx_swm *s, int nt) {
+static int build(imx_swm *s, int nt, int scheme) {
   const int nv = s->nv, NE = s->NE, NTri = s->NT;
-  const bool ap = s->f_apvm;
+  const bool ap = scheme == kApvm, px = scheme == kPerot, df = scheme == kDiff;
   const int LC = cap_a(nt), CL = cap_l(nt, ap), TC = cap_t(nt, ap), GC = cap_g(nt);
   const double ea = s->o.erad;
   std::vector<int32_t> nbr, bA, bB, oth, tab, teb;
@@ -606,8 +703,13 @@ static int build(imx_swm *s, int nt) {
     return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
   std::vector<Quad<T>> awc, awt;
   std::vector<int32_t> atn;
-  if (ap && (!down(awc, s->x_ap_wc, (size_t)MX * nv) || !down(awt, s->x_ap_wt, (size_t)3 * NTri) ||
-             !down(atn, s->x_ap_tnb, (size_t)3 * NTri)))
+  std::vector<Quad<T>> pn;
+  std::vector<T> pq, kh, kt;
+  std::vector<double> iaa;
+  if (((ap || px) && !down(awc, s->x_ap_wc, (size_t)MX * nv)) ||
+      (ap && (!down(awt, s->x_ap_wt, (size_t)3 * NTri) || !down(atn, s->x_ap_tnb, (size_t)3 * NTri))) ||
+      (px && (!down(pn, s->x_px_n, NE) || !down(pq, s->x_px_wq, (size_t)MX * nv))) ||
+      (df && (!down(kh, s->x_kh, nv) || !down(kt, s->x_kt, NTri) || !down(iaa, s->x_c_iaa, nv))))
     return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
 
   auto tri_of = [&](int c, int j) {
@@ -698,7 +800,7 @@ static int build(imx_swm *s, int nt) {
     if (!ok) return IMX_OK;
   if (nblk > 1 && (int64_t)nblk * nt > (int64_t)3 * nv) return IMX_OK;
   // the kernel addresses its tables by 32-bit byte offsets
-  if ((uint64_t)NE * sizeof(Pair<T>) >> 32) return IMX_OK;
+  if ((uint64_t)NE * sizeof(Tri<T>) >> 32) return IMX_OK;
 
   std::vector<int4> head(nblk);
   std::vector<int32_t> halo((size_t)nblk * nt, 0);
@@ -708,7 +810,10 @@ static int build(imx_swm *s, int nt) {
   std::vector<uint16_t> loth(NE, 0xFFFF), tslot((size_t)nblk * TC, 0);
   std::vector<uint32_t> tv((size_t)nblk * TC, 0);
   std::vector<T> tfv((size_t)nblk * TC, (T)0);
-  std::vector<Tri<T>> wc(ap ? (size_t)nblk * MX * CL : 0, Tri<T>{0, 0, 0}),
+  std::vector<Tri<T>> eno(px ? NE : 0);
+  for (int e = 0; px && e < NE; ++e) eno[e] = Tri<T>{pn[e].x, pn[e].y, pn[e].z};
+  std::vector<T> tktv(df ? (size_t)nblk * TC : 0, (T)0);
+  std::vector<Tri<T>> wc(ap || px ? (size_t)nblk * MX * CL : 0, Tri<T>{0, 0, 0}),
       wt(ap ? (size_t)nblk * 3 * GC : 0, Tri<T>{0, 0, 0});
   std::vector<ushort4> tn(ap ? (size_t)nblk * GC : 0, ushort4{0, 0, 0, 0});
   for (int e = 0; e < NE; ++e) eld[e] = Pair<T>{(T)leng[e], (T)dleng[e]};
@@ -750,17 +855,18 @@ static int build(imx_swm *s, int nt) {
           f[j] |= ((bA[c] >> (BA_TNR + j)) & 1u) << SB_TNR;
           t3 |= ((bB[c] >> (BB_TSEL + 2 * j)) & 3u) << (2 * j);
           t3 |= ((bB[c] >> (BB_KT + j)) & 1u) << (SW_KT + j);
-          r[j] = R[(size_t)j * nv + c];
+          if (df) t3 |= ((bA[c] >> (BA_FZ + j)) & 1u) << (SW_FZ + j);
+          r[j] = px ? pq[(size_t)j * nv + c] : R[(size_t)j * nv + c];
         }
         topo[(size_t)b * CL + k] = uint4{f[0] | f[1] << 16, f[2] | f[3] << 16, f[4] | f[5] << 16, t3};
-        for (int j = 0; ap && j < MX; ++j) {
+        for (int j = 0; (ap || px) && j < MX; ++j) {
           const Quad<T> &q = awc[(size_t)j * nv + c];
           wc[((size_t)b * MX + j) * CL + k] = Tri<T>{q.x, q.y, q.z};
         }
         if (k >= nC) continue;
         cw[((size_t)b * 2) * nt + k] = Quad<T>{r[0], r[1], r[2], r[3]};
         // ika = 1 / sum (l l~ / 4)
-        cw[((size_t)b * 2 + 1) * nt + k] = Quad<T>{r[4], r[5], (T)0.25 * ika[c], (T)0};
+        cw[((size_t)b * 2 + 1) * nt + k] = Quad<T>{r[4], r[5], (T)0.25 * ika[c], df ? (T)((double)kh[c] * iaa[c]) : (T)0};
       }
       for (int k = 0; k < (int)tris.size(); ++k) {
         const int t = tris[k];
@@ -772,6 +878,7 @@ static int build(imx_swm *s, int nt) {
         tslot[p] = (uint16_t)(2 * id(t / 2) + t % 2);
         tk[p] = Quad<T>{kap[t], kap[(size_t)NTri + t], kap[(size_t)2 * NTri + t], (T)(1.0 / (tarea[t] * ea))};
         tfv[p] = tf[t];
+        if (df) tktv[p] = kt[t];
         if (!ap || k >= w.nG) continue;
         auto slot = [&](int i) { return (unsigned short)(2 * id(i / 2) + i % 2); };
         tn[(size_t)b * GC + k] = ushort4{slot(atn[t]), slot(atn[(size_t)NTri + t]), slot(atn[(size_t)2 * NTri + t]),
@@ -803,9 +910,11 @@ static int build(imx_swm *s, int nt) {
   g->tslot = A.put(tslot);
   g->tk = A.put(tk);
   g->tf = A.put(tfv);
-  g->ap = ap;
+  g->scheme = scheme;
+  if (ap || px) g->wc = A.put(wc);
+  if (px) g->en = A.put(eno);
+  if (df) g->tkt = A.put(tktv);
   if (ap) {
-    g->wc = A.put(wc);
     g->wt = A.put(wt);
     g->tn = A.put(tn);
   }
@@ -817,41 +926,42 @@ static int build(imx_swm *s, int nt) {
   return IMX_OK;
 }
 
-int stage_build(imx_swm *s, int nt) {
+int stage_build(imx_swm *s, int nt, int scheme) {
   stage_free(s);
   try {
-    return s->single ? build<float>(s, nt) : build<double>(s, nt);
+    return s->single ? build<float>(s, nt, scheme) : build<double>(s, nt, scheme);
   } catch (const std::bad_alloc &) {
     return set_error(IMX_ENOMEM, "stage tables: host out of memory");
   }
 }
 
-template <typename T, int NT, bool AP>
-static void launch_nt(const StageArgs<T> &a, int stage, int grid, hipStream_t st) {
+template <typename T, int NT, int S>
+static void launch_nt(const StageOpts<T> &a, int stage, int grid, hipStream_t st) {
+  using Args = std::conditional_t<S == kPlain, StageArgs<T>, StageOpts<T>>;
   switch (stage) {
-    case 0: fast_stage<T, NT, 0, AP><<<grid, NT, 0, st>>>(a); break;
+    case 0: fast_stage<T, NT, 0, S, Args><<<grid, NT, 0, st>>>(a); break;
     case 1:
-    case 2: fast_stage<T, NT, 1, AP><<<grid, NT, 0, st>>>(a); break;
-    case 3: fast_stage<T, NT, 2, AP><<<grid, NT, 0, st>>>(a); break;
-    default: fast_stage<T, NT, 3, AP><<<grid, NT, 0, st>>>(a); break;
+    case 2: fast_stage<T, NT, 1, S, Args><<<grid, NT, 0, st>>>(a); break;
+    case 3: fast_stage<T, NT, 2, S, Args><<<grid, NT, 0, st>>>(a); break;
+    default: fast_stage<T, NT, 3, S, Args><<<grid, NT, 0, st>>>(a); break;
   }
 }
 
-template <typename T, bool AP>
-static void launch_threads(const StageArgs<T> &a, int nt, int stage, int grid, hipStream_t st) {
+template <typename T, int S>
+static void launch_threads(const StageOpts<T> &a, int nt, int stage, int grid, hipStream_t st) {
   switch (nt) {
-    case 128: launch_nt<T, 128, AP>(a, stage, grid, st); break;
+    case 128: launch_nt<T, 128, S>(a, stage, grid, st); break;
     case 512:
-      if constexpr (sizeof(T) == 4) launch_nt<T, 512, AP>(a, stage, grid, st);
+      if constexpr (sizeof(T) == 4) launch_nt<T, 512, S>(a, stage, grid, st);
       break;
-    default: launch_nt<T, 256, AP>(a, stage, grid, st); break;
+    default: launch_nt<T, 256, S>(a, stage, grid, st); break;
   }
 }
 
 template <typename T>
 void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *uout) {
   const Stage &g = *s->stg;
-  StageArgs<T> a;
+  StageOpts<T> a;
   a.head = g.head;
   a.halo = g.halo;
   a.topo = g.topo;
@@ -865,6 +975,8 @@ void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *u
   a.wc = (const Tri<T> *)g.wc;
   a.wt = (const Tri<T> *)g.wt;
   a.tn = g.tn;
+  a.en = (const Tri<T> *)g.en;
+  a.tkt = (const T *)g.tkt;
   a.pvsdt = (T)(s->sc.pvspar * s->o.dt);
   a.iaa = s->x_c_iaa;
   a.hs = hs;
@@ -898,8 +1010,12 @@ void stage_launch(imx_swm *s, int stage, const T *hs, const T *us, T *hout, T *u
   a.flin = s->f_lin ? 1 : 0;
   a.zero_mom = s->o.testcase <= 1;
   const int grid = (g.nblk + NXCD - 1) / NXCD * NXCD;
-  if (g.ap) launch_threads<T, true>(a, g.nt, stage, grid, s->stream);
-  else launch_threads<T, false>(a, g.nt, stage, grid, s->stream);
+  switch (g.scheme) {
+    case kApvm: launch_threads<T, kApvm>(a, g.nt, stage, grid, s->stream); break;
+    case kPerot: launch_threads<T, kPerot>(a, g.nt, stage, grid, s->stream); break;
+    case kDiff: launch_threads<T, kDiff>(a, g.nt, stage, grid, s->stream); break;
+    default: launch_threads<T, kPlain>(a, g.nt, stage, grid, s->stream); break;
+  }
 }
 template void stage_launch<float>(imx_swm *, int, const float *, const float *, float *, float *);
 template void stage_launch<double>(imx_swm *, int, const double *, const double *, double *, double *);

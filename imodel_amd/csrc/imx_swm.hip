@@ -1786,15 +1786,21 @@ static void launch_ref_step(imx_swm *s) {
     default: CALL(256); break;   \
   }
 
-// The schemes imx_stage.hip evaluates in one launch per stage: trsk10's
-// methods without options or with APVM, HTC or HC, with any topography and
-// Coriolis term.
-static bool stage_scheme(const imx_swm *s) {
-  return !(s->f_gass || s->f_melv || s->f_perhx || s->f_nopv || s->f_bary || s->f_pered || s->f_gk || s->f_dtred ||
-           s->f_diff || s->f_hyper);
+// The schemes imx_stage.hip evaluates in one launch per stage, with any
+// topography and Coriolis term: trsk10's methods without options (0), with
+// APVM (1) or with diffusion (3), HTC or HC, and pxt16's three methods on HTC
+// (2). -1, their combinations and the other methods: the passes below, which
+// at glevel 7 FP32 take 78, 126, 89 and 105 us a step for 0, 1, 3 and 2 where
+// one launch takes 44, 77, 49 and 56.
+static int one_launch_scheme(const imx_swm *s) {
+  if (s->f_gass || s->f_melv || s->f_nopv || s->f_gk || s->f_dtred || s->f_hyper) return -1;
+  const bool any = s->f_bary || s->f_pered || s->f_perhx;
+  if (s->f_apvm + s->f_diff + any > 1) return -1;
+  if (any) return s->f_bary && s->f_pered && s->f_perhx && !s->f_pxhc ? 2 : -1;
+  return s->f_apvm ? 1 : s->f_diff ? 3 : 0;
 }
 static bool stage_on(const imx_swm *s) {
-  return s->stg && !s->stg_stale && stage_scheme(s) && stage_apvm(s) == s->f_apvm;
+  return s->stg && !s->stg_stale && stage_scheme(s) == one_launch_scheme(s);
 }
 
 // One FAST stage: stage<0 evaluates the tendency of (hs, us) into dh_out/du_out.
@@ -2691,6 +2697,8 @@ static int validate_desc(const imx_mesh_desc &d) {
 //   glevel 8 FP32   256: 317    512: 291   512, no remap: 285
 //   glevel 8 FP64   256: 695               256, no remap: 686
 //   glevel 9 FP32   256: 1206              512, no remap: 1124
+// pxt16 and diffusion take the plain scheme's: no other choice was more than
+// 2 % faster (pxt16 glevel 8 256: 158, 512: 155).
 static bool stage_large(const imx_swm *s) { return (size_t)s->nv * (s->single ? 4 : 8) > ((size_t)8 << 20); }
 static void stage_defaults(imx_swm *s) {
   s->stg_nt[0] = s->nv < 30000 ? 128 : stage_large(s) && s->single ? 512 : 256;
@@ -2698,23 +2706,28 @@ static void stage_defaults(imx_swm *s) {
   const bool apvm_large = (size_t)s->nv * (s->single ? 4 : 8) > ((size_t)2 << 20);
   s->stg_nt[1] = s->nv < 30000 ? 128 : apvm_large && s->single ? 512 : 256;
   s->stg_remap[1] = apvm_large ? 0 : 1;
+  for (int k = 2; k < 4; ++k) {
+    s->stg_nt[k] = s->stg_nt[0];
+    s->stg_remap[k] = s->stg_remap[0];
+  }
 }
 
 // (Re)builds the stage tables for the handle's scheme: they follow its
 // staggering, triangle weights and Coriolis parameter, and are made again
 // when a scheme that has them is back.
 static int stage_make(imx_swm *s) {
-  const int rc = stage_build(s, s->stg_nt[s->f_apvm]);
-  stage_set_remap(s, s->stg_remap[s->f_apvm]);
+  const int k = one_launch_scheme(s), rc = stage_build(s, s->stg_nt[k], k);
+  stage_set_remap(s, s->stg_remap[k]);
   s->stg_stale = false;
   return rc;
 }
 static int stage_refresh(imx_swm *s) {
   s->stg_stale = true;
-  if (!s->stg_local || !stage_scheme(s)) return IMX_OK;
+  const int k = one_launch_scheme(s);
+  if (!s->stg_local || k < 0) return IMX_OK;
   const int rc = stage_make(s);
-  if (!s->f_apvm || !rc) return rc;
-  // no room for APVM's tables: the three passes need none
+  if (!k || !rc) return rc;
+  // no room for an option's tables: the passes need none
   (void)hipGetLastError();
   return IMX_OK;
 }
@@ -3131,10 +3144,11 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   if (stage_on(s)) {
     // one launch per stage: block threads (which cut the mesh anew) x remap
     double best = 1e30;
-    int &bb = s->stg_nt[s->f_apvm], &br = s->stg_remap[s->f_apvm];
+    int &bb = s->stg_nt[stage_scheme(s)], &br = s->stg_remap[stage_scheme(s)];
+    const int scheme = stage_scheme(s);
     for (int bs : {128, 256, 512}) {
       if (bs == 512 && !s->single) continue;  // over 64 KB of LDS
-      if ((rc = stage_build(s, bs))) break;
+      if ((rc = stage_build(s, bs, scheme))) break;
       if (!s->stg) continue;
       for (int r = 0; r < 2 && !rc; ++r) {
         stage_set_remap(s, r);
