@@ -219,7 +219,7 @@ struct imx_swm {
   int nparts = 0;
 
   // REF state and fields
-  double *rh = nullptr, *ru = nullptr, *rhn = nullptr, *run = nullptr;
+  double *rh = nullptr, *ru = nullptr, *rhn = nullptr, *rhm = nullptr, *run = nullptr;
   double *massf = nullptr, *momf = nullptr;
   double *f_h_ed = nullptr, *f_uh = nullptr, *f_eta = nullptr, *f_h_tr = nullptr,
          *f_q_tr = nullptr, *f_q_ed = nullptr, *f_divuh = nullptr, *f_ke = nullptr,

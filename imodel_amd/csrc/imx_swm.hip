@@ -72,6 +72,7 @@ static inline int grid_bs(int n, int bs) {
 
 // epsilon(1.)/1e5 of the reference zero guard (swm_operators.f90:1603)
 #define HTR_GUARD (1.1920928955078125e-07 / 100000.0)
+#define REF_ONE_MAX 65536  // edges; see ref_one
 
 // ============================================================ REF kernels ==
 // What ode_rk4 does with a tendency value (swm.f90:2647-2678), by the kernel
@@ -113,59 +114,72 @@ __device__ __forceinline__ void ref_edge_flux(int l, int ne, const int32_t *__re
   uh[l] = u[l] * he;
 }
 
+struct RefPre {
+  int ne, nt, nbe;  // nbe blocks of edges, then blocks of triangles
+  const int32_t *e_v;
+  const double *hb;
+  const int32_t *hv;
+  const double *h, *u;
+  double *h_ed, *uh;
+  const int32_t *t_ed;
+  const int8_t *t_tg;
+  const int32_t *t_v;
+  const double *t_area, *t_f, *t_trhx, *e_leng;
+  int hmode;
+  const double *t_w;
+  double erad;
+  int use_pv, flin;
+  double *eta, *zeta, *h_tr, *q_tr;
+  int *flag;
+};
+
+struct RefTri {
+  double zeta, eta, h, q;
+};
+
 // vort_tr + rel_vort_tr + scalar_hx2tr + scalar_elem_divide
 // (swm_operators.f90:551-611, :780-827, :258-263, :1579-1615)
 // h at triangles: trsk area weights (hmode 0), barycentric coordinates t_w
 // (1, pxt16), or edge values weighted by the edge's sub-triangle areas t_w
 // (2, gass18: scalar_edtr2trcc, swm_operators.f90:286-346)
-__device__ __forceinline__ void ref_tri(int k, int nt, const int32_t *__restrict__ t_ed,
-                                               const int8_t *__restrict__ t_tg,
-                                               const int32_t *__restrict__ t_v,
-                                               const double *__restrict__ t_area,
-                                               const double *__restrict__ t_f,
-                                               const double *__restrict__ t_trhx,
-                                               const double *__restrict__ e_leng,
-                                               const double *__restrict__ u,
-                                               const double *__restrict__ h, int hmode,
-                                               const double *__restrict__ t_w,
-                                               const double *__restrict__ h_ed, double erad,
-                                               int use_pv, int flin, double *__restrict__ eta,
-                                               double *__restrict__ zeta,
-                                               double *__restrict__ h_tr,
-                                               double *__restrict__ q_tr, int *__restrict__ flag) {
-  if (k >= nt || t_ed[k] < 0) return;
+__device__ __forceinline__ RefTri ref_tri_value(const RefPre &a, int k) {
+  const int nt = a.nt;
+  RefTri r;
   double e = 0.0;
 #pragma unroll
   for (int l = 0; l < 3; ++l) {
-    const int ed = t_ed[l * nt + k];
-    e = e + u[ed] * e_leng[ed] * (double)t_tg[l * nt + k];
+    const int ed = a.t_ed[l * nt + k];
+    e = e + a.u[ed] * a.e_leng[ed] * (double)a.t_tg[l * nt + k];
   }
-  const double z = e / t_area[k] / erad;
-  zeta[k] = z;
+  r.zeta = e / a.t_area[k] / a.erad;
   // absolute vorticity; the linearised f-sphere keeps f alone
-  const double et = flin ? t_f[k] : z + t_f[k];
-  eta[k] = et;
-  double s = 0.0, ht;
-  if (hmode == 1) {
+  r.eta = a.flin ? a.t_f[k] : r.zeta + a.t_f[k];
+  double s = 0.0;
+  if (a.hmode == 1) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) s = s + t_w[i * nt + k] * h[t_v[i * nt + k]];
-    ht = s;
-  } else if (hmode == 2) {
+    for (int i = 0; i < 3; ++i) s = s + a.t_w[i * nt + k] * a.h[a.t_v[i * nt + k]];
+    r.h = s;
+  } else if (a.hmode == 2) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) s = s + t_w[i * nt + k] * h_ed[t_ed[i * nt + k]];
-    ht = s / t_area[k];
+    for (int i = 0; i < 3; ++i) s = s + a.t_w[i * nt + k] * a.h_ed[a.t_ed[i * nt + k]];
+    r.h = s / a.t_area[k];
   } else {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) s = s + t_trhx[i * nt + k] * h[t_v[i * nt + k]];
-    ht = s / t_area[k];
+    for (int i = 0; i < 3; ++i) s = s + a.t_trhx[i * nt + k] * a.h[a.t_v[i * nt + k]];
+    r.h = s / a.t_area[k];
   }
-  h_tr[k] = ht;
-  double q = 0.0;
-  if (use_pv) {
-    if (fabs(ht) < HTR_GUARD) flag[0] = 1;
-    else q = et / ht;
-  }
-  q_tr[k] = q;
+  r.q = a.use_pv && !(fabs(r.h) < HTR_GUARD) ? r.eta / r.h : 0.0;
+  return r;
+}
+
+__device__ __forceinline__ void ref_tri(const RefPre &a, int k) {
+  if (k >= a.nt || a.t_ed[k] < 0) return;
+  const RefTri r = ref_tri_value(a, k);
+  a.zeta[k] = r.zeta;
+  a.eta[k] = r.eta;
+  a.h_tr[k] = r.h;
+  if (a.use_pv && fabs(r.h) < HTR_GUARD) a.flag[0] = 1;
+  a.q_tr[k] = r.q;
 }
 
 // PV at edges: scalar_tr2ed of q, simple average (qmode 0, trsk10,
@@ -234,7 +248,10 @@ __global__ __launch_bounds__(TPB) void ref_ketr(int nt, const int32_t *__restric
 
 // div_hx(uh), div_hx(u), kinetic_energy_hx, g(h+b)+K
 // (swm_operators.f90:613-661, :1132-1217; swm.f90:2533-2536)
-__device__ __forceinline__ void ref_cell(int i, int nv, const int32_t *__restrict__ c_nnb,
+// ONE: uh is formed here, from the edges' two cells (e_v)
+template <bool ONE>
+__device__ __forceinline__ void ref_cell(int i, int nv, int ne, const int32_t *__restrict__ e_v,
+                                                const int32_t *__restrict__ c_nnb,
                                                 const int32_t *__restrict__ c_ed,
                                                 const int8_t *__restrict__ c_ttg,
                                                 const double *__restrict__ c_area,
@@ -261,10 +278,10 @@ __device__ __forceinline__ void ref_cell(int i, int nv, const int32_t *__restric
   double gu[MX], guh[MX], gl[MX], gd[MX], sgn[MX];
 #pragma unroll
   for (int j = 0; j < MX; ++j) {
-    const int l = c_ed[j * nv + i];  // padded slots name edge slot 0
+    const int l = c_ed[j * nv + i];  // padded slots name edge slot 0, which may have no edge
     sgn[j] = (double)c_ttg[j * nv + i];
     gu[j] = u[l];
-    guh[j] = uh[l];
+    guh[j] = ONE ? u[l] * ((h[max(e_v[l], 0)] + h[max(e_v[ne + l], 0)]) * 0.5) : uh[l];
     gl[j] = e_leng[l];
     gd[j] = e_dleng[l];
   }
@@ -307,38 +324,18 @@ __device__ __forceinline__ void ref_cell(int i, int nv, const int32_t *__restric
   }
   ke[i] = kk;
   ghbk[i] = grav * (h[i] + bt[i]) + kk;
-  rk.update(i, -dv);  // may overwrite h[i], which no other cell reads
+  rk.update(i, -dv);
 }
 
 // Two operators that do not read each other's results share a launch: flux
 // and depth at edges with the triangles (which take gass18's depth from the
 // edges: there the triangles come second), and PV at edges with the cells.
 // A launch costs 1.8 us of the step's 80 at glevel 5.
-struct RefPre {
-  int ne, nt, nbe;  // nbe blocks of edges, then blocks of triangles
-  const int32_t *e_v;
-  const double *hb;
-  const int32_t *hv;
-  const double *h, *u;
-  double *h_ed, *uh;
-  const int32_t *t_ed;
-  const int8_t *t_tg;
-  const int32_t *t_v;
-  const double *t_area, *t_f, *t_trhx, *e_leng;
-  int hmode;
-  const double *t_w;
-  double erad;
-  int use_pv, flin;
-  double *eta, *zeta, *h_tr, *q_tr;
-  int *flag;
-};
 __global__ __launch_bounds__(TPB) void ref_pre(const RefPre a) {
   if ((int)blockIdx.x < a.nbe)
     ref_edge_flux(part_index(blockIdx.x, a.nbe), a.ne, a.e_v, a.hb, a.hv, a.h, a.u, a.h_ed, a.uh);
   else
-    ref_tri(part_index(blockIdx.x - a.nbe, gridDim.x - a.nbe), a.nt, a.t_ed, a.t_tg, a.t_v, a.t_area, a.t_f, a.t_trhx,
-            a.e_leng, a.u, a.h, a.hmode, a.t_w, a.h_ed, a.erad, a.use_pv, a.flin, a.eta, a.zeta, a.h_tr, a.q_tr,
-            a.flag);
+    ref_tri(a, part_index(blockIdx.x - a.nbe, gridDim.x - a.nbe));
 }
 
 struct RefMid {
@@ -359,14 +356,44 @@ struct RefMid {
   double *divuh, *masseq, *divu, *ke, *ghbk;
   RefRk rk;
 };
+template <bool ONE>
+__device__ __forceinline__ void ref_mid_cell(const RefMid &a, const int32_t *e_v, int i) {
+  ref_cell<ONE>(i, a.nv, a.ne, e_v, a.c_nnb, a.c_ed, a.c_ttg, a.c_area, a.e_leng, a.e_dleng, a.u, a.uh, a.h, a.bt,
+                a.kmode, a.vhx, a.vuh, a.ketr, a.c_tr, a.c_hxtr, a.gcoef, a.erad, a.grav, a.divuh, a.masseq, a.divu,
+                a.ke, a.ghbk, a.rk);
+}
 __global__ __launch_bounds__(TPB) void ref_mid(const RefMid a) {
   if ((int)blockIdx.x < a.nbe)
     ref_edge_q(part_index(blockIdx.x, a.nbe), a.ne, a.qmode, a.e_sh, a.e_dw, a.t_area, a.eta, a.h_tr, a.q_tr, a.q_ed,
                a.eta_ed, a.flag);
   else
-    ref_cell(part_index(blockIdx.x - a.nbe, gridDim.x - a.nbe), a.nv, a.c_nnb, a.c_ed, a.c_ttg, a.c_area, a.e_leng,
-             a.e_dleng, a.u, a.uh, a.h, a.bt, a.kmode, a.vhx, a.vuh, a.ketr, a.c_tr, a.c_hxtr, a.gcoef, a.erad, a.grav,
-             a.divuh, a.masseq, a.divu, a.ke, a.ghbk, a.rk);
+    ref_mid_cell<false>(a, nullptr, part_index(blockIdx.x - a.nbe, gridDim.x - a.nbe));
+}
+
+// Up to where all values follow from u and h alone (trsk interpolation and
+// kinetic energy) both launches in one: edges and cells form the depths,
+// fluxes and PV they need again, in the same order, instead of waiting for
+// those stored. A launch of these, at a few thousand entities, is mostly its
+// gathers' latency: a step takes 37.3 us instead of 43.9 at glevel 5 (32.6
+// instead of 40.4 at 3), but at glevel 6 the values formed twice already cost
+// as much as the launch (83.4 to 82.4).
+__global__ __launch_bounds__(TPB) void ref_one(const RefPre a, const RefMid m, int nbt) {
+  int b = blockIdx.x;
+  if (b < a.nbe) {
+    const int l = part_index(b, a.nbe), ne = a.ne;
+    if (l >= ne || a.e_v[l] < 0) return;
+    const double he = (a.h[a.e_v[l]] + a.h[a.e_v[ne + l]]) * 0.5;
+    a.h_ed[l] = he;
+    a.uh[l] = a.u[l] * he;
+    if (m.e_sh[l] < 0) return;
+    const RefTri t1 = ref_tri_value(a, m.e_sh[l]), t2 = ref_tri_value(a, m.e_sh[ne + l]);
+    m.q_ed[l] = 0.5 * (t1.q + t2.q);
+    if (m.eta_ed) m.eta_ed[l] = 0.5 * (t1.eta + t2.eta);
+    return;
+  }
+  b -= a.nbe;
+  if (b < nbt) ref_tri(a, part_index(b, nbt));
+  else ref_mid_cell<true>(m, a.e_v, part_index(b - nbt, gridDim.x - a.nbe - nbt));
 }
 
 // grad_ed (HTC) + coriolis_ed (trsk, PV form) -> momeq
@@ -1673,7 +1700,10 @@ static bool launch_ref_tendency(imx_swm *s, const double *h, const double *u, do
              s->t_ed, tsg, s->t_v, s->t_area, s->t_f, s->t_trhx, s->e_leng, sint, s->t_w, s->o.erad,
              s->o.testcase >= 2, s->f_lin ? 1 : 0, s->f_eta, s->f_zeta, s->f_h_tr, s->f_q_tr, s->flag};
   const int gt = grid_bs(NT, bs);
-  if (sint == IMX_SINT_GASS) {  // the triangles read the edges' depths
+  const bool one = sint == IMX_SINT_TRSK && rec == IMX_REC_TRSK && NE < REF_ONE_MAX;
+  if (one) {
+    // with the next launch's edges and cells, below
+  } else if (sint == IMX_SINT_GASS) {  // the triangles read the edges' depths
     ref_pre<<<pre.nbe, bs, 0, st>>>(pre);
     pre.nbe = 0;
     ref_pre<<<gt, bs, 0, st>>>(pre);
@@ -1695,7 +1725,8 @@ static bool launch_ref_tendency(imx_swm *s, const double *h, const double *u, do
                    s->e_leng, s->e_dleng, u, s->f_uh, h, s->bt, rec, s->f_vhx,
                    (hc && rec == IMX_REC_MELV) ? s->f_vuh : nullptr, s->f_ketr, s->c_tr, s->c_hxtr, s->sc_gcoef,
                    s->o.erad, s->o.grav, s->f_divuh, masseq, s->f_divu, s->f_ke, s->f_ghbk, rkh};
-  ref_mid<<<mid.nbe + grid_bs(nv, bs), bs, 0, st>>>(mid);
+  if (one) ref_one<<<pre.nbe + gt + grid_bs(nv, bs), bs, 0, st>>>(pre, mid, gt);
+  else ref_mid<<<mid.nbe + grid_bs(nv, bs), bs, 0, st>>>(mid);
   if (cor == IMX_COR_DTRED)  // vhq_tr (swm.f90:2501-2503)
     ref_lte_tr<<<grid_for(NT), TPB, 0, st>>>(NT, NE, s->t_ed, tsg, epc, s->t_c, s->e_leng, s->t_area, s->f_uh,
                                              s->f_q_tr, s->f_vhq);
@@ -1769,10 +1800,12 @@ static void launch_ref_step(imx_swm *s) {
     rh.kind = ru.kind = k < 2 ? 1 : k;
     rh.dt = ru.dt = s->o.dt;
     rh.y = s->rh, ru.y = s->ru;
-    rh.out = k < 3 ? s->rhn : s->rh, ru.out = k < 3 ? s->run : s->ru;
+    // h: cells of other blocks read the stage's while this one writes
+    double *const hs[4] = {s->rhn, s->rhm, s->rhn, s->rh};
+    rh.out = hs[k], ru.out = k < 3 ? s->run : s->ru;
     rh.k0 = m[0], rh.k1 = m[1], rh.k2 = m[2];
     ru.k0 = f[0], ru.k1 = f[1], ru.k2 = f[2];
-    if (launch_ref_tendency(s, k ? s->rhn : s->rh, k ? s->run : s->ru, m[k], f[k], rh, ru))
+    if (launch_ref_tendency(s, k ? hs[k - 1] : s->rh, k ? s->run : s->ru, m[k], f[k], rh, ru))
       ref_rk<<<grid_for(NE), TPB, 0, s->stream>>>(NE, f[k], ru);
   }
 }
@@ -2888,6 +2921,7 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
     s->rh = A.get<double>(nv);
     s->ru = A.get<double>(NE);
     s->rhn = A.get<double>(nv);
+    s->rhm = A.get<double>(nv);
     s->run = A.get<double>(NE);
     s->massf = A.get<double>((size_t)4 * nv);
     s->momf = A.get<double>((size_t)4 * NE);
