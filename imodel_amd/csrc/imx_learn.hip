@@ -238,16 +238,33 @@ struct FeatLoader {
   }
 };
 
-// out_c = (D F)_c - t_c (t may be NULL), F = the flux output Y[.][1]
+// (D F)_c of the flux output F = Y[.][1]: all gathers in flight, then the sum
+// in ring order
+__device__ __forceinline__ float div_flux(int c, int nv, const int32_t *__restrict__ c_nnb,
+                                          const int32_t *__restrict__ c_ed, const float *__restrict__ dc,
+                                          const float *__restrict__ Y) {
+  const int n = c_nnb[c];
+  float f[IMX_MAXNB], d[IMX_MAXNB];
+#pragma unroll
+  for (int j = 0; j < IMX_MAXNB; ++j) {  // padded slots name edge slot 0
+    f[j] = Y[2 * c_ed[j * nv + c] + 1];
+    d[j] = dc[j * nv + c];
+  }
+  float v = 0.f;
+#pragma unroll
+  for (int j = 0; j < IMX_MAXNB; ++j)
+    if (j < n) v += d[j] * f[j];
+  return v;
+}
+
+// out_c = (D F)_c - t_c (t may be NULL)
 __global__ __launch_bounds__(LTPB) void learn_div(int nv, const int32_t *__restrict__ c_nnb,
                                                   const int32_t *__restrict__ c_ed,
                                                   const float *__restrict__ dc, const float *__restrict__ Y,
                                                   const float *__restrict__ t, float *__restrict__ out) {
   const int c = blockIdx.x * LTPB + threadIdx.x;
   if (c >= nv) return;
-  const int n = c_nnb[c];
-  float v = 0.f;
-  for (int j = 0; j < n; ++j) v += dc[j * nv + c] * Y[2 * c_ed[j * nv + c] + 1];
+  const float v = div_flux(c, nv, c_nnb, c_ed, dc, Y);
   out[c] = t ? v - t[c] : v;
 }
 
@@ -296,9 +313,24 @@ __global__ __launch_bounds__(1024) void learn_norm2(int na, const float *__restr
   if (threadIdx.x == 0) out[0] = take_sqrt ? sqrt(red[0]) : red[0];
 }
 
+// Sum of one value per thread of a block, the same in every thread: lanes by
+// butterfly, then the waves in order.
+__device__ __forceinline__ double block_sum(double v) {
+  __shared__ double red[LTPB / 64];
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
+  __syncthreads();
+  double r = red[0];
+#pragma unroll
+  for (int w = 1; w < LTPB / 64; ++w) r += red[w];
+  return r;
+}
+
 // (D F)_c of the flux output into dhc, and per-block partial sums of the
 // correction's squared norm sum_e w_e Y0^2 + (1/nv) sum_c (D F)_c^2
-// (grid-stride over max(nv, NE), LPART blocks)
+// (grid-stride over max(nv, NE), LPART blocks). 17.4 us at glevel 8 and 4.8 at
+// 6, with each gather waiting for the one before 24.5 and 6.5; 57 MB at glevel
+// 8, mostly latency still.
 __global__ __launch_bounds__(LTPB) void learn_div_part(int nv, int NE, const int32_t *__restrict__ c_nnb,
                                                        const int32_t *__restrict__ c_ed,
                                                        const float *__restrict__ dc,
@@ -308,29 +340,23 @@ __global__ __launch_bounds__(LTPB) void learn_div_part(int nv, int NE, const int
   double s = 0.0, t = 0.0;
   const int nmax = nv > NE ? nv : NE;
   for (int i = blockIdx.x * LTPB + threadIdx.x; i < nmax; i += gridDim.x * LTPB) {
-    if (i < nv) {
-      const int n = c_nnb[i];
-      float v = 0.f;
-      for (int j = 0; j < n; ++j) v += dc[j * nv + i] * Y[2 * c_ed[j * nv + i] + 1];
-      dhc[i] = v;
-      t += (double)v * (double)v;
-    }
     if (i < NE) s += (double)w[i] * (double)Y[2 * i] * (double)Y[2 * i];
+    if (i >= nv) continue;
+    const float v = div_flux(i, nv, c_nnb, c_ed, dc, Y);
+    dhc[i] = v;
+    t += (double)v * (double)v;
   }
-  __shared__ double red[LTPB];
-  red[threadIdx.x] = s + t / nv;
-  __syncthreads();
-  for (int o = LTPB / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  const double r = block_sum(s + t / nv);
+  if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
 // every block sums the LPART partials (fixed order: the same RMS in every
 // block), then the state u, h becomes the plain step's up, hp plus Y0/tsu and
-// (D F)/tsh, or the plain step's where RMS > bound
-template <typename T>
+// (D F)/tsh, or the plain step's where RMS > bound. K elements a thread, their
+// operands loaded before the sum's barrier: with one a thread every element's
+// block sums the partials first, 15.4 us at glevel 8 against 9.0 with four (47
+// MB at a copy's rate); from half a million elements on there are blocks enough.
+template <typename T, int K>
 __global__ __launch_bounds__(LTPB) void learn_apply(int nv, int NE, const float *__restrict__ wv,
                                                     const float *__restrict__ Y,
                                                     const float *__restrict__ dhc, float inv_tsu,
@@ -338,31 +364,40 @@ __global__ __launch_bounds__(LTPB) void learn_apply(int nv, int NE, const float 
                                                     const double *__restrict__ bound, const T *__restrict__ up,
                                                     const T *__restrict__ hp, T *__restrict__ u, T *__restrict__ h,
                                                     double *__restrict__ rms, int *__restrict__ nfb) {
-  __shared__ double red[LTPB];
-  double p = 0.0;
-  for (int k = threadIdx.x; k < LPART; k += LTPB) p += part[k];
-  red[threadIdx.x] = p;
-  __syncthreads();
-  for (int o = LTPB / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+  const int i0 = blockIdx.x * (LTPB * K) + threadIdx.x;
+  float y[K], d[K], wt[K];
+  T us[K], hq[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = i0 + k * LTPB, e = min(i, NE - 1), c = min(i, nv - 1);
+    wt[k] = wv[e];
+    y[k] = Y[2 * e];
+    us[k] = up[e];
+    d[k] = dhc[c];
+    hq[k] = hp[c];
   }
+  double p = 0.0;
+#pragma unroll
+  for (int k = 0; k < LPART; k += LTPB) p += part[k + threadIdx.x];
   // limiter (bound[0] the RMS bound, bound[1] the mode): a correction whose
   // RMS exceeds the bound is dropped and the plain step kept (mode 0), or
   // scaled down to the bound (mode 1); a non-finite one (or bound 0) always
   // leaves the plain step untouched
-  const double r = sqrt(red[0]);
+  const double r = sqrt(block_sum(p));
   const bool ok = r <= bound[0];
   const bool scale = bound[1] > 0.5;
   const float sc = ok ? 1.f : ((scale && r < 1e300) ? (float)(bound[0] / r) : 0.f);
-  const int i = blockIdx.x * LTPB + threadIdx.x;
-  if (i == 0) {
+  if (i0 == 0) {
     rms[0] = r;
     if (!ok) nfb[0] = nfb[0] + 1;  // one thread of the grid counts
   }
   const bool on = sc > 0.f;
-  if (i < NE && wv[i] > 0.f) u[i] = on ? (T)((float)up[i] + sc * (Y[2 * i] * inv_tsu)) : up[i];
-  if (i < nv) h[i] = on ? (T)((float)hp[i] + sc * (dhc[i] * inv_tsh)) : hp[i];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = i0 + k * LTPB;
+    if (i < NE && wt[k] > 0.f) u[i] = on ? (T)((float)us[k] + sc * (y[k] * inv_tsu)) : us[k];
+    if (i < nv) h[i] = on ? (T)((float)hq[k] + sc * (d[k] * inv_tsh)) : hq[k];
+  }
 }
 
 namespace imx {
@@ -424,10 +459,13 @@ static int learn_enqueue_step(imx_learn *L) {
   const int nmax = s->nv > L->NE ? s->nv : L->NE;
   learn_div_part<<<LPART, LTPB, 0, st>>>(s->nv, L->NE, s->c_nnb, s->c_ed, L->dc, L->Y, L->wv, L->dhc,
                                          L->part);
-  learn_apply<T><<<(nmax + LTPB - 1) / LTPB, LTPB, 0, st>>>(s->nv, L->NE, L->wv, L->Y, L->dhc,
-                                                           1.f / L->tsu, 1.f / L->tsh, L->part, L->bound,
-                                                           (const T *)L->uq, (const T *)L->hq, (T *)s->u0,
-                                                           (T *)s->h0, L->rms, L->nfb);
+  auto apply = [&](auto kern, int k) {
+    kern<<<(nmax + k * LTPB - 1) / (k * LTPB), LTPB, 0, st>>>(
+        s->nv, L->NE, L->wv, L->Y, L->dhc, 1.f / L->tsu, 1.f / L->tsh, L->part, L->bound, (const T *)L->uq,
+        (const T *)L->hq, (T *)s->u0, (T *)s->h0, L->rms, L->nfb);
+  };
+  if (nmax < 1 << 19) apply(learn_apply<T, 1>, 1);
+  else apply(learn_apply<T, 4>, 4);
   LTRY(hipGetLastError(), "learn_apply");
   return IMX_OK;
 }
