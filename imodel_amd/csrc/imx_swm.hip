@@ -330,7 +330,7 @@ __device__ __forceinline__ void ref_cell(int i, int nv, int ne, const int32_t *_
 // Two operators that do not read each other's results share a launch: flux
 // and depth at edges with the triangles (which take gass18's depth from the
 // edges: there the triangles come second), and PV at edges with the cells.
-// A launch costs 1.8 us of the step's 80 at glevel 5.
+// A launch costs 1.8 us of the step's 82 at glevel 6.
 __global__ __launch_bounds__(TPB) void ref_pre(const RefPre a) {
   if ((int)blockIdx.x < a.nbe)
     ref_edge_flux(part_index(blockIdx.x, a.nbe), a.ne, a.e_v, a.hb, a.hv, a.h, a.u, a.h_ed, a.uh);

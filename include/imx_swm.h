@@ -414,8 +414,8 @@ void imx_swm_destroy(imx_swm *s);
 
 /* Autotuner (no counterpart in the reference): times every block size
    (64/128/256/512) x XCD-remap choice of each fused kernel over nsteps steps
-   and keeps the fastest; out = {bs, remap} for tri, cell, edge. The state is
-   restored. FAST precisions only. */
+   and keeps the fastest; out = {bs, remap} for tri, cell, edge, those of the
+   one-launch stage under cell. The state is restored. FAST precisions only. */
 int  imx_swm_tune(imx_swm *s, int32_t nsteps, int32_t out[6]);
 
 /* ---- ensembles: many independent instances in one set of launches --------
@@ -475,7 +475,7 @@ void imx_mlp_destroy(imx_mlp *m);
    steps); the network's second output is an edge mass flux whose
    divergence is the h correction, so corrections conserve total mass.
    loss[2] receives the scaled u and h losses. imx_learn_step runs corrected
-   steps (one graph launch each): plain step + MLP correction; a
+   steps (up to 16 per graph launch): plain step + MLP correction; a
    correction whose RMS (scaled units) exceeds `bound` is dropped and the
    plain step kept (IMX_LIMIT_FALLBACK, the default), or scaled down to RMS
    `bound` (IMX_LIMIT_SCALE, imx_learn_set_limiter); a non-finite one, or
