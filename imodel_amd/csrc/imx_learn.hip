@@ -170,11 +170,10 @@ __global__ __launch_bounds__(LTPB) void learn_featx(int NE, const int32_t *__res
 // Input fragments of the network formed in its own kernel: the features of
 // learn_featx in the slots of mlp_feature_slot. The four lanes of an edge read
 // its record as consecutive 32-byte quarters and gather six ids each; the
-// normalised row (96 bytes written and read per edge) never exists: 385 us at
-// glevel 8 instead of 147 for the rows and 301 for the network on them. The
-// kernel is bound by its activations, two waves a SIMD; fetching the next
-// tile's record, or its gathers too, a tile ahead did not help (395 us, and
-// 424 with registers spilled). norm: per lane group 12 means, 12 deviations.
+// normalised row (96 bytes written and read per edge) never exists: 382 us at
+// glevel 8 instead of 147 for the rows and 259 for the network on them. The
+// kernel is bound by its activations, two waves a SIMD; gathering a tile ahead
+// takes 1 % off there and adds as much at glevel 6. norm: per lane group 12 means, 12 deviations.
 template <typename T>
 struct FeatLoader {
   static constexpr int kNorm = 24;
