@@ -387,13 +387,12 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
       T z = flip(sA[e0], (v << 2) & 0x80000000u);
       z += flip(sA[e1], (v << 1) & 0x80000000u);
       z += flip(sA[e2], v & 0x80000000u);
-      z *= k.w;
-      if (!a.flin) eta += z;
-      if constexpr (DF) sZ[sl] = tkt[r] * z;
+      if (!a.flin) eta = fma_(z, k.w, eta);
+      if constexpr (DF) sZ[sl] = tkt[r] * (z * k.w);
     }
     T hsum = k.x * sH[o];
-    hsum += k.y * sH[va];
-    hsum += k.z * sH[vb];
+    hsum = fma_(k.y, sH[va], hsum);
+    hsum = fma_(k.z, sH[vb], hsum);
     const T ht = href + hsum;
     T qq = (T)0;
     if (a.use_pv) {
@@ -452,11 +451,7 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
       // cancels exactly between them
       const double he = fma_(0.5, (double)hc + (double)sH[nb[j]], a.href);
       double g = (double)flip(u, f[j] & 0x80000000u) * he * (double)dl;
-      T k = sA[ed[j]] * (u * dl);
-      if (!valid) {
-        g = 0.0;
-        k = (T)0;
-      }
+      if (!valid) g = 0.0;
       if (j == 0) dv = g;
       else two_sum(dv, dvc, g);
       if constexpr (PX) {
@@ -468,7 +463,7 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
         v.z = fma_(wc[0][j].z, u, v.z);
       } else {
         G[j] = (T)g;
-        ke += k;
+        ke = fma_(valid ? sA[ed[j]] : (T)0, u * dl, ke);
       }
       if constexpr (DF) du += valid ? (double)flip(u, f[j] & 0x80000000u) * (double)dl : 0.0;
     }
@@ -486,9 +481,8 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
     }
     // a pentagon's padded slot may name a triangle that is not local
     if (!hex) qt[MX - 1] = (T)0;
-    T pot = a.grav * hc;
-    if (a.gb) pot += at(a.gb, tid < nown ? own0 + tid : halo[tid - nown]);
-    sPhi[tid] = (pot + K) * a.inv_a;
+    if (a.gb) K += at(a.gb, tid < nown ? own0 + tid : halo[tid - nown]);
+    sPhi[tid] = fma_(a.grav, hc, K) * a.inv_a;
     if (tid < nown) {
       const double dh = -(dv + dvc) * iaa;
       // the step over the stage's share of it (1, 2 halves) and over 6 or 3
