@@ -49,8 +49,15 @@
 //
 // Blocks are cut greedily along the curve so that |C| fills the block's
 // threads and |L| its LDS. Ids inside a block are 10-bit, which packs the
-// topology of a cell into 16 bytes; lengths are stored once per edge and the
-// kinetic-energy and vorticity coefficients are formed from them.
+// topology of a cell into 16 bytes; lengths are stored once per edge, as 1 / l
+// and l~, and the kinetic-energy and vorticity coefficients are formed from
+// them. The momentum tendency is multiplied by 1 / l: an error of that factor
+// is the same in every step and adds up over a run. With l stored, rounded once
+// and inverted (a second rounding), h' at glevel 4 after 48 steps was 2.35e-7
+// off (FP32, trsk10, eight seeds; HC 4.54e-7) where the three passes, which
+// read 1 / l, are 2.14e-7 off (3.84e-7); with 1 / l stored it is 2.02e-7 (3.83e-7).
+// The lengths, which the other terms take, bear the second rounding without
+// effect. Three reciprocals a thread more: 1 % at glevel 5, less from 6 on.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -125,7 +132,7 @@ struct Stage {
   uint4 *topo = nullptr;     // [nblk][cap_l]
   void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~, with diffusion K / A;
                              // pxt16: PV weights of the earlier triangle at edges 0-3; 4, 5
-  void *eld = nullptr;       // [NE] Pair: length, dual length
+  void *eld = nullptr;       // [NE] Pair: 1 / length, dual length
   uint16_t *oth = nullptr;   // [NE] local id of the edge's other cell | it is v1 << 10; 0xFFFF dummy
   uint32_t *tv = nullptr;    // [nblk][cap_t] vertices a, b (10 bits each), edge bits (9), curl signs (3)
   uint16_t *tslot = nullptr; // [nblk][cap_t] local slot 2 owner + k
@@ -322,7 +329,7 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
     if (i < 3 * nown) {
       sU[i] = eu[r];
       sD[i] = el[r].y;
-      sA[i] = eu[r] * el[r].x;
+      sA[i] = eu[r] * recip(el[r].x);
     }
   }
   if (tid < nown) sH[tid] = ho;
@@ -333,7 +340,7 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
     for (int k = 0; k < 3; ++k) {
       sU[3 * lc + k] = hu[k];
       sD[3 * lc + k] = hl[k].y;
-      sA[3 * lc + k] = hu[k] * hl[k].x;
+      sA[3 * lc + k] = hu[k] * recip(hl[k].x);
     }
   }
   ushort4 tn[NG];
@@ -599,11 +606,11 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
       const T uhq = (T)0.25 * (en[r].x * (ql * (A1.x + A2.x) + (B1.x + B2.x)) +
                                en[r].y * (ql * (A1.y + A2.y) + (B1.y + B2.y)) +
                                en[r].z * (ql * (A1.z + A2.z) + (B1.z + B2.z)));
-      du = -d * recip(el[r].x) - uhq;
+      du = -d * el[r].x - uhq;
     } else {
       T P = sP[i] + sPo[i];
-      if constexpr (DF) P += el[r].x * recip(el[r].y) * a.inv_a * sE[i];
-      du = -(d + P) * recip(el[r].x);
+      if constexpr (DF) P += recip(el[r].x * el[r].y) * a.inv_a * sE[i];
+      du = -(d + P) * el[r].x;
     }
     if (a.zero_mom) du = (T)0;
     T ca = a.cat, cb = a.cbt;
@@ -810,7 +817,7 @@ static int build(imx_swm *s, int nt, int scheme) {
   std::vector<Tri<T>> wc(ap || px ? (size_t)nblk * MX * CL : 0, Tri<T>{0, 0, 0}),
       wt(ap ? (size_t)nblk * 3 * GC : 0, Tri<T>{0, 0, 0});
   std::vector<ushort4> tn(ap ? (size_t)nblk * GC : 0, ushort4{0, 0, 0, 0});
-  for (int e = 0; e < NE; ++e) eld[e] = Pair<T>{(T)leng[e], (T)dleng[e]};
+  for (int e = 0; e < NE; ++e) eld[e] = Pair<T>{(T)(1.0 / leng[e]), (T)dleng[e]};
   each_segment([&](int g) {
     LocalSets w;
     for (int b = seg0[g]; b < seg0[g + 1]; ++b) {
