@@ -2779,7 +2779,7 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
   s->nt = d.nt;
   s->fast = o.precision != IMX_PREC_FP64_REF;
   s->single = o.precision == IMX_PREC_FP32;
-  if (o.h_ref != 0.0) {
+  if (s->fast && o.h_ref != 0.0) {  // the reference-order kernels take h itself
     s->href = o.h_ref;
     s->href_set = true;
   }

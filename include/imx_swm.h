@@ -97,8 +97,8 @@ typedef struct imx_swm_opts {
   double  grav;        /* gravity [m s^-2]         (constants.f90:61)         */
   double  omega;       /* rotation rate [s^-1]     (constants.f90:67)         */
   double  dt;          /* time step [s]                                       */
-  double  h_ref;       /* FP32 mode stores h - h_ref; 0 -> area mean of the
-                          first state set                                     */
+  double  h_ref;       /* the fused modes store h - h_ref; 0 -> area mean of
+                          the first state set. IMX_PREC_FP64_REF stores h     */
 } imx_swm_opts;
 
 typedef struct imx_mesh imx_mesh;  /* host mesh built by the library */
