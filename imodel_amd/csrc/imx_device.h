@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <vector>
 
 #include "imx_internal.h"
@@ -110,8 +111,12 @@ struct imx_swm {
   imx::Layout lay;             // caller -> internal maps
   int32_t *d_cell = nullptr, *d_edge = nullptr;  // the cell and edge maps on the device
   // pinned memory the kernels read states from and write them to in caller
-  // order (at most kHostStage bytes: larger states go through it in parts)
+  // order (at most kHostStage bytes: larger states go through it in parts).
+  // One area for all threads that move states of the handle (the instances of
+  // an ensemble share its handle): hstage_mu is held from the first value put
+  // there until the device, or the host, has read the last.
   static constexpr size_t kHostStage = (size_t)64 << 20;
+  std::mutex hstage_mu;
   void *hstage = nullptr;
   size_t hstage_bytes = 0;
   hipStream_t stream = nullptr;

@@ -2993,7 +2993,7 @@ static constexpr int kHostGrain = 1 << 17;
 // nu edge values from edge e0) to internal order: the host rounds h - href
 // and u into the staging area in the caller's order, a sequential pass, and
 // state_in puts every value in its place, so the scattered writes are the
-// device's. The call returns when the device has the state.
+// device's. The caller holds hstage_mu until the stream has been waited for.
 template <typename T>
 static int upload_state(imx_swm *s, const double *h, const double *u, T *hd, T *ud, int c0, int nh, int e0, int nu) {
   const int n = nh + nu;
@@ -3017,8 +3017,9 @@ static int upload_state(imx_swm *s, const double *h, const double *u, T *hd, T *
 }
 
 // The way back: state_out writes the values in the caller's order, as D, to
-// the staging area; the host adds href to the cells' ones. With `what` the
-// caller's arrays are written only when no kernel met a vanishing depth.
+// the staging area (the caller holds hstage_mu); the host adds href to the
+// cells' ones. With `what` the caller's arrays are written only when no kernel
+// met a vanishing depth.
 template <typename D, typename TH, typename TU>
 static int download_state(imx_swm *s, double *h, double *u, const TH *hd, const TU *ud, double href, int c0, int nh,
                           int e0, int nu, const char *what = nullptr) {
@@ -3047,6 +3048,7 @@ static int download_state(imx_swm *s, double *h, double *u, const TH *hd, const 
 
 template <typename T>
 static int set_state(imx_swm *s, const double *h, const double *u, T *hd, T *ud) {
+  std::lock_guard<std::mutex> lk(s->hstage_mu);
   const int rc = upload_state<T>(s, h, u, hd, ud, 0, s->nv, 0, s->ne);
   if (rc) return rc;
   HIPTRY(hipStreamSynchronize(s->stream), "upload");
@@ -3055,6 +3057,7 @@ static int set_state(imx_swm *s, const double *h, const double *u, T *hd, T *ud)
 
 template <typename T>
 static int get_state(imx_swm *s, double *h, double *u, const T *hd, const T *ud) {
+  std::lock_guard<std::mutex> lk(s->hstage_mu);
   return download_state<T>(s, h, u, hd, ud, s->href, 0, s->nv, 0, s->ne);
 }
 
@@ -3370,6 +3373,7 @@ int imx_swm_tendency(imx_swm *s, const double *h, const double *u, double *masse
   const int nv = s->nv, ne = s->ne;
   const char *me = "imx_swm_tendency";
   int rc;
+  std::lock_guard<std::mutex> lk(s->hstage_mu);
   if (!s->fast) {
     if ((rc = imx::upload_state<double>(s, h, u, s->rhn, s->run, 0, nv, 0, ne))) return rc;
     imx::launch_ref_tendency(s, s->rhn, s->run, s->massf, s->momf);
@@ -4271,6 +4275,7 @@ namespace imx {
 template <typename T>
 static int ens_upload(imx_ens *E, int i, const double *h, const double *u) {
   imx_swm *s = E->s;
+  std::lock_guard<std::mutex> lk(s->hstage_mu);
   const int rc = upload_state<T>(s, h, u, (T *)s->h0, (T *)s->u0, E->cv0[i], E->nv[i], E->ce0[i], E->ne[i]);
   if (rc) return rc;
   HIPTRY(hipStreamSynchronize(s->stream), "imx_ens_set_state");
@@ -4280,6 +4285,7 @@ static int ens_upload(imx_ens *E, int i, const double *h, const double *u) {
 template <typename T>
 static int ens_download(imx_ens *E, int i, double *h, double *u) {
   imx_swm *s = E->s;
+  std::lock_guard<std::mutex> lk(s->hstage_mu);
   return download_state<T>(s, h, u, (const T *)s->h0, (const T *)s->u0, s->href, E->cv0[i], E->nv[i], E->ce0[i],
                            E->ne[i]);
 }
