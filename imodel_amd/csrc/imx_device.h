@@ -66,8 +66,9 @@ struct StepGraphs {
       graph[k] = nullptr;
     }
   }
-  // captures what a run of nsteps launches; one(): enqueues a step, 0 or an
-  // IMX_E* code, which is returned (a hipError_t comes back in err)
+  // captures what a run of nsteps launches; one(last): enqueues a step (last: of
+  // its graph), 0 or an IMX_E* code, which is returned (a hipError_t comes back
+  // in err)
   template <typename F>
   int ensure(int nsteps, hipStream_t st, F one, hipError_t &err) {
     err = hipSuccess;
@@ -77,7 +78,7 @@ struct StepGraphs {
       if (count == 0 || exec[k]) continue;
       if ((err = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal)) != hipSuccess) return 0;
       int rc = 0;
-      for (int i = 0; i < kSteps[k] && rc == 0; ++i) rc = one();
+      for (int i = 0; i < kSteps[k] && rc == 0; ++i) rc = one(i == kSteps[k] - 1);
       hipGraph_t g = nullptr;
       err = hipStreamEndCapture(st, &g);
       if (rc == 0 && err == hipSuccess) err = hipGraphInstantiate(&exec[k], g, nullptr, nullptr, 0);

@@ -49,7 +49,7 @@ struct imx_learn {
   int32_t *stn = nullptr;   // [NE][SREC] stencil record per edge slot (see learn_featx)
   float *dc = nullptr;      // [6][nv] coefficient of F_{c_ed[j][c]} in (D F)_c
   float *de = nullptr;      // [2][NE] coefficient of F_e in (D F) at e_v[0/1][e]
-  void *hn = nullptr, *un = nullptr;  // state before the step (T)
+  void *hn = nullptr, *un = nullptr;  // state before the last step or sample (T)
   float *raw = nullptr;     // [NE][NF]
   float *mu = nullptr, *sig = nullptr, *norm = nullptr;  // norm: FeatLoader's order
   void *hq = nullptr, *uq = nullptr;  // state after the plain step of a corrected one (T)
@@ -412,14 +412,20 @@ static int lfail(hipError_t e, const char *what) {
 
 static void learn_drop_graph(imx_learn *L) { L->graphs.drop(); }
 
-// enqueue: save x_n, one plain step
+// enqueue: save x_n
 template <typename T>
-static void learn_enqueue_sample(imx_learn *L) {
+static void learn_enqueue_save(imx_learn *L) {
   imx_swm *s = L->s;
   const int g = (L->NE + LTPB - 1) / LTPB;
   learn_save<T><<<g, LTPB, 0, s->stream>>>(s->nv, L->NE, (const T *)s->h0, (const T *)s->u0, (T *)L->hn,
                                            (T *)L->un);
-  swm_launch_step(s);
+}
+
+// enqueue: save x_n, one plain step
+template <typename T>
+static void learn_enqueue_sample(imx_learn *L) {
+  learn_enqueue_save<T>(L);
+  swm_launch_step(L->s);
 }
 
 // enqueue: features of (saved state, current state) into raw and/or X
@@ -447,11 +453,15 @@ static void learn_free_store(imx_learn *L) {
 
 // enqueue: one corrected step: the plain step into hq, uq, the network on
 // features gathered from both states, the correction (with the RMS bound)
-// back into the handle's state
+// back into the handle's state. save: x_n is kept as a sample's is; the last
+// step of a run has it (with every graph's last step, 1 of up to 16: a copy of
+// the state, 15 us at glevel 8), so that imx_learn_train and imx_learn_store
+// after it take that step's features
 template <typename T>
-static int learn_enqueue_step(imx_learn *L) {
+static int learn_enqueue_step(imx_learn *L, bool save) {
   imx_swm *s = L->s;
   hipStream_t st = s->stream;
+  if (save) learn_enqueue_save<T>(L);
   swm_launch_step(s, L->hq, L->uq);
   const FeatLoader<T> ld{L->stn, (const T *)s->u0, (const T *)s->h0, (const T *)L->uq, (const T *)L->hq, L->norm};
   LTRY(mlp_fwd_launch(L->m->F1g, L->m->Ff32, L->m->P, L->NE, ld, L->Y, st), "mlp_fwd_lds");
@@ -481,8 +491,8 @@ static int learn_ensure_graphs(imx_learn *L, int nsteps) {
   if (L->gen != L->s->generation) learn_drop_graph(L);
   L->gen = L->s->generation;
   hipError_t e;
-  const int rc = L->graphs.ensure(nsteps, L->s->stream, [&] {
-    return L->s->single ? learn_enqueue_step<float>(L) : learn_enqueue_step<double>(L);
+  const int rc = L->graphs.ensure(nsteps, L->s->stream, [&](bool last) {
+    return L->s->single ? learn_enqueue_step<float>(L, last) : learn_enqueue_step<double>(L, last);
   }, e);
   if (rc) return rc;
   LTRY(e, "learn graph capture");

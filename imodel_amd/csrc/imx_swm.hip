@@ -3091,7 +3091,7 @@ static void drop_graph(imx_swm *s) {
 
 static int ensure_graphs(imx_swm *s, int nsteps) {
   hipError_t e;
-  const int rc = s->graphs.ensure(nsteps, s->stream, [&] { launch_step(s); return 0; }, e);
+  const int rc = s->graphs.ensure(nsteps, s->stream, [&](bool) { launch_step(s); return 0; }, e);
   HIPTRY(e, "step graph capture");
   return rc;
 }

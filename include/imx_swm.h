@@ -472,7 +472,7 @@ void imx_mlp_destroy(imx_mlp *m);
    raw != NULL). imx_learn_set_scaling gives the feature mean/std and the
    target scales (scaled target = tscale * physical). imx_learn_train fits
    the MLP to the correction du[ne], dh[nv] of that step (`epochs` AdamW
-   steps); the network's second output is an edge mass flux whose
+   steps), or of the last corrected step where imx_learn_step ran since; the network's second output is an edge mass flux whose
    divergence is the h correction, so corrections conserve total mass.
    loss[2] receives the scaled u and h losses. imx_learn_step runs corrected
    steps (up to 16 per graph launch): plain step + MLP correction; a
