@@ -168,6 +168,8 @@ def lib():
             "imx_swm_destroy": (None, [vp]),
             "imx_copy_probe": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int32, _F64P]),
             "imx_swm_tune": (ctypes.c_int, [vp, ctypes.c_int32, _I32P]),
+            "imx_swm_get_launch": (ctypes.c_int, [vp, _I32P]),
+            "imx_swm_set_launch": (ctypes.c_int, [vp, _I32P]),
             "imx_ens_create": (ctypes.c_int, [ctypes.c_int32, ctypes.POINTER(MeshDesc), _F64P,
                                               ctypes.POINTER(SwmOpts), ctypes.POINTER(vp)]),
             "imx_ens_set_state": (ctypes.c_int, [vp, ctypes.c_int32, _F64P, _F64P]),

@@ -3240,6 +3240,51 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   return check_flag(s, "imx_swm_tune");
 }
 
+// The launch shapes in use, {threads, remap} for tri, cell, edge; the one-launch
+// stage's under cell.
+static void launch_shapes(const imx_swm *s, int32_t *out) {
+  for (int k = 0; k < 3; ++k) {
+    out[2 * k] = s->kbs[k];
+    out[2 * k + 1] = s->kremap[k];
+  }
+  if (!stage_on(s)) return;
+  out[2] = s->stg_nt[stage_scheme(s)];
+  out[3] = s->stg_remap[stage_scheme(s)];
+}
+
+static int set_launch(imx_swm *s, const int32_t *cfg) {
+  const char *bad = "imx_swm_set_launch: not a launch shape of the handle";
+  const bool one = stage_on(s);
+  for (int k = 0; k < 3; ++k) {
+    if (one && k != 1) continue;
+    const int n = cfg[2 * k], r = cfg[2 * k + 1];
+    const bool fits = n == 128 || n == 256 || (n == 64 && !one) || (n == 512 && (!one || s->single));
+    if (!fits || r < 0 || r > 1) return set_error(IMX_EINVAL, bad);
+  }
+  if (!one) {
+    for (int k = 0; k < 3; ++k) {
+      s->kbs[k] = cfg[2 * k];
+      s->kremap[k] = cfg[2 * k + 1];
+    }
+    drop_graph(s);
+    return IMX_OK;
+  }
+  const int k = stage_scheme(s), nt0 = s->stg_nt[k], remap0 = s->stg_remap[k];
+  s->stg_nt[k] = cfg[2];
+  s->stg_remap[k] = cfg[3];
+  drop_graph(s);
+  if (stage_threads(s) == cfg[2]) {
+    stage_set_remap(s, cfg[3]);
+    return IMX_OK;
+  }
+  const int rc = stage_make(s);
+  if (!rc && s->stg) return IMX_OK;
+  s->stg_nt[k] = nt0;
+  s->stg_remap[k] = remap0;
+  (void)stage_make(s);
+  return rc ? rc : set_error(IMX_EINVAL, bad);  // no cut of the mesh into such blocks
+}
+
 int swm_check_flag(imx_swm *s, const char *what) { return check_flag(s, what); }
 
 }  // namespace imx
@@ -4254,6 +4299,19 @@ void imx_swm_destroy(imx_swm *s) {
 int imx_swm_tune(imx_swm *s, int32_t nsteps, int32_t out[6]) {
   if (!s) return imx::set_error(IMX_EINVAL, "imx_swm_tune: NULL handle");
   return imx::tune(s, nsteps, out);
+}
+
+int imx_swm_get_launch(imx_swm *s, int32_t cfg[6]) {
+  if (!s || !cfg) return imx::set_error(IMX_EINVAL, "imx_swm_get_launch: NULL argument");
+  if (!s->fast) return imx::set_error(IMX_ENOTSUP, "imx_swm_get_launch: FAST precisions only");
+  imx::launch_shapes(s, cfg);
+  return IMX_OK;
+}
+
+int imx_swm_set_launch(imx_swm *s, const int32_t cfg[6]) {
+  if (!s || !cfg) return imx::set_error(IMX_EINVAL, "imx_swm_set_launch: NULL argument");
+  if (!s->fast) return imx::set_error(IMX_ENOTSUP, "imx_swm_set_launch: FAST precisions only");
+  return imx::set_launch(s, cfg);
 }
 
 }  // extern "C"

@@ -366,6 +366,18 @@ class Swm:
         capi.check(capi.lib().imx_swm_tune(self._h, int(nsteps), capi.i32p(out)), "imx_swm_tune")
         return {k: (int(out[2 * i]), int(out[2 * i + 1])) for i, k in enumerate(("tri", "cell", "edge"))}
 
+    def launch(self):
+        """The launch shapes in use, as tune returns them."""
+        out = np.zeros(6, dtype=np.int32)
+        capi.check(capi.lib().imx_swm_get_launch(self._h, capi.i32p(out)), "imx_swm_get_launch")
+        return {k: (int(out[2 * i]), int(out[2 * i + 1])) for i, k in enumerate(("tri", "cell", "edge"))}
+
+    def set_launch(self, shapes):
+        """Launch shapes to use from now on, as tune or launch return them; a
+        scheme that runs as one launch per stage takes that under "cell"."""
+        cfg = np.array([v for k in ("tri", "cell", "edge") for v in shapes[k]], dtype=np.int32)
+        capi.check(capi.lib().imx_swm_set_launch(self._h, capi.i32p(cfg)), "imx_swm_set_launch")
+
 
 class Ensemble:
     """Independent instances (meshes, time steps) advanced together on the GPU."""

@@ -417,6 +417,13 @@ void imx_swm_destroy(imx_swm *s);
    and keeps the fastest; out = {bs, remap} for tri, cell, edge, those of the
    one-launch stage under cell. The state is restored. FAST precisions only. */
 int  imx_swm_tune(imx_swm *s, int32_t nsteps, int32_t out[6]);
+/* The launch shapes in use, laid out as imx_swm_tune returns them, and shapes
+   to use from now on (those of an earlier imx_swm_tune, say): block threads and
+   remap (0/1) for tri, cell, edge, or, where the handle's scheme runs as one
+   launch per stage, that launch's under cell alone (128, 256 or, FP32, 512
+   threads). IMX_EINVAL, and the shapes as they were, for others. */
+int  imx_swm_get_launch(imx_swm *s, int32_t cfg[6]);
+int  imx_swm_set_launch(imx_swm *s, const int32_t cfg[6]);
 
 /* ---- ensembles: many independent instances in one set of launches --------
    (no counterpart in the reference; the batched configuration). Instance i

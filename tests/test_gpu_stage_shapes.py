@@ -1,0 +1,75 @@
+"""Every launch shape of the one-launch stage (csrc/imx_stage.hip), forced by
+imx_swm_set_launch on a mesh of many blocks: a result does not depend on how the
+mesh is cut, so all shapes give the same bits, and these are the passes' of the
+same precision (a handle on the mesh's own numbering) within the fused paths'
+tolerances; FP64_REF is no reference for FP64 from glevel 5 on, where the kite
+areas that both fused paths rebuild the TRiSK weights from carry more (HC 2e-12)."""
+import numpy as np
+import pytest
+
+from imodel_amd.capi import ImxError
+from imodel_amd.swm import Mesh, Swm
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+SCHEMES = {"plain": {}, "hc": {"stag": "HC"}, "apvm": {"pv": "apvm", "pvspar": 0.5},
+           "apvm-hc": {"pv": "apvm", "pvspar": 0.5, "stag": "HC"}, "pxt16": {"wrap": "pxt16"},
+           "k2": {"k2": 1e5, "diffus": "const"}, "k2-hc": {"k2": 1e5, "diffus": "diam", "stag": "HC"}}
+# the fused paths' tolerances with scheme options: tendency, h and u after 6 steps
+TOL = {"fp64": (1e-12, 1e-12, 1e-11), "fp32": (5e-5, 1e-6, 1e-5)}
+
+
+def evaluate(s, h, u):
+    t = s.tendency(h, u)
+    s.set_state(h, u)
+    s.step(6)
+    return t + s.get_state()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("scheme", list(SCHEMES))
+def test_shapes(scheme, prec):
+    m = Mesh.icos(5)
+    h, u = m.spectral(35)
+    kw, dt = SCHEMES[scheme], 300.0
+    with Swm(m, precision=prec, dt=dt, use_sfc=False) as s:
+        s.set_scheme(**kw)
+        ref = evaluate(s, h, u)
+        assert len(s.profile(1)) == 3
+    got = {}
+    with Swm(m, precision=prec, dt=dt) as s:
+        s.set_scheme(**kw)
+        shape = s.launch()
+        for threads in (128, 256, 512) if prec == "fp32" else (128, 256):
+            for remap in (0, 1):
+                print("[gpu-case] stage shape", scheme, prec, threads, remap, flush=True)
+                s.set_launch({**shape, "cell": (threads, remap)})
+                assert s.launch()["cell"] == (threads, remap)
+                got[threads, remap] = evaluate(s, h, u)
+                assert list(s.profile(1)) == ["fast_stage"]
+        for bad in ((64, 1), (192, 1), (256, 2), (1024, 1)) + (((512, 1),) if prec == "fp64" else ()):
+            with pytest.raises(ImxError):
+                s.set_launch({**shape, "cell": bad})
+        assert s.launch()["cell"] == (threads, remap)
+    first = got[128, 0]
+    for shape, x in got.items():
+        assert all(np.array_equal(a, b) for a, b in zip(x, first)), shape
+    t, th, tu = TOL[prec]
+    for g, r, tol in zip(first, ref, (t, t, th, tu)):
+        assert rel_l2(g, r) < tol, rel_l2(g, r)
+
+
+def test_shapes_of_the_passes():
+    """A scheme without the one-launch stage takes the three kernels' shapes."""
+    print("[gpu-case] shapes of the passes", flush=True)
+    m = Mesh.icos(4)
+    h, u = m.spectral(35)
+    with Swm(m, precision="fp32", dt=300.0) as s:
+        s.set_scheme(wrap="gass18")
+        first = evaluate(s, h, u)
+        s.set_launch({"tri": (64, 0), "cell": (512, 1), "edge": (128, 0)})
+        assert s.launch() == {"tri": (64, 0), "cell": (512, 1), "edge": (128, 0)}
+        assert all(np.array_equal(a, b) for a, b in zip(evaluate(s, h, u), first))
+        with pytest.raises(ImxError):
+            s.set_launch({"tri": (64, 0), "cell": (32, 1), "edge": (128, 0)})
