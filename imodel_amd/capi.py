@@ -170,6 +170,7 @@ def lib():
             "imx_swm_tune": (ctypes.c_int, [vp, ctypes.c_int32, _I32P]),
             "imx_swm_get_launch": (ctypes.c_int, [vp, _I32P]),
             "imx_swm_set_launch": (ctypes.c_int, [vp, _I32P]),
+            "imx_swm_set_stage_limit": (ctypes.c_int, [vp, ctypes.c_int64]),
             "imx_ens_create": (ctypes.c_int, [ctypes.c_int32, ctypes.POINTER(MeshDesc), _F64P,
                                               ctypes.POINTER(SwmOpts), ctypes.POINTER(vp)]),
             "imx_ens_set_state": (ctypes.c_int, [vp, ctypes.c_int32, _F64P, _F64P]),

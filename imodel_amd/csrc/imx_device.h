@@ -13,12 +13,16 @@ namespace imx {
 
 struct Alloc {
   std::vector<void *> ptrs;
-  size_t bytes = 0;
+  size_t bytes = 0, limit = 0;  // limit: the most it may take, 0 for any
   hipError_t err = hipSuccess;
   template <typename X>
   X *get(size_t n) {
     void *p = nullptr;
     if (n == 0) n = 1;
+    if (limit && bytes + n * sizeof(X) > limit) {
+      err = hipErrorOutOfMemory;
+      return nullptr;
+    }
     hipError_t e = hipMalloc(&p, n * sizeof(X));
     if (e != hipSuccess) {
       err = e;
@@ -289,11 +293,14 @@ struct imx_swm {
   // XCD remap, chosen by imx_swm_tune
   int kbs[3] = {256, 256, 256};
   int kremap[3] = {1, 1, 1};
-  // one launch per stage; stg_local: the numbering is local. stg_stale: the
-  // tables no longer match the handle's staggering, triangle weights or
-  // Coriolis parameter. stg_nt, stg_remap: block threads and XCD remap of
-  // each scheme it has (one_launch_scheme).
+  // one launch per stage; null where its tables find no memory: the passes need
+  // none. stg_local: the numbering is local. stg_stale: the tables no longer
+  // match the handle's staggering, triangle weights or Coriolis parameter.
+  // stg_limit: the most device memory they may take (0: any). stg_nt,
+  // stg_remap: block threads and XCD remap of each scheme it has
+  // (one_launch_scheme).
   imx::Stage *stg = nullptr;
+  size_t stg_limit = 0;
   bool stg_stale = false, stg_local = false;
   int stg_nt[4] = {256, 256, 256, 256}, stg_remap[4] = {1, 1, 1, 1};
 };
@@ -325,10 +332,11 @@ void swm_launch_step(imx_swm *s, void *hout = nullptr, void *uout = nullptr);
 int swm_check_flag(imx_swm *s, const char *what);
 
 // One launch per RK stage (imx_stage.hip). stage_build makes the block
-// tables from the handle's device tables for blocks of nt threads and leaves
-// s->stg null where the numbering cuts into blocks that are mostly rim;
+// tables from the handle's device tables for blocks of nt threads. It leaves
+// s->stg null, and *local false, where the numbering cuts into blocks that are
+// mostly rim, and null with IMX_ENOMEM where device or host memory is short;
 // stage_launch evaluates stage 0..3 of (hs, us), or a tendency (stage -1).
-int stage_build(imx_swm *s, int nt, int scheme);
+int stage_build(imx_swm *s, int nt, int scheme, bool *local);
 void stage_free(imx_swm *s);
 int stage_threads(const imx_swm *s);
 int stage_scheme(const imx_swm *s);

@@ -63,6 +63,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <memory>
 #include <new>
 #include <string>
 #include <thread>
@@ -687,7 +688,7 @@ struct LocalSets {
 };
 
 template <typename T>
-static int build(imx_swm *s, int nt, int scheme) {
+static int build(imx_swm *s, int nt, int scheme, bool *local) {
   const int nv = s->nv, NE = s->NE, NTri = s->NT;
   const bool ap = scheme == kApvm, px = scheme == kPerot, df = scheme == kDiff;
   const int LC = cap_a(nt), CL = cap_l(nt, ap), TC = cap_t(nt, ap), GC = cap_g(nt);
@@ -797,9 +798,9 @@ static int build(imx_swm *s, int nt, int scheme) {
   start.push_back(nv);
   // Numberings that are not local (a mesh in its caller's order) cut into
   // blocks that are mostly rim: the three passes run instead.
-  for (char ok : fine)
-    if (!ok) return IMX_OK;
-  if (nblk > 1 && (int64_t)nblk * nt > (int64_t)3 * nv) return IMX_OK;
+  *local = nblk <= 1 || (int64_t)nblk * nt <= (int64_t)3 * nv;
+  for (char ok : fine) *local = *local && ok;
+  if (!*local) return IMX_OK;
   // the kernel addresses its tables by 32-bit byte offsets
   if ((uint64_t)NE * sizeof(Tri<T>) >> 32) return IMX_OK;
 
@@ -897,8 +898,16 @@ static int build(imx_swm *s, int nt, int scheme) {
   });
 
   if (!memory) return set_error(IMX_ENOMEM, out_of);
-  Stage *g = s->stg = new Stage();
+  // the handle has the tables once they are whole
+  struct Drop {
+    void operator()(Stage *p) const {
+      p->A.release();
+      delete p;
+    }
+  };
+  std::unique_ptr<Stage, Drop> g(new Stage());
   Alloc &A = g->A;
+  A.limit = s->stg_limit;
   g->nt = nt;
   g->nblk = nblk;
   g->head = A.put(head);
@@ -919,18 +928,18 @@ static int build(imx_swm *s, int nt, int scheme) {
     g->wt = A.put(wt);
     g->tn = A.put(tn);
   }
-  if (A.err != hipSuccess) {
-    const std::string why = hipGetErrorString(A.err);
-    stage_free(s);
-    return set_error(IMX_EDEVICE, "stage tables: " + why);
-  }
+  if (A.err != hipSuccess)
+    return set_error(A.err == hipErrorOutOfMemory ? IMX_ENOMEM : IMX_EDEVICE,
+                     std::string("stage tables: ") + hipGetErrorString(A.err));
+  s->stg = g.release();
   return IMX_OK;
 }
 
-int stage_build(imx_swm *s, int nt, int scheme) {
+int stage_build(imx_swm *s, int nt, int scheme, bool *local) {
   stage_free(s);
+  *local = true;
   try {
-    return s->single ? build<float>(s, nt, scheme) : build<double>(s, nt, scheme);
+    return s->single ? build<float>(s, nt, scheme, local) : build<double>(s, nt, scheme, local);
   } catch (const std::bad_alloc &) {
     return set_error(IMX_ENOMEM, "stage tables: host out of memory");
   }

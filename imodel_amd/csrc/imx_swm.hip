@@ -2747,21 +2747,27 @@ static void stage_defaults(imx_swm *s) {
 
 // (Re)builds the stage tables for the handle's scheme: they follow its
 // staggering, triangle weights and Coriolis parameter, and are made again
-// when a scheme that has them is back.
-static int stage_make(imx_swm *s) {
-  const int k = one_launch_scheme(s), rc = stage_build(s, s->stg_nt[k], k);
+// when a scheme that has them is back. Where they find no memory, the handle
+// runs the passes, whose tables it has.
+static int stage_make(imx_swm *s, bool *local) {
+  const int k = one_launch_scheme(s);
+  int rc = stage_build(s, s->stg_nt[k], k, local);
+  if (rc == IMX_ENOMEM) {
+    (void)hipGetLastError();
+    rc = IMX_OK;
+  }
   stage_set_remap(s, s->stg_remap[k]);
   s->stg_stale = false;
   return rc;
 }
+static int stage_make(imx_swm *s) {
+  bool local;
+  return stage_make(s, &local);
+}
 static int stage_refresh(imx_swm *s) {
   s->stg_stale = true;
-  const int k = one_launch_scheme(s);
-  if (!s->stg_local || k < 0) return IMX_OK;
-  const int rc = stage_make(s);
-  if (!k || !rc) return rc;
-  // no room for an option's tables: the passes need none
-  (void)hipGetLastError();
+  if (one_launch_scheme(s) < 0) stage_free(s);
+  else if (s->stg_local) return stage_make(s);
   return IMX_OK;
 }
 
@@ -2955,8 +2961,7 @@ static int create(const imx_mesh_desc &d, const imx_swm_opts &o, imx_swm *s,
   HIPTRY(hipDeviceSynchronize(), "imx_swm_create");
   if (s->fast) {
     stage_defaults(s);
-    if ((rc = stage_make(s))) return rc;
-    s->stg_local = s->stg != nullptr;
+    if ((rc = stage_make(s, &s->stg_local))) return rc;
   }
   return IMX_OK;
 }
@@ -3185,7 +3190,13 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
     const int scheme = stage_scheme(s);
     for (int bs : {128, 256, 512}) {
       if (bs == 512 && !s->single) continue;  // over 64 KB of LDS
-      if ((rc = stage_build(s, bs, scheme))) break;
+      bool local;
+      rc = stage_build(s, bs, scheme, &local);
+      if (rc == IMX_ENOMEM) {  // not a candidate
+        (void)hipGetLastError();
+        rc = IMX_OK;
+      }
+      if (rc) break;
       if (!s->stg) continue;
       for (int r = 0; r < 2 && !rc; ++r) {
         stage_set_remap(s, r);
@@ -4306,6 +4317,15 @@ int imx_swm_get_launch(imx_swm *s, int32_t cfg[6]) {
   if (!s->fast) return imx::set_error(IMX_ENOTSUP, "imx_swm_get_launch: FAST precisions only");
   imx::launch_shapes(s, cfg);
   return IMX_OK;
+}
+
+int imx_swm_set_stage_limit(imx_swm *s, int64_t bytes) {
+  if (!s) return imx::set_error(IMX_EINVAL, "imx_swm_set_stage_limit: NULL handle");
+  if (bytes < 0) return imx::set_error(IMX_EINVAL, "imx_swm_set_stage_limit: negative size");
+  if (!s->fast) return imx::set_error(IMX_ENOTSUP, "imx_swm_set_stage_limit: FAST precisions only");
+  s->stg_limit = (size_t)bytes;
+  imx::drop_graph(s);
+  return imx::stage_refresh(s);
 }
 
 int imx_swm_set_launch(imx_swm *s, const int32_t cfg[6]) {

@@ -378,6 +378,11 @@ class Swm:
         cfg = np.array([v for k in ("tri", "cell", "edge") for v in shapes[k]], dtype=np.int32)
         capi.check(capi.lib().imx_swm_set_launch(self._h, capi.i32p(cfg)), "imx_swm_set_launch")
 
+    def set_stage_limit(self, nbytes):
+        """The device memory the one-launch stage's tables may take (0: any); a
+        scheme whose tables take more runs as one kernel per pass."""
+        capi.check(capi.lib().imx_swm_set_stage_limit(self._h, int(nbytes)), "imx_swm_set_stage_limit")
+
 
 class Ensemble:
     """Independent instances (meshes, time steps) advanced together on the GPU."""

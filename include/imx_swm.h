@@ -424,6 +424,11 @@ int  imx_swm_tune(imx_swm *s, int32_t nsteps, int32_t out[6]);
    threads). IMX_EINVAL, and the shapes as they were, for others. */
 int  imx_swm_get_launch(imx_swm *s, int32_t cfg[6]);
 int  imx_swm_set_launch(imx_swm *s, const int32_t cfg[6]);
+/* The device memory [bytes] the tables of one launch per stage may take (about
+   200 bytes a cell in FP32, 560 with APVM; 0, the default: any). A scheme whose
+   tables take more, or find no memory, runs as one kernel per pass instead, from
+   tables every handle has: the same results within rounding. */
+int  imx_swm_set_stage_limit(imx_swm *s, int64_t bytes);
 
 /* ---- ensembles: many independent instances in one set of launches --------
    (no counterpart in the reference; the batched configuration). Instance i
