@@ -3150,9 +3150,22 @@ static int diag_range(imx_swm *s, int c0, int c1, double *out) {
   return IMX_OK;
 }
 
-// Autotuner: for each fused kernel, time every (block size, XCD remap)
-// candidate over `nsteps` steps with the other kernels fixed, keep the
-// fastest. The state is restored afterwards.
+// The launch shapes in use, {threads, remap} for tri, cell, edge; the one-launch
+// stage's under cell.
+static void launch_shapes(const imx_swm *s, int32_t *out) {
+  for (int k = 0; k < 3; ++k) {
+    out[2 * k] = s->kbs[k];
+    out[2 * k + 1] = s->kremap[k];
+  }
+  if (!stage_on(s)) return;
+  out[2] = s->stg_nt[stage_scheme(s)];
+  out[3] = s->stg_remap[stage_scheme(s)];
+}
+
+// Autotuner: time every (block threads, XCD remap) candidate over `nsteps`
+// steps and keep the fastest: of the one-launch stage where the scheme runs as
+// one (the scheme's own shape; the passes keep theirs), else of each of the
+// three kernels with the others fixed. The state is restored afterwards.
 static int tune(imx_swm *s, int nsteps, int32_t *out) {
   if (!s->fast) return set_error(IMX_ENOTSUP, "imx_swm_tune: FAST precisions only");
   if (nsteps < 1) nsteps = 1;
@@ -3213,8 +3226,6 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
     const int r2 = !s->stg || stage_threads(s) != bb ? stage_make(s) : IMX_OK;
     if (!rc) rc = r2;
     stage_set_remap(s, br);
-    s->kbs[1] = bb;
-    s->kremap[1] = br;
   } else {
   for (int k = 0; k < 3 && !rc; ++k) {
     double best = 1e30;
@@ -3243,24 +3254,8 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
   (void)hipFree(su);
   drop_graph(s);
   if (rc) return rc;
-  if (out)
-    for (int k = 0; k < 3; ++k) {
-      out[2 * k] = s->kbs[k];
-      out[2 * k + 1] = s->kremap[k];
-    }
+  if (out) launch_shapes(s, out);
   return check_flag(s, "imx_swm_tune");
-}
-
-// The launch shapes in use, {threads, remap} for tri, cell, edge; the one-launch
-// stage's under cell.
-static void launch_shapes(const imx_swm *s, int32_t *out) {
-  for (int k = 0; k < 3; ++k) {
-    out[2 * k] = s->kbs[k];
-    out[2 * k + 1] = s->kremap[k];
-  }
-  if (!stage_on(s)) return;
-  out[2] = s->stg_nt[stage_scheme(s)];
-  out[3] = s->stg_remap[stage_scheme(s)];
 }
 
 static int set_launch(imx_swm *s, const int32_t *cfg) {

@@ -73,3 +73,27 @@ def test_shapes_of_the_passes():
         assert all(np.array_equal(a, b) for a, b in zip(evaluate(s, h, u), first))
         with pytest.raises(ImxError):
             s.set_launch({"tri": (64, 0), "cell": (32, 1), "edge": (128, 0)})
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_tuning_leaves_the_passes_alone(prec):
+    """The one-launch stage and the passes have shapes of their own: tuning the
+    plain scheme changes neither the passes' nor another scheme's."""
+    print("[gpu-case] tune and the passes", prec, flush=True)
+    m = Mesh.icos(4)
+    passes = {"tri": (64, 0), "cell": (64, 0), "edge": (128, 0)}
+    with Swm(m, precision=prec, dt=300.0) as s:
+        s.set_scheme(wrap="gass18")
+        s.set_launch(passes)
+        s.set_scheme(wrap="pxt16")
+        other = s.launch()["cell"]
+        s.set_scheme()
+        s.set_state(*m.spectral(1))
+        best = s.tune(1)
+        assert best == s.launch() and best["cell"][0] in (128, 256, 512)
+        s.set_scheme(wrap="pxt16")
+        assert s.launch()["cell"] == other
+        s.set_scheme(wrap="gass18")
+        assert s.launch() == passes
+        s.set_scheme()
+        assert s.launch() == best
