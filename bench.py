@@ -208,6 +208,7 @@ def main():
         log("autotuned", tuned)
         s.set_state(h0, u0)
     s.step(args.warmup)
+    s.prepare(args.steps)  # graphs of other sizes than the warm-up's
     s.set_state(h0, u0)
     t0 = time.perf_counter()
     ev_ms = s.step_timed(args.steps)
@@ -456,6 +457,7 @@ def bench_ensemble(args):
     cfg = E.tune(2)
     log("autotuned", cfg)
     E.step(args.warmup)
+    E.prepare(args.steps)
     for i, (h, u) in enumerate(states):
         E.set_state(i, h, u)
     t0 = time.perf_counter()
@@ -511,11 +513,13 @@ def bench_mlp(args):
     fwd_ms = m.forward_timed(ne_slots, reps=args.steps)
     s.set_state(h0, u0)
     L.step(args.warmup, 1e30)
+    L.prepare(args.steps)
     t = time.perf_counter()
     nfb = L.step(args.steps, 1e30)
     learned_us = 1e6 * (time.perf_counter() - t) / args.steps
     s.set_state(h0, u0)
     s.step(args.warmup)
+    s.prepare(args.steps)
     t = time.perf_counter()
     s.step(args.steps)
     plain_us = 1e6 * (time.perf_counter() - t) / args.steps

@@ -160,6 +160,7 @@ def lib():
             "imx_swm_get_field": (ctypes.c_int, [vp, ctypes.c_int32, _F64P]),
             "imx_swm_set_scheme": (ctypes.c_int, [vp, ctypes.POINTER(MeshDesc), ctypes.POINTER(Scheme)]),
             "imx_swm_step": (ctypes.c_int, [vp, ctypes.c_int32]),
+            "imx_swm_prepare": (ctypes.c_int, [vp, ctypes.c_int32, _I32P]),
             "imx_swm_step_timed": (ctypes.c_int, [vp, ctypes.c_int32, _F64P]),
             "imx_swm_profile": (ctypes.c_int, [vp, ctypes.c_int32, _F64P, _I32P]),
             "imx_swm_kernel_name": (ctypes.c_char_p, [vp, ctypes.c_int32]),
@@ -176,6 +177,7 @@ def lib():
             "imx_ens_set_state": (ctypes.c_int, [vp, ctypes.c_int32, _F64P, _F64P]),
             "imx_ens_get_state": (ctypes.c_int, [vp, ctypes.c_int32, _F64P, _F64P]),
             "imx_ens_step": (ctypes.c_int, [vp, ctypes.c_int32]),
+            "imx_ens_prepare": (ctypes.c_int, [vp, ctypes.c_int32, _I32P]),
             "imx_ens_step_timed": (ctypes.c_int, [vp, ctypes.c_int32, _F64P]),
             "imx_ens_diagnostics": (ctypes.c_int, [vp, ctypes.c_int32, _F64P]),
             "imx_ens_tune": (ctypes.c_int, [vp, ctypes.c_int32, _I32P]),
@@ -201,6 +203,7 @@ def lib():
     "imx_learn_fit": (ctypes.c_int, [vp, ctypes.c_int32, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                      ctypes.c_uint64, _F64P]),
     "imx_learn_step": (ctypes.c_int, [vp, ctypes.c_int32, ctypes.c_double, _I32P]),
+            "imx_learn_prepare": (ctypes.c_int, [vp, ctypes.c_int32, _I32P]),
             "imx_learn_last_rms": (ctypes.c_int, [vp, _F64P]),
             "imx_learn_set_limiter": (ctypes.c_int, [vp, ctypes.c_int32]),
             "imx_learn_destroy": (None, [vp]),

@@ -486,14 +486,14 @@ static int learn_sample(imx_learn *L) {
   return IMX_OK;
 }
 
-static int learn_ensure_graphs(imx_learn *L, int nsteps) {
+static int learn_ensure_graphs(imx_learn *L, int nsteps, int32_t *made = nullptr) {
   // recapture when the handle's step changed (scheme, tuning, topography, h_ref)
   if (L->gen != L->s->generation) learn_drop_graph(L);
   L->gen = L->s->generation;
   hipError_t e;
   const int rc = L->graphs.ensure(nsteps, L->s->stream, [&](bool last) {
     return L->s->single ? learn_enqueue_step<float>(L, last) : learn_enqueue_step<double>(L, last);
-  }, e);
+  }, e, made);
   if (rc) return rc;
   LTRY(e, "learn graph capture");
   return IMX_OK;
@@ -741,6 +741,11 @@ int imx_learn_set_limiter(imx_learn *L, int32_t mode) {
   LTRY(hipMemcpyAsync(L->bound + 1, &m, 8, hipMemcpyHostToDevice, L->s->stream), "imx_learn_set_limiter");
   LTRY(hipStreamSynchronize(L->s->stream), "imx_learn_set_limiter");
   return IMX_OK;
+}
+
+int imx_learn_prepare(imx_learn *L, int32_t nsteps, int32_t *made) {
+  if (!L || nsteps < 0) return imx::set_error(IMX_EINVAL, "imx_learn_prepare: bad argument");
+  return imx::learn_ensure_graphs(L, nsteps, made);
 }
 
 int imx_learn_step(imx_learn *L, int32_t nsteps, double bound, int32_t *nlimited) {

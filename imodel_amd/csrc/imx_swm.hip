@@ -3094,9 +3094,9 @@ static void drop_graph(imx_swm *s) {
   s->graphs.drop();
 }
 
-static int ensure_graphs(imx_swm *s, int nsteps) {
+static int ensure_graphs(imx_swm *s, int nsteps, int32_t *made = nullptr) {
   hipError_t e;
-  const int rc = s->graphs.ensure(nsteps, s->stream, [&](bool) { launch_step(s); return 0; }, e);
+  const int rc = s->graphs.ensure(nsteps, s->stream, [&](bool) { launch_step(s); return 0; }, e, made);
   HIPTRY(e, "step graph capture");
   return rc;
 }
@@ -4110,6 +4110,12 @@ int imx_swm_step(imx_swm *s, int32_t nsteps) {
   return imx::check_flag(s, "imx_swm_step");
 }
 
+int imx_swm_prepare(imx_swm *s, int32_t nsteps, int32_t *made) {
+  if (!s || nsteps < 0) return imx::set_error(IMX_EINVAL, "imx_swm_prepare: bad argument");
+  if (made) *made = 0;
+  return s->o.use_graph ? imx::ensure_graphs(s, nsteps, made) : IMX_OK;
+}
+
 int imx_swm_step_timed(imx_swm *s, int32_t nsteps, double *ms) {
   if (!s || !ms) return imx::set_error(IMX_EINVAL, "imx_swm_step_timed: NULL argument");
   if (nsteps < 0) return imx::set_error(IMX_EINVAL, "imx_swm_step_timed: nsteps < 0");
@@ -4576,6 +4582,11 @@ int imx_ens_get_state(imx_ens *E, int32_t i, double *h, double *u) {
 int imx_ens_step(imx_ens *E, int32_t nsteps) {
   if (!E) return imx::set_error(IMX_EINVAL, "imx_ens_step: NULL handle");
   return imx_swm_step(E->s, nsteps);
+}
+
+int imx_ens_prepare(imx_ens *E, int32_t nsteps, int32_t *made) {
+  if (!E) return imx::set_error(IMX_EINVAL, "imx_ens_prepare: NULL handle");
+  return imx_swm_prepare(E->s, nsteps, made);
 }
 
 int imx_ens_step_timed(imx_ens *E, int32_t nsteps, double *ms) {

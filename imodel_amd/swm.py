@@ -338,6 +338,13 @@ class Swm:
     def step(self, nsteps=1):
         capi.check(capi.lib().imx_swm_step(self._h, int(nsteps)), "imx_swm_step")
 
+    def prepare(self, nsteps):
+        """Capture the graphs a run of nsteps launches (no step is run);
+        returns how many were missing."""
+        made = np.zeros(1, dtype=np.int32)
+        capi.check(capi.lib().imx_swm_prepare(self._h, int(nsteps), capi.i32p(made)), "imx_swm_prepare")
+        return int(made[0])
+
     def step_timed(self, nsteps):
         ms = ctypes.c_double()
         capi.check(capi.lib().imx_swm_step_timed(self._h, int(nsteps), ctypes.byref(ms)), "imx_swm_step_timed")
@@ -436,6 +443,13 @@ class Ensemble:
 
     def step(self, nsteps=1):
         capi.check(capi.lib().imx_ens_step(self._h, int(nsteps)), "imx_ens_step")
+
+    def prepare(self, nsteps):
+        """Capture the graphs a run of nsteps launches (no step is run);
+        returns how many were missing."""
+        made = np.zeros(1, dtype=np.int32)
+        capi.check(capi.lib().imx_ens_prepare(self._h, int(nsteps), capi.i32p(made)), "imx_ens_prepare")
+        return int(made[0])
 
     def step_timed(self, nsteps):
         ms = ctypes.c_double()

@@ -393,6 +393,12 @@ int  imx_swm_lte(imx_swm *s, const imx_mesh *m, double *err, double *mim);
 int  imx_swm_lte_hol(imx_swm *s, const imx_mesh *m, double hollgw, double *err, double *mim);
 /* nsteps x ode_rk4 on the resident state            src/swm.f90:2600-2683 */
 int  imx_swm_step(imx_swm *s, int32_t nsteps);
+/* Captures, without running a step, the graphs a run of nsteps launches (of 16,
+   4 and 1 steps), which the first such run does otherwise: for a program that
+   times its steps. *made (may be NULL) counts those that were missing; they are
+   again after a change of scheme, launch shapes, topography or Coriolis
+   parameter. */
+int  imx_swm_prepare(imx_swm *s, int32_t nsteps, int32_t *made);
 /* as imx_swm_step, returns device time (HIP events on the handle's stream)  */
 int  imx_swm_step_timed(imx_swm *s, int32_t nsteps, double *ms);
 /* per-kernel average device time [ms] over nsteps, one entry per kernel of
@@ -442,6 +448,7 @@ int  imx_ens_create(int32_t n, const imx_mesh_desc *descs, const double *dt,
 int  imx_ens_set_state(imx_ens *e, int32_t i, const double *h, const double *u);
 int  imx_ens_get_state(imx_ens *e, int32_t i, double *h, double *u);
 int  imx_ens_step(imx_ens *e, int32_t nsteps);
+int  imx_ens_prepare(imx_ens *e, int32_t nsteps, int32_t *made);  /* as imx_swm_prepare */
 int  imx_ens_step_timed(imx_ens *e, int32_t nsteps, double *ms);
 int  imx_ens_diagnostics(imx_ens *e, int32_t i, double out[IMX_NDIAG]);
 int  imx_ens_tune(imx_ens *e, int32_t nsteps, int32_t out[6]);
@@ -513,6 +520,7 @@ int  imx_learn_store(imx_learn *l, const double *du, const double *dh, int32_t *
 int  imx_learn_fit(imx_learn *l, int32_t nsteps, float lr0, float lr1, float wd, uint64_t seed,
                    double loss[2]);
 int  imx_learn_step(imx_learn *l, int32_t nsteps, double bound, int32_t *nlimited);
+int  imx_learn_prepare(imx_learn *l, int32_t nsteps, int32_t *made);  /* as imx_swm_prepare */
 int  imx_learn_set_limiter(imx_learn *l, int32_t mode);
 int  imx_learn_last_rms(imx_learn *l, double *rms);
 void imx_learn_destroy(imx_learn *l);
