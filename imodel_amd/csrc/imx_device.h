@@ -4,7 +4,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <map>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "imx_internal.h"
@@ -40,13 +42,17 @@ struct Alloc {
     return (X *)p;
   }
   template <typename X>
-  X *put(const std::vector<X> &h) {
-    X *p = get<X>(h.size());
-    if (p && !h.empty()) {
-      hipError_t e = hipMemcpy(p, h.data(), h.size() * sizeof(X), hipMemcpyHostToDevice);
+  X *put(const X *h, size_t n) {
+    X *p = get<X>(n);
+    if (p && n) {
+      hipError_t e = hipMemcpy(p, h, n * sizeof(X), hipMemcpyHostToDevice);
       if (e != hipSuccess) err = e;
     }
     return p;
+  }
+  template <typename X>
+  X *put(const std::vector<X> &h) {
+    return put(h.data(), h.size());
   }
   void release() {
     for (void *p : ptrs) (void)hipFree(p);
@@ -304,6 +310,7 @@ struct imx_swm {
   // (one_launch_scheme).
   imx::Stage *stg = nullptr;
   size_t stg_limit = 0;
+  std::map<std::pair<int, bool>, std::vector<int32_t>> stg_start;  // cuts: first cells, by threads and ring
   bool stg_stale = false, stg_local = false;
   int stg_nt[4] = {256, 256, 256, 256}, stg_remap[4] = {1, 1, 1, 1};
 };
@@ -335,7 +342,8 @@ void swm_launch_step(imx_swm *s, void *hout = nullptr, void *uout = nullptr);
 int swm_check_flag(imx_swm *s, const char *what);
 
 // One launch per RK stage (imx_stage.hip). stage_build makes the block
-// tables from the handle's device tables for blocks of nt threads. It leaves
+// tables from the handle's device tables for blocks of nt threads, keeping the
+// cut of the mesh where it has it; graphs captured before are stale. It leaves
 // s->stg null, and *local false, where the numbering cuts into blocks that are
 // mostly rim, and null with IMX_ENOMEM where device or host memory is short;
 // stage_launch evaluates stage 0..3 of (hs, us), or a tendency (stage -1).

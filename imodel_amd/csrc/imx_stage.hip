@@ -123,10 +123,16 @@ static constexpr int cap_l(int nt, bool ap) { return ap ? nt + nt / 4 + 64 : nt;
 static constexpr int cap_t(int nt, bool ap) { return ap ? 3 * nt : 2 * nt + nt / 2 + 64; }
 static constexpr int cap_g(int nt) { return 2 * nt + nt / 4 + 32; }
 
+//
+// Which cells, triangles and edges a block holds follows from the mesh, the
+// block's threads and whether it holds APVM's wider ring: the cut, made on the
+// host. What the handle's tables say of them (signs, weights, the Coriolis
+// parameter) is filled in by stage_fill, again whenever those tables change.
 struct Stage {
   int nt = 0, nblk = 0, remap = 1;
   int scheme = kPlain;
-  Alloc A;
+  bool wide = false;  // the cut holds APVM's ring
+  Alloc A, O;         // the cut and the plain scheme's values; an option's
   int4 *head = nullptr;      // [nblk] first own cell, own cells | |L| << 16, |C| | triangles around C << 16,
                              // local cells | triangles << 16
   int32_t *halo = nullptr;   // [nblk][nt] cells of the local ids past the own ones
@@ -632,15 +638,29 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
 }
 
 // ------------------------------------------------------------- host side ---
+// an array whose elements are written before they are read
 template <typename X>
-static bool down(std::vector<X> &h, const void *d, size_t n) {
-  h.resize(n);
-  return n == 0 || hipMemcpy(h.data(), d, n * sizeof(X), hipMemcpyDeviceToHost) == hipSuccess;
+struct Raw {
+  std::unique_ptr<X[]> p;
+  size_t n = 0;
+  explicit Raw(size_t count = 0) : p(new X[count]), n(count) {}
+  X &operator[](size_t i) { return p[i]; }
+  const X &operator[](size_t i) const { return p[i]; }
+};
+template <typename X>
+static bool down(Raw<X> &h, const void *d, size_t n) {
+  h = Raw<X>(n);
+  return n == 0 || hipMemcpy(h.p.get(), d, n * sizeof(X), hipMemcpyDeviceToHost) == hipSuccess;
+}
+template <typename X>
+static X *up(Alloc &A, const Raw<X> &h) {
+  return A.put(h.p.get(), h.n);
 }
 
 void stage_free(imx_swm *s) {
   if (!s->stg) return;
   s->stg->A.release();
+  s->stg->O.release();
   delete s->stg;
   s->stg = nullptr;
 }
@@ -650,7 +670,7 @@ int stage_scheme(const imx_swm *s) { return s->stg ? s->stg->scheme : -1; }
 void stage_set_remap(imx_swm *s, int remap) {
   if (s->stg) s->stg->remap = remap;
 }
-size_t stage_bytes(const imx_swm *s) { return s->stg ? s->stg->A.bytes : 0; }
+size_t stage_bytes(const imx_swm *s) { return s->stg ? s->stg->A.bytes + s->stg->O.bytes : 0; }
 
 // A block's local cells and triangles: small open-addressing tables that are
 // emptied by raising the stamp (a block holds far fewer entries than slots).
@@ -687,31 +707,25 @@ struct LocalSets {
   }
 };
 
-template <typename T>
-static int build(imx_swm *s, int nt, int scheme, bool *local) {
+// The cut of the curve into blocks of nt threads, as the device takes it, with
+// every value that stage_fill writes zero.
+struct Cut {
+  int nblk = 0;
+  Raw<int4> head;
+  Raw<int32_t> halo;
+  Raw<uint4> topo;
+  Raw<uint16_t> oth, tslot;
+  Raw<uint32_t> tv;
+  Raw<ushort4> tn;
+};
+
+static int cut_blocks(imx_swm *s, int nt, bool wide, Cut &C, bool *local) {
   const int nv = s->nv, NE = s->NE, NTri = s->NT;
-  const bool ap = scheme == kApvm, px = scheme == kPerot, df = scheme == kDiff;
-  const int LC = cap_a(nt), CL = cap_l(nt, ap), TC = cap_t(nt, ap), GC = cap_g(nt);
-  const double ea = s->o.erad;
-  std::vector<int32_t> nbr, bA, bB, oth, tab, teb;
-  std::vector<T> R, ika, ceta, kap, tf;
-  std::vector<double> leng, dleng, tarea;
+  const int LC = cap_a(nt), CL = cap_l(nt, wide), TC = cap_t(nt, wide), GC = cap_g(nt);
+  Raw<int32_t> nbr, bA, bB, oth, tab, teb, atn;
   if (!down(nbr, s->x_c_nb, (size_t)MX * nv) || !down(bA, s->x_c_bitsA, nv) || !down(bB, s->x_c_bitsB, nv) ||
       !down(oth, s->x_e_oth, NE) || !down(tab, s->x_t_ab, (size_t)2 * NTri) || !down(teb, s->x_t_eb, NTri) ||
-      !down(R, s->x_c_R, (size_t)MX * nv) || !down(ika, s->x_c_ika, nv) ||
-      !down(ceta, s->x_t_ceta, (size_t)3 * NTri) || !down(kap, s->x_t_kap, (size_t)3 * NTri) ||
-      !down(tf, s->x_t_f, NTri) || !down(leng, s->e_leng, NE) || !down(dleng, s->e_dleng, NE) ||
-      !down(tarea, s->t_area, NTri))
-    return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
-  std::vector<Quad<T>> awc, awt;
-  std::vector<int32_t> atn;
-  std::vector<Quad<T>> pn;
-  std::vector<T> pq, kh, kt;
-  std::vector<double> iaa;
-  if (((ap || px) && !down(awc, s->x_ap_wc, (size_t)MX * nv)) ||
-      (ap && (!down(awt, s->x_ap_wt, (size_t)3 * NTri) || !down(atn, s->x_ap_tnb, (size_t)3 * NTri))) ||
-      (px && (!down(pn, s->x_px_n, NE) || !down(pq, s->x_px_wq, (size_t)MX * nv))) ||
-      (df && (!down(kh, s->x_kh, nv) || !down(kt, s->x_kt, NTri) || !down(iaa, s->x_c_iaa, nv))))
+      (wide && !down(atn, s->x_ap_tnb, (size_t)3 * NTri)))
     return set_error(IMX_EDEVICE, "stage tables: copy from the device failed");
 
   auto tri_of = [&](int c, int j) {
@@ -726,7 +740,7 @@ static int build(imx_swm *s, int nt, int scheme, bool *local) {
       if (q.level) return;
       q.level = 1;
       ++w.nL;
-      if (!ap) return;
+      if (!wide) return;
       // APVM takes the velocity at k and the PV of the triangles around it
       const int n = bA[k] & 7;
       for (int j = 0; j < n; ++j) {
@@ -755,149 +769,227 @@ static int build(imx_swm *s, int nt, int scheme, bool *local) {
     ++w.own;
     const int nA = (int)w.L.keys.size();
     return w.nC <= nt && nA <= LC && nA - w.own <= nt && (int)w.tri.keys.size() <= TC &&
-           (!ap || (w.nL <= CL && w.nG <= GC));
+           (!wide || (w.nL <= CL && w.nG <= GC));
   };
 
-  // cut the curve into at most 16 segments, one host thread each, and every
-  // segment greedily into blocks
-  const int seg = std::max(64 * nt, (nv + 15) / 16), nseg = (nv + seg - 1) / seg;
-  std::vector<std::vector<int32_t>> cuts(nseg);
-  std::vector<char> fine(nseg, 1);
+  // Where the blocks start: the curve in at most 16 segments, one host thread
+  // each, and every segment greedily into blocks. Kept with the handle (a few
+  // thousand numbers), so that a scheme that is back need not look for them.
+  std::vector<int32_t> &start = s->stg_start[{nt, wide}];
   std::atomic<bool> memory{true};
-  auto each_segment = [&](auto fn) {
-    parallel_ranges(nseg, [&](int g0, int g1) {
+  auto parallel = [&](int n, auto fn) {
+    parallel_ranges(n, [&](int i0, int i1) {
       try {
-        for (int g = g0; g < g1; ++g) fn(g);
+        fn(i0, i1);
       } catch (const std::bad_alloc &) {
         memory = false;
       }
     }, 1);
   };
-  each_segment([&](int g) {
-    const int c0 = g * seg, c1 = std::min(nv, c0 + seg);
-    LocalSets w;
-    int first = c0;
-    cuts[g].push_back(first);
-    for (int c = c0; c < c1 && fine[g]; ++c) {
-      if (add(w, c)) continue;
-      first = c;
-      cuts[g].push_back(first);
-      w.clear();
-      fine[g] = add(w, c);  // a single cell within the caps
-    }
-  });
   const char *out_of = "stage tables: host out of memory";
-  if (!memory) return set_error(IMX_ENOMEM, out_of);
-  std::vector<int32_t> start, seg0;
-  for (int g = 0; g < nseg; ++g) {
-    seg0.push_back((int32_t)start.size());
-    start.insert(start.end(), cuts[g].begin(), cuts[g].end());
+  if (start.empty()) {
+    const int seg = std::max(64 * nt, (nv + 15) / 16), nseg = (nv + seg - 1) / seg;
+    std::vector<std::vector<int32_t>> cuts(nseg);
+    std::vector<char> fine(nseg, 1);
+    parallel(nseg, [&](int g0, int g1) {
+      LocalSets w;
+      for (int g = g0; g < g1; ++g) {
+        const int c0 = g * seg, c1 = std::min(nv, c0 + seg);
+        w.clear();
+        cuts[g].push_back(c0);
+        for (int c = c0; c < c1 && fine[g]; ++c) {
+          if (add(w, c)) continue;
+          cuts[g].push_back(c);
+          w.clear();
+          fine[g] = add(w, c);  // a single cell within the caps
+        }
+      }
+    });
+    if (!memory) return set_error(IMX_ENOMEM, out_of);
+    std::vector<int32_t> all;
+    for (const auto &c : cuts) all.insert(all.end(), c.begin(), c.end());
+    // Numberings that are not local (a mesh in its caller's order) cut into
+    // blocks that are mostly rim: the three passes run instead.
+    *local = all.size() <= 1 || (int64_t)all.size() * nt <= (int64_t)3 * nv;
+    for (char ok : fine) *local = *local && ok;
+    if (!*local) return IMX_OK;
+    all.push_back(nv);
+    start.swap(all);
   }
-  const int nblk = (int)start.size();
-  seg0.push_back(nblk);
-  start.push_back(nv);
-  // Numberings that are not local (a mesh in its caller's order) cut into
-  // blocks that are mostly rim: the three passes run instead.
-  *local = nblk <= 1 || (int64_t)nblk * nt <= (int64_t)3 * nv;
-  for (char ok : fine) *local = *local && ok;
-  if (!*local) return IMX_OK;
-  // the kernel addresses its tables by 32-bit byte offsets
-  if ((uint64_t)NE * sizeof(Tri<T>) >> 32) return IMX_OK;
+  const int nblk = (int)start.size() - 1;
 
-  std::vector<int4> head(nblk);
-  std::vector<int32_t> halo((size_t)nblk * nt, 0);
-  std::vector<uint4> topo((size_t)nblk * CL, uint4{0, 0, 0, 0});
-  std::vector<Quad<T>> cw((size_t)nblk * 2 * nt, Quad<T>{0, 0, 0, 0}), tk((size_t)nblk * TC, Quad<T>{0, 0, 0, 0});
-  std::vector<Pair<T>> eld(NE);
-  std::vector<uint16_t> loth(NE, 0xFFFF), tslot((size_t)nblk * TC, 0);
-  std::vector<uint32_t> tv((size_t)nblk * TC, 0);
-  std::vector<T> tfv((size_t)nblk * TC, (T)0);
-  std::vector<Tri<T>> eno(px ? NE : 0);
-  for (int e = 0; px && e < NE; ++e) eno[e] = Tri<T>{pn[e].x, pn[e].y, pn[e].z};
-  std::vector<T> tktv(df ? (size_t)nblk * TC : 0, (T)0);
-  std::vector<Tri<T>> wc(ap || px ? (size_t)nblk * MX * CL : 0, Tri<T>{0, 0, 0}),
-      wt(ap ? (size_t)nblk * 3 * GC : 0, Tri<T>{0, 0, 0});
-  std::vector<ushort4> tn(ap ? (size_t)nblk * GC : 0, ushort4{0, 0, 0, 0});
-  for (int e = 0; e < NE; ++e) eld[e] = Pair<T>{(T)(1.0 / leng[e]), (T)dleng[e]};
-  each_segment([&](int g) {
+  C.nblk = nblk;
+  C.head = Raw<int4>(nblk);
+  C.halo = Raw<int32_t>((size_t)nblk * nt);
+  C.topo = Raw<uint4>((size_t)nblk * CL);
+  C.oth = Raw<uint16_t>(NE);
+  C.tslot = Raw<uint16_t>((size_t)nblk * TC);
+  C.tv = Raw<uint32_t>((size_t)nblk * TC);
+  C.tn = Raw<ushort4>(wide ? (size_t)nblk * GC : 0);
+  parallel(nblk, [&](int b0, int b1) {
     LocalSets w;
-    for (int b = seg0[g]; b < seg0[g + 1]; ++b) {
+    std::vector<uint64_t> cells, tris;  // rank above the id
+    for (int b = b0; b < b1; ++b) {
       const int o0 = start[b], nown = start[b + 1] - o0;
       w.clear();
       for (int c = o0; c < o0 + nown; ++c) (void)add(w, c);
       // own cells, the rest of C, the rest of L, the others, each ascending;
       // own triangles, the others around C, the others
       auto own = [&](int k) { return k >= o0 && k < o0 + nown; };
-      std::vector<int32_t> cells = w.L.keys, tris = w.tri.keys;
-      auto rank = [&](int k) { return own(k) ? 0 : 3 - w.L.at(k).level; };
-      auto trank = [&](int k) { return own(k / 2) ? 0 : 2 - w.tri.at(k).level; };
-      std::sort(cells.begin(), cells.end(), [&](int x, int y) {
-        const int rx = rank(x), ry = rank(y);
-        return rx != ry ? rx < ry : x < y;
-      });
-      std::sort(tris.begin(), tris.end(), [&](int x, int y) {
-        const int rx = trank(x), ry = trank(y);
-        return rx != ry ? rx < ry : x < y;
-      });
-      const int nA = (int)cells.size(), nL = w.nL, nC = w.nC;
-      for (int k = 0; k < nA; ++k) w.L.at(cells[k]).id = k;
+      auto ranked = [](uint64_t rank, int k) { return rank << 32 | (uint32_t)k; };
+      cells.clear();
+      for (int k : w.L.keys) cells.push_back(ranked(own(k) ? 0 : 3 - w.L.at(k).level, k));
+      tris.clear();
+      for (int k : w.tri.keys) tris.push_back(ranked(own(k / 2) ? 0 : 2 - w.tri.at(k).level, k));
+      std::sort(cells.begin(), cells.end());
+      std::sort(tris.begin(), tris.end());
+      const int nA = (int)cells.size(), nTri = (int)tris.size(), nL = w.nL, nC = w.nC;
+      for (int k = 0; k < nA; ++k) w.L.at((int32_t)cells[k]).id = k;
       auto id = [&](int k) { return (uint32_t)w.L.at(k).id; };
-      for (int k = nown; k < nA; ++k) halo[(size_t)b * nt + k - nown] = cells[k];
-      head[b] = int4{o0, nown | nL << 16, nC | w.nG << 16, nA | (int)tris.size() << 16};
-      for (int k = 0; k < (ap ? nL : nC); ++k) {
-        const int c = cells[k];
-        const bool hex = (bA[c] & 7) == MX;
-        uint32_t f[MX], t3 = (uint32_t)hex << SW_HEX;
-        T r[MX];
+      int32_t *halo = &C.halo[(size_t)b * nt];
+      for (int k = 0; k < nt; ++k) halo[k] = nown + k < nA ? (int32_t)cells[nown + k] : 0;
+      C.head[b] = int4{o0, nown | nL << 16, nC | w.nG << 16, nA | nTri << 16};
+      uint4 *topo = &C.topo[(size_t)b * CL];
+      for (int k = 0; k < CL; ++k) {
+        topo[k] = uint4{0, 0, 0, 0};
+        if (k >= (wide ? nL : nC)) continue;
+        const int c = (int32_t)cells[k];
+        uint32_t f[MX], t3 = (uint32_t)((bA[c] & 7) == MX) << SW_HEX;
         for (int j = 0; j < MX; ++j) {
           f[j] = id(nbr[(size_t)j * nv + c]);
           f[j] |= ((bA[c] >> (BA_OWN + j)) & 1u) << SB_OWN;
           f[j] |= ((bB[c] >> (2 * j)) & 3u) << SB_K;
-          f[j] |= ((bA[c] >> (BA_TTG + j)) & 1u) << SB_TTG;
-          f[j] |= ((bA[c] >> (BA_TNR + j)) & 1u) << SB_TNR;
           t3 |= ((bB[c] >> (BB_TSEL + 2 * j)) & 3u) << (2 * j);
           t3 |= ((bB[c] >> (BB_KT + j)) & 1u) << (SW_KT + j);
-          if (df) t3 |= ((bA[c] >> (BA_FZ + j)) & 1u) << (SW_FZ + j);
-          r[j] = px ? pq[(size_t)j * nv + c] : R[(size_t)j * nv + c];
         }
-        topo[(size_t)b * CL + k] = uint4{f[0] | f[1] << 16, f[2] | f[3] << 16, f[4] | f[5] << 16, t3};
-        for (int j = 0; (ap || px) && j < MX; ++j) {
-          const Quad<T> &q = awc[(size_t)j * nv + c];
-          wc[((size_t)b * MX + j) * CL + k] = Tri<T>{q.x, q.y, q.z};
-        }
-        if (k >= nC) continue;
-        cw[((size_t)b * 2) * nt + k] = Quad<T>{r[0], r[1], r[2], r[3]};
-        // ika = 1 / sum (l l~ / 4)
-        cw[((size_t)b * 2 + 1) * nt + k] = Quad<T>{r[4], r[5], (T)0.25 * ika[c], df ? (T)((double)kh[c] * iaa[c]) : (T)0};
+        topo[k] = uint4{f[0] | f[1] << 16, f[2] | f[3] << 16, f[4] | f[5] << 16, t3};
       }
-      for (int k = 0; k < (int)tris.size(); ++k) {
-        const int t = tris[k];
+      for (int k = 0; k < TC; ++k) {
         const size_t p = (size_t)b * TC + k;
-        uint32_t v = id(tab[t]) | id(tab[(size_t)NTri + t]) << 10;
-        v |= (uint32_t)(teb[t] & 511) << 20;
-        for (int m = 0; m < 3; ++m) v |= (ceta[(size_t)m * NTri + t] < 0 ? 1u : 0u) << (29 + m);
-        tv[p] = v;
-        tslot[p] = (uint16_t)(2 * id(t / 2) + t % 2);
-        tk[p] = Quad<T>{kap[t], kap[(size_t)NTri + t], kap[(size_t)2 * NTri + t], (T)(1.0 / (tarea[t] * ea))};
-        tfv[p] = tf[t];
-        if (df) tktv[p] = kt[t];
-        if (!ap || k >= w.nG) continue;
+        C.tv[p] = 0;
+        C.tslot[p] = 0;
+        if (k >= nTri) continue;
+        const int t = (int32_t)tris[k];
+        C.tv[p] = id(tab[t]) | id(tab[(size_t)NTri + t]) << 10 | (uint32_t)(teb[t] & 511) << 20;
+        C.tslot[p] = (uint16_t)(2 * id(t / 2) + t % 2);
+      }
+      for (int k = 0; wide && k < GC; ++k) {
+        ushort4 &q = C.tn[(size_t)b * GC + k];
+        q = ushort4{0, 0, 0, 0};
+        if (k >= w.nG) continue;
+        const int t = (int32_t)tris[k];
         auto slot = [&](int i) { return (unsigned short)(2 * id(i / 2) + i % 2); };
-        tn[(size_t)b * GC + k] = ushort4{slot(atn[t]), slot(atn[(size_t)NTri + t]), slot(atn[(size_t)2 * NTri + t]),
-                                         slot(t)};
-        for (int m = 0; m < 3; ++m) {
-          const Quad<T> &q = awt[(size_t)m * NTri + t];
-          wt[((size_t)b * 3 + m) * GC + k] = Tri<T>{q.x, q.y, q.z};
-        }
+        q = ushort4{slot(atn[t]), slot(atn[(size_t)NTri + t]), slot(atn[(size_t)2 * NTri + t]), slot(t)};
       }
-      for (int e = 3 * o0; e < 3 * (o0 + nown); ++e) {
-        if (oth[e] < 0) continue;
-        loth[e] = (uint16_t)(id(oth[e] & OTH_MASK) | ((uint32_t)(oth[e] >> OTH_V2) & 1u) << SB_OWN);
-      }
+      for (int e = 3 * o0; e < 3 * (o0 + nown); ++e)
+        C.oth[e] = oth[e] < 0 ? (uint16_t)0xFFFF : (uint16_t)id(oth[e] & OTH_MASK);
     }
   });
+  return memory ? IMX_OK : set_error(IMX_ENOMEM, out_of);
+}
 
-  if (!memory) return set_error(IMX_ENOMEM, out_of);
+// The handle's tables, and where their values go in the blocks' order.
+template <typename T>
+struct FillArgs {
+  const int4 *head;
+  const int32_t *halo;
+  const uint16_t *tslot;
+  const int32_t *bitsA, *e_oth;
+  const T *R, *ika, *kh, *kt, *ceta, *kap, *f;
+  const double *iaa, *leng, *dleng, *tarea;
+  const Quad<T> *awc, *awt, *pn;
+  uint4 *topo;
+  Quad<T> *cw, *tk;
+  Pair<T> *eld;
+  uint16_t *oth;
+  uint32_t *tv;
+  T *tf, *tkt;
+  Tri<T> *wc, *wt, *en;
+  int nv, NE, NT, nt, CL, TC, GC;
+  double ea;
+};
+
+// One block per block of the stage. The values are those of the host's
+// arithmetic (IEEE divisions in FP64, rounded once to T). 0.3 ms at glevel 8,
+// where making the tables on the host and copying them took 67.
+template <typename T, int SCHEME>
+__global__ __launch_bounds__(256) void stage_fill(const FillArgs<T> a) {
+  constexpr bool AP = SCHEME == kApvm, PX = SCHEME == kPerot, DF = SCHEME == kDiff;
+  const int b = blockIdx.x, nv = a.nv, NT = a.NT;
+  const int4 hd = a.head[b];
+  const int own0 = hd.x, nown = hd.y & 0xFFFF, nL = hd.y >> 16, nC = hd.z & 0xFFFF, nG = hd.z >> 16;
+  const int nTri = hd.w >> 16;
+  const int32_t *halo = a.halo + (size_t)b * a.nt;
+  auto cell = [&](int k) { return k < nown ? own0 + k : halo[k - nown]; };
+  for (int k = threadIdx.x; k < (AP ? nL : nC); k += blockDim.x) {
+    const int c = cell(k), A = a.bitsA[c];
+    uint4 &tp = a.topo[(size_t)b * a.CL + k];
+    uint32_t w[3] = {tp.x & 0x3FFF3FFFu, tp.y & 0x3FFF3FFFu, tp.z & 0x3FFF3FFFu};
+    for (int j = 0; j < MX; ++j) {
+      const uint32_t f = ((A >> (BA_TTG + j)) & 1u) << SB_TTG | ((A >> (BA_TNR + j)) & 1u) << SB_TNR;
+      w[j / 2] |= f << (16 * (j % 2));
+    }
+    const uint32_t fz = DF ? ((uint32_t)A >> BA_FZ & 63u) << SW_FZ : 0u;
+    tp = uint4{w[0], w[1], w[2], (tp.w & ~(63u << SW_FZ)) | fz};
+    if constexpr (AP || PX)
+      for (int j = 0; j < MX; ++j) {
+        const Quad<T> q = a.awc[(size_t)j * nv + c];
+        a.wc[((size_t)b * MX + j) * a.CL + k] = Tri<T>{q.x, q.y, q.z};
+      }
+    if (k >= nC) continue;
+    T r[MX];
+    for (int j = 0; j < MX; ++j) r[j] = a.R[(size_t)j * nv + c];
+    a.cw[((size_t)b * 2) * a.nt + k] = Quad<T>{r[0], r[1], r[2], r[3]};
+    // ika = 1 / sum (l l~ / 4)
+    a.cw[((size_t)b * 2 + 1) * a.nt + k] =
+        Quad<T>{r[4], r[5], (T)0.25 * a.ika[c], DF ? (T)((double)a.kh[c] * a.iaa[c]) : (T)0};
+  }
+  for (int k = threadIdx.x; k < nTri; k += blockDim.x) {
+    const size_t p = (size_t)b * a.TC + k;
+    const int sl = a.tslot[p], t = 2 * cell(sl >> 1) + (sl & 1);
+    uint32_t v = a.tv[p] & 0x1FFFFFFFu;
+    for (int m = 0; m < 3; ++m) v |= (a.ceta[(size_t)m * NT + t] < (T)0 ? 1u : 0u) << (29 + m);
+    a.tv[p] = v;
+    a.tk[p] = Quad<T>{a.kap[t], a.kap[(size_t)NT + t], a.kap[(size_t)2 * NT + t], (T)(1.0 / (a.tarea[t] * a.ea))};
+    a.tf[p] = a.f[t];
+    if constexpr (DF) a.tkt[p] = a.kt[t];
+    if constexpr (AP) {
+      if (k >= nG) continue;
+      for (int m = 0; m < 3; ++m) {
+        const Quad<T> q = a.awt[(size_t)m * NT + t];
+        a.wt[((size_t)b * 3 + m) * a.GC + k] = Tri<T>{q.x, q.y, q.z};
+      }
+    }
+  }
+  for (int e = 3 * own0 + threadIdx.x; e < 3 * (own0 + nown); e += blockDim.x) {
+    a.eld[e] = Pair<T>{(T)(1.0 / a.leng[e]), (T)a.dleng[e]};
+    const int o = a.e_oth[e];
+    if (o < 0) continue;
+    a.oth[e] = (uint16_t)((a.oth[e] & LID) | ((uint32_t)(o >> OTH_V2) & 1u) << SB_OWN);
+    if constexpr (PX) {
+      const Quad<T> q = a.pn[e];
+      a.en[e] = Tri<T>{q.x, q.y, q.z};
+    }
+  }
+}
+
+static int no_memory(hipError_t e) {
+  return set_error(e == hipErrorOutOfMemory ? IMX_ENOMEM : IMX_EDEVICE,
+                   std::string("stage tables: ") + hipGetErrorString(e));
+}
+
+// The cut for nt threads, or that the handle has where it fits the scheme too.
+template <typename T>
+static int ensure_cut(imx_swm *s, int nt, bool wide, bool *local) {
+  if (s->stg && s->stg->nt == nt && s->stg->wide == wide &&
+      (!s->stg_limit || s->stg->A.bytes <= s->stg_limit))
+    return IMX_OK;
+  stage_free(s);
+  // the kernel addresses its tables by 32-bit byte offsets
+  if ((uint64_t)s->NE * sizeof(Tri<T>) >> 32) return IMX_OK;
+  Cut C;
+  const int rc = cut_blocks(s, nt, wide, C, local);
+  if (rc || !*local) return rc;
   // the handle has the tables once they are whole
   struct Drop {
     void operator()(Stage *p) const {
@@ -908,39 +1000,111 @@ static int build(imx_swm *s, int nt, int scheme, bool *local) {
   std::unique_ptr<Stage, Drop> g(new Stage());
   Alloc &A = g->A;
   A.limit = s->stg_limit;
+  const size_t nc = (size_t)C.nblk * nt, ntr = C.tv.n;
   g->nt = nt;
-  g->nblk = nblk;
-  g->head = A.put(head);
-  g->halo = A.put(halo);
-  g->topo = A.put(topo);
-  g->cw = A.put(cw);
-  g->eld = A.put(eld);
-  g->oth = A.put(loth);
-  g->tv = A.put(tv);
-  g->tslot = A.put(tslot);
-  g->tk = A.put(tk);
-  g->tf = A.put(tfv);
-  g->scheme = scheme;
-  if (ap || px) g->wc = A.put(wc);
-  if (px) g->en = A.put(eno);
-  if (df) g->tkt = A.put(tktv);
-  if (ap) {
-    g->wt = A.put(wt);
-    g->tn = A.put(tn);
-  }
-  if (A.err != hipSuccess)
-    return set_error(A.err == hipErrorOutOfMemory ? IMX_ENOMEM : IMX_EDEVICE,
-                     std::string("stage tables: ") + hipGetErrorString(A.err));
+  g->nblk = C.nblk;
+  g->wide = wide;
+  g->head = up(A, C.head);
+  g->halo = up(A, C.halo);
+  g->topo = up(A, C.topo);
+  g->oth = up(A, C.oth);
+  g->tv = up(A, C.tv);
+  g->tslot = up(A, C.tslot);
+  if (wide) g->tn = up(A, C.tn);
+  g->cw = A.get<Quad<T>>(2 * nc);
+  g->eld = A.get<Pair<T>>(s->NE);
+  g->tk = A.get<Quad<T>>(ntr);
+  g->tf = A.get<T>(ntr);
+  if (A.err != hipSuccess) return no_memory(A.err);
   s->stg = g.release();
   return IMX_OK;
 }
 
-int stage_build(imx_swm *s, int nt, int scheme, bool *local) {
+template <typename T, int SCHEME>
+static void fill(const FillArgs<T> &a, int nblk, hipStream_t st) {
+  stage_fill<T, SCHEME><<<nblk, 256, 0, st>>>(a);
+}
+
+template <typename T>
+static int build(imx_swm *s, int nt, int scheme, bool *local) {
+  const bool ap = scheme == kApvm, px = scheme == kPerot, df = scheme == kDiff;
+  int rc = ensure_cut<T>(s, nt, ap, local);
+  if (rc || !s->stg) return rc;
+  Stage &g = *s->stg;
+  const int CL = cap_l(nt, ap), TC = cap_t(nt, ap), GC = cap_g(nt);
+  Alloc &O = g.O;
+  O.release();
+  O = Alloc();
+  g.wc = g.wt = g.en = g.tkt = nullptr;
+  if (s->stg_limit) O.limit = std::max<size_t>(s->stg_limit - g.A.bytes, 1);
+  if (ap || px) g.wc = O.get<Tri<T>>((size_t)g.nblk * MX * CL);
+  if (ap) g.wt = O.get<Tri<T>>((size_t)g.nblk * 3 * GC);
+  if (px) g.en = O.get<Tri<T>>(s->NE);
+  if (df) g.tkt = O.get<T>((size_t)g.nblk * TC);
+  if (O.err != hipSuccess) {
+    rc = no_memory(O.err);
+    stage_free(s);
+    return rc;
+  }
+  g.scheme = scheme;
+  FillArgs<T> a;
+  a.head = g.head;
+  a.halo = g.halo;
+  a.tslot = g.tslot;
+  a.bitsA = s->x_c_bitsA;
+  a.e_oth = s->x_e_oth;
+  a.R = (const T *)(px ? s->x_px_wq : s->x_c_R);
+  a.ika = (const T *)s->x_c_ika;
+  a.kh = (const T *)s->x_kh;
+  a.kt = (const T *)s->x_kt;
+  a.ceta = (const T *)s->x_t_ceta;
+  a.kap = (const T *)s->x_t_kap;
+  a.f = (const T *)s->x_t_f;
+  a.iaa = s->x_c_iaa;
+  a.leng = s->e_leng;
+  a.dleng = s->e_dleng;
+  a.tarea = s->t_area;
+  a.awc = (const Quad<T> *)s->x_ap_wc;
+  a.awt = (const Quad<T> *)s->x_ap_wt;
+  a.pn = (const Quad<T> *)s->x_px_n;
+  a.topo = g.topo;
+  a.cw = (Quad<T> *)g.cw;
+  a.tk = (Quad<T> *)g.tk;
+  a.eld = (Pair<T> *)g.eld;
+  a.oth = g.oth;
+  a.tv = g.tv;
+  a.tf = (T *)g.tf;
+  a.tkt = (T *)g.tkt;
+  a.wc = (Tri<T> *)g.wc;
+  a.wt = (Tri<T> *)g.wt;
+  a.en = (Tri<T> *)g.en;
+  a.nv = s->nv;
+  a.NE = s->NE;
+  a.NT = s->NT;
+  a.nt = nt;
+  a.CL = CL;
+  a.TC = TC;
+  a.GC = GC;
+  a.ea = s->o.erad;
+  switch (scheme) {
+    case kApvm: fill<T, kApvm>(a, g.nblk, s->stream); break;
+    case kPerot: fill<T, kPerot>(a, g.nblk, s->stream); break;
+    case kDiff: fill<T, kDiff>(a, g.nblk, s->stream); break;
+    default: fill<T, kPlain>(a, g.nblk, s->stream); break;
+  }
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+  if (e == hipSuccess) return IMX_OK;
   stage_free(s);
+  return set_error(IMX_EDEVICE, std::string("stage tables: ") + hipGetErrorString(e));
+}
+
+int stage_build(imx_swm *s, int nt, int scheme, bool *local) {
   *local = true;
   try {
     return s->single ? build<float>(s, nt, scheme, local) : build<double>(s, nt, scheme, local);
   } catch (const std::bad_alloc &) {
+    stage_free(s);
     return set_error(IMX_ENOMEM, "stage tables: host out of memory");
   }
 }

@@ -19,9 +19,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -2394,41 +2396,48 @@ static int fast_stagger(imx_swm *s, const imx_mesh_desc &d, bool hc) {
   }
   std::vector<int32_t> bitsA(nv), e_oth(NE, -1);
   HIPTRY(hipMemcpy(bitsA.data(), s->x_c_bitsA, nv * sizeof(int32_t), hipMemcpyDeviceToHost), "set_scheme");
-  for (int co = 0; co < nv; ++co) {
-    const int c = cn[co];
-    bitsA[c] &= ~((((1 << MX) - 1) << BA_TTG) | (((1 << MX) - 1) << BA_TNR));
-    for (int j = 0; j < d.v_nnb[co]; ++j) {
-      const int sf = hc ? hcc[(size_t)j * nv + c] : d.hx_ttgout[MX * co + j];
-      const int sn = hc ? hcc[(size_t)j * nv + c] : d.hx_tnrccw[MX * co + j];
-      if (sf < 0) bitsA[c] |= 1 << (BA_TTG + j);
-      if (sn < 0) bitsA[c] |= 1 << (BA_TNR + j);
+  parallel_ranges(nv, [&](int co0, int co1) {
+    for (int co = co0; co < co1; ++co) {
+      const int c = cn[co];
+      bitsA[c] &= ~((((1 << MX) - 1) << BA_TTG) | (((1 << MX) - 1) << BA_TNR));
+      for (int j = 0; j < d.v_nnb[co]; ++j) {
+        const int sf = hc ? hcc[(size_t)j * nv + c] : d.hx_ttgout[MX * co + j];
+        const int sn = hc ? hcc[(size_t)j * nv + c] : d.hx_tnrccw[MX * co + j];
+        if (sf < 0) bitsA[c] |= 1 << (BA_TTG + j);
+        if (sn < 0) bitsA[c] |= 1 << (BA_TNR + j);
+      }
     }
-  }
-  for (int eo = 0; eo < d.ne; ++eo) {
-    const int e = en[eo];
-    const int o = e / 3;
-    int v1 = cn[d.ed_v[2 * eo] - 1], v2 = cn[d.ed_v[2 * eo + 1] - 1];
-    if (hc && hg[e] < 0) std::swap(v1, v2);
-    e_oth[e] = (o == v1) ? v2 : (v1 | (1 << OTH_V2));
-  }
-  std::vector<double> t_ceta((size_t)3 * NT, 0.0);
-  for (int ko = 0; ko < d.nt; ++ko) {
-    const int t = tn[ko];
-    int r = -1;
-    for (int l = 0; l < 3; ++l)
-      if (cn[d.tr_v[3 * ko + l] - 1] == t / 2) r = l;
-    if (r < 0) return set_error(IMX_EINVAL, "imx_swm_set_scheme: triangle owner not found");
-    for (int m = 0; m < 3; ++m) {
-      const int lr = (r + m) % 3;
-      const int eo = d.tr_ed[3 * ko + lr] - 1;
-      const double sg = hc ? (double)hct[(size_t)lr * NT + t] : (double)d.tr_tg[3 * ko + lr];
-      t_ceta[(size_t)m * NT + t] = d.ed_leng[eo] * sg / (d.tr_areag[ko] * a);
+  });
+  parallel_ranges(d.ne, [&](int eo0, int eo1) {
+    for (int eo = eo0; eo < eo1; ++eo) {
+      const int e = en[eo];
+      const int o = e / 3;
+      int v1 = cn[d.ed_v[2 * eo] - 1], v2 = cn[d.ed_v[2 * eo + 1] - 1];
+      if (hc && hg[e] < 0) std::swap(v1, v2);
+      e_oth[e] = (o == v1) ? v2 : (v1 | (1 << OTH_V2));
     }
-  }
-  const std::vector<T> tcT = cvt<T>(t_ceta);
+  });
+  std::vector<T> t_ceta((size_t)3 * NT, (T)0);
+  std::atomic<bool> owned{true};
+  parallel_ranges(d.nt, [&](int ko0, int ko1) {
+    for (int ko = ko0; ko < ko1; ++ko) {
+      const int t = tn[ko];
+      int r = -1;
+      for (int l = 0; l < 3; ++l)
+        if (cn[d.tr_v[3 * ko + l] - 1] == t / 2) r = l;
+      if (r < 0) owned = false;
+      for (int m = 0; m < 3 && r >= 0; ++m) {
+        const int lr = (r + m) % 3;
+        const int eo = d.tr_ed[3 * ko + lr] - 1;
+        const double sg = hc ? (double)hct[(size_t)lr * NT + t] : (double)d.tr_tg[3 * ko + lr];
+        t_ceta[(size_t)m * NT + t] = (T)(d.ed_leng[eo] * sg / (d.tr_areag[ko] * a));
+      }
+    }
+  });
+  if (!owned) return set_error(IMX_EINVAL, "imx_swm_set_scheme: triangle owner not found");
   HIPTRY(hipMemcpy(s->x_c_bitsA, bitsA.data(), nv * sizeof(int32_t), hipMemcpyHostToDevice), "set_scheme");
   HIPTRY(hipMemcpy(s->x_e_oth, e_oth.data(), NE * sizeof(int32_t), hipMemcpyHostToDevice), "set_scheme");
-  HIPTRY(hipMemcpy(s->x_t_ceta, tcT.data(), tcT.size() * sizeof(T), hipMemcpyHostToDevice), "set_scheme");
+  HIPTRY(hipMemcpy(s->x_t_ceta, t_ceta.data(), t_ceta.size() * sizeof(T), hipMemcpyHostToDevice), "set_scheme");
   return IMX_OK;
 }
 
@@ -2445,32 +2454,39 @@ template <typename T>
 static int fast_cell_weights(imx_swm *s, const imx_mesh_desc &d) {
   const int nv = s->nv;
   const std::vector<int32_t> &cn = s->lay.cell_new;
-  std::vector<double> wc((size_t)4 * MX * nv, 0.0);
+  const size_t n = (size_t)4 * MX * nv;
+  const std::unique_ptr<T[]> wc(new (std::nothrow) T[n]);
+  if (!wc) return set_error(IMX_ENOMEM, "imx_swm_set_scheme: host out of memory");
   // HC: hx%nr signs and the Voronoi edge midpoints
   std::vector<int8_t> hcc;
   if (s->sc_hc) {
     hcc.resize((size_t)MX * nv);
     HIPTRY(hipMemcpy(hcc.data(), s->hc_c, hcc.size(), hipMemcpyDeviceToHost), "set_scheme");
   }
-  for (int co = 0; co < nv; ++co) {
-    const double *p = d.v_p + 3 * co;
-    for (int j = 0; j < d.v_nnb[co]; ++j) {
-      const int eo = d.v_ed[MX * co + j] - 1;
-      // ttgout u (ed%c - v%p) edhx%leng / hx%areag (swm_operators.f90:474-505)
-      const double sg = s->sc_hc ? (double)hcc[(size_t)j * nv + cn[co]] : (double)d.hx_ttgout[MX * co + j];
-      const double *pe = s->sc_hc ? d.edhx_c + 3 * eo : d.ed_c + 3 * eo;
-      const double f = sg * d.edhx_leng[eo] / d.hx_areag[co];
-      double w[3];
-      for (int q = 0; q < 3; ++q) w[q] = f * (pe[q] - p[q]);
-      put_projected(&wc[4 * ((size_t)j * nv + cn[co])], w, p);
+  parallel_ranges(nv, [&](int co0, int co1) {
+    for (int co = co0; co < co1; ++co) {
+      const double *p = d.v_p + 3 * co;
+      for (int j = 0; j < MX; ++j) {
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
+        if (j < d.v_nnb[co]) {
+          const int eo = d.v_ed[MX * co + j] - 1;
+          // ttgout u (ed%c - v%p) edhx%leng / hx%areag (swm_operators.f90:474-505)
+          const double sg = s->sc_hc ? (double)hcc[(size_t)j * nv + cn[co]] : (double)d.hx_ttgout[MX * co + j];
+          const double *pe = s->sc_hc ? d.edhx_c + 3 * eo : d.ed_c + 3 * eo;
+          const double f = sg * d.edhx_leng[eo] / d.hx_areag[co];
+          double w[3];
+          for (int q = 0; q < 3; ++q) w[q] = f * (pe[q] - p[q]);
+          put_projected(v, w, p);
+        }
+        for (int q = 0; q < 4; ++q) wc[4 * ((size_t)j * nv + cn[co]) + q] = (T)v[q];
+      }
     }
-  }
+  });
   if (!s->x_ap_wc) {
-    s->x_ap_wc = s->A.get<T>((size_t)4 * MX * nv);
+    s->x_ap_wc = s->A.get<T>(n);
     if (s->A.err != hipSuccess) return hip_fail(s->A.err, "imx_swm_set_scheme");
   }
-  const std::vector<T> wcT = cvt<T>(wc);
-  HIPTRY(hipMemcpy(s->x_ap_wc, wcT.data(), wcT.size() * sizeof(T), hipMemcpyHostToDevice), "set_scheme");
+  HIPTRY(hipMemcpy(s->x_ap_wc, wc.get(), n * sizeof(T), hipMemcpyHostToDevice), "set_scheme");
   return IMX_OK;
 }
 
@@ -2624,40 +2640,49 @@ static int fast_apvm(imx_swm *s, const imx_mesh_desc &d, const imx_scheme &sc) {
   const int nv = s->nv, NT = s->NT;
   const std::vector<int32_t> &cn = s->lay.cell_new, &tn = s->lay.tri_new;
   const double a = s->o.erad;
-  // weights as (x, y, z, 0) records: wt [3][NT]
-  std::vector<double> wt((size_t)4 * 3 * NT, 0.0);
+  // weights as (x, y, z, 0) records: wt [3][NT]; triangle slots without one -1
+  std::vector<T> wt((size_t)4 * 3 * NT, (T)0);
   std::vector<int32_t> tnb((size_t)3 * NT, -1);
   int rc = fast_cell_weights<T>(s, d);
   if (rc) return rc;
-  for (int ko = 0; ko < d.nt; ++ko) {
-    const int t = tn[ko];
-    const double *p = d.tr_c + 3 * ko;
-    int r = -1;  // slot m of the fused kernels is reference edge (r + m) % 3
-    for (int l = 0; l < 3; ++l)
-      if (cn[d.tr_v[3 * ko + l] - 1] == t / 2) r = l;
-    if (r < 0) return set_error(IMX_EINVAL, "imx_swm_set_scheme: triangle owner not found");
-    for (int m = 0; m < 3; ++m) {
-      const int lr = (r + m) % 3;
-      const int eo = d.tr_ed[3 * ko + lr] - 1;
-      const int s1 = d.ed_sh[2 * eo] - 1, s2 = d.ed_sh[2 * eo + 1] - 1;
-      if (s1 != ko && s2 != ko) return set_error(IMX_EINVAL, "imx_swm_set_scheme: triangle not on its edge");
-      const double *pa = d.v_p + 3 * (d.ed_v[2 * eo] - 1), *pb = d.v_p + 3 * (d.ed_v[2 * eo + 1] - 1);
-      double nr[3];
-      cross3(pa, pb, nr);
-      double dp = 0.0;
-      for (int q = 0; q < 3; ++q) dp = dp + nr[q] * (d.tr_c[3 * s2 + q] - d.tr_c[3 * s1 + q]);
-      const double nrs = std::signbit(dp) ? -1.0 : 1.0;
-      const double side = (ko == s1) ? 1.0 : -1.0;  // q(across) - q(t) = +-(q(sh2) - q(sh1))
-      tnb[(size_t)m * NT + t] = tn[ko == s1 ? s2 : s1];
-      // grad q at the edge: ed%nr-sign (q(sh2) - q(sh1)) / (|e*| a); its Perot
-      // term: -tr%tg |e| (ed%c - tr%c) / tr%areag (swm_operators.f90:1427-1462)
-      const double f = -(double)d.tr_tg[3 * ko + lr] * d.ed_leng[eo] / d.tr_areag[ko] * nrs /
-                       (d.edhx_leng[eo] * a) * side;
-      double w[3];
-      for (int q = 0; q < 3; ++q) w[q] = f * (d.ed_c[3 * eo + q] - p[q]);
-      put_projected(&wt[4 * ((size_t)m * NT + t)], w, p);
+  std::atomic<int> bad{0};
+  parallel_ranges(d.nt, [&](int ko0, int ko1) {
+    for (int ko = ko0; ko < ko1; ++ko) {
+      const int t = tn[ko];
+      const double *p = d.tr_c + 3 * ko;
+      int r = -1;  // slot m of the fused kernels is reference edge (r + m) % 3
+      for (int l = 0; l < 3; ++l)
+        if (cn[d.tr_v[3 * ko + l] - 1] == t / 2) r = l;
+      if (r < 0) bad = 1;
+      for (int m = 0; m < 3 && r >= 0; ++m) {
+        const int lr = (r + m) % 3;
+        const int eo = d.tr_ed[3 * ko + lr] - 1;
+        const int s1 = d.ed_sh[2 * eo] - 1, s2 = d.ed_sh[2 * eo + 1] - 1;
+        if (s1 != ko && s2 != ko) {
+          bad = 2;
+          break;
+        }
+        const double *pa = d.v_p + 3 * (d.ed_v[2 * eo] - 1), *pb = d.v_p + 3 * (d.ed_v[2 * eo + 1] - 1);
+        double nr[3];
+        cross3(pa, pb, nr);
+        double dp = 0.0;
+        for (int q = 0; q < 3; ++q) dp = dp + nr[q] * (d.tr_c[3 * s2 + q] - d.tr_c[3 * s1 + q]);
+        const double nrs = std::signbit(dp) ? -1.0 : 1.0;
+        const double side = (ko == s1) ? 1.0 : -1.0;  // q(across) - q(t) = +-(q(sh2) - q(sh1))
+        tnb[(size_t)m * NT + t] = tn[ko == s1 ? s2 : s1];
+        // grad q at the edge: ed%nr-sign (q(sh2) - q(sh1)) / (|e*| a); its Perot
+        // term: -tr%tg |e| (ed%c - tr%c) / tr%areag (swm_operators.f90:1427-1462)
+        const double f = -(double)d.tr_tg[3 * ko + lr] * d.ed_leng[eo] / d.tr_areag[ko] * nrs /
+                         (d.edhx_leng[eo] * a) * side;
+        double w[3], v[3];
+        for (int q = 0; q < 3; ++q) w[q] = f * (d.ed_c[3 * eo + q] - p[q]);
+        put_projected(v, w, p);
+        for (int q = 0; q < 3; ++q) wt[4 * ((size_t)m * NT + t) + q] = (T)v[q];
+      }
     }
-  }
+  });
+  if (bad == 1) return set_error(IMX_EINVAL, "imx_swm_set_scheme: triangle owner not found");
+  if (bad) return set_error(IMX_EINVAL, "imx_swm_set_scheme: triangle not on its edge");
   Alloc &A = s->A;
   if (!s->x_ap_tnb) {
     s->x_ap_tnb = A.get<int32_t>((size_t)3 * NT);
@@ -2666,9 +2691,8 @@ static int fast_apvm(imx_swm *s, const imx_mesh_desc &d, const imx_scheme &sc) {
     s->x_ap_g = A.get<T>((size_t)4 * NT);
     if (A.err != hipSuccess) return hip_fail(A.err, "imx_swm_set_scheme");
   }
-  const std::vector<T> wtT = cvt<T>(wt);
   HIPTRY(hipMemcpy(s->x_ap_tnb, tnb.data(), tnb.size() * sizeof(int32_t), hipMemcpyHostToDevice), "set_scheme");
-  HIPTRY(hipMemcpy(s->x_ap_wt, wtT.data(), wtT.size() * sizeof(T), hipMemcpyHostToDevice), "set_scheme");
+  HIPTRY(hipMemcpy(s->x_ap_wt, wt.data(), wt.size() * sizeof(T), hipMemcpyHostToDevice), "set_scheme");
   s->f_apvm = true;
   return IMX_OK;
 }
