@@ -4586,14 +4586,18 @@ int imx_ens_create(int32_t n, const imx_mesh_desc *descs, const double *dt, cons
 int imx_ens_set_state(imx_ens *E, int32_t i, const double *h, const double *u) {
   if (!E || !h || !u || i < 0 || i >= E->n) return imx::set_error(IMX_EINVAL, "imx_ens_set_state: bad argument");
   imx_swm *s = E->s;
-  if (!s->href_set) {  // FP32 storage reference: area mean of the first state set
-    double sa = 0.0, sh = 0.0;
-    for (int k = 0; k < E->nv[i]; ++k) {
-      sa += E->area[E->cv0[i] + k];
-      sh += E->area[E->cv0[i] + k] * h[k];
+  {
+    std::lock_guard<std::mutex> lk(s->hstage_mu);
+    if (!s->href_set) {  // FP32 storage reference: area mean of the first state set
+      double sa = 0.0, sh = 0.0;
+      for (int k = 0; k < E->nv[i]; ++k) {
+        sa += E->area[E->cv0[i] + k];
+        sh += E->area[E->cv0[i] + k] * h[k];
+      }
+      s->href = sh / sa;
+      s->href_set = true;
+      imx::drop_graph(s);  // a step captured before holds href = 0
     }
-    s->href = sh / sa;
-    s->href_set = true;
   }
   return s->single ? imx::ens_upload<float>(E, i, h, u) : imx::ens_upload<double>(E, i, h, u);
 }

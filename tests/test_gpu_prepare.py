@@ -47,6 +47,27 @@ def test_prepare_of_ensembles_and_corrected_steps():
         L.close()
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_prepared_before_the_first_state(prec):
+    """Without h_ref the first state sets the storage offset, which the captured
+    steps hold: graphs captured before it are not used after it."""
+    say("prepare before the first state", prec)
+    m = Mesh.icos(3)
+    h, u = m.spectral(2)
+    got = []
+    for early in (0, 5):
+        with Ensemble([m, m], [600.0, 300.0], precision=prec) as E, Swm(m, precision=prec, dt=600.0) as s:
+            E.prepare(early)
+            s.prepare(early)
+            for i in range(2):
+                E.set_state(i, h, u)
+            s.set_state(h, u)
+            E.step(5)
+            s.step(5)
+            got.append(E.get_state(0) + E.get_state(1) + s.get_state())
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
 def test_evaluation_times_no_capture(monkeypatch):
     say("evaluation")
     timed, seen = [False], []
