@@ -49,15 +49,16 @@
 //
 // Blocks are cut greedily along the curve so that |C| fills the block's
 // threads and |L| its LDS. Ids inside a block are 10-bit, which packs the
-// topology of a cell into 16 bytes; lengths are stored once per edge, as 1 / l
-// and l~, and the kinetic-energy and vorticity coefficients are formed from
-// them. The momentum tendency is multiplied by 1 / l: an error of that factor
-// is the same in every step and adds up over a run. With l stored, rounded once
-// and inverted (a second rounding), h' at glevel 4 after 48 steps was 2.35e-7
-// off (FP32, trsk10, eight seeds; HC 4.54e-7) where the three passes, which
-// read 1 / l, are 2.14e-7 off (3.84e-7); with 1 / l stored it is 2.02e-7 (3.83e-7).
-// The lengths, which the other terms take, bear the second rounding without
-// effect. Three reciprocals a thread more: 1 % at glevel 5, less from 6 on.
+// topology of a cell into 16 bytes; lengths are stored once per edge, in FP32 as
+// 1 / l and l~, and the kinetic-energy and vorticity coefficients are formed
+// from them. The momentum tendency is multiplied by 1 / l: an error of that
+// factor is the same in every step and adds up over a run. With l stored, rounded
+// to FP32 and then inverted (a second rounding), h' at glevel 4 after 48 steps
+// was 2.39e-7 off (trsk10, ten seeds; HC 4.53e-7) where the three passes, which
+// read 1 / l, are 2.14e-7 off (3.84e-7); with 1 / l stored it is 2.04e-7
+// (3.83e-7). The lengths, which the other terms take, bear the second rounding
+// without effect. Three reciprocals a thread more: 1 % at glevel 5, less from 6
+// on; a table of 1 / l beside l took 3 % at glevels 7 to 9.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -139,7 +140,7 @@ struct Stage {
   uint4 *topo = nullptr;     // [nblk][cap_l]
   void *cw = nullptr;        // [nblk][2][nt] Quad: kite fractions 0-3; 4, 5, 1 / sum l l~, with diffusion K / A;
                              // pxt16: PV weights of the earlier triangle at edges 0-3; 4, 5
-  void *eld = nullptr;       // [NE] Pair: 1 / length, dual length
+  void *eld = nullptr;       // [NE] Pair: 1 / length (FP64: length), dual length
   uint16_t *oth = nullptr;   // [NE] local id of the edge's other cell | it is v1 << 10; 0xFFFF dummy
   uint32_t *tv = nullptr;    // [nblk][cap_t] vertices a, b (10 bits each), edge bits (9), curl signs (3)
   uint16_t *tslot = nullptr; // [nblk][cap_t] local slot 2 owner + k
@@ -211,6 +212,19 @@ __device__ __forceinline__ double recip(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
   return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+// l, 1 / l and l / l~ of the stored length: 1 / l in FP32; in FP64 l, whose reciprocal
+// is as good as a stored one and which three edges a thread fewer then need
+// (glevel 7: 68.4 us a step, with 1 / l stored 69.1)
+__device__ __forceinline__ float length(float s) { return recip(s); }
+__device__ __forceinline__ float inverse_length(float s) { return s; }
+__device__ __forceinline__ float length_ratio(float s, float dl) { return recip(s * dl); }
+__device__ __forceinline__ double length(double s) { return s; }
+__device__ __forceinline__ double inverse_length(double s) { return recip(s); }
+__device__ __forceinline__ double length_ratio(double s, double dl) { return s * recip(dl); }
+template <typename T>
+__device__ __forceinline__ T stored_length(double l) {
+  return sizeof(T) == 4 ? (T)(1.0 / l) : (T)l;
 }
 // element i of a table, by a 32-bit byte offset (tables are under 4 GiB; see
 // stage_build): one scalar base and one vector register for the address
@@ -336,7 +350,7 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
     if (i < 3 * nown) {
       sU[i] = eu[r];
       sD[i] = el[r].y;
-      sA[i] = eu[r] * recip(el[r].x);
+      sA[i] = eu[r] * length(el[r].x);
     }
   }
   if (tid < nown) sH[tid] = ho;
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
     for (int k = 0; k < 3; ++k) {
       sU[3 * lc + k] = hu[k];
       sD[3 * lc + k] = hl[k].y;
-      sA[3 * lc + k] = hu[k] * recip(hl[k].x);
+      sA[3 * lc + k] = hu[k] * length(hl[k].x);
     }
   }
   ushort4 tn[NG];
@@ -613,11 +627,11 @@ __global__ __launch_bounds__(NT, SCHEME == kApvm && NT == 512 ? 4 : 1) void fast
       const T uhq = (T)0.25 * (en[r].x * (ql * (A1.x + A2.x) + (B1.x + B2.x)) +
                                en[r].y * (ql * (A1.y + A2.y) + (B1.y + B2.y)) +
                                en[r].z * (ql * (A1.z + A2.z) + (B1.z + B2.z)));
-      du = -d * el[r].x - uhq;
+      du = -d * inverse_length(el[r].x) - uhq;
     } else {
       T P = sP[i] + sPo[i];
-      if constexpr (DF) P += recip(el[r].x * el[r].y) * a.inv_a * sE[i];
-      du = -(d + P) * el[r].x;
+      if constexpr (DF) P += length_ratio(el[r].x, el[r].y) * a.inv_a * sE[i];
+      du = -(d + P) * inverse_length(el[r].x);
     }
     if (a.zero_mom) du = (T)0;
     T ca = a.cat, cb = a.cbt;
@@ -962,7 +976,7 @@ __global__ __launch_bounds__(256) void stage_fill(const FillArgs<T> a) {
     }
   }
   for (int e = 3 * own0 + threadIdx.x; e < 3 * (own0 + nown); e += blockDim.x) {
-    a.eld[e] = Pair<T>{(T)(1.0 / a.leng[e]), (T)a.dleng[e]};
+    a.eld[e] = Pair<T>{stored_length<T>(a.leng[e]), (T)a.dleng[e]};
     const int o = a.e_oth[e];
     if (o < 0) continue;
     a.oth[e] = (uint16_t)((a.oth[e] & LID) | ((uint32_t)(o >> OTH_V2) & 1u) << SB_OWN);
@@ -1007,14 +1021,14 @@ static int ensure_cut(imx_swm *s, int nt, bool wide, bool *local) {
   g->head = up(A, C.head);
   g->halo = up(A, C.halo);
   g->topo = up(A, C.topo);
+  g->cw = A.get<Quad<T>>(2 * nc);
+  g->eld = A.get<Pair<T>>(s->NE);
   g->oth = up(A, C.oth);
   g->tv = up(A, C.tv);
   g->tslot = up(A, C.tslot);
-  if (wide) g->tn = up(A, C.tn);
-  g->cw = A.get<Quad<T>>(2 * nc);
-  g->eld = A.get<Pair<T>>(s->NE);
   g->tk = A.get<Quad<T>>(ntr);
   g->tf = A.get<T>(ntr);
+  if (wide) g->tn = up(A, C.tn);
   if (A.err != hipSuccess) return no_memory(A.err);
   s->stg = g.release();
   return IMX_OK;
