@@ -170,10 +170,13 @@ __global__ __launch_bounds__(LTPB) void learn_featx(int NE, const int32_t *__res
 // Input fragments of the network formed in its own kernel: the features of
 // learn_featx in the slots of mlp_feature_slot. The four lanes of an edge read
 // its record as consecutive 32-byte quarters and gather six ids each; the
-// normalised row (96 bytes written and read per edge) never exists: 382 us at
-// glevel 8 instead of 147 for the rows and 259 for the network on them. The
-// kernel is bound by its activations, two waves a SIMD; gathering a tile ahead
-// takes 1 % off there and adds as much at glevel 6. norm: per lane group 12 means, 12 deviations.
+// normalised row (96 bytes written and read per edge) never exists: 355 to 382 us
+// at glevel 8 instead of 147 for the rows and 259 to 279 for the network on them.
+// Both kernels keep the vector units busy 92 % of the time (counters: 46 % of
+// each wave's cycles issue vector work, two waves a SIMD). Of the cycles that the
+// gathers add, 45 % are vector work (27 % more instructions: ids, signs, the
+// normalisation's divisions) and 41 % waits, mostly for memory; gathering a tile
+// ahead takes 1 % off there and adds as much at glevel 6. norm: per lane group 12 means, 12 deviations.
 template <typename T>
 struct FeatLoader {
   static constexpr int kNorm = 24;

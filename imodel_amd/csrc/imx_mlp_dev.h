@@ -156,10 +156,6 @@ __device__ __forceinline__ v8s gelu_chunk(const v4f &z0, const v4f &z1) {
   return __builtin_bit_cast(v8s, p);
 }
 
-// Hidden layer zn = b + W^T g(z) (K = N = 128), chunk-outer: chunk c of
-// the input needs only tiles 2c, 2c+1 of z, so the activation of chunk
-// c + 1 can issue while the MFMAs of chunk c run. Each output tile still
-// sums its chunks in ascending order.
 // The biases of output tile b (of the 24 of layers 1-3) in the gaps of layer
 // 4's fragments behind the loader's constants. Read from memory, as 24 vector
 // loads a tile in the order of the others, they took registers ahead of their
@@ -170,6 +166,10 @@ __device__ __forceinline__ F *lds_bias(F *sh, int b) {
   return sh + 64 * (4 + b / 3) + 16 * (b % 3);
 }
 
+// Hidden layer zn = b + W^T g(z) (K = N = 128), chunk-outer: chunk c of
+// the input needs only tiles 2c, 2c+1 of z, so the activation of chunk
+// c + 1 can issue while the MFMAs of chunk c run. Each output tile still
+// sums its chunks in ascending order.
 template <int ET>
 __device__ __forceinline__ void layer_pipe(const short *Ws, const float *sh, int layer, const v4f (&z)[8][ET],
                                            v4f (&zn)[8][ET], int lane) {

@@ -29,10 +29,10 @@
 // Measured (us per RK4 step, three passes -> this; 16-step graphs on both
 // sides would take 6 off the first figures): glevel 5 FP32 43 -> 19.7, glevel
 // 7 78 -> 43.5, FP64 105 -> 68, glevel 8 191 -> 110.6, FP64 380 -> 211,
-// glevel 9 948 -> 547. The three passes moved 252 MB per stage at glevel 8;
+// glevel 9 948 -> 516. The three passes moved 252 MB per stage at glevel 8;
 // this moves 181 (FETCH_SIZE x 2 + WRITE_SIZE) at 6.6 TB/s, against 7.8 for a
 // copy that stays in the last-level cache. What bounds it there: the vector
-// units are busy 47 % of the time (693 instructions a wave), memory most of
+// units are busy 47 % of the time (686 instructions a wave), memory most of
 // the rest. What was worth most: every load issued before the first barrier
 // (with each phase loading its own tables a glevel-8 stage took 45 us instead
 // of 32), then fewer vector instructions (32 -> 27.6).

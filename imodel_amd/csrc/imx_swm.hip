@@ -3226,7 +3226,7 @@ static int tune(imx_swm *s, int nsteps, int32_t *out) {
     int &bb = s->stg_nt[stage_scheme(s)], &br = s->stg_remap[stage_scheme(s)];
     const int scheme = stage_scheme(s);
     for (int bs : {128, 256, 512}) {
-      if (bs == 512 && !s->single) continue;  // over 64 KB of LDS
+      if (bs == 512 && !s->single) continue;  // 109 to 159 KB of LDS: one block, two waves a SIMD, per CU
       bool local;
       rc = stage_build(s, bs, scheme, &local);
       if (rc == IMX_ENOMEM) {  // not a candidate

@@ -418,10 +418,11 @@ int  imx_swm_diagnostics_dev(imx_swm *s, double *out_dev);
 int  imx_swm_info(imx_swm *s, int64_t out[8]);   /* nv ne nt bytes_dev ... */
 void imx_swm_destroy(imx_swm *s);
 
-/* Autotuner (no counterpart in the reference): times every block size
-   (64/128/256/512) x XCD-remap choice of each fused kernel over nsteps steps
-   and keeps the fastest; out = {bs, remap} for tri, cell, edge, those of the
-   one-launch stage under cell. The state is restored. FAST precisions only. */
+/* Autotuner (no counterpart in the reference): times the block sizes x
+   XCD-remap choices of the one-launch stage where the scheme runs as one
+   (128/256/512 threads; FP64 without 512), else those of each fused kernel
+   (64/128/256/512), over nsteps steps and keeps the fastest; out = {bs, remap}
+   for tri, cell, edge, the one-launch stage's under cell. The state is restored. FAST precisions only. */
 int  imx_swm_tune(imx_swm *s, int32_t nsteps, int32_t out[6]);
 /* The launch shapes in use, laid out as imx_swm_tune returns them, and shapes
    to use from now on (those of an earlier imx_swm_tune, say): block threads and
@@ -439,7 +440,7 @@ int  imx_swm_set_stage_limit(imx_swm *s, int64_t bytes);
 /* ---- ensembles: many independent instances in one set of launches --------
    (no counterpart in the reference; the batched configuration). Instance i
    has its own mesh descs[i] and time step dt[i]; all instances advance
-   together, one launch per fused kernel per RK stage, one hipGraph per step.
+   together, one launch per RK stage (or fused kernel), up to 16 steps per hipGraph.
    FAST precisions only. States and diagnostics are per instance, in that
    instance's own (caller, 1-based) numbering. */
 typedef struct imx_ens imx_ens;
@@ -456,8 +457,8 @@ int  imx_ens_info(imx_ens *e, int64_t out[8]);  /* as imx_swm_info, out[7] = n *
 void imx_ens_destroy(imx_ens *e);
 
 /* ---- learned correction (no counterpart in the reference) -----------------
-   Per-edge MLP 48 -> 128 -> 128 -> 128 -> 2, activation x*clamp(0.5+0.4255x, 0, 1) (hard-sigmoid GELU), BF16 weights
-   and activations on MFMA with FP32 accumulation; FP32 master parameters
+   Per-edge MLP 48 -> 128 -> 128 -> 128 -> 2, activation GELU in its tanh form, BF16 weights and activations
+   on MFMA with FP32 accumulation; FP32 master parameters
    updated by AdamW. Parameters are flat FP32: W1[48][128] b1[128]
    W2[128][128] b2 W3[128][128] b3 W4[128][2] b4[2] (W stored [in][out]). */
 typedef struct imx_mlp imx_mlp;
