@@ -13,6 +13,11 @@
 
 namespace imx {
 
+// What an earlier HIP call of the thread failed with (the program's own, or an
+// allocation that did not fit) stays to be read until somebody does; before a
+// launch whose error is looked at, it is read away.
+inline void forget_error() { (void)hipGetLastError(); }
+
 struct Alloc {
   std::vector<void *> ptrs;
   size_t bytes = 0, limit = 0;  // limit: the most it may take, 0 for any

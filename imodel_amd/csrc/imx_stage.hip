@@ -1100,6 +1100,7 @@ static int build(imx_swm *s, int nt, int scheme, bool *local) {
   a.TC = TC;
   a.GC = GC;
   a.ea = s->o.erad;
+  forget_error();
   switch (scheme) {
     case kApvm: fill<T, kApvm>(a, g.nblk, s->stream); break;
     case kPerot: fill<T, kPerot>(a, g.nblk, s->stream); break;

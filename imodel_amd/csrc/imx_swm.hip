@@ -3038,6 +3038,7 @@ static int upload_state(imx_swm *s, const double *h, const double *u, T *hd, T *
       for (int k = a; k < cells; ++k) st[k] = (T)(h[i0 + k] - href);
       for (int k = cells; k < b; ++k) st[k] = (T)u[i0 + k - nh];
     }, kHostGrain);
+    forget_error();
     state_in<T><<<(m + TPB - 1) / TPB, TPB, 0, s->stream>>>(i0, m, nh, s->d_cell + c0, s->d_edge + e0, st, hd, ud);
     HIPTRY(hipGetLastError(), "upload");
     if (i0 + m < n) HIPTRY(hipStreamSynchronize(s->stream), "upload");
@@ -3061,6 +3062,7 @@ static int download_state(imx_swm *s, double *h, double *u, const TH *hd, const 
   const int part = (int)std::min<size_t>(n, s->hstage_bytes / sizeof(D));
   for (int i0 = 0; i0 < n; i0 += part) {
     const int m = std::min(part, n - i0);
+    forget_error();
     state_out<D, TH, TU><<<(m + TPB - 1) / TPB, TPB, 0, s->stream>>>(i0, m, nh, s->d_cell + c0, s->d_edge + e0, hd, ud,
                                                                     st);
     HIPTRY(hipGetLastError(), "download");
